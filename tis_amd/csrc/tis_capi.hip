@@ -35,7 +35,8 @@ __global__ void k_lpair(DevPtrs, const double *, const double *, const EwTask *,
                         int, int);
 __global__ void k_advance(uint64_t *, uint64_t, unsigned long long *);
 __global__ void k_count_rebuild(unsigned long long *);
-__global__ void k_energy(DevPtrs, const double *, const double *, const int32_t *, double *, int);
+__global__ void k_energy(DevPtrs, const double *, const double *, const EwTask *, const int32_t *, int, double *, int);
+__global__ void k_energy_sum(const int32_t *, const int32_t *, int, const double *, double *, int);
 __global__ void k_label_apply(DevPtrs, LabelDev, const int32_t *, const int32_t *, const double *);
 __global__ void k_stack_status(DevPtrs, const double *, const double *, int, int, int32_t *);
 }  // namespace tis
@@ -116,6 +117,7 @@ struct HostSys {
   int32_t pt_begin = 0, pt_count = 0;    // periodic electrostatic chunk-pair tasks
   int32_t bp_begin = 0, bp_count = 0;    // bead tile pairs of the tile-pair list build
   int32_t qp_begin = 0, qp_count = 0;    // charge tile pairs
+  int32_t et_begin = 0, et_count = 0;    // energy tasks
   std::vector<double> mass, fric;
   std::vector<double> lc_fric, lc_mass;   // its Langevin classes
   std::vector<int32_t> stack_ids;       // global stack indices
@@ -157,17 +159,21 @@ struct tis_ctx {
   Tile *d_btiles = nullptr, *d_qtiles = nullptr;
   Tile *d_btiles_xcd = nullptr;          // the bead tiles in k_main's whole-batch launch order
   int32_t nbtile = 0, nqtile = 0;
-  int32_t *d_systask = nullptr, *d_sysidx = nullptr;
+  int32_t *d_systask = nullptr;
   int32_t nsystask = 0;
   int32_t *d_hbdense = nullptr;          // hbond lanes (DevPtrs::hb_dense)
   int32_t nhbdense = 0;
   std::vector<int32_t> systask_of;       // index into d_systask per system or -1
   int32_t *d_ststat = nullptr;           // st_status output of tis_term_status [nsttot]
   double *d_energy = nullptr;
-  int32_t *d_eset = nullptr;             // tis_energy_sumup_set: system list and energies
+  EwTask *d_etask = nullptr;             // energy tasks (system, part, parts) in live order
+  int32_t *d_efirst = nullptr;           // first task of each live system, and the end
+  double *d_epart = nullptr;             // their sums [n_etask][kEnergyTerms]
+  int32_t n_etask = 0;
+  int32_t *d_eset = nullptr;             // tis_energy_sumup_set: live positions, then task list
   double *d_eset_out = nullptr;
   size_t eset_cap = 0, eset_out_cap = 0;
-  double *d_eunit = nullptr;   // raw per-unit-pair energies [nunit^2][25]
+  double *d_eunit = nullptr;   // raw per-unit-pair energies [nunit^2][25], then their parts
   size_t eunit_cap = 0;
   unsigned long long *d_counters = nullptr;
   uint64_t *d_stepbase = nullptr;
@@ -394,7 +400,6 @@ struct Range {
   int isys;                 // else this system
   int bt0, btn, qt0, qtn, task0, taskn;
   int hd0, hdn;             // hbond lanes
-  const int32_t *sysidx; int nsel;
   int b0, nb, a0, na, s0, ns;
   int ek0, ekn, ef0, efn;   // Ewald tasks
   int pt0, ptn;             // periodic electrostatic chunk-pair tasks
@@ -446,7 +451,6 @@ Range range_of(tis_ctx *c, int32_t isys) {
     r.all = true;
     r.bt0 = 0; r.btn = c->nbtile; r.qt0 = 0; r.qtn = c->nqtile; r.task0 = 0; r.taskn = c->nsystask;
     r.hd0 = 0; r.hdn = c->nhbdense;
-    r.sysidx = c->d_sysidx; r.nsel = c->nlive;
     r.b0 = 0; r.nb = c->stage.nbd; r.a0 = 0; r.na = c->stage.nba; r.s0 = 0; r.ns = c->stage.nst;
     r.ek0 = 0; r.ekn = c->n_ewsk; r.ef0 = 0; r.efn = c->n_ewf;
     r.pt0 = 0; r.ptn = c->n_ptask;
@@ -457,7 +461,6 @@ Range range_of(tis_ctx *c, int32_t isys) {
     r.task0 = c->systask_of[isys] < 0 ? 0 : c->systask_of[isys];
     r.taskn = c->systask_of[isys] < 0 ? 0 : 1;
     r.hd0 = h.hd_begin; r.hdn = h.hd_count;
-    r.sysidx = c->d_sysidx + h.live_pos; r.nsel = 1;
     r.b0 = h.d.boff; r.nb = h.d.nbd; r.a0 = h.d.aoff; r.na = h.d.nba; r.s0 = h.d.soff; r.ns = h.d.nst;
     r.ek0 = h.esk_begin; r.ekn = h.esk_count; r.ef0 = h.ef_begin; r.efn = h.ef_count;
     r.pt0 = h.pt_begin; r.ptn = h.pt_count;
@@ -988,8 +991,8 @@ int build_tables(tis_ctx *c) {
   c->tab_allocs.clear();
   c->tab_bytes = 0;
   std::vector<Tile> btiles, qtiles;
-  std::vector<EwTask> ptask, bpair, qpair, ewsk, ewf;
-  std::vector<int32_t> systask, sysidx, hbdense;
+  std::vector<EwTask> ptask, bpair, qpair, ewsk, ewf, etask;
+  std::vector<int32_t> systask, hbdense, efirst;
   c->systask_of.assign(c->nsys, -1);
   c->any_ele = false;
   c->any_periodic = false;
@@ -999,7 +1002,7 @@ int build_tables(tis_ctx *c) {
     DSys &d = h.d;
     h.bt_begin = h.bt_count = h.qt_begin = h.qt_count = h.esk_begin = h.esk_count = 0;
     h.ef_begin = h.ef_count = h.pt_begin = h.pt_count = h.bp_begin = h.bp_count = h.qp_begin = h.qp_count = 0;
-    h.hd_begin = h.hd_count = 0;
+    h.hd_begin = h.hd_count = h.et_begin = h.et_count = 0;
     if (!h.live) { std::memset(&dsys[is], 0, sizeof(DSys)); dsys[is].nmp = 0; continue; }
     if (d.periodic) c->any_periodic = true;
     if (d.ele_form >= 0) c->any_ele = true;
@@ -1043,11 +1046,16 @@ int build_tables(tis_ctx *c) {
         for (int kc = 0; kc < d.nkc; ++kc) ewf.push_back(EwTask{is, qt, kc});
       h.ef_count = (int32_t)ewf.size() - h.ef_begin;
     }
-    h.live_pos = (int32_t)sysidx.size();
-    sysidx.push_back(is);
+    h.et_begin = (int32_t)etask.size();
+    h.et_count = energy_parts(d.nmp, d.ele_form != TIS_ELE_NONE ? d.nqt : 0, d.ele_form == TIS_ELE_EWALD ? d.nk : 0);
+    for (int k = 0; k < h.et_count; ++k) etask.push_back(EwTask{is, k, h.et_count});
+    h.live_pos = (int32_t)efirst.size();
+    efirst.push_back(h.et_begin);
     dsys[is] = d;
   }
-  c->nlive = (int32_t)sysidx.size();
+  efirst.push_back((int32_t)etask.size());
+  c->n_etask = (int32_t)etask.size();
+  c->nlive = (int32_t)efirst.size() - 1;
   c->P.nsys = c->nsys;
   c->nbtile = (int32_t)btiles.size(); c->nqtile = (int32_t)qtiles.size(); c->nsystask = (int32_t)systask.size();
   c->nhbdense = (int32_t)hbdense.size();
@@ -1069,8 +1077,8 @@ int build_tables(tis_ctx *c) {
     UPT(c->d_btiles_xcd, xt);
   }
   UPT(c->d_ptask, ptask); UPT(c->d_ptask_lpt, lpt); UPT(c->d_bpair, bpair); UPT(c->d_qpair, qpair);
-  UPT(c->d_ewsk, ewsk); UPT(c->d_ewf, ewf); UPT(c->d_systask, systask); UPT(c->d_sysidx, sysidx);
-  UPT(c->d_hbdense, hbdense);
+  UPT(c->d_ewsk, ewsk); UPT(c->d_ewf, ewf); UPT(c->d_systask, systask);
+  UPT(c->d_hbdense, hbdense); UPT(c->d_etask, etask); UPT(c->d_efirst, efirst);
 #undef UPT
   c->P.hb_dense = c->d_hbdense;
   const size_t nbt = std::max<size_t>(btiles.size(), 1), nqt = std::max<size_t>(qtiles.size(), 1);
@@ -1078,6 +1086,7 @@ int build_tables(tis_ctx *c) {
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.qbbox, nqt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.sbox, 4 * nbt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.ttop, 2 * nbt, &c->tab_bytes))) return rc;
+  if ((rc = dalloc_in(c, c->tab_allocs, &c->d_epart, (size_t)c->n_etask * kEnergyTerms, &c->tab_bytes))) return rc;
   c->dev_bytes += c->tab_bytes;
   for (int k = 0; k < 2; ++k)
     if (c->graph[k]) { (void)hipGraphExecDestroy(c->graph[k]); c->graph[k] = nullptr; }
@@ -1611,11 +1620,14 @@ int32_t tis_energy_sumup(tis_ctx *c, int32_t isys, double *energy_out) {
   const int ek0 = isys < 0 ? 0 : c->hs[isys].esk_begin, ekn = isys < 0 ? c->n_ewsk : c->hs[isys].esk_count;
   if (ekn > 0)
     hipLaunchKernelGGL(k_ewald_sk, dim3(ekn), dim3(kTile), 0, c->stream, c->P, PXc(c), c->d_ewsk + ek0, 1);
-  // one block per live system (in live-list order); the output is by
-  // system index, zeros for retired systems
-  const int nsel = isys < 0 ? c->nlive : 1;
-  hipLaunchKernelGGL(k_energy, dim3(nsel), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c),
-                     c->d_sysidx + (isys < 0 ? 0 : c->hs[isys].live_pos), c->d_energy, 0);
+  // every live system (in live-list order) or one; the output is by system
+  // index, zeros for retired systems
+  const int nsel = isys < 0 ? c->nlive : 1, pos0 = isys < 0 ? 0 : c->hs[isys].live_pos;
+  const int t0 = isys < 0 ? 0 : c->hs[isys].et_begin, nt = isys < 0 ? c->n_etask : c->hs[isys].et_count;
+  hipLaunchKernelGGL(k_energy, dim3(nt), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c), c->d_etask,
+                     (const int32_t *)nullptr, t0, c->d_epart, 0);
+  hipLaunchKernelGGL(k_energy_sum, dim3(nsel), dim3(kTile), 0, c->stream, c->d_efirst, (const int32_t *)nullptr, pos0,
+                     c->d_epart, c->d_energy, 0);
   HIPCHK(c, hipGetLastError());
   std::vector<double> e(25 * (size_t)nsel);
   HIPCHK(c, hipMemcpyAsync(e.data(), c->d_energy, e.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
@@ -1648,13 +1660,22 @@ int32_t tis_energy_sumup_set(tis_ctx *c, int32_t n, const int32_t *isys, double 
       hipLaunchKernelGGL(k_ewald_sk, dim3(h.esk_count), dim3(kTile), 0, c->stream, c->P, PXc(c),
                          c->d_ewsk + h.esk_begin, 1);
   }
-  // k_energy takes a list of system indices, one block each (the same
-  // kernel as the whole-batch launch)
-  if ((size_t)n > c->eset_cap) {
+  // the live position of each entry, then the tasks of the systems listed
+  // (each system's once, however often it is listed)
+  std::vector<int32_t> arg(n);
+  std::vector<char> seen(c->nlive, 0);
+  for (int k = 0; k < n; ++k) {
+    const HostSys &h = c->hs[isys[k]];
+    arg[k] = h.live_pos;
+    if (seen[h.live_pos]) continue;
+    seen[h.live_pos] = 1;
+    for (int q = 0; q < h.et_count; ++q) arg.push_back(h.et_begin + q);
+  }
+  if (arg.size() > c->eset_cap) {
     if (c->d_eset) { (void)hipFree(c->d_eset); c->d_eset = nullptr; c->dev_bytes -= c->eset_cap * sizeof(int32_t); }
     c->eset_cap = 0;
-    HIPCHK(c, hipMalloc(&c->d_eset, (size_t)n * sizeof(int32_t)));
-    c->eset_cap = (size_t)n;
+    HIPCHK(c, hipMalloc(&c->d_eset, arg.size() * sizeof(int32_t)));
+    c->eset_cap = arg.size();
     c->dev_bytes += c->eset_cap * sizeof(int32_t);
   }
   if ((size_t)n * 25 > c->eset_out_cap) {
@@ -1664,8 +1685,11 @@ int32_t tis_energy_sumup_set(tis_ctx *c, int32_t n, const int32_t *isys, double 
     c->eset_out_cap = (size_t)n * 25;
     c->dev_bytes += c->eset_out_cap * sizeof(double);
   }
-  HIPCHK(c, hipMemcpyAsync(c->d_eset, isys, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_energy, dim3(n), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c), c->d_eset, c->d_eset_out, 0);
+  HIPCHK(c, hipMemcpyAsync(c->d_eset, arg.data(), arg.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+  hipLaunchKernelGGL(k_energy, dim3((unsigned)(arg.size() - n)), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c),
+                     c->d_etask, c->d_eset + n, 0, c->d_epart, 0);
+  hipLaunchKernelGGL(k_energy_sum, dim3(n), dim3(kTile), 0, c->stream, c->d_efirst, c->d_eset, 0, c->d_epart,
+                     c->d_eset_out, 0);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipMemcpyAsync(energy_out, c->d_eset_out, (size_t)n * 25 * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
@@ -1683,19 +1707,23 @@ int32_t tis_energy_unit(tis_ctx *c, int32_t isys, int32_t style, double *energy_
   const int nu = c->hs[isys].d.nunit;
   const size_t nn = (size_t)nu * nu;
   if (nu < 1 || nn > 65535) return fail(c, TIS_ERR_ARG, "system %d has %d units", isys, nu);
-  if (c->eunit_cap < nn * 25) {
+  const HostSys &h = c->hs[isys];
+  const size_t nraw = nn * (25 + (size_t)kEnergyTerms * h.et_count);
+  if (c->eunit_cap < nraw) {
     if (c->d_eunit) {
       (void)hipFree(c->d_eunit);
       c->allocs.erase(std::remove(c->allocs.begin(), c->allocs.end(), (void *)c->d_eunit), c->allocs.end());
       c->dev_bytes -= c->eunit_cap * sizeof(double);
       c->d_eunit = nullptr;
     }
-    rc = dalloc(c, &c->d_eunit, nn * 25);
+    rc = dalloc(c, &c->d_eunit, nraw);
     if (rc) return rc;
-    c->eunit_cap = nn * 25;
+    c->eunit_cap = nraw;
   }
-  hipLaunchKernelGGL(k_energy, dim3(1, (unsigned)nn), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c),
-                     c->d_sysidx + c->hs[isys].live_pos, c->d_eunit, 1);
+  hipLaunchKernelGGL(k_energy, dim3(h.et_count, (unsigned)nn), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c),
+                     c->d_etask, (const int32_t *)nullptr, h.et_begin, c->d_eunit + nn * 25, 1);
+  hipLaunchKernelGGL(k_energy_sum, dim3(1, (unsigned)nn), dim3(kTile), 0, c->stream, c->d_efirst,
+                     (const int32_t *)nullptr, h.live_pos, c->d_eunit + nn * 25, c->d_eunit, 1);
   HIPCHK(c, hipGetLastError());
   std::vector<double> raw(nn * 25);
   HIPCHK(c, hipMemcpyAsync(raw.data(), c->d_eunit, raw.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));

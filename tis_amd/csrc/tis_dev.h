@@ -87,6 +87,21 @@ struct EwTask { int32_t sys, a, b; };
 struct LangClass { double r[4], rcm, fric, mass, pad; };
 constexpr int kEwKChunk = 256;   // reciprocal vectors per block of the force pass
 
+// Blocks of the energy pass for a system of nmp beads, nqt charge chunks and
+// nk reciprocal vectors: 256 beads or vectors, or two chunk pairs (32 of their
+// 128 rows for each of its four waves; four pairs a block measured 126 us for
+// the call below against 116), per block, up to four blocks per CU.
+constexpr int kEnergyTerms = 9;
+constexpr int kEnergyPartsMax = 1024;
+inline int energy_parts(int nmp, int nqt, int nk) {
+  const int64_t pairs = (int64_t)nqt * (nqt + 1) / 2;
+  int64_t p = (nmp + 255) / 256;
+  p = p > (pairs + 1) / 2 ? p : (pairs + 1) / 2;
+  p = p > (nk + 255) / 256 ? p : (nk + 255) / 256;
+  p = p < kEnergyPartsMax ? p : kEnergyPartsMax;
+  return (int)(p > 1 ? p : 1);
+}
+
 struct Tile { int32_t sys, start; };
 
 // bonds [b0, b0+nb), angles [a0, a0+na), consecutive stacks [s0, s0+ns);

@@ -2001,39 +2001,135 @@ __global__ void k_count_rebuild(unsigned long long *counters) {
 }
 
 // ------------------------------------------------------------------ energies
-// energy_sumup.F90:149-529 for one system per block; deterministic tree sum.
+// energy_sumup.F90:149-529.  A system's terms are shared out over
+// energy_parts blocks (tis_dev.h), and k_energy_sum adds the blocks' sums in
+// a fixed order; the split depends on the system alone, so its energies do
+// not depend on what else is evaluated.
+// Bound: FP64 VALU (a square root, an exponential and a division per
+// electrostatic pair).  With one block per system and one thread per charge
+// row the largest system set the time, each row's loads following its bit
+// tests one by one.  The pairs are taken by chunk pair now: the lane's charge
+// of chunk J and its row's list bits in registers, row by row through lane
+// reads, so the inner loop has no load; at four waves per SIMD (the compiler's
+// own 179 VGPRs left two: 146 us).  The batch call of 576 systems (237,111
+// beads, its copy to the host included): 557 -> 116 us.
 constexpr int kEBlock = 256;
-constexpr int kNE = 10;  // bond angle stack tstack hbond thbond exv ele velo spare
-__device__ inline double block_sum(double v, double *red) {
-  const int t = threadIdx.x;
-  red[t] = v;
-  __syncthreads();
-  for (int w = kEBlock / 2; w > 0; w >>= 1) {
-    if (t < w) red[t] += red[t + w];
-    __syncthreads();
+constexpr int kNE = kEnergyTerms;  // bond angle stack tstack hbond thbond exv ele velo
+
+// sums of the block's kNE values per thread, thread k gets sum k
+__device__ inline double block_sums(const double (&e)[kNE], double (*red)[kNE]) {
+  const int t = threadIdx.x, w = t / kTile;
+#pragma unroll
+  for (int k = 0; k < kNE; ++k) {
+    double v = e[k];
+#pragma unroll
+    for (int off = kTile / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
+    if ((t & (kTile - 1)) == 0) red[w][k] = v;
   }
-  double r = red[0];
   __syncthreads();
+  double r = 0.0;
+  if (t < kNE)
+    for (int q = 0; q < kEBlock / kTile; ++q) r += red[q][t];
   return r;
 }
 
+// The value of v at lane r (the same for every lane) of the wave.
+__device__ inline double at_lane(double v, int r) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, r);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), r);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Electrostatic pair energies of wave w of nw over system s: the chunk pairs
+// (I <= J) in task order, 64 rows each, in nw runs of consecutive rows.  A
+// pair counts once, by its lower charge (qj > qi).
+// Debye-Hueckel (energy_ele_DH.F90:33-100), plain Coulomb
+// (energy_ele_coulomb.F90:55-66), the Ewald real-space term
+// (energy_ele_coulomb_ewld.F90:126-138).
+__device__ inline double ele_energy(const DevPtrs &P, const DSys &s, const double *Y, int w, int nw, int unit_mode,
+                                    int ua, int ub) {
+  const int lane = threadIdx.x & (kTile - 1);
+  const int n = P.ntot;
+  const int64_t nrow = (int64_t)s.nqt * (s.nqt + 1) / 2 * kTile;
+  const int64_t r0 = nrow * w / nw, r1 = nrow * (w + 1) / nw;
+  const double cut2 = s.ele_form == 0 ? s.dh_ecut2 : s.cl_cut2;
+  double e = 0.0;
+  int I = 0;
+  int64_t first = 0;   // chunk pairs before row I of them
+  while (I + 1 < s.nqt && r0 / kTile >= first + (s.nqt - I)) { first += s.nqt - I; ++I; }
+  int J = I + (int)(r0 / kTile - first);
+  for (int64_t p = r0 / kTile; p * kTile < r1; ++p) {
+    const int ra = (int)max((int64_t)0, r0 - p * kTile), rb = (int)min((int64_t)kTile, r1 - p * kTile);
+    // lane l: charge l of chunk I with its list bits against chunk J, and
+    // charge l of chunk J
+    const int qi = I * kTile + lane, qj = J * kTile + lane;
+    double xi[3] = {0, 0, 0}, xj[3] = {0, 0, 0}, ci = 0.0, cj = 0.0;
+    uint64_t m64 = 0;
+    int ui = 0, uj = 0;
+    if (qi < s.nq) {
+      const int g = P.qbead[s.qoff + qi];
+      ld3(Y, n, g, xi);
+      ci = P.charge[g];
+      ui = P.unit[g];
+      const uint32_t *row = P.qmask + s.moff + (int64_t)qi * s.mwords;
+      m64 = row[2 * J];
+      if (2 * J + 1 < s.mwords) m64 |= (uint64_t)row[2 * J + 1] << 32;
+    }
+    if (qj < s.nq) {
+      const int g = P.qbead[s.qoff + qj];
+      ld3(Y, n, g, xj);
+      cj = P.charge[g];
+      uj = P.unit[g];
+    }
+    if (I == J) m64 &= lane < kTile - 1 ? ~0ull << (lane + 1) : 0ull;
+    const uint32_t mlo = (uint32_t)m64, mhi = (uint32_t)(m64 >> 32);
+    for (int r = ra; r < rb; ++r) {
+      const uint64_t row = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mlo, r) |
+                           (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)mhi, r) << 32;
+      if (row == 0) continue;
+      if (unit_mode && __builtin_amdgcn_readlane(ui, r) != ua) continue;
+      bool on = (row >> lane) & 1u;
+      if (unit_mode) on = on && uj == ub;
+      double v[3] = {xj[0] - at_lane(xi[0], r), xj[1] - at_lane(xi[1], r), xj[2] - at_lane(xi[2], r)};
+      if (s.periodic) {
+        const int c = on ? (int)P.qmirror[s.mioff + (int64_t)(I * kTile + r) * s.nq + qj] : 26;
+        for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, c, d);
+      }
+      const double d2 = dot3(v, v);
+      if (!on || d2 > cut2) continue;
+      const double d1 = sqrt(d2);
+      const double cij = (at_lane(ci, r) * cj) * s.ele_coef;
+      if (s.ele_form == 0) e += cij / d1 * exp(-d1 * s.rcdist);
+      else if (s.ele_form == 1) e += cij * (1.0 / d1 - s.cl_rcinv);
+      else e += cij * erfc(s.ew_alpha * d1) / d1;
+    }
+    if (++J == s.nqt) { ++I; J = I; }
+  }
+  return e;
+}
+
+// One block per task (system, part of its nparts): task ids[blockIdx.x], or
+// t0 + blockIdx.x without ids; the sums of task k go to part[k].
 // unit_mode 1: block (x, y) sums only the terms whose unit pair, taken as
 // energy_sumup.F90's terms take it, is (y mod nunit, y / nunit): raw
 // energy_unit entries (the Ewald terms add none, as in
-// energy_ele_coulomb_ewld.F90:168-170).
-__global__ __launch_bounds__(kEBlock) void k_energy(DevPtrs P, const double *X, const double *PX,
-                                                    const int32_t *sysidx, double *out, int unit_mode) {
-  __shared__ double red[kEBlock];
-  const int t = threadIdx.x;
-  const int is = sysidx[blockIdx.x];
-  const DSys s = P.sys[is];
+// energy_ele_coulomb_ewld.F90:168-170); their sums go to part[y ntask + k - t0].
+__global__ __launch_bounds__(kEBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_energy(DevPtrs P, const double *X, const double *PX,
+                                                    const EwTask *tasks, const int32_t *ids, int t0, double *part,
+                                                    int unit_mode) {
+  __shared__ double red[kEBlock / kTile][kNE];
+  const int task = ids ? ids[blockIdx.x] : t0 + (int)blockIdx.x;
+  const EwTask tk = tasks[task];
+  const DSys s = P.sys[tk.sys];
+  const int t = tk.a * kEBlock + (int)threadIdx.x, nt = tk.b * kEBlock;   // this thread of the system's
   const int n = P.ntot;
   const int ua = unit_mode ? (int)blockIdx.y % s.nunit : 0, ub = unit_mode ? (int)blockIdx.y / s.nunit : 0;
   auto take = [&](int gi, int gj) { return !unit_mode || (P.unit[gi] == ua && P.unit[gj] == ub); };
   double e[kNE];
   for (int k = 0; k < kNE; ++k) e[k] = 0.0;
   // bonds (energy_bond.F90:39-57)
-  for (int b = s.boff + t; b < s.boff + s.nbd; b += kEBlock) {
+  for (int b = s.boff + t; b < s.boff + s.nbd; b += nt) {
     if (!take(P.bd_mp[2 * b], P.bd_mp[2 * b + 1])) continue;
     double v[3];
     vsub(X, n, P.bd_mp[2 * b + 1], P.bd_mp[2 * b], v);
@@ -2041,7 +2137,7 @@ __global__ __launch_bounds__(kEBlock) void k_energy(DevPtrs P, const double *X, 
     e[0] += P.bd_coef[b] * (dd * dd);
   }
   // angles (energy_bangle.F90:36-52)
-  for (int a = s.aoff + t; a < s.aoff + s.nba; a += kEBlock) {
+  for (int a = s.aoff + t; a < s.aoff + s.nba; a += nt) {
     if (!take(P.ba_mp[3 * a], P.ba_mp[3 * a + 1])) continue;
     double v21[3], v32[3];
     vsub(X, n, P.ba_mp[3 * a + 1], P.ba_mp[3 * a], v21);
@@ -2052,7 +2148,7 @@ __global__ __launch_bounds__(kEBlock) void k_energy(DevPtrs P, const double *X, 
     e[1] += P.ba_coef[a] * (dba * dba);
   }
   // consecutive stacks (energy_dtrna_stack.F90:85-160)
-  for (int st = s.soff + t; st < s.soff + s.nst; st += kEBlock) {
+  for (int st = s.soff + t; st < s.soff + s.nst; st += nt) {
     if (!take(P.st_mp[7 * st], P.st_mp[7 * st])) continue;
     if (!stack_on(P, X, PX, st)) continue;
     const int32_t *m7 = P.st_mp + 7 * st;
@@ -2072,7 +2168,7 @@ __global__ __launch_bounds__(kEBlock) void k_energy(DevPtrs P, const double *X, 
     e[2] += cf[0] / ediv;
   }
   // tertiary stacks (energy_dtrna_stack_nlocal.F90:55-230)
-  for (int k = s.toff + t; k < s.toff + s.ntst; k += kEBlock) {
+  for (int k = s.toff + t; k < s.toff + s.ntst; k += nt) {
     if (!take(P.tst_mp[6 * k], P.tst_mp[6 * k + 1])) continue;
     const int32_t *m6 = P.tst_mp + 6 * k;
     const double *nat = P.tst_nat + 6 * k, *cf = P.tst_coef + 7 * k;
@@ -2103,91 +2199,62 @@ __global__ __launch_bounds__(kEBlock) void k_energy(DevPtrs P, const double *X, 
     e[3] += cf[0] / ediv;
   }
   // hbonds: energies of the last force evaluation (energy_dtrna_hbond15.F90:119-148)
-  for (int h = s.hoff + t; h < s.hoff + s.nhb; h += kEBlock)
+  for (int h = s.hoff + t; h < s.hoff + s.nhb; h += nt)
     if (P.hb_inlist[h] && P.hb_status[h] && take(P.hb_mp[6 * h], P.hb_mp[6 * h + 1]))
       e[P.hb_tert[h] ? 5 : 4] += P.hb_ene[h];
-  // excluded volume, each pair once by its lower bead (energy_exv_dt15.F90:60-116)
+  // excluded volume, each pair once by its lower bead
+  // (energy_exv_dt15.F90:60-116): the entries of four neighbours, then their
+  // beads, are loaded together
   {
     const double *Y = s.periodic ? PX : X;
     const double a = s.exv_a;
-    for (int li = t; li < s.nmp; li += kEBlock) {
-      int g = s.off + li;
+    for (int li = t; li < s.nmp; li += nt) {
+      const int g = s.off + li;
       double xi[3];
       ld3(Y, n, g, xi);
-      int cnt = min(P.nb_cnt[g], P.nb_cap);
-      for (int m = 0; m < cnt; ++m) {
-        uint32_t ent = P.nb[(size_t)m * n + g];
-        int j = (int)(ent & kIdxMask);
-        if (j < g || !take(g, j)) continue;
-        double v[3] = {Y[j] - xi[0], Y[n + j] - xi[1], Y[2 * n + j] - xi[2]};
-        if (s.periodic) { int c = (int)(ent >> kMirrorShift); for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, c, d); }
-        int ti = P.mptype[g], tj = P.mptype[j];
-        double dij;
-        if ((ti == 2 && tj == 4) || (ti == 4 && tj == 2)) dij = s.exv_dist_PS;
-        else if (P.iclass[g] == 2 && P.iclass[j] == 2) dij = s.exv_dist;
-        else dij = P.exv_rad[g] + P.exv_rad[j];
-        double dist = sqrt(dot3(v, v));
-        if (dist > dij) continue;
-        dist = dist + a - dij;
-        if (dist > s.exv_inf) {
-          double r = a / dist, r2 = r * r, r6 = r2 * r2 * r2;
-          e[6] += ((double)P.exv_eps[g] * (double)P.exv_eps[j]) * (r6 * r6 - 2.0 * r6 + 1.0);
-        } else {
-          e[6] += kHighEnergy;
+      const int cnt = min(P.nb_cnt[g], P.nb_cap);
+      const SpPair *tab = P.sptab + s.sptab + (int)P.species[g] * s.nspecies;
+      for (int m0 = 0; m0 < cnt; m0 += 4) {
+        uint32_t ent[4];
+        double y[4][3];
+        SpPair tp[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ent[u] = P.nb[(size_t)min(m0 + u, cnt - 1) * n + g];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int j = (int)(ent[u] & kIdxMask);
+          ld3(Y, n, j, y[u]);
+          tp[u] = tab[P.species[j]];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int j = (int)(ent[u] & kIdxMask);
+          if (m0 + u >= cnt || j < g) continue;
+          double v[3] = {y[u][0] - xi[0], y[u][1] - xi[1], y[u][2] - xi[2]};
+          if (s.periodic) {
+            const int c = (int)(ent[u] >> kMirrorShift);
+            for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, c, d);
+          }
+          double dist = sqrt(dot3(v, v));
+          if (dist > tp[u].dij || !take(g, j)) continue;
+          dist = dist + a - tp[u].dij;
+          if (dist > s.exv_inf) {
+            double r = a / dist, r2 = r * r, r6 = r2 * r2 * r2;
+            e[6] += ((double)P.exv_eps[g] * (double)P.exv_eps[j]) * (r6 * r6 - 2.0 * r6 + 1.0);
+          } else {
+            e[6] += kHighEnergy;
+          }
         }
       }
     }
   }
-  // Debye-Hueckel, each pair once (energy_ele_DH.F90:33-100)
-  if (s.ele_form == 0) {
-    const double *Y = s.periodic ? PX : X;
-    for (int qi = t; qi < s.nq; qi += kEBlock) {
-      if (unit_mode && P.unit[P.qbead[s.qoff + qi]] != ua) continue;
-      int gi = P.qbead[s.qoff + qi];
-      double xi[3];
-      ld3(Y, n, gi, xi);
-      const uint32_t *row = P.qmask + s.moff + (int64_t)qi * s.mwords;
-      for (int qj = qi + 1; qj < s.nq; ++qj) {
-        if (!((row[qj >> 5] >> (qj & 31)) & 1u)) continue;
-        int gj = P.qbead[s.qoff + qj];
-        if (unit_mode && P.unit[gj] != ub) continue;
-        double v[3] = {Y[gj] - xi[0], Y[n + gj] - xi[1], Y[2 * n + gj] - xi[2]};
-        if (s.periodic) { int c = P.qmirror[s.mioff + (int64_t)qi * s.nq + qj]; for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, c, d); }
-        double d2 = dot3(v, v);
-        if (d2 > s.dh_ecut2) continue;
-        double d1 = sqrt(d2);
-        e[7] += (P.charge[gi] * P.charge[gj]) * s.ele_coef / d1 * exp(-d1 * s.rcdist);
-      }
-    }
-  }
-  // plain Coulomb (energy_ele_coulomb.F90:55-66) and the Ewald real-space
-  // term (energy_ele_coulomb_ewld.F90:126-138), each pair once
-  if (s.ele_form == 1 || (s.ele_form == 2 && !unit_mode)) {
-    const double *Y = s.periodic ? PX : X;
-    for (int qi = t; qi < s.nq; qi += kEBlock) {
-      if (unit_mode && P.unit[P.qbead[s.qoff + qi]] != ua) continue;
-      int gi = P.qbead[s.qoff + qi];
-      double xi[3];
-      ld3(Y, n, gi, xi);
-      const uint32_t *row = P.qmask + s.moff + (int64_t)qi * s.mwords;
-      for (int qj = qi + 1; qj < s.nq; ++qj) {
-        if (!((row[qj >> 5] >> (qj & 31)) & 1u)) continue;
-        int gj = P.qbead[s.qoff + qj];
-        if (unit_mode && P.unit[gj] != ub) continue;
-        double v[3] = {Y[gj] - xi[0], Y[n + gj] - xi[1], Y[2 * n + gj] - xi[2]};
-        if (s.periodic) { int c = P.qmirror[s.mioff + (int64_t)qi * s.nq + qj]; for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, c, d); }
-        double d2 = dot3(v, v);
-        if (d2 > s.cl_cut2) continue;
-        double d1 = sqrt(d2);
-        const double cij = (P.charge[gi] * P.charge[gj]) * s.ele_coef;
-        e[7] += s.ele_form == 1 ? cij * (1.0 / d1 - s.cl_rcinv) : cij * erfc(s.ew_alpha * d1) / d1;
-      }
-    }
-  }
+  if (s.ele_form == 0 || s.ele_form == 1 || (s.ele_form == 2 && !unit_mode))
+    e[7] += ele_energy(P, s, s.periodic ? PX : X, __builtin_amdgcn_readfirstlane(t / kTile), nt / kTile, unit_mode, ua,
+                       ub);
   // Ewald Fourier sum (energy_ele_coulomb_ewld.F90:70-90) from the partial
   // structure factors of the last k_ewald_sk pass, plus the self term
   if (s.ele_form == 2 && !unit_mode) {
-    for (int k = t; k < s.nk; k += kEBlock) {
+    for (int k = t; k < s.nk; k += nt) {
       double sc = 0.0, ss = 0.0;
       for (int c = 0; c < s.nqc; ++c) {
         const double *ps = P.psk + s.psk_off + 2 * ((int64_t)c * s.nk + k);
@@ -2198,23 +2265,56 @@ __global__ __launch_bounds__(kEBlock) void k_energy(DevPtrs P, const double *X, 
     if (t == 0) e[7] += s.ew_self;
   }
   // kinetic (energy_kinetic.F90:33-44)
-  for (int li = t; li < s.nmp; li += kEBlock) {
+  for (int li = t; li < s.nmp; li += nt) {
     int g = s.off + li;
     if (!take(g, g)) continue;
     double v[3] = {P.v[g], P.v[n + g], P.v[2 * n + g]};
     e[8] += 0.5 * P.mass[g] * dot3(v, v);
   }
+  const double tot = block_sums(e, red);
+  const size_t slot = unit_mode ? (size_t)blockIdx.y * gridDim.x + blockIdx.x : (size_t)task;
+  if ((int)threadIdx.x < kNE) part[slot * kNE + threadIdx.x] = tot;
+}
+
+// The parts of entry k (tasks [first[i], first[i + 1]) with i = pos[k], or k0
+// + k without pos; unit_mode: all parts of block row blockIdx.y) added in a
+// fixed order into the 25 E_TYPE slots of out[k]; TOTAL excludes VELO.
+__global__ __launch_bounds__(kTile) void k_energy_sum(const int32_t *first, const int32_t *pos, int k0,
+                                                      const double *part, double *out, int unit_mode) {
+  const int i = pos ? pos[blockIdx.x] : k0 + (int)blockIdx.x, t = (int)threadIdx.x;
+  const int np = first[i + 1] - first[i];
+  const double *p = part + (unit_mode ? (size_t)blockIdx.y * np : (size_t)first[i]) * kNE;
+  // lane l adds parts l, l + 64, ..; then the lanes' sums
   double tot[kNE];
-  for (int k = 0; k < kNE; ++k) tot[k] = block_sum(e[k], red);
-  if (t == 0) {
-    double *o = out + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * 25;
-    for (int k = 0; k < 25; ++k) o[k] = 0.0;
-    o[2] = tot[0]; o[3] = tot[1]; o[15] = tot[2]; o[18] = tot[3]; o[16] = tot[4]; o[19] = tot[5];
-    o[17] = tot[6]; o[7] = tot[7]; o[1] = tot[8];
-    double sum = 0.0;
-    for (int k = 2; k < 25; ++k) sum += o[k];
-    o[0] = sum;
+#pragma unroll
+  for (int k = 0; k < kNE; ++k) tot[k] = 0.0;
+  for (int q = t; q < np; q += kTile)
+#pragma unroll
+    for (int k = 0; k < kNE; ++k) tot[k] += p[(size_t)q * kNE + k];
+#pragma unroll
+  for (int k = 0; k < kNE; ++k)
+#pragma unroll
+    for (int off = kTile / 2; off > 0; off >>= 1) tot[k] += __shfl_xor(tot[k], off);
+  double *o = out + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * 25;
+  if (t >= 25) return;
+  // E_TYPE slots of the kNE sums
+  double v = 0.0;
+  switch (t) {
+    case 0:   // in slot order
+      v = ((((((tot[0] + tot[1]) + tot[7]) + tot[2]) + tot[4]) + tot[6]) + tot[3]) + tot[5];
+      break;
+    case 1: v = tot[8]; break;
+    case 2: v = tot[0]; break;
+    case 3: v = tot[1]; break;
+    case 7: v = tot[7]; break;
+    case 15: v = tot[2]; break;
+    case 16: v = tot[4]; break;
+    case 17: v = tot[6]; break;
+    case 18: v = tot[3]; break;
+    case 19: v = tot[5]; break;
+    default: break;
   }
+  o[t] = v;
 }
 
 // ------------------------------------------------------------------ labels
