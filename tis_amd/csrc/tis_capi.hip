@@ -33,7 +33,8 @@ __global__ void k_lists(DevPtrs, const double *, const double *, const Tile *, i
                         int, int);
 __global__ void k_lpair(DevPtrs, const double *, const double *, const EwTask *, int, const EwTask *, int, int, int,
                         int, int);
-__global__ void k_advance(uint64_t *, uint64_t, unsigned long long *);
+__global__ void k_advance(uint64_t *, uint64_t, uint64_t, uint64_t, unsigned long long *);
+__global__ void k_window(DevPtrs, const int32_t *, int, int, int, int, int);
 __global__ void k_count_rebuild(unsigned long long *);
 __global__ void k_energy(DevPtrs, const double *, const double *, const EwTask *, const int32_t *, int, double *, int);
 __global__ void k_energy_sum(const int32_t *, const int32_t *, int, const double *, double *, int);
@@ -163,6 +164,8 @@ struct tis_ctx {
   int32_t nsystask = 0;
   int32_t *d_hbdense = nullptr;          // hbond lanes (DevPtrs::hb_dense)
   int32_t nhbdense = 0;
+  int32_t *d_wsys = nullptr;             // live systems, largest first, when k_window takes the batch
+  int32_t win_rows = 0, win_lds = 0;     // its list rows and bytes in LDS; win_lds 0: per-step passes
   std::vector<int32_t> systask_of;       // index into d_systask per system or -1
   int32_t *d_ststat = nullptr;           // st_status output of tis_term_status [nsttot]
   double *d_energy = nullptr;
@@ -899,7 +902,7 @@ int alloc_arena(tis_ctx *c, const Caps &k, std::vector<void *> &list, DevPtrs &P
   P.nb_cap = std::max(nb_cap, 64);
   AL(P.nb, (size_t)P.nb_cap * B);
   AL(P.dxyz, 3 * B); AL(P.dlast, 3 * B);
-  AL(P.sys_flag, k.nsys);
+  AL(P.sys_flag, k.nsys); AL(P.win_at, k.nsys);
   AL(P.pp, k.pp); AL(P.qmask, k.m); AL(P.qmirror, k.mi); AL(P.lcnt, k.lp * kTile);
   AL(A.ewh, 3 * k.k); AL(A.ewc, k.k); AL(P.psk, k.psk); AL(P.pf, k.pf);
   AL(A.counters, TIS_CNT_MAX); AL(A.stepbase, 1); AL(A.energy, 25 * k.nsys);
@@ -981,6 +984,50 @@ StageMarks marks_of(const Stage &g) {
   return m;
 }
 
+// Whether k_window can take system d: no periodic image, no tertiary stack,
+// indices within its 16-bit entries.
+bool window_fits(const DSys &d) {
+  return !d.periodic && d.ele_form != TIS_ELE_EWALD && d.ntst == 0 && d.nmp <= kWinThreads &&
+         d.nspecies <= kWinSpecies && d.nunit <= kWinUnits && win_slots(d) <= 65535 && d.nhb <= 65535 &&
+         d.nsite < 0xFFFF;
+}
+
+// Batched runs take k_window when every live system fits it and is small (see
+// kWindowBeads).  *wsys gets the systems, the largest first (blocks start in
+// order).
+// Measured, us a step with a rebuild every 10 (per-step passes / k_window), 1
+// system and 512: 95 beads 16.3 / 10.9 and 26 / 20; 254 beads 19.4 / 15.7 and
+// 40 / 31; 446 beads 20.8 / 24.6 and 62 / 50: one workgroup falls behind on
+// its own near 400 beads and stays ahead when the batch fills the chip.
+constexpr int kWindowBeads = 448;
+constexpr int kWindowSteps = 500;   // steps per k_window launch (a few ms)
+
+void choose_window(tis_ctx *c, std::vector<int32_t> &wsys) {
+  c->win_rows = c->win_lds = 0;
+  const int room = kLdsBytes - 256;
+  int rows = kWinRows;
+  for (int is = 0; is < c->nsys; ++is) {
+    const HostSys &h = c->hs[is];
+    if (!h.live) continue;
+    if (!window_fits(h.d) || h.d.nmp > kWindowBeads) { wsys.clear(); return; }
+    const int base = win_layout(h.d, 0).total;
+    if (base > room) { wsys.clear(); return; }
+    rows = std::min(rows, (room - base - 8) / (2 * h.d.nmp));
+    wsys.push_back(is);
+  }
+  if (wsys.empty()) return;
+  std::stable_sort(wsys.begin(), wsys.end(), [&](int a, int b) { return c->hs[a].d.nmp > c->hs[b].d.nmp; });
+  int bytes = 0;
+  for (int is : wsys) bytes = std::max(bytes, win_layout(c->hs[is].d, rows).total);
+  if (hipFuncSetAttribute((const void *)k_window, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    wsys.clear();
+    return;
+  }
+  c->win_rows = rows;
+  c->win_lds = bytes;
+}
+
 // The launch tables of the live systems (tiles, chunk pairs, tile pairs,
 // Ewald tasks, hbond / tertiary-stack systems, the live list) and every
 // system's DSys; tables are rebuilt whole on each change of the live set.
@@ -992,7 +1039,7 @@ int build_tables(tis_ctx *c) {
   c->tab_bytes = 0;
   std::vector<Tile> btiles, qtiles;
   std::vector<EwTask> ptask, bpair, qpair, ewsk, ewf, etask;
-  std::vector<int32_t> systask, hbdense, efirst;
+  std::vector<int32_t> systask, hbdense, efirst, wsys;
   c->systask_of.assign(c->nsys, -1);
   c->any_ele = false;
   c->any_periodic = false;
@@ -1078,6 +1125,8 @@ int build_tables(tis_ctx *c) {
   }
   UPT(c->d_ptask, ptask); UPT(c->d_ptask_lpt, lpt); UPT(c->d_bpair, bpair); UPT(c->d_qpair, qpair);
   UPT(c->d_ewsk, ewsk); UPT(c->d_ewf, ewf); UPT(c->d_systask, systask);
+  choose_window(c, wsys);
+  UPT(c->d_wsys, wsys);
   UPT(c->d_hbdense, hbdense); UPT(c->d_etask, etask); UPT(c->d_efirst, efirst);
 #undef UPT
   c->P.hb_dense = c->d_hbdense;
@@ -1910,6 +1959,7 @@ int32_t tis_langevin_init(tis_ctx *c, double tstep, int32_t rebuild_every, uint6
   // displacements since this rebuild start at zero, no rebuild pending
   HIPCHK(c, hipMemsetAsync(c->P.dxyz, 0, 3 * sizeof(double) * (size_t)std::max(c->P.ntot, 1), c->stream));
   HIPCHK(c, hipMemsetAsync(c->P.sys_flag, 0, (size_t)c->caps.nsys, c->stream));
+  HIPCHK(c, hipMemsetAsync(c->P.win_at, 0, sizeof(uint64_t) * (size_t)c->caps.nsys, c->stream));
   HIPCHK(c, hipMemsetAsync(c->P.ttop, 0, 2 * sizeof(double) * (size_t)std::max(c->nbtile, 1), c->stream));
   Range r = range_of(c, -1);
   const int cu = c->cur;
@@ -1973,17 +2023,20 @@ static int capture_graph(tis_ctx *c, int parity) {
   HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   int cu = parity;
   Range r = range_of(c, -1);
+  // one rebuild per graph, at its start: counted with the steps
+  const bool one = !c->P.dyn && L == c->rebuild_every;
   for (int t = 0; t < L; ++t) {
     if (c->P.dyn) {
       launch_lists(c, r, c->P.x[cu], c->P.px[cu], c->P.px[cu ^ 1], 1, 1);
     } else if (t % c->rebuild_every == 0) {
       launch_lists(c, r, c->P.x[cu], c->P.px[cu], c->P.px[cu ^ 1], 1, 0);
-      hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
+      if (!one) hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
     }
     launch_force_pair(c, r, c->P.x[cu ^ 1], c->P.px[cu ^ 1], c->P.x[cu], c->P.px[cu], t, 1, 1);
     cu ^= 1;
   }
-  hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)L, c->d_counters);
+  hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)L,
+                     (uint64_t)(one ? 1 : 0), (uint64_t)0, c->d_counters);
   hipError_t e = hipStreamEndCapture(c->stream, &g);
   if (e != hipSuccess) return fail(c, TIS_ERR_HIP, "stream capture failed: %s", hipGetErrorString(e));
   e = hipGraphInstantiate(&c->graph[parity], g, nullptr, nullptr, 0);
@@ -1998,7 +2051,21 @@ static int capture_graph(tis_ctx *c, int parity) {
 static int run_steps(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch) {
   int64_t done = 0;
   const int L = steps_per_graph(c);
-  if (mode == TIS_MODE_GRAPH) {
+  if (mode == TIS_MODE_GRAPH && c->win_lds > 0) {
+    // every system small: launches of up to kWindowSteps steps
+    while (done < nsteps) {
+      const int n = (int)std::min<int64_t>(nsteps - done, kWindowSteps);
+      const int re = c->P.dyn ? 0 : c->rebuild_every;
+      const int phase = re > 0 ? (int)(c->t_since_init % re) : 0;
+      const int nreb = re > 0 ? (phase + n - 1) / re + (phase == 0 ? 1 : 0) : 0;   // multiples of re in [phase, phase + n)
+      hipLaunchKernelGGL(k_window, dim3(c->nlive), dim3(kWinThreads), c->win_lds, c->stream, c->P, c->d_wsys,
+                         c->win_rows, c->cur, n, phase, re);
+      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)n, (uint64_t)nreb,
+                         (uint64_t)n, c->d_counters);
+      c->cur ^= n & 1;
+      done += n; c->t_since_init += n; *nlaunch += 1;
+    }
+  } else if (mode == TIS_MODE_GRAPH) {
     while (done < nsteps) {
       if (c->t_since_init % L == 0 && nsteps - done >= L) {
         if (!c->graph[c->cur]) { int rc = capture_graph(c, c->cur); if (rc) return rc; }
@@ -2007,7 +2074,8 @@ static int run_steps(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch)
         *nlaunch += 1;
       } else {
         eager_step(c, -1);
-        hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)1, c->d_counters);
+        hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)1, (uint64_t)0,
+                         (uint64_t)0, c->d_counters);
         c->cur ^= 1; ++done; ++c->t_since_init; *nlaunch += 2;
       }
     }
@@ -2016,7 +2084,8 @@ static int run_steps(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch)
     c->tev_used = 0;
     for (; done < nsteps; ++done) {
       eager_step(c, -1);
-      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)1, c->d_counters);
+      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)1, (uint64_t)0,
+                         (uint64_t)0, c->d_counters);
       c->cur ^= 1; ++c->t_since_init; *nlaunch += 2;
     }
   } else {
@@ -2030,7 +2099,8 @@ static int run_steps(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch)
         if (c->hs[is].live) eager_lists(c, is);
       for (int is = 0; is < c->nsys; ++is)
         if (c->hs[is].live) eager_forces(c, is, is == last);
-      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)1, c->d_counters);
+      hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)1, (uint64_t)0,
+                         (uint64_t)0, c->d_counters);
       c->cur ^= 1; ++c->t_since_init; *nlaunch += 2 * c->nlive;
     }
   }

@@ -102,6 +102,11 @@ inline int energy_parts(int nmp, int nqt, int nk) {
   return (int)(p > 1 ? p : 1);
 }
 
+// The staged J chunk of a chunk pair (twice over) as the unrolled pair loop
+// reads it.  Arrays, not records, so that the 64 lanes' reads of consecutive
+// entries fall in distinct LDS banks.
+struct EleWave { double x[2 * kTile], y[2 * kTile], z[2 * kTile]; float q[2 * kTile]; };
+
 struct Tile { int32_t sys, start; };
 
 // bonds [b0, b0+nb), angles [a0, a0+na), consecutive stacks [s0, s0+ns);
@@ -115,6 +120,54 @@ struct SpPair { double dij, dij2, coef; };
 
 // axis-aligned bounding box of a tile of beads (or charges)
 struct BBox { double lo[3], hi[3]; };
+
+// k_window: one bead per thread of the workgroup; beads numbered in 10 bits
+// and species in 6 of a 16-bit list entry; list rows held in LDS.
+constexpr int kWinThreads = 512;
+constexpr int kWinSpecies = 64, kWinRows = 64, kWinUnits = 16;
+constexpr int kLdsBytes = 160 * 1024;
+
+// LDS of one k_window workgroup: byte offsets of its system's arrays.  Sizes
+// depend on the system; rows is the part of the excluded-volume lists held
+// (the rest is read from memory).
+struct WinLds {
+  int32_t x, e, g, pp, je, sptab, mask, rl2, ene, bd, ba, st, hb, qic, slot, meta, cnt, val, list, inc, incoff, nb, bdm,
+      bam, stm, hbm, hbsite, seq, qidx, qb, spec, stat, inl, total;
+};
+
+__host__ __device__ inline int win_slots(const DSys &d) {
+  return 2 * d.nbd + 3 * d.nba + 7 * d.nst + 6 * d.nhb;   // slots = incidence entries
+}
+
+__host__ __device__ inline WinLds win_layout(const DSys &d, int rows) {
+  WinLds L;
+  int32_t at = 0;
+  auto take = [&](int32_t bytes) { const int32_t o = at; at += (bytes + 7) & ~7; return o; };
+  const int nb3 = 24 * d.nmp, nqt = d.ele_form >= 0 ? d.nqt : 0, nq = d.ele_form >= 0 ? d.nq : 0;
+  const int np = nqt * (nqt + 1) / 2, ns = win_slots(d), nv = d.hb_excess_possible ? d.nhb : 0;
+  L.x = take(nb3); L.e = take(2 * nb3); L.g = take(nb3);
+  L.pp = take(np * 6 * kTile * 8);
+  L.je = take(nqt * (int)sizeof(EleWave));
+  L.sptab = take(d.nspecies * d.nspecies * (int)sizeof(SpPair));
+  L.mask = take(np * kTile * 8);
+  L.rl2 = take(8 * d.nunit * d.nunit);
+  L.ene = take(8 * nv);
+  // term parameters, one array per component
+  L.bd = take(16 * d.nbd); L.ba = take(16 * d.nba); L.st = take(56 * d.nst); L.hb = take(104 * d.nhb);
+  L.qic = take(nqt * kTile * 4);
+  // slot forces; during a list build the accept masks of 64-bead segments
+  const int seg = 8 * d.nmp * ((d.nmp + kTile - 1) / kTile);
+  L.slot = take(12 * ns > seg ? 12 * ns : seg);
+  L.meta = take(4 * d.nmp);
+  L.cnt = take(nv ? 4 * d.nsite : 0); L.val = take(nv ? 4 * d.nsite : 0);
+  L.inc = take(2 * ns); L.incoff = take(2 * (d.nmp + 1)); L.nb = take(2 * d.nmp);
+  L.bdm = take(4 * d.nbd); L.bam = take(6 * d.nba); L.stm = take(14 * d.nst); L.hbm = take(12 * d.nhb);
+  L.hbsite = take(12 * nv); L.seq = take(2 * nv);
+  L.qidx = take(2 * d.nmp); L.qb = take(2 * nq); L.spec = take(d.nmp); L.stat = take(nv); L.inl = take(d.nhb);
+  L.list = take(2 * d.nmp * rows);
+  L.total = at;
+  return L;
+}
 
 // All device pointers of a context, passed by value to kernels.
 struct DevPtrs {
@@ -183,6 +236,9 @@ struct DevPtrs {
   double *dxyz, *dlast;      // [3][ntot]
   double *ttop;              // [nbtile][2]
   uint8_t *sys_flag;         // [nsys]
+  // k_window: the step a system has reached ahead of *stepbase (a launch that
+  // another system's list overflow cut short), << 1 | the buffer of its x
+  uint64_t *win_at;          // [nsys]
   // counters / timing
   unsigned long long *counters;  // TIS_CNT_*
   uint64_t *stepbase;

@@ -12,9 +12,30 @@
 //   neighbor_list.F90:56-87 + neighbor_assign.F90:481-559, neighbor_list_ele.F90:123-210,
 //   neighbor_list_hb.F90:59-78, util_periodic.F90:26-36, time_integral.F90:149-183,
 //   time_integral_pre.F90:176-179, energy_*.F90.
+#include <type_traits>
+
 #include "tis_dev.h"
 
+// Multiply-adds are fused where one expression writes them, and nowhere else:
+// a term evaluated by two kernels (the per-step passes and k_window) then has
+// the same bits in both, whatever code surrounds it.
+#pragma clang fp contract(on)
+
 namespace tis {
+
+// Coordinates as the terms read them: component d of bead g, from an SoA
+// array in global memory or (k_window) from the workgroup's copy of its
+// system's beads in LDS.
+struct GlobalX {
+  const double *p;
+  int n;
+  __device__ double operator()(int d, int g) const { return p[(size_t)d * n + g]; }
+};
+struct LocalX {
+  const double *p;   // [3][n], bead off first
+  int n, off;
+  __device__ double operator()(int d, int g) const { return p[d * n + g - off]; }
+};
 
 __device__ inline void ld3(const double *X, int n, int g, double r[3]) {
   r[0] = X[g]; r[1] = X[n + g]; r[2] = X[2 * n + g];
@@ -35,35 +56,46 @@ __device__ inline double wrap_pi(double d) {
 __device__ inline void vsub(const double *X, int n, int a, int b, double v[3]) {
   v[0] = X[a] - X[b]; v[1] = X[n + a] - X[n + b]; v[2] = X[2 * n + a] - X[2 * n + b];
 }
+template <class XA>
+__device__ inline void vsub(const XA &X, int a, int b, double v[3]) {
+  v[0] = X(0, a) - X(0, b); v[1] = X(1, a) - X(1, b); v[2] = X(2, a) - X(2, b);
+}
+
+// The value of v at lane r (the same for every lane) of the wave.
+__device__ inline double at_lane(double v, int r) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, r);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), r);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
 
 // ------------------------------------------------------------------ bonded
 // Each bonded term is evaluated once (one lane per term) and its per-bead
 // forces are written to the slots of the beads' incidence lists.
 
 // force_bond.F90:40-58: fo[0..2] on bead 1, fo[3..5] on bead 2
-__device__ inline void bond_eval(const DevPtrs &P, const double *X, int b, double fo[6]) {
-  int i = P.bd_mp[2 * b], j = P.bd_mp[2 * b + 1];
+template <class XA>
+__device__ inline void bond_eval(const XA &X, int i, int j, double nat, double coef, double fo[6]) {
   double v[3];
-  vsub(X, P.ntot, j, i, v);
+  vsub(X, j, i, v);
   double dist = sqrt(dot3(v, v));
-  double dd = dist - P.bd_nat[b];
-  double fr = P.bd_coef[b] * (-2.0 * dd / dist);
+  double dd = dist - nat;
+  double fr = coef * (-2.0 * dd / dist);
   for (int d = 0; d < 3; ++d) { fo[d] = -(fr * v[d]); fo[3 + d] = fr * v[d]; }
 }
 
 // force_bangle.F90:40-84
-__device__ inline void angle_eval(const DevPtrs &P, const double *X, int a, double fo[9]) {
+template <class XA>
+__device__ inline void angle_eval(const XA &X, int i1, int i2, int i3, double nat, double coef, double fo[9]) {
   for (int k = 0; k < 9; ++k) fo[k] = 0.0;
-  double coef = P.ba_coef[a];
   if (coef < 1.0e-6) return;
-  int i1 = P.ba_mp[3 * a], i2 = P.ba_mp[3 * a + 1], i3 = P.ba_mp[3 * a + 2];
   double v21[3], v32[3];
-  vsub(X, P.ntot, i2, i1, v21);
-  vsub(X, P.ntot, i3, i2, v32);
+  vsub(X, i2, i1, v21);
+  vsub(X, i3, i2, v32);
   double c11 = dot3(v21, v21), c22 = dot3(v32, v32), c21 = dot3(v32, v21);
   double ct = -c21 / sqrt(c11 * c22);
   ct = ct > 1.0 ? 1.0 : (ct < -1.0 ? -1.0 : ct);
-  double dba = acos(ct) - P.ba_nat[a];
+  double dba = acos(ct) - nat;
   double t3 = c11 * c22 - c21 * c21;
   if (t3 <= 1.0) t3 = 1.0;
   double fr = 2.0 * coef * dba / sqrt(t3);
@@ -75,16 +107,15 @@ __device__ inline void angle_eval(const DevPtrs &P, const double *X, int a, doub
 }
 
 // force_dtrna_stack.F90:53-165: fo[3*k + d] on bead k of B1 B2 P1 S1 P2 S2 P3
-__device__ inline void stack_eval(const DevPtrs &P, const double *X, int st, double fo[21]) {
-  const int n = P.ntot;
-  const int32_t *m7 = P.st_mp + 7 * st;
-  const double *nat = P.st_nat + 3 * st, *cf = P.st_coef + 4 * st;
+template <class XA>
+__device__ inline void stack_eval(const XA &X, const int m7[7], const double nat[3], const double cf[4],
+                                  double fo[21]) {
   double v21[3], v34[3], v54[3], v56[3], v76[3], m[3], nn[3], fi[3], fl[3];
-  vsub(X, n, m7[1], m7[0], v21);
-  vsub(X, n, m7[2], m7[3], v34);
-  vsub(X, n, m7[4], m7[3], v54);
-  vsub(X, n, m7[4], m7[5], v56);
-  vsub(X, n, m7[6], m7[5], v76);
+  vsub(X, m7[1], m7[0], v21);
+  vsub(X, m7[2], m7[3], v34);
+  vsub(X, m7[4], m7[3], v54);
+  vsub(X, m7[4], m7[5], v56);
+  vsub(X, m7[6], m7[5], v76);
   double ediv = 1.0;
   double dist = sqrt(dot3(v21, v21));
   double dd = dist - nat[0];
@@ -162,14 +193,17 @@ __device__ inline void bonded_lane(const DevPtrs &P, const double *X, const doub
   t = t < ns ? t + nb + na : (t < ns + na ? t - ns + nb : t - ns - na);   // stacks, angles, bonds
   if (t < nb) {
     double fo[6];
-    bond_eval(P, X, b0 + t, fo);
+    const int b = b0 + t;
+    bond_eval(GlobalX{X, P.ntot}, P.bd_mp[2 * b], P.bd_mp[2 * b + 1], P.bd_nat[b], P.bd_coef[b], fo);
     put_slots(P, P.sb_bd, b0 + t, 2, fo);
     return;
   }
   t -= nb;
   if (t < na) {
     double fo[9];
-    angle_eval(P, X, a0 + t, fo);
+    const int a = a0 + t;
+    angle_eval(GlobalX{X, P.ntot}, P.ba_mp[3 * a], P.ba_mp[3 * a + 1], P.ba_mp[3 * a + 2], P.ba_nat[a], P.ba_coef[a],
+               fo);
     put_slots(P, P.sb_ba, a0 + t, 3, fo);
     return;
   }
@@ -177,7 +211,8 @@ __device__ inline void bonded_lane(const DevPtrs &P, const double *X, const doub
   if (t < ns) {
     const int st = s0 + t;
     double fo[21];
-    if (stack_on(P, X, PX, st)) stack_eval(P, X, st, fo);
+    if (stack_on(P, X, PX, st))
+      stack_eval(GlobalX{X, P.ntot}, P.st_mp + 7 * st, P.st_nat + 3 * st, P.st_coef + 4 * st, fo);
     else for (int k = 0; k < 21; ++k) fo[k] = 0.0;
     put_slots(P, P.sb_st, st, 7, fo);
   }
@@ -279,15 +314,13 @@ __device__ void tstack_eval(const DevPtrs &P, const DSys &s, const double *X, co
 // ------------------------------------------------------------------ hbond15
 // force_dtrna_hbond15.F90:91-353 (default branch).  Returns 1 and fills
 // fo[18], *ene when |r12 - r0| <= hb_cutoff_dist.
-__device__ int hbond_eval(const DevPtrs &P, const DSys &s, const double *X, const double *PX,
-                          int h, double fo[18], double *ene) {
-  const int n = P.ntot;
+template <class XA>
+__device__ inline int hbond_eval(const DSys &s, const XA &X, const XA &PX, const int m6[6], const double nat[6],
+                                 const double cf[7], double fo[18], double *ene) {
   const double MAXC = cos((double)(0.57f / 180.0f) * kPi);  // const_physical.F90:37-38
-  const int32_t *m6 = P.hb_mp + 6 * h;
-  const double *nat = P.hb_nat + 6 * h, *cf = P.hb_coef + 7 * h;
   double v12[3], v13[3], v53[3], v42[3], v46[3], fi[3], fk[3], fl[3];
-  if (s.periodic) { vsub(PX, n, m6[0], m6[1], v12); pbneighbor(s, v12); }
-  else vsub(X, n, m6[0], m6[1], v12);
+  if (s.periodic) { vsub(PX, m6[0], m6[1], v12); pbneighbor(s, v12); }
+  else vsub(X, m6[0], m6[1], v12);
   double d1212 = dot3(v12, v12), a12 = sqrt(d1212);
   double dd = a12 - nat[0];
   if (fabs(dd) > s.hb_cut) return 0;
@@ -297,10 +330,10 @@ __device__ int hbond_eval(const DevPtrs &P, const DSys &s, const double *X, cons
     fo[d] = fi[d]; fo[3 + d] = -fi[d];
   }
   for (int k = 6; k < 18; ++k) fo[k] = 0.0;
-  vsub(X, n, m6[0], m6[2], v13);
-  vsub(X, n, m6[4], m6[2], v53);
-  vsub(X, n, m6[3], m6[1], v42);
-  vsub(X, n, m6[3], m6[5], v46);
+  vsub(X, m6[0], m6[2], v13);
+  vsub(X, m6[4], m6[2], v53);
+  vsub(X, m6[3], m6[1], v42);
+  vsub(X, m6[3], m6[5], v46);
   if (s.periodic) { pbneighbor(s, v13); pbneighbor(s, v53); pbneighbor(s, v42); pbneighbor(s, v46); }
   double d1313 = dot3(v13, v13), d4242 = dot3(v42, v42);
   double a13 = sqrt(d1313), a42 = sqrt(d4242);
@@ -382,6 +415,12 @@ __device__ int hbond_eval(const DevPtrs &P, const DSys &s, const double *X, cons
   return 1;
 }
 
+__device__ inline int hbond_at(const DevPtrs &P, const DSys &s, const double *X, const double *PX, int h,
+                               double fo[18], double *ene) {
+  return hbond_eval(s, GlobalX{X, P.ntot}, GlobalX{PX, P.ntot}, P.hb_mp + 6 * h, P.hb_nat + 6 * h, P.hb_coef + 7 * h,
+                    fo, ene);
+}
+
 __device__ inline int site_count(const DevPtrs &P, int site) {
   return __hip_atomic_load(&P.site_cnt[site], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -406,42 +445,67 @@ __device__ inline bool site_in_excess(const DevPtrs &P, int site) {
   return site_count(P, site) - P.site_val[site] > 0;
 }
 
+// The hbond state the valence pass works on, in global memory: candidates q
+// and sites k are numbered within the system.
+struct GlobalHb {
+  const DevPtrs &P;
+  const DSys &s;
+  __device__ bool excess(int k) const { return site_in_excess(P, s.sitoff + k); }
+  __device__ bool formed(int q) const { return P.hb_inlist[s.hoff + q] && P.hb_status[s.hoff + q]; }
+  __device__ int site(int q, int k) const {
+    const int st = P.hb_site[6 * (s.hoff + q) + k];
+    return st < 0 ? -1 : st - s.sitoff;
+  }
+  __device__ double ene(int q) const { return P.hb_ene[s.hoff + q]; }
+  __device__ int seq(int i) const { return P.hb_seq[s.hoff + i]; }
+  __device__ void set_seq(int i, int q) const { P.hb_seq[s.hoff + i] = q; }
+  // lane 0: hbond q deleted
+  __device__ void drop(int q) const {
+    P.hb_status[s.hoff + q] = 0;
+    P.hb_ene[s.hoff + q] = 0.0;
+  }
+  __device__ void drop_site(int k) const { atomicSub(&P.site_cnt[s.sitoff + k], 1); }
+};
+
 // Valence-limit deletion of force_dtrna_hbond15.F90:373-510 for one system,
 // run by the whole wave (every lane calls it).  The scans are wave-wide:
 // sites in excess are counted and the pick-th one found by ballots over
 // chunks of 64 sites, and the listed, formed hbonds of the picked site are
 // gathered in list order by ballots over chunks of 64 candidates into the
-// system's scratch sequence (P.hb_seq, one entry per candidate, so any
-// length fits).  A sequence of at most 64 is moved into registers (lane i
-// holds element i) and the shuffle and the Metropolis choice run on every
-// lane alike; a longer one is shuffled and chosen from by lane 0 in the
-// scratch copy.  Either way the draws of the counter-based generator are
-// taken in the order of a serial pass, so that the result equals the
-// oracle's bit for bit.  Lane 0 applies each deletion; the fence after it
-// orders the next scan's reads.
-__device__ int hbond_valence_wave(const DevPtrs &P, const DSys &s, uint64_t step, int lane) {
+// system's scratch sequence (one entry per candidate, so any length fits).
+// A sequence of at most 64 is moved into registers (lane i holds element i);
+// a longer one is shuffled and chosen from by lane 0 in the scratch copy.
+// The generator is counter-based, so a deletion's draws (the site, one per
+// element for the shuffle, one per element but the first for the Metropolis
+// choice) are taken by the lanes at once, lane i draw i, and the choice tests
+// every remaining element against the current one together, taking the first
+// that is accepted: the draws and decisions of a serial pass, so that the
+// result equals the oracle's bit for bit, without a Philox evaluation and an
+// exponential per element in series.  Lane 0 applies each deletion; the fence
+// after it orders the next scan's reads.
+template <class Hb>
+__device__ inline int hbond_valence_wave(const DevPtrs &P, const DSys &s, uint64_t step, int lane, const Hb &hb) {
   const uint64_t below = (1ull << lane) - 1ull;
-  int32_t *seq = P.hb_seq + s.hoff;
   int ndel = 0;
   uint32_t draw = 0;
   for (int iter = 0; iter < (1 << 20); ++iter) {
     int nex = 0;
     for (int k0 = 0; k0 < s.nsite; k0 += kTile) {
       const int k = k0 + lane;
-      nex += __popcll(__ballot(k < s.nsite && site_in_excess(P, s.sitoff + k)));
+      nex += __popcll(__ballot(k < s.nsite && hb.excess(k)));
     }
     if (nex == 0) break;
-    double rnd = uniform01(P.seed, s.key, step, 0, draw++);
-    const int pick = (int)ceil(rnd * nex) - 1;  // rnd in (0,1): 0 <= pick < nex
+    const double u0 = uniform01(P.seed, s.key, step, 0, draw + (uint32_t)lane);
+    const int pick = (int)ceil(at_lane(u0, 0) * nex) - 1;  // uniform in (0,1): 0 <= pick < nex
     int site = -1;
     for (int k0 = 0, c = 0; k0 < s.nsite; k0 += kTile) {
       const int k = k0 + lane;
-      const bool ex = k < s.nsite && site_in_excess(P, s.sitoff + k);
+      const bool ex = k < s.nsite && hb.excess(k);
       const uint64_t b = __ballot(ex);
       const int n = __popcll(b);
       if (pick < c + n) {
         const uint64_t w = __ballot(ex && c + __popcll(b & below) == pick);
-        site = s.sitoff + k0 + __builtin_ctzll(w);
+        site = k0 + __builtin_ctzll(w);
         break;
       }
       c += n;
@@ -450,66 +514,68 @@ __device__ int hbond_valence_wave(const DevPtrs &P, const DSys &s, uint64_t step
     int nseq = 0;
     for (int q0 = 0; q0 < s.nhb; q0 += kTile) {
       const int q = q0 + lane;
-      const int h = s.hoff + q;
       bool m = false;
-      if (q < s.nhb && P.hb_inlist[h] && P.hb_status[h])
-        for (int k = 0; k < 6; ++k) m = m || P.hb_site[6 * h + k] == site;
+      if (q < s.nhb && hb.formed(q))
+        for (int k = 0; k < 6; ++k) m = m || hb.site(q, k) == site;
       const uint64_t b = __ballot(m);
-      if (m) seq[nseq + __popcll(b & below)] = h;
+      if (m) hb.set_seq(nseq + __popcll(b & below), q);
       nseq += __popcll(b);
     }
     if (nseq == 0) break;
     wave_sync();
     int del;
     if (nseq <= kTile) {
-      int myh = lane < nseq ? seq[lane] : -1;
+      // draws 1 .. nseq shuffle, nseq + 1 .. 2 nseq - 1 choose
+      const double u1 = 2 * nseq > kTile ? uniform01(P.seed, s.key, step, 0, draw + (uint32_t)(kTile + lane)) : 0.0;
+      int myh = lane < nseq ? hb.seq(lane) : -1;
       for (int i = 0; i < nseq; ++i) {
-        rnd = uniform01(P.seed, s.key, step, 0, draw++);
+        const double rnd = i + 1 < kTile ? at_lane(u0, i + 1) : at_lane(u1, i + 1 - kTile);
         const int isw = (int)ceil(rnd * nseq) - 1;  // 0 <= isw < nseq
-        const int a = __shfl(myh, i), c = __shfl(myh, isw);
+        const int a = __builtin_amdgcn_readlane(myh, i), c = __builtin_amdgcn_readlane(myh, isw);
         if (lane == i) myh = c;
         if (lane == isw) myh = a;
       }
-      const double myene = lane < nseq ? P.hb_ene[myh] : 0.0;
-      del = __shfl(myh, 0);
-      double edel = __shfl(myene, 0);
-      for (int i = 1; i < nseq; ++i) {
-        const int j = __shfl(myh, i);
-        const double ej = __shfl(myene, i);
-        const double ratio = exp((ej - edel) * s.beta_hb);
-        rnd = uniform01(P.seed, s.key, step, 0, draw++);
-        if (rnd < ratio) { del = j; edel = ej; }
+      const double myene = lane < nseq ? hb.ene(myh) : 0.0;
+      const int ir = nseq + lane;
+      const double r0 = __shfl(u0, ir & (kTile - 1)), r1 = __shfl(u1, ir & (kTile - 1));
+      const double myrnd = ir < kTile ? r0 : r1;
+      int at = 0;
+      for (;;) {
+        const double ratio = exp((myene - at_lane(myene, at)) * s.beta_hb);
+        const uint64_t b = __ballot(lane > at && lane < nseq && myrnd < ratio);
+        if (b == 0) break;
+        at = __builtin_ctzll(b);
       }
+      del = __builtin_amdgcn_readlane(myh, at);
     } else {
       del = -1;
       if (lane == 0) {
-        uint32_t d = draw;
+        uint32_t d = draw + 1u;
         for (int i = 0; i < nseq; ++i) {
           const double r = uniform01(P.seed, s.key, step, 0, d++);
           const int isw = (int)ceil(r * nseq) - 1;
-          const int a = seq[i];
-          seq[i] = seq[isw];
-          seq[isw] = a;
+          const int a = hb.seq(i);
+          hb.set_seq(i, hb.seq(isw));
+          hb.set_seq(isw, a);
         }
-        del = seq[0];
-        double edel = P.hb_ene[del];
+        del = hb.seq(0);
+        double edel = hb.ene(del);
         for (int i = 1; i < nseq; ++i) {
-          const int j = seq[i];
-          const double ej = P.hb_ene[j];
+          const int j = hb.seq(i);
+          const double ej = hb.ene(j);
           const double ratio = exp((ej - edel) * s.beta_hb);
           if (uniform01(P.seed, s.key, step, 0, d++) < ratio) { del = j; edel = ej; }
         }
       }
       del = __shfl(del, 0);
-      draw += 2u * (uint32_t)nseq - 1u;
     }
+    draw += 2u * (uint32_t)nseq;
     if (lane == 0) {
-      P.hb_status[del] = 0;
-      P.hb_ene[del] = 0.0;
+      hb.drop(del);
       // excess -= 1 where positive; count kept as valence + excess
       for (int k = 0; k < 6; ++k) {
-        const int st = P.hb_site[6 * del + k];
-        if (st >= 0 && site_in_excess(P, st)) atomicSub(&P.site_cnt[st], 1);
+        const int st = hb.site(del, k);
+        if (st >= 0 && hb.excess(st)) hb.drop_site(st);
       }
     }
     ++ndel;
@@ -525,7 +591,7 @@ __device__ inline void hbond_lane(const DevPtrs &P, const double *X, const doubl
   const DSys &s = P.sys[P.hb_sys[h]];
   int st = 0;
   double e = 0.0, fo[18];
-  if (P.hb_inlist[h]) st = hbond_eval(P, s, X, PX, h, fo, &e);
+  if (P.hb_inlist[h]) st = hbond_at(P, s, X, PX, h, fo, &e);
   if (!st) for (int q = 0; q < 18; ++q) fo[q] = 0.0;
   P.hb_status[h] = (uint8_t)st;
   P.hb_ene[h] = e;
@@ -557,7 +623,7 @@ __device__ void terms_wave(const DevPtrs &P, const double *X, const double *PX, 
     int h = s.hoff + k;
     int st = 0;
     double e = 0.0, fo[18];
-    if (P.hb_inlist[h]) st = hbond_eval(P, s, X, PX, h, fo, &e);
+    if (P.hb_inlist[h]) st = hbond_at(P, s, X, PX, h, fo, &e);
     P.hb_status[h] = (uint8_t)st;
     P.hb_ene[h] = e;
     if (st) {
@@ -573,7 +639,7 @@ __device__ void terms_wave(const DevPtrs &P, const double *X, const double *PX, 
   for (int k = lane; k < s.nsite; k += nt)
     if (site_count(P, s.sitoff + k) - P.site_val[s.sitoff + k] > 0) any = 1;
   if (__any(any)) {
-    const int nd = hbond_valence_wave(P, s, step, lane);
+    const int nd = hbond_valence_wave(P, s, step, lane, GlobalHb{P, s});
     if (nd && lane == 0) atomicAdd(&P.counters[2], (unsigned long long)nd);
   }
   wave_sync();
@@ -615,12 +681,9 @@ __device__ inline float ele_dv(const DSys &s, float qq, float d2, unsigned &ncla
   }
 }
 
-// Staging of the J chunk of each wave's chunk pair.
-// The J chunk of each wave's chunk pair: ele_pair_task uses the first 64
-// entries of each array, ele_pair_unrolled keeps the chunk twice over (so
-// that its reads need no wrap-around).  Arrays, not records, so that the 64
-// lanes' reads of consecutive entries fall in distinct LDS banks.
-struct EleWave { double x[2 * kTile], y[2 * kTile], z[2 * kTile]; float q[2 * kTile]; };
+// Staging of the J chunk of each wave's chunk pair: ele_pair_task uses the
+// first 64 entries of each array, ele_pair_unrolled keeps the chunk twice over
+// (so that its reads need no wrap-around).
 struct EleLds {
   EleWave w[kWaves];
 };
@@ -767,48 +830,24 @@ __device__ inline void ele_pair_task(const DevPtrs &P, const DSys &s, const doub
 // are turned into the same order once (bit k of mr is the pair of step k); a
 // pair that is not on gets charge product 0, so its force is exactly zero
 // and adds nothing, with no branch; the DE_MAX clamps are counted per wave.
-template <int FORM>
-__device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const double *Y, int I, int J, int dir,
-                                         EleWave *JE) {
-  // the chunk pair is the wave's: uniform, so the step loops below are scalar
-  I = __builtin_amdgcn_readfirstlane(I);
-  J = __builtin_amdgcn_readfirstlane(J);
+// Absent charges sit far apart (kFar, charge 0; -kFar on the I side): their
+// pairs stay finite and off.
+constexpr double kFar = 1e15;
+
+// Where lane l's charge of a chunk is staged (and again 64 entries on).
+__device__ inline int stage_at(int lane, int dir) { return dir == 1 ? lane : kTile - 1 - lane; }
+
+// The pairs of one chunk pair from registers (chunk I: position, charge
+// product factor, list bits m64 of its row against chunk J, nj charges) and
+// the staged chunk J: sums on chunk I in F, on chunk J in G (the diagonal
+// chunk's are added to F).  Returns the clamps (the same on every lane).
+template <int FORM, bool DPP>
+__device__ inline uint32_t ele_pair_sums(const DSys &s, bool diag, int nj, bool valid, uint64_t m64, double xi0,
+                                         double xi1, double xi2, float qiC, int dir, const EleWave *JE, double F[3],
+                                         double G[3]) {
   const int lane = threadIdx.x & (kTile - 1);
-  const int c = dir == 1 ? lane : kTile - 1 - lane;
-  const int n = P.ntot;
-  const int qi = I * kTile + lane;
-  const bool valid = qi < s.nq;
-  // absent charges sit far apart (+-1e15, charge 0): their pairs stay
-  // finite and off
-  constexpr double kFar = 1e15;
-  double xi0 = -kFar, xi1 = -kFar, xi2 = -kFar, chi = 0.0;
-  if (valid) {
-    const int gi = P.qbead[s.qoff + qi];
-    xi0 = Y[gi]; xi1 = Y[n + gi]; xi2 = Y[2 * n + gi];
-    chi = P.charge[gi];
-  }
-  const int jt = J * kTile;
-  {
-    const bool vj = jt + lane < s.nq;
-    const int gj = vj ? P.qbead[s.qoff + jt + lane] : 0;
-    const double x = vj ? Y[gj] : kFar, y = vj ? Y[n + gj] : kFar, z = vj ? Y[2 * n + gj] : kFar;
-    const float q = vj ? (float)P.charge[gj] : 0.0f;
-    JE->x[c] = x; JE->y[c] = y; JE->z[c] = z; JE->q[c] = q;
-    JE->x[c + kTile] = x; JE->y[c + kTile] = y; JE->z[c + kTile] = z; JE->q[c + kTile] = q;
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const float qiC = (float)(chi * s.ele_coef);
+  const int c = stage_at(lane, dir);
   const double cut2 = FORM == 0 ? s.dh_cut2 : s.cl_cut2;
-  const uint32_t *row = P.qmask + s.moff + (int64_t)(valid ? qi : 0) * s.mwords;
-  uint64_t m64 = 0;
-  if (valid) {
-    const int wb = jt >> 5;
-    m64 = row[wb];
-    if (wb + 1 < s.mwords) m64 |= (uint64_t)row[wb + 1] << 32;
-  }
-  const bool diag = I == J;
   // bit k of mr: the pair of step k, j = (lane + dir k) mod 64
   uint64_t mr = __builtin_rotateright64(dir == 1 ? m64 : __builtin_bitreverse64(m64), (uint64_t)c);
   if (diag && lane >= 32) mr &= ~(1ull << 32);   // step 32 of the diagonal chunk: lanes < 32 only
@@ -845,12 +884,11 @@ __device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const 
       const double dd = (double)dv;
       F0 -= dd * v0; F1 -= dd * v1; F2 -= dd * v2;
       G0 += dd * v0; G1 += dd * v1; G2 += dd * v2;
-      G0 = wave_rot(G0); G1 = wave_rot(G1); G2 = wave_rot(G2);
+      G0 = rot_next<DPP>(G0); G1 = rot_next<DPP>(G1); G2 = rot_next<DPP>(G2);
     }
   };
   if (__any(m64 != 0)) {
     // every valid j listed for every valid lane (off-diagonal chunk pairs)
-    const int nj = s.nq - jt < kTile ? s.nq - jt : kTile;
     const uint64_t vjm = nj >= kTile ? ~0ull : (1ull << nj) - 1ull;
     const bool all_listed = !diag && __all(!valid || (m64 & vjm) == vjm);
     if (all_listed) {
@@ -862,14 +900,61 @@ __device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const 
       for (int k0 = k_begin; k0 < k_end; k0 += 8) steps8(k0, (uint32_t)(mr >> k0), std::true_type{});
     }
   }
-  double *pp = P.pp + s.pp_off + ele_task_index(I, J, s.nqt) * (6 * kTile);
   if (diag) {
     const int src = (lane - dir * 33) & (kTile - 1);
     F0 += __shfl(G0, src); F1 += __shfl(G1, src); F2 += __shfl(G2, src);
-  } else {
-    pp[3 * kTile + lane] = G0; pp[4 * kTile + lane] = G1; pp[5 * kTile + lane] = G2;
   }
-  pp[lane] = F0; pp[kTile + lane] = F1; pp[2 * kTile + lane] = F2;
+  F[0] = F0; F[1] = F1; F[2] = F2;
+  G[0] = G0; G[1] = G1; G[2] = G2;
+  return nclamp;
+}
+
+template <int FORM>
+__device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const double *Y, int I, int J, int dir,
+                                         EleWave *JE) {
+  // the chunk pair is the wave's: uniform, so the step loops are scalar
+  I = __builtin_amdgcn_readfirstlane(I);
+  J = __builtin_amdgcn_readfirstlane(J);
+  const int lane = threadIdx.x & (kTile - 1);
+  const int c = stage_at(lane, dir);
+  const int n = P.ntot;
+  const int qi = I * kTile + lane;
+  const bool valid = qi < s.nq;
+  double xi0 = -kFar, xi1 = -kFar, xi2 = -kFar, chi = 0.0;
+  if (valid) {
+    const int gi = P.qbead[s.qoff + qi];
+    xi0 = Y[gi]; xi1 = Y[n + gi]; xi2 = Y[2 * n + gi];
+    chi = P.charge[gi];
+  }
+  const int jt = J * kTile;
+  {
+    const bool vj = jt + lane < s.nq;
+    const int gj = vj ? P.qbead[s.qoff + jt + lane] : 0;
+    const double x = vj ? Y[gj] : kFar, y = vj ? Y[n + gj] : kFar, z = vj ? Y[2 * n + gj] : kFar;
+    const float q = vj ? (float)P.charge[gj] : 0.0f;
+    JE->x[c] = x; JE->y[c] = y; JE->z[c] = z; JE->q[c] = q;
+    JE->x[c + kTile] = x; JE->y[c + kTile] = y; JE->z[c + kTile] = z; JE->q[c + kTile] = q;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const float qiC = (float)(chi * s.ele_coef);
+  const uint32_t *row = P.qmask + s.moff + (int64_t)(valid ? qi : 0) * s.mwords;
+  uint64_t m64 = 0;
+  if (valid) {
+    const int wb = jt >> 5;
+    m64 = row[wb];
+    if (wb + 1 < s.mwords) m64 |= (uint64_t)row[wb + 1] << 32;
+  }
+  const bool diag = I == J;
+  const int nj = s.nq - jt < kTile ? s.nq - jt : kTile;
+  double F[3], G[3];
+  const uint32_t nclamp = ele_pair_sums<FORM, true>(s, diag, nj, valid, m64, xi0, xi1, xi2, qiC, dir, JE, F, G);
+  double *pp = P.pp + s.pp_off + ele_task_index(I, J, s.nqt) * (6 * kTile);
+  if (!diag) {
+    pp[3 * kTile + lane] = G[0]; pp[4 * kTile + lane] = G[1]; pp[5 * kTile + lane] = G[2];
+  }
+  pp[lane] = F[0]; pp[kTile + lane] = F[1]; pp[2 * kTile + lane] = F[2];
   if (lane == 0 && nclamp) atomicAdd(&P.counters[1], (unsigned long long)nclamp);
 }
 
@@ -1084,19 +1169,30 @@ __device__ inline void load_state(const DevPtrs &P, const DSys &s, int g, const 
   }
 }
 
+// One component: force, noise, velocity and acceleration (both updated);
+// returns the displacement of the next position update.
+__device__ inline double langevin_update(const double r[4], double rcm, double tstep2, int mode, double F, double gs,
+                                         double &v, double &a) {
+#pragma clang fp contract(off)
+  double af = F * rcm + r[0] * gs;
+  double vv = v;
+  const double a0 = a;
+  if (mode == 3) af = a0;
+  if (mode == 1) vv = r[1] * vv + r[2] * (a0 + af);
+  v = vv;
+  a = af;
+  return r[3] * vv + tstep2 * af;
+}
+
 __device__ inline void integrate(const DevPtrs &P, const DSys &s, int g, const BeadState &b, const double gs[3],
                                  const double F[3], double *XN, double *PXN, int mode, double dxo[3]) {
 #pragma clang fp contract(off)
   const int n = P.ntot;
   for (int d = 0; d < 3; ++d) {
-    double af = F[d] * b.rcm + b.r[0] * gs[d];
-    double vv = b.v[d];
-    const double a0 = b.a[d];
-    if (mode == 3) af = a0;
-    if (mode == 1) vv = b.r[1] * vv + b.r[2] * (a0 + af);
-    P.v[d * n + g] = vv;
-    P.a[d * n + g] = af;
-    double dx = b.r[3] * vv + P.tstep2 * af;
+    double v = b.v[d], a = b.a[d];
+    const double dx = langevin_update(b.r, b.rcm, P.tstep2, mode, F[d], gs[d], v, a);
+    P.v[d * n + g] = v;
+    P.a[d * n + g] = a;
     dxo[d] = dx;
     XN[d * n + g] = b.x[d] + dx;
     if (s.periodic) PXN[d * n + g] = b.px[d] + dx;
@@ -1129,21 +1225,36 @@ __device__ inline void tile_boxes(double p0, double p1, double p2, BBox *tile, B
   }
 }
 
-// Two waves share a tile of 64 beads: wave 0 sums each bead's bonded slots,
-// wave 1 draws its Langevin noise and adds its electrostatic sums, and the
-// two waves take alternate groups of four excluded-volume neighbours; the
-// partial sums are added in wave order (a fixed order: results are bitwise
-// reproducible), then wave 0 integrates.
+// The force on a bead is (S + Q) + ((E0 + E2) + (E1 + E3)): its bonded slots
+// S in incidence order, its electrostatic sums Q (ele_sums) and its
+// excluded-volume neighbours in groups of four, group k of the list in E of
+// k mod 4 -- a fixed order that every pass keeps (k_main, k_window), however
+// it shares the parts out, so results are bitwise reproducible.
 __device__ inline void exv_entries(const DevPtrs &P, int g, int m0, int cnt, uint32_t e[4]) {
   // entries past cnt re-read entry cnt - 1 (m0 < cnt) and are skipped
 #pragma unroll
   for (int u = 0; u < 4; ++u) e[u] = P.nb[(size_t)min(m0 + u, cnt - 1) * P.ntot + g];
 }
 
-// e: the group's list entries (exv_entries); the entries of the wave's next
-// group (m0 + 8) are loaded into en while this group's neighbours are read
+// One neighbour within its contact distance (force_exv_dt15.F90:53-115): the
+// mWCA factor (a/dr)^14 amplifies rounding 14-fold, so this formula runs in
+// FP64 (only pairs within D_ij reach it).  Returns whether it was clamped.
+__device__ inline bool exv_contact(double a, double dij, double coef, const double v[3], double d2, double F[3]) {
+  const double dist = sqrt(d2);
+  const double dr = dist + a - dij;
+  const double id = 1.0 / dr, ar = a * id, r2 = ar * ar, r6 = r2 * r2 * r2, r12 = r6 * r6;
+  double dv = fabs(12.0 * coef * (r12 - r6) * id / dist);
+  const bool cl = dv > kDeMax;
+  if (cl) dv = kDeMax;
+  F[0] -= dv * v[0]; F[1] -= dv * v[1]; F[2] -= dv * v[2];
+  return cl;
+}
+
+// The wave's group of four neighbours at m0, added to E[hi]; e: the group's
+// list entries (exv_entries); the entries of the wave's next group (m0 + 8)
+// are loaded into en while this group's neighbours are read
 __device__ inline void exv_group(const DevPtrs &P, const DSys &s, const double *Y, int g, int m0, int cnt,
-                                 double xi0, double xi1, double xi2, const SpPair *tab, double F[3],
+                                 double xi0, double xi1, double xi2, const SpPair *tab, double (&E)[2][3], bool hi,
                                  unsigned &nclamp, const uint32_t e[4], uint32_t en[4]) {
   const int n = P.ntot;
   // every load of the group is issued before the arithmetic
@@ -1160,36 +1271,36 @@ __device__ inline void exv_group(const DevPtrs &P, const DSys &s, const double *
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     if (m0 + u >= cnt) continue;
-    double v0 = y0[u] - xi0, v1 = y1[u] - xi1, v2 = y2[u] - xi2;
+    double v[3] = {y0[u] - xi0, y1[u] - xi1, y2[u] - xi2};
     if (s.periodic) {
       const int code = (int)(e[u] >> kMirrorShift);
-      v0 += mirror_shift(s, code, 0); v1 += mirror_shift(s, code, 1); v2 += mirror_shift(s, code, 2);
+      for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, code, d);
     }
     const SpPair t = tp[u];
-    const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+    const double d2 = dot3(v, v);
     if (d2 > t.dij2) continue;
-    // contact pair: the mWCA factor (a/dr)^14 amplifies rounding 14-fold, so
-    // this formula runs in FP64 (only pairs within D_ij reach it)
-    const double dist = sqrt(d2);
-    const double dr = dist + a - t.dij;
-    const double id = 1.0 / dr, ar = a * id, r2 = ar * ar, r6 = r2 * r2 * r2, r12 = r6 * r6;
-    double dv = fabs(12.0 * t.coef * (r12 - r6) * id / dist);
-    if (dv > kDeMax) { dv = kDeMax; if (g < (int)(e[u] & kIdxMask)) ++nclamp; }
-    F[0] -= dv * v0; F[1] -= dv * v1; F[2] -= dv * v2;
+    const bool cl = hi ? exv_contact(a, t.dij, t.coef, v, d2, E[1]) : exv_contact(a, t.dij, t.coef, v, d2, E[0]);
+    if (cl && g < (int)(e[u] & kIdxMask)) ++nclamp;
   }
 }
 
-// The two largest squared displacements of a bead tile since the last
-// rebuild (wave merge of top-2 pairs; -1 marks lanes without a bead), for
-// the rebuild decision of the next step (system_trigger).
-__device__ inline void tile_top2(const DevPtrs &P, int tile, double d2) {
-  double a = d2, b = -1.0;
+// The two largest values over the wave (merge of top-2 pairs).
+__device__ inline void top2_wave(double d2, double &a, double &b) {
+  a = d2; b = -1.0;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     const double a2 = __shfl_xor(a, off), b2 = __shfl_xor(b, off);
     const double hi = fmax(a, a2), lo = fmax(fmin(a, a2), fmax(b, b2));
     a = hi; b = lo;
   }
+}
+
+// The two largest squared displacements of a bead tile since the last
+// rebuild (-1 marks lanes without a bead), for the rebuild decision of the
+// next step (system_trigger).
+__device__ inline void tile_top2(const DevPtrs &P, int tile, double d2) {
+  double a, b;
+  top2_wave(d2, a, b);
   if ((threadIdx.x & (kTile - 1)) == 0) { P.ttop[2 * tile] = a; P.ttop[2 * tile + 1] = b; }
 }
 
@@ -1244,11 +1355,12 @@ __device__ inline uint64_t noise_step(const DevPtrs &P, const DSys &s, int32_t t
 // with the noise gs; returns the squared displacement since the last
 // rebuild before this step's update (and accumulates the update) when
 // rebuilds are displacement-triggered.
-__device__ inline double main_tail(const DevPtrs &P, const DSys &s, int g, double F[3], double (*red)[2][kTile],
-                                   const BeadState &b, const double gs[3], int lane, double *XN, double *PXN,
+__device__ inline double main_tail(const DevPtrs &P, const DSys &s, int g, const double S[3], const double E02[3],
+                                   double (*red)[2][kTile], const BeadState &b, const double gs[3], int lane, double *XN, double *PXN,
                                    int mode) {
   const int n = P.ntot;
-  for (int d = 0; d < 3; ++d) F[d] = red[d][0][lane] + red[d][1][lane];
+  double F[3];
+  for (int d = 0; d < 3; ++d) F[d] = (S[d] + red[d][0][lane]) + (E02[d] + red[d][1][lane]);
   P.f[g] = F[0]; P.f[n + g] = F[1]; P.f[2 * n + g] = F[2];
   if (mode == 0) return -1.0;
   double dx[3];
@@ -1278,7 +1390,9 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
   const bool valid = li < s.nmp;
   const int g = s.off + (valid ? li : 0);
   const int n = P.ntot;
-  double F[3] = {0.0, 0.0, 0.0};
+  // wave 0: the bonded slots S, wave 1: the electrostatic sums Q, in F; both:
+  // their excluded-volume groups (k mod 4 = w and w + 2) in E
+  double F[3] = {0.0, 0.0, 0.0}, E[2][3] = {};
   if (valid) {
     if (w == 1) {
       // the Langevin noise of the bead (wave 0 integrates after the
@@ -1328,13 +1442,16 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
     uint32_t e[4] = {0u, 0u, 0u, 0u}, en[4] = {0u, 0u, 0u, 0u};
     if (4 * w < cnt) exv_entries(P, g, 4 * w, cnt, e);
     for (int m0 = 4 * w; m0 < cnt; m0 += 8) {
-      exv_group(P, s, Y, g, m0, cnt, xi0, xi1, xi2, tab, F, nclamp, e, en);
+      exv_group(P, s, Y, g, m0, cnt, xi0, xi1, xi2, tab, E, (m0 & 8) != 0, nclamp, e, en);
 #pragma unroll
       for (int u = 0; u < 4; ++u) e[u] = en[u];
     }
     if (nclamp) atomicAdd(&P.counters[0], (unsigned long long)nclamp);
   }
-  for (int d = 0; d < 3; ++d) red[d][w][lane] = F[d];
+  double Ew[3];   // wave 0: E0 + E2, wave 1: E1 + E3
+  for (int d = 0; d < 3; ++d) Ew[d] = E[0][d] + E[1][d];
+  if (w == 1)
+    for (int d = 0; d < 3; ++d) { red[d][0][lane] = F[d]; red[d][1][lane] = Ew[d]; }
   BeadState bs;
   if (w == 0 && valid && mode != 0) load_state(P, s, g, X, PX, bs);
   __syncthreads();
@@ -1342,19 +1459,20 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
   double d2 = -1.0;   // squared displacement since the last rebuild, before this update
   if (valid) {
     const double gs[3] = {gsh[0][lane], gsh[1][lane], gsh[2][lane]};
-    d2 = main_tail(P, s, g, F, red, bs, gs, lane, XN, PXN, mode);
+    d2 = main_tail(P, s, g, F, Ew, red, bs, gs, lane, XN, PXN, mode);
   }
   if (P.dyn && mode != 0) {
     const int it = s.bt0 + tl.start / kTile;
     tile_top2(P, it, d2);
-    // the tile's boxes at the new positions, which a displacement-triggered
-    // rebuild of the next step culls by (k_lists then runs without k_prep;
-    // lanes past the last bead take the tile's first bead, as bbox_tile)
+    // the tile's boxes at this step's positions, which a displacement-triggered
+    // rebuild before the next step builds its lists from and culls by (k_lists
+    // then runs without k_prep; lanes past the last bead take the tile's first
+    // bead, as bbox_tile)
     if (!s.periodic) {
       double p[3] = {0.0, 0.0, 0.0};
       if (valid) {
 #pragma unroll
-        for (int d = 0; d < 3; ++d) p[d] = XN[d * n + g];   // this lane's own store
+        for (int d = 0; d < 3; ++d) p[d] = bs.x[d];
       }
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
@@ -1463,6 +1581,26 @@ __device__ inline double point_box_d2(const double p[3], const BBox &b) {
   return s2;
 }
 
+// The candidate pair (li, lj2) of a non-periodic system at squared distance
+// d2, every test evaluated and combined (no branch per test): the unit-pair
+// radius of neighbor_list.F90 and the exclusions of neighbor_assign.F90
+// (exv_keep, by selects).  tcj: type | class << 8 of bead lj2.
+template <bool ONE_UNIT>
+__device__ inline bool exv_listed(const DSys &s, double d2, int li, int ui, int ti, int ci, int lj2, int uj, int tcj,
+                                  const double *rl2) {
+  const bool own_lo = li < lj2;
+  const int ulo = own_lo ? ui : uj, uhi = own_lo ? uj : ui;
+  const double r2 = ONE_UNIT ? s.rl2max : rl2[ulo * s.nunit + uhi];
+  const int tlo = own_lo ? ti : (tcj & 0xFF), clo = own_lo ? ci : (tcj >> 8);
+  const int lo = own_lo ? li : lj2, hi = own_lo ? lj2 : li;
+  int sep = -1;
+  sep = tlo == 2 ? s.nsep[0] : sep;
+  sep = tlo == 4 ? s.nsep[1] : sep;
+  sep = tlo == 3 ? s.nsep[2] : sep;
+  const bool keep = (ulo != uhi) | (clo != 2) | ((sep >= 0) & (hi >= lo + sep));
+  return (lj2 != li) & (d2 < s.rl2max) & (d2 < r2) & keep;
+}
+
 // One wave per bead tile sweeps the system's bead tiles in order; tiles and
 // 16-bead groups whose boxes no bead of the tile can reach within the
 // largest list radius are skipped.  The tile boxes are tested 64 at a time
@@ -1548,20 +1686,9 @@ __device__ inline void list_exv_tile_t(const DevPtrs &P, const DSys &s, const do
             if (k >= q1) continue;   // (the same for every lane)
             const int lj2 = jt + k;
             const double d2 = sq3_separate(sx[k] - xi[0], sy[k] - xi[1], sz[k] - xi[2]);
-            const bool own_lo = li < lj2;
             // one unit: its radius is rl2max and both beads are in it
-            const int uj = ONE_UNIT ? ui : su[k], tcj = stc[k];
-            const int ulo = own_lo ? ui : uj, uhi = own_lo ? uj : ui;
-            const double r2 = ONE_UNIT ? s.rl2max
-                                       : (RL2_LDS ? L.rl2[ulo * s.nunit + uhi] : P.rl2[s.uoff + ulo * s.nunit + uhi]);
-            const int tlo = own_lo ? ti : (tcj & 0xFF), clo = own_lo ? ci : (tcj >> 8);
-            const int lo = own_lo ? li : lj2, hi = own_lo ? lj2 : li;
-            int sep = -1;   // exv_keep's separation by the lower bead's type, as selects
-            sep = tlo == 2 ? s.nsep[0] : sep;
-            sep = tlo == 4 ? s.nsep[1] : sep;
-            sep = tlo == 3 ? s.nsep[2] : sep;
-            const bool keep = (ulo != uhi) | (clo != 2) | ((sep >= 0) & (hi >= lo + sep));
-            if ((lj2 != li) & (d2 < s.rl2max) & (d2 < r2) & keep) {
+            if (exv_listed<ONE_UNIT>(s, d2, li, ui, ti, ci, lj2, ONE_UNIT ? ui : su[k], stc[k],
+                                     RL2_LDS ? L.rl2 : P.rl2 + s.uoff)) {
               if (cnt < P.nb_cap) P.nb[(size_t)cnt * n + g] = (uint32_t)(s.off + lj2);
               ++cnt;
             }
@@ -1667,23 +1794,22 @@ __device__ inline void list_ele_tile(const DevPtrs &P, const DSys &s, const doub
   }
 }
 
-// hb candidate list (neighbor_list_hb.F90:59-78; radius mloop_dtrna.F90:149)
-__device__ inline void list_hb_entry(const DevPtrs &P, const DSys &s, const double *X, const double *PX, int h) {
+// hb candidate list (neighbor_list_hb.F90:59-78; radius mloop_dtrna.F90:149):
+// whether the bases at (wrapped) difference v are listed
+__device__ inline bool hb_listed(const DSys &s, const double v[3], double nat0) {
 #pragma clang fp contract(off)
-  const int n = P.ntot;
-  int a = P.hb_mp[6 * h], b = P.hb_mp[6 * h + 1];
-  double v[3];
-  if (s.periodic) {
-    v[0] = __dadd_rn(PX[a], -PX[b]); v[1] = __dadd_rn(PX[n + a], -PX[n + b]); v[2] = __dadd_rn(PX[2 * n + a], -PX[2 * n + b]);
-    pbneighbor(s, v);
-  } else {
-    v[0] = __dadd_rn(X[a], -X[b]); v[1] = __dadd_rn(X[n + a], -X[n + b]); v[2] = __dadd_rn(X[2 * n + a], -X[2 * n + b]);
-  }
-  double d2 = sq3_exact(v[0], v[1], v[2]);
-  double r = __dadd_rn(__dadd_rn(P.hb_nat[6 * h], s.hb_cut), s.margin);
-  P.hb_inlist[h] = (uint8_t)(d2 < __dmul_rn(r, r));
+  const double d2 = sq3_exact(v[0], v[1], v[2]);
+  const double r = __dadd_rn(__dadd_rn(nat0, s.hb_cut), s.margin);
+  return d2 < __dmul_rn(r, r);
 }
-
+__device__ inline void list_hb_entry(const DevPtrs &P, const DSys &s, const double *X, const double *PX, int h) {
+  const int n = P.ntot;
+  const int a = P.hb_mp[6 * h], b = P.hb_mp[6 * h + 1];
+  const double *Y = s.periodic ? PX : X;
+  double v[3] = {__dadd_rn(Y[a], -Y[b]), __dadd_rn(Y[n + a], -Y[n + b]), __dadd_rn(Y[2 * n + a], -Y[2 * n + b])};
+  if (s.periodic) pbneighbor(s, v);
+  P.hb_inlist[h] = (uint8_t)hb_listed(s, v, P.hb_nat[6 * h]);
+}
 
 // ------------------------------------------------------------------ lists by tile pairs
 // Periodic systems (no box culling, so one wave per tile would sweep every
@@ -1975,6 +2101,594 @@ __global__ __launch_bounds__(kTile) void k_lists(DevPtrs P, const double *X, con
   list_hb_entry(P, P.sys[P.hb_sys[h]], X, PX, h);
 }
 
+// ------------------------------------------------------------------ windows of steps
+// Steps of small systems without leaving the workgroup: one workgroup takes
+// one system through n Langevin steps with its list rebuilds, its
+// coordinates, slot forces, pair sums, term parameters, incidence and
+// neighbour lists in LDS (win_layout), velocities and accelerations in the
+// registers of one thread per bead.
+// Bound: a step of a 64-nt hairpin is some 8,000 wave instructions, most of
+// them FP64, on the four SIMDs of one CU; its longest chain is the 32
+// dependent pair steps of a charge chunk.  As two launches per step (k_force,
+// k_main) and three per rebuild every hand-over went through L2: 17.6 us a
+// step for that hairpin against 11.4 here, 64 of them 18.1 against 12.4.
+// Per step: (1) the terms as tasks of one wave each, longest first, taken
+// from a counter in LDS (chunk pairs of charges, 64 hbonds, 64 stacks, the
+// noise of 64 beads, half the neighbour groups of 64 beads, 64 angles, 64
+// bonds); (2) after a barrier, each bead's thread sums them, integrates, and
+// stages the next position where the next step's tasks read it.  Systems with
+// valence-limited hbonds take the hbonds first and run the valence pass (one
+// wave) beside the remaining tasks.
+// Every term, list and sum is that of the per-step passes, in their order, so
+// results do not depend on which of them ran.
+//
+// cu: the buffer of the current positions at *stepbase; phase: steps since
+// the last fixed rebuild was due; rebuild: the interval, 0 for the
+// displacement trigger.  A rebuild that overflows the list capacity raises
+// TIS_CNT_NB_OVERFLOW and the system stops before that step; the others
+// complete the launch, and win_at keeps how far each system came, so the
+// launch can be repeated when the capacity has grown.
+
+// The hbond state of the valence pass in LDS.
+struct LocalHb {
+  double *e;
+  int32_t *cnt;
+  const int32_t *val;
+  const uint16_t *hbsite;   // 0xFFFF: none
+  uint16_t *sq;
+  uint8_t *stat;
+  float *slot;              // the hbonds' slot forces
+  __device__ bool excess(int k) const { return *(volatile int32_t *)&cnt[k] - val[k] > 0; }
+  __device__ bool formed(int q) const { return *(volatile uint8_t *)&stat[q] != 0; }
+  __device__ int site(int q, int k) const {
+    const int st = hbsite[6 * q + k];
+    return st == 0xFFFF ? -1 : st;
+  }
+  __device__ double ene(int q) const { return e[q]; }
+  __device__ int seq(int i) const { return sq[i]; }
+  __device__ void set_seq(int i, int q) const { sq[i] = (uint16_t)q; }
+  __device__ void drop(int q) const {
+    stat[q] = 0;
+    e[q] = 0.0;
+    for (int k = 0; k < 18; ++k) slot[18 * q + k] = 0.0f;
+  }
+  __device__ void drop_site(int k) const { *(volatile int32_t *)&cnt[k] = cnt[k] - 1; }
+};
+
+// the next task of the workgroup's counter, the same for the whole wave
+__device__ inline int take_task(int *next) {
+  int k = 0;
+  if ((threadIdx.x & (kTile - 1)) == 0) k = atomicAdd(next, 1);
+  return __builtin_amdgcn_readfirstlane(k);
+}
+
+// (I, J), I <= J, of chunk pair k of nqt chunks
+__device__ inline void chunk_pair(int k, int nqt, int &I, int &J) {
+  int i = 0, first = 0;
+  while (k >= first + (nqt - i)) { first += nqt - i; ++i; }
+  I = i;
+  J = i + k - first;
+}
+
+__global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_window(
+    DevPtrs P, const int32_t *wsys, int rows, int cu, int n, int phase, int rebuild) {
+  extern __shared__ __align__(16) char lds[];
+  constexpr int T = kWinThreads, W = T / kTile;
+  __shared__ int next[3];
+  __shared__ unsigned over;
+  __shared__ double top[W][2];
+  if (run_stopped(P)) return;
+  const int isys = wsys[blockIdx.x];
+  const DSys s = P.sys[isys];
+  const uint64_t base = *P.stepbase;
+  const int ce = cu ^ (n & 1);
+  int from = 0, cb = cu;
+  {
+    const uint64_t at = P.win_at[isys];
+    if ((at >> 1) > base) { from = (int)min((at >> 1) - base, (uint64_t)n); cb = (int)(at & 1); }
+  }
+  if (from == n && cb == ce) return;
+  const WinLds L = win_layout(s, rows);
+  const int tid = (int)threadIdx.x, lane = tid & (kTile - 1), w = tid / kTile, N = P.ntot, nb = s.nmp;
+  double *x = (double *)(lds + L.x), *e = (double *)(lds + L.e), *gn = (double *)(lds + L.g),
+         *pp = (double *)(lds + L.pp), *hene = (double *)(lds + L.ene), *rl2 = (double *)(lds + L.rl2),
+         *bdp = (double *)(lds + L.bd), *bap = (double *)(lds + L.ba), *stp = (double *)(lds + L.st),
+         *hbp = (double *)(lds + L.hb);
+  EleWave *je = (EleWave *)(lds + L.je);
+  SpPair *sptab = (SpPair *)(lds + L.sptab);
+  uint64_t *mask = (uint64_t *)(lds + L.mask), *seg = (uint64_t *)(lds + L.slot);
+  float *qic = (float *)(lds + L.qic), *slot = (float *)(lds + L.slot);
+  uint32_t *meta = (uint32_t *)(lds + L.meta);   // type | class << 8 | unit << 16
+  int32_t *scnt = (int32_t *)(lds + L.cnt), *sval = (int32_t *)(lds + L.val);
+  uint16_t *list = (uint16_t *)(lds + L.list), *inc = (uint16_t *)(lds + L.inc), *incoff = (uint16_t *)(lds + L.incoff),
+           *nbc = (uint16_t *)(lds + L.nb), *bdm = (uint16_t *)(lds + L.bdm), *bam = (uint16_t *)(lds + L.bam),
+           *stm = (uint16_t *)(lds + L.stm), *hbm = (uint16_t *)(lds + L.hbm), *hbsite = (uint16_t *)(lds + L.hbsite),
+           *sq = (uint16_t *)(lds + L.seq), *qb = (uint16_t *)(lds + L.qb);
+  int16_t *qidx = (int16_t *)(lds + L.qidx);
+  uint8_t *spec = (uint8_t *)(lds + L.spec), *stat = (uint8_t *)(lds + L.stat), *inl = (uint8_t *)(lds + L.inl);
+  const int nq = s.ele_form >= 0 ? s.nq : 0, nqt = s.ele_form >= 0 ? s.nqt : 0, np = nqt * (nqt + 1) / 2;
+  const int nbt = s.nbt, nbd = s.nbd, nba = s.nba, nst = s.nst, nhb = s.nhb;
+  const bool vlim = s.hb_excess_possible != 0, dyn = rebuild == 0;
+  const int wdir = wave_dir(), dir = wdir ? wdir : 1;   // 0: rotation by shuffles (ele_pair_task)
+  // slot bases within the system
+  const int lb_ba = 2 * nbd, lb_st = lb_ba + 3 * nba, lb_hb = lb_st + 7 * nst;
+  float *hslot = slot + 3 * lb_hb;
+
+  // ---- the system into LDS and registers
+  const double *XC = P.x[cb], *XP = P.x[cb ^ 1];
+  const bool own = tid < nb;
+  const int g = s.off + (own ? tid : 0);
+  double xc[3], v[3], a[3], ds[3] = {0.0, 0.0, 0.0}, dl[3] = {0.0, 0.0, 0.0}, lr[4], rcm;
+  {
+    const LangClass &lc = P.lcls[s.lc0 + P.lcl[g]];
+    for (int k = 0; k < 4; ++k) lr[k] = lc.r[k];
+    rcm = lc.rcm;
+    for (int d = 0; d < 3; ++d) {
+      xc[d] = XC[(size_t)d * N + g]; v[d] = P.v[(size_t)d * N + g]; a[d] = P.a[(size_t)d * N + g];
+      if (dyn) { ds[d] = P.dxyz[(size_t)d * N + g]; dl[d] = P.dlast[(size_t)d * N + g]; }
+    }
+  }
+  const int ib0 = P.inc_off[s.off];
+  if (own) {
+    for (int d = 0; d < 3; ++d) x[d * nb + tid] = XP[(size_t)d * N + g];
+    meta[tid] = (uint32_t)(uint8_t)P.mptype[g] | (uint32_t)(uint8_t)P.iclass[g] << 8 | (uint32_t)P.unit[g] << 16;
+    incoff[tid] = (uint16_t)(P.inc_off[g] - ib0);
+    qidx[tid] = (int16_t)(nq > 0 && P.qidx[g] >= 0 ? P.qidx[g] - s.qoff : -1);
+    spec[tid] = P.species[g];
+  }
+  const int ninc = P.inc_off[s.off + nb] - ib0;
+  if (tid == 0) {
+    incoff[nb] = (uint16_t)ninc;
+    next[0] = next[1] = next[2] = 0;
+    over = 0;
+  }
+  for (int k = tid; k < ninc; k += T) {
+    const int64_t at = P.inc_slot[ib0 + k];
+    int64_t l;
+    if (at >= P.sb_hb) l = at - P.sb_hb - 6 * (int64_t)s.hoff + lb_hb;
+    else if (at >= P.sb_st) l = at - P.sb_st - 7 * (int64_t)s.soff + lb_st;
+    else if (at >= P.sb_ba) l = at - P.sb_ba - 3 * (int64_t)s.aoff + lb_ba;
+    else l = at - 2 * (int64_t)s.boff;
+    inc[k] = (uint16_t)l;
+  }
+  for (int k = tid; k < nbd; k += T) {
+    const int t = s.boff + k;
+    for (int q = 0; q < 2; ++q) bdm[q * nbd + k] = (uint16_t)(P.bd_mp[2 * t + q] - s.off);
+    bdp[k] = P.bd_nat[t]; bdp[nbd + k] = P.bd_coef[t];
+  }
+  for (int k = tid; k < nba; k += T) {
+    const int t = s.aoff + k;
+    for (int q = 0; q < 3; ++q) bam[q * nba + k] = (uint16_t)(P.ba_mp[3 * t + q] - s.off);
+    bap[k] = P.ba_nat[t]; bap[nba + k] = P.ba_coef[t];
+  }
+  for (int k = tid; k < nst; k += T) {
+    const int t = s.soff + k;
+    for (int q = 0; q < 7; ++q) stm[q * nst + k] = (uint16_t)(P.st_mp[7 * t + q] - s.off);
+    for (int q = 0; q < 3; ++q) stp[q * nst + k] = P.st_nat[3 * t + q];
+    for (int q = 0; q < 4; ++q) stp[(3 + q) * nst + k] = P.st_coef[4 * t + q];
+  }
+  for (int k = tid; k < nhb; k += T) {
+    const int t = s.hoff + k;
+    for (int q = 0; q < 6; ++q) hbm[q * nhb + k] = (uint16_t)(P.hb_mp[6 * t + q] - s.off);
+    for (int q = 0; q < 6; ++q) hbp[q * nhb + k] = P.hb_nat[6 * t + q];
+    for (int q = 0; q < 7; ++q) hbp[(6 + q) * nhb + k] = P.hb_coef[7 * t + q];
+    inl[k] = P.hb_inlist[t];
+  }
+  for (int k = tid; k < s.nspecies * s.nspecies; k += T) sptab[k] = P.sptab[s.sptab + k];
+  for (int k = tid; k < s.nunit * s.nunit; k += T) rl2[k] = P.rl2[s.uoff + k];
+  for (int k = tid; k < nqt * kTile; k += T) {
+    const int c = stage_at(k % kTile, dir);
+    const bool val = k < nq;
+    const int gq = val ? P.qbead[s.qoff + k] : 0;
+    EleWave &E = je[k / kTile];
+    const double px = val ? XP[gq] : kFar, py = val ? XP[N + gq] : kFar, pz = val ? XP[2 * (size_t)N + gq] : kFar;
+    const float q = val ? (float)P.charge[gq] : 0.0f;
+    E.x[c] = px; E.y[c] = py; E.z[c] = pz; E.q[c] = q;
+    E.x[c + kTile] = px; E.y[c + kTile] = py; E.z[c + kTile] = pz; E.q[c + kTile] = q;
+    qic[k] = val ? (float)(P.charge[gq] * s.ele_coef) : 0.0f;
+    if (val) qb[k] = (uint16_t)(gq - s.off);
+  }
+  if (vlim) {
+    for (int k = tid; k < s.nsite; k += T) { scnt[k] = 0; sval[k] = P.site_val[s.sitoff + k]; }
+    for (int k = tid; k < 6 * nhb; k += T) {
+      const int st = P.hb_site[6 * (size_t)s.hoff + k];
+      hbsite[k] = (uint16_t)(st < 0 ? 0xFFFF : st - s.sitoff);
+    }
+  }
+  if (dyn && lane == 0) {
+    top[w][0] = w < nbt ? P.ttop[2 * (s.bt0 + w)] : 0.0;
+    top[w][1] = w < nbt ? P.ttop[2 * (s.bt0 + w) + 1] : 0.0;
+  }
+  const uint64_t step0 = base + 1u - s.step_origin;
+  const LocalX lx{x, nb, 0};
+  const LocalHb hb{hene, scnt, sval, hbsite, sq, stat, hslot};
+  // tasks of a step, in the order they are taken; valence-limited systems
+  // take the first nfirst (hbonds, stacks) before the others
+  const int t_hb = (nhb + kTile - 1) / kTile, t_st = (nst + kTile - 1) / kTile;
+  const int t_ba = (nba + kTile - 1) / kTile, t_bd = (nbd + kTile - 1) / kTile;
+  const int nfirst = vlim ? t_hb + t_st : 0;
+  const int nrest = np + (vlim ? 0 : t_hb + t_st) + 3 * nbt + t_ba + t_bd;
+  unsigned clamp_exv = 0, clamp_ele = 0, ndel = 0, nfire = 0;
+  __syncthreads();
+
+  // whether the lists are rebuilt before step t: at the fixed interval, or by
+  // the displacement trigger (system_trigger on the tiles' two largest)
+  auto due = [&](int t) {
+    if (!dyn) return (phase + t) % rebuild == 0;
+    double m1 = 0.0, m2 = 0.0;
+    for (int q = 0; q < nbt; ++q) {
+      const double hi = fmax(m1, top[q][0]), lo = fmax(fmin(m1, top[q][0]), fmax(m2, top[q][1]));
+      m1 = hi; m2 = lo;
+    }
+    return sqrt(m1) + sqrt(m2) > s.margin;
+  };
+  if (from < n && !due(from)) {
+    // the lists as they stand
+    if (own) {
+      const int cnt = min(P.nb_cnt[g], P.nb_cap);
+      nbc[tid] = (uint16_t)cnt;
+    }
+    __syncthreads();
+    for (int k = tid; k < rows * nb; k += T) {
+      const int m = k / nb, i = k % nb;
+      if (m >= nbc[i]) continue;
+      const int j = (int)(P.nb[(size_t)m * N + s.off + i] & kIdxMask) - s.off;
+      list[k] = (uint16_t)(j | (int)spec[j] << 10);
+    }
+    for (int k = tid; k < np * kTile; k += T) {
+      int I, J;
+      chunk_pair(k / kTile, nqt, I, J);
+      const int qi = I * kTile + k % kTile;
+      uint64_t m = 0;
+      if (qi < nq) {
+        const uint32_t *row = P.qmask + s.moff + (int64_t)qi * s.mwords;
+        m = row[2 * J];
+        if (2 * J + 1 < s.mwords) m |= (uint64_t)row[2 * J + 1] << 32;
+      }
+      mask[k] = m;
+    }
+    __syncthreads();
+  }
+
+  int t = from;
+  double xp[3] = {0.0, 0.0, 0.0};
+  for (; t < n; ++t) {
+    const bool last = t == n - 1;
+    if (due(t)) {
+      // ---- lists from the current positions (k_lists' tests; entries in
+      // ascending order); to memory too when no later rebuild of this launch
+      // replaces them
+      const bool keep = dyn || t + rebuild >= n;
+      if (own)
+        for (int d = 0; d < 3; ++d) { xp[d] = x[d * nb + tid]; x[d * nb + tid] = xc[d]; }
+      __syncthreads();
+      for (;;) {
+        int k = take_task(&next[2]);
+        if (k >= nbt * nbt + nqt * nqt) break;
+        if (k < nbt * nbt) {
+          // 64 beads against 64: the accept bits of each lane's bead
+          const int i = (k / nbt) * kTile + lane, j0 = (k % nbt) * kTile, kend = min(kTile, nb - j0);
+          const int ic = i < nb ? i : 0;
+          const double x0 = x[ic], x1 = x[nb + ic], x2 = x[2 * nb + ic];
+          const int mi = (int)meta[ic], ui = mi >> 16, ti = mi & 0xFF, ci = (mi >> 8) & 0xFF;
+          uint64_t m = 0;
+#pragma unroll 4
+          for (int q = 0; q < kend; ++q) {
+            const int j = j0 + q, mj = (int)meta[j];
+            const double d2 = sq3_separate(x[j] - x0, x[nb + j] - x1, x[2 * nb + j] - x2);
+            const bool ok = s.nunit == 1 ? exv_listed<true>(s, d2, i, ui, ti, ci, j, ui, mj & 0xFFFF, rl2)
+                                         : exv_listed<false>(s, d2, i, ui, ti, ci, j, mj >> 16, mj & 0xFFFF, rl2);
+            m |= (uint64_t)(ok ? 1 : 0) << q;
+          }
+          if (i < nb) seg[(k % nbt) * nb + i] = m;
+          continue;
+        }
+        k -= nbt * nbt;
+        const int I = k / nqt, J = k % nqt, qi = I * kTile + lane, jt = J * kTile;
+        if (J < I && !keep) continue;
+        const int bi = qi < nq ? qb[qi] : 0, kend = min(kTile, nq - jt);
+        const double xi[3] = {x[bi], x[nb + bi], x[2 * nb + bi]};
+        uint64_t m = 0;
+#pragma unroll 4
+        for (int q = 0; q < kend; ++q) {
+          const int bj = qb[jt + q];
+          double dv[3];
+          pair_vec(s, x[bj], x[nb + bj], x[2 * nb + bj], xi, true, dv);
+          const bool ok = jt + q != qi && sq3_exact(dv[0], dv[1], dv[2]) < s.ele_rl2;
+          m |= (uint64_t)(ok ? 1 : 0) << q;
+        }
+        if (qi >= nq) m = 0;
+        if (J >= I) mask[ele_task_index(I, J, nqt) * kTile + lane] = m;
+        if (keep && qi < nq) {
+          uint32_t *row = P.qmask + s.moff + (int64_t)qi * s.mwords;
+          row[2 * J] = (uint32_t)m;
+          if (2 * J + 1 < s.mwords) row[2 * J + 1] = (uint32_t)(m >> 32);
+        }
+      }
+      for (int k = tid; k < nhb; k += T) {
+        const int b0 = hbm[k], b1 = hbm[nhb + k];
+        const double dv[3] = {__dadd_rn(x[b0], -x[b1]), __dadd_rn(x[nb + b0], -x[nb + b1]),
+                              __dadd_rn(x[2 * nb + b0], -x[2 * nb + b1])};
+        inl[k] = (uint8_t)hb_listed(s, dv, hbp[k]);
+        if (keep) P.hb_inlist[s.hoff + k] = inl[k];
+      }
+      __syncthreads();
+      if (own)
+        for (int d = 0; d < 3; ++d) x[d * nb + tid] = xp[d];
+      if (tid == 0) next[2] = 0;
+      for (int k = tid; k < nb * nbt; k += T) {
+        const int i = k % nb, sg = k / nb;
+        int m = 0;
+        for (int q = 0; q < sg; ++q) m += __popcll(seg[q * nb + i]);
+        uint64_t bits = seg[k];
+        const int tot = m + __popcll(bits);
+        for (; bits; bits &= bits - 1, ++m) {
+          const int j = sg * kTile + (int)__builtin_ctzll(bits);
+          if (m < rows) list[m * nb + i] = (uint16_t)(j | (int)spec[j] << 10);
+          if ((keep || m >= rows) && m < P.nb_cap) P.nb[(size_t)m * N + s.off + i] = (uint32_t)(s.off + j);
+        }
+        if (sg == nbt - 1) {
+          nbc[i] = (uint16_t)tot;
+          if (keep) P.nb_cnt[s.off + i] = tot;
+          if (tot > P.nb_cap) {
+            atomicMax(&over, (unsigned)tot);
+            atomicMax(&P.counters[5], (unsigned long long)tot);
+          }
+        }
+      }
+      __syncthreads();
+      if (over) break;   // (no thread writes it before the next rebuild)
+      if (dyn) {
+        ++nfire;
+        for (int d = 0; d < 3; ++d) ds[d] = dl[d];
+      }
+    }
+    // ---- the terms
+    auto hb_task = [&](int q0) {
+      const int q = q0 + lane;
+      if (q >= nhb) return;
+      const int m6[6] = {hbm[q], hbm[nhb + q], hbm[2 * nhb + q], hbm[3 * nhb + q], hbm[4 * nhb + q], hbm[5 * nhb + q]};
+      double fo[18], ene = 0.0;
+      int st = 0;
+      if (inl[q]) {
+        double nat[6], cf[7];
+        for (int k = 0; k < 6; ++k) nat[k] = hbp[k * nhb + q];
+        for (int k = 0; k < 7; ++k) cf[k] = hbp[(6 + k) * nhb + q];
+        st = hbond_eval(s, lx, lx, m6, nat, cf, fo, &ene);
+      }
+      if (!st) for (int k = 0; k < 18; ++k) fo[k] = 0.0;
+      for (int k = 0; k < 18; ++k) hslot[18 * q + k] = (float)fo[k];
+      if (vlim) {
+        stat[q] = (uint8_t)st;
+        hene[q] = ene;
+        if (st)
+          for (int k = 0; k < 6; ++k)
+            if (hbsite[6 * q + k] != 0xFFFF) atomicAdd(&scnt[hbsite[6 * q + k]], 1);
+      } else if (last) {
+        P.hb_status[s.hoff + q] = (uint8_t)st;
+        P.hb_ene[s.hoff + q] = ene;
+      }
+    };
+    auto st_task = [&](int k0) {
+      const int k = k0 + lane;
+      if (k >= nst) return;
+      int m7[7];
+      double nat[3], cf[4], fo[21];
+      for (int q = 0; q < 7; ++q) m7[q] = stm[q * nst + k];
+      for (int q = 0; q < 3; ++q) nat[q] = stp[q * nst + k];
+      for (int q = 0; q < 4; ++q) cf[q] = stp[(3 + q) * nst + k];
+      stack_eval(lx, m7, nat, cf, fo);
+      float *o = slot + 3 * (lb_st + 7 * k);
+      for (int q = 0; q < 21; ++q) o[q] = (float)fo[q];
+    };
+    if (vlim) {
+      for (;;) {
+        const int k = take_task(&next[0]);
+        if (k >= nfirst) break;
+        if (k < t_hb) hb_task(k * kTile);
+        else st_task((k - t_hb) * kTile);
+      }
+      __syncthreads();
+      if (w == 0) {
+        bool any = false;
+        for (int k = lane; k < s.nsite; k += kTile) any = any || hb.excess(k);
+        if (__any(any)) ndel += (unsigned)hbond_valence_wave(P, s, step0 + (uint64_t)t, lane, hb);
+        // the counts of the next step start at zero
+        wave_sync();
+        for (int k = lane; k < s.nsite; k += kTile) scnt[k] = 0;
+        if (last)
+          for (int q = lane; q < nhb; q += kTile) {
+            P.hb_status[s.hoff + q] = stat[q];
+            P.hb_ene[s.hoff + q] = hene[q];
+          }
+      }
+    }
+    for (;;) {
+      int k = take_task(&next[1]);
+      if (k >= nrest) break;
+      if (k < np) {
+        int I, J;
+        chunk_pair(k, nqt, I, J);
+        const int qi = I * kTile + lane, c = stage_at(lane, dir);
+        const bool val = qi < nq;
+        const double x0 = val ? je[I].x[c] : -kFar, x1 = val ? je[I].y[c] : -kFar, x2 = val ? je[I].z[c] : -kFar;
+        const int nj = nq - J * kTile < kTile ? nq - J * kTile : kTile;
+        double F[3], G[3];
+        auto sums = [&](auto form, auto dpp) {
+          return ele_pair_sums<decltype(form)::value, decltype(dpp)::value>(s, I == J, nj, val, mask[k * kTile + lane],
+                                                                            x0, x1, x2, qic[qi], dir, &je[J], F, G);
+        };
+        using F0 = std::integral_constant<int, 0>;
+        using F1 = std::integral_constant<int, 1>;
+        const uint32_t nc = wdir ? (s.ele_form == 0 ? sums(F0{}, std::true_type{}) : sums(F1{}, std::true_type{}))
+                                 : (s.ele_form == 0 ? sums(F0{}, std::false_type{}) : sums(F1{}, std::false_type{}));
+        double *o = pp + (size_t)k * (6 * kTile) + lane;
+        for (int d = 0; d < 3; ++d) { o[d * kTile] = F[d]; o[(3 + d) * kTile] = G[d]; }
+        clamp_ele += nc;
+        continue;
+      }
+      k -= np;
+      if (!vlim) {
+        if (k < t_hb) { hb_task(k * kTile); continue; }
+        k -= t_hb;
+        if (k < t_st) { st_task(k * kTile); continue; }
+        k -= t_st;
+      }
+      if (k < nbt) {
+        const int i = k * kTile + lane;
+        if (i < nb) {
+          double gs[3];
+          gauss3(P.seed, s.key, step0 + (uint64_t)t, (uint32_t)i, gs);
+          for (int d = 0; d < 3; ++d) gn[d * nb + i] = gs[d];
+        }
+        continue;
+      }
+      k -= nbt;
+      if (k < 2 * nbt) {
+        // half h of the neighbour groups of 64 beads: groups k mod 4 = h and
+        // h + 2 (exv_group's order)
+        const int h = k & 1, i = (k >> 1) * kTile + lane;
+        if (i < nb) {
+          const double xi0 = x[i], xi1 = x[nb + i], xi2 = x[2 * nb + i];
+          const int cnt = nbc[i];
+          const SpPair *tab = sptab + (int)spec[i] * s.nspecies;
+          double E[2][3] = {};
+          int en[4], enn[4] = {0, 0, 0, 0};
+          auto entries = [&](int m0, int (&o)[4]) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int m = min(m0 + u, cnt - 1);
+              if (m < rows) {
+                o[u] = list[m * nb + i];
+              } else {
+                const int j = (int)(P.nb[(size_t)m * N + s.off + i] & kIdxMask) - s.off;
+                o[u] = j | (int)spec[j] << 10;
+              }
+            }
+          };
+          if (4 * h < cnt) entries(4 * h, en);
+          for (int m0 = 4 * h; m0 < cnt; m0 += 8) {
+            double d2[4], dv[4][3], lim[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int j = en[u] & 1023;
+              dv[u][0] = x[j] - xi0; dv[u][1] = x[nb + j] - xi1; dv[u][2] = x[2 * nb + j] - xi2;
+              lim[u] = tab[en[u] >> 10].dij2;
+            }
+            if (m0 + 8 < cnt) entries(m0 + 8, enn);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) d2[u] = dot3(dv[u], dv[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              if (m0 + u >= cnt || d2[u] > lim[u]) continue;
+              const SpPair tp = tab[en[u] >> 10];
+              const bool cl = (m0 & 8) ? exv_contact(s.exv_a, tp.dij, tp.coef, dv[u], d2[u], E[1])
+                                       : exv_contact(s.exv_a, tp.dij, tp.coef, dv[u], d2[u], E[0]);
+              if (cl && i < (en[u] & 1023)) ++clamp_exv;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) en[u] = enn[u];
+          }
+          for (int d = 0; d < 3; ++d) e[(3 * h + d) * nb + i] = E[0][d] + E[1][d];
+        }
+        continue;
+      }
+      k -= 2 * nbt;
+      if (k < t_ba) {
+        const int q = k * kTile + lane;
+        if (q < nba) {
+          double fo[9];
+          angle_eval(lx, bam[q], bam[nba + q], bam[2 * nba + q], bap[q], bap[nba + q], fo);
+          float *o = slot + 3 * (lb_ba + 3 * q);
+          for (int u = 0; u < 9; ++u) o[u] = (float)fo[u];
+        }
+        continue;
+      }
+      k -= t_ba;
+      const int q = k * kTile + lane;
+      if (q < nbd) {
+        double fo[6];
+        bond_eval(lx, bdm[q], bdm[nbd + q], bdp[q], bdp[nbd + q], fo);
+        float *o = slot + 6 * q;
+        for (int u = 0; u < 6; ++u) o[u] = (float)fo[u];
+      }
+    }
+    __syncthreads();
+    // ---- sums and integration, one thread per bead
+    if (tid == 0) { next[0] = 0; next[1] = 0; }
+    double d2 = -1.0;   // squared displacement since the last rebuild, before this update
+    if (own) {
+      double S[3] = {0.0, 0.0, 0.0}, Q[3] = {0.0, 0.0, 0.0};
+      const int k1 = incoff[tid + 1];
+      for (int k = incoff[tid]; k < k1; ++k) {
+        const float *sl = slot + 3 * inc[k];
+        S[0] += (double)sl[0]; S[1] += (double)sl[1]; S[2] += (double)sl[2];
+      }
+      const int q = qidx[tid];
+      if (q >= 0) {
+        const int C = q / kTile, lc = q % kTile;
+        for (int I = 0; I < nqt; ++I) {
+          const int ta = I <= C ? I : C, tb = I <= C ? C : I;
+          const double *o = pp + ele_task_index(ta, tb, nqt) * (6 * kTile) + (I < C ? 3 * kTile : 0) + lc;
+          Q[0] += o[0]; Q[1] += o[kTile]; Q[2] += o[2 * kTile];
+        }
+      }
+      double dx[3];
+      for (int d = 0; d < 3; ++d) {
+        const double F = (S[d] + Q[d]) + (e[d * nb + tid] + e[(3 + d) * nb + tid]);
+        xc[d] = x[d * nb + tid];
+        dx[d] = langevin_update(lr, rcm, P.tstep2, 1, F, gn[d * nb + tid], v[d], a[d]);
+        xp[d] = __dadd_rn(xc[d], dx[d]);
+        x[d * nb + tid] = xp[d];
+        if (last) P.f[(size_t)d * N + g] = F;
+      }
+      if (q >= 0) {
+        EleWave &E = je[q / kTile];
+        const int c = stage_at(q % kTile, dir);
+        E.x[c] = xp[0]; E.y[c] = xp[1]; E.z[c] = xp[2];
+        E.x[c + kTile] = xp[0]; E.y[c + kTile] = xp[1]; E.z[c + kTile] = xp[2];
+      }
+      if (dyn) {
+#pragma clang fp contract(off)
+        d2 = ds[0] * ds[0] + ds[1] * ds[1] + ds[2] * ds[2];
+        for (int d = 0; d < 3; ++d) { ds[d] = ds[d] + dx[d]; dl[d] = dx[d]; }
+      }
+    }
+    if (dyn && w < nbt) {
+      double m1, m2;
+      top2_wave(d2, m1, m2);
+      if (lane == 0) { top[w][0] = m1; top[w][1] = m2; }
+    }
+    __syncthreads();
+  }
+  // ---- the state back: at the end of the launch, or (t < n) before the step
+  // whose rebuild overflowed, in the buffers of the launch's start
+  const int cw = t == n ? ce : cu;
+  if (own)
+    for (int d = 0; d < 3; ++d) {
+      const size_t o = (size_t)d * N + g;
+      const double nx = x[d * nb + tid];
+      P.x[cw][o] = xc[d];
+      P.x[cw ^ 1][o] = nx;
+      P.v[o] = v[d];
+      P.a[o] = a[d];
+      if (dyn) { P.dxyz[o] = ds[d]; P.dlast[o] = dl[d]; }
+    }
+  if (dyn && w < nbt) {
+    if (lane == 0) { P.ttop[2 * (s.bt0 + w)] = top[w][0]; P.ttop[2 * (s.bt0 + w) + 1] = top[w][1]; }
+    double p[3];
+    for (int d = 0; d < 3; ++d) { const double p0 = __shfl(xc[d], 0); p[d] = own ? xc[d] : p0; }
+    tile_boxes(p[0], p[1], p[2], &P.bbox[s.bt0 + w], &P.sbox[4 * (s.bt0 + w)]);
+  }
+  if (clamp_exv) atomicAdd(&P.counters[0], (unsigned long long)clamp_exv);
+  if (lane == 0 && clamp_ele) atomicAdd(&P.counters[1], (unsigned long long)clamp_ele);
+  if (tid == 0) {
+    P.win_at[isys] = (base + (uint64_t)t) << 1 | (uint64_t)cw;
+    if (ndel) atomicAdd(&P.counters[2], (unsigned long long)ndel);
+    if (nfire) atomicAdd(&P.counters[3], (unsigned long long)nfire);
+  }
+}
+
 // st_status of the consecutive stacks [s0, s0 + ns) at the given
 // coordinates (force_dtrna_stack_nlocal.F90:83-92 via stack_on), for output.
 __global__ __launch_bounds__(256) void k_stack_status(DevPtrs P, const double *X, const double *PX, int s0, int ns,
@@ -1983,17 +2697,16 @@ __global__ __launch_bounds__(256) void k_stack_status(DevPtrs P, const double *X
   if (k < ns) out[k] = stack_on(P, X, PX, s0 + k) ? 1 : 0;
 }
 
-// The step counter: by steps at once after a captured window, one step per
-// eager step.  A stopped run does not advance it (the host reads it to know
-// where to resume).
-__global__ void k_advance(uint64_t *stepbase, uint64_t by, unsigned long long *counters) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && counters[5] == 0ull) { *stepbase += by; counters[4] += by; }
-}
-
-// One step of a captured window: the step counter moves per step, so a stop
-// inside a window leaves it at the step to resume from.
-__global__ void k_advance_step(uint64_t *stepbase, unsigned long long *counters) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && counters[5] == 0ull) { *stepbase += 1ull; counters[4] += 1ull; }
+// The step counter: by steps at once after a captured run of steps or a
+// k_window launch, one step per eager step; with its whole-batch list
+// rebuilds and its completed steps where its kernels do not count them
+// (rebuilds, completed).  A stopped run does not advance it (the host reads
+// it to know where to resume).
+__global__ void k_advance(uint64_t *stepbase, uint64_t by, uint64_t rebuilds, uint64_t completed,
+                          unsigned long long *counters) {
+  if (threadIdx.x == 0 && blockIdx.x == 0 && counters[5] == 0ull) {
+    *stepbase += by; counters[4] += by; counters[3] += rebuilds; counters[6] += completed;
+  }
 }
 
 __global__ void k_count_rebuild(unsigned long long *counters) {
@@ -2031,14 +2744,6 @@ __device__ inline double block_sums(const double (&e)[kNE], double (*red)[kNE]) 
   if (t < kNE)
     for (int q = 0; q < kEBlock / kTile; ++q) r += red[q][t];
   return r;
-}
-
-// The value of v at lane r (the same for every lane) of the wave.
-__device__ inline double at_lane(double v, int r) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, r);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), r);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
 // Electrostatic pair energies of wave w of nw over system s: the chunk pairs
