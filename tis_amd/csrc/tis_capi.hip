@@ -25,10 +25,12 @@ __global__ void k_force(DevPtrs, const double *, const double *, const int32_t *
                         BondedRange, int32_t);
 __global__ void k_ewald_sk(DevPtrs, const double *, const EwTask *, int);
 __global__ void k_ewald_f(DevPtrs, const double *, const EwTask *);
-__global__ void k_main(DevPtrs, const double *, const double *, double *, double *, const Tile *, int, int32_t, int, int,
-                       int);
-__global__ void k_prep(DevPtrs, const double *, double *, double *, const Tile *, int, int, const Tile *, int, int,
-                       int, int);
+template <int XW>
+__global__ void k_main(DevPtrs, const double *, const double *, const float4 *, double *, double *, float4 *,
+                       const Tile *, int, int32_t, int, int, int);
+__global__ void k_near(DevPtrs, const double *, float4 *, int, int);
+__global__ void k_prep(DevPtrs, const double *, double *, double *, float4 *, float4 *, const Tile *, int, int,
+                       const Tile *, int, int, int, int);
 __global__ void k_lists(DevPtrs, const double *, const double *, const Tile *, int, int, const Tile *, int, int, int,
                         int, int);
 __global__ void k_lpair(DevPtrs, const double *, const double *, const EwTask *, int, const EwTask *, int, int, int,
@@ -484,13 +486,14 @@ static void launch_lpair(tis_ctx *c, const Range &r, const double *X, const doub
                        c->d_qpair + qp0, nqp, h0, 0, mode, 1);
 }
 
-// The lists of the range from X (wrapped copies into PXcur, predicted
-// wrapped positions into PXpred when with_pred): k_prep, then k_lists by
+// The lists of the range from the positions in buffer cu (wrapped copies into
+// px[cu], predicted wrapped positions into the other when with_pred): k_prep, then k_lists by
 // bead / charge tile for non-periodic systems and the hbond candidates, and
 // k_lpair by tile pair for periodic systems; with gate, only the systems
 // whose displacement trigger fired.
-int launch_lists(tis_ctx *c, const Range &r, const double *X, double *PXcur, double *PXpred, int with_pred,
-                 int gate) {
+int launch_lists(tis_ctx *c, const Range &r, int cu, int with_pred, int gate) {
+  const double *X = c->P.x[cu];
+  double *PXcur = c->P.px[cu], *PXpred = c->P.px[cu ^ 1];
   const int h0 = r.all ? 0 : c->hs[r.isys].d.hoff, nh = r.all ? c->nhbtot : c->hs[r.isys].d.nhb;
   const bool periodic = r.all ? c->any_periodic : c->hs[r.isys].d.periodic != 0;
   if (gate && !periodic) {
@@ -504,8 +507,8 @@ int launch_lists(tis_ctx *c, const Range &r, const double *X, double *PXcur, dou
     return 0;
   }
   if (r.btn + r.qtn > 0)
-    hipLaunchKernelGGL(k_prep, dim3(r.btn + r.qtn), dim3(kTile), 0, c->stream, c->P, X, PXcur, PXpred, c->d_btiles,
-                       r.bt0, r.btn, c->d_qtiles, r.qt0, r.qtn, with_pred, gate);
+    hipLaunchKernelGGL(k_prep, dim3(r.btn + r.qtn), dim3(kTile), 0, c->stream, c->P, X, PXcur, PXpred,
+                       c->P.xf[cu], c->P.xf[cu ^ 1], c->d_btiles, r.bt0, r.btn, c->d_qtiles, r.qt0, r.qtn, with_pred, gate);
   const int nblk = r.btn + r.qtn + (nh + kTile - 1) / kTile;
   if (nblk > 0)
     hipLaunchKernelGGL(k_lists, dim3(nblk), dim3(kTile), 0, c->stream, c->P, X, PXcur, c->d_btiles, r.bt0, r.btn,
@@ -744,6 +747,9 @@ int stage_system(tis_ctx *c, Stage &g, HostSys &h, const tis_system &s, int is, 
         dij = A.r + B.r;
       g.sptab.push_back(SpPair{dij, dij * dij, A.e * B.e});
     }
+  double dmax = 0.0;
+  for (int k = 0; k < NS * NS; ++k) dmax = std::max(dmax, g.sptab[d.sptab + k].dij);
+  d.exv_near2 = (float)((dmax + kNearMargin) * (dmax + kNearMargin));
   // its Langevin classes (constants r[] set by tis_langevin_init)
   d.lc0 = (int32_t)g.lcls.size();
   d.nlc = (int32_t)h.lc_fric.size();
@@ -876,6 +882,7 @@ int alloc_arena(tis_ctx *c, const Caps &k, std::vector<void *> &list, DevPtrs &P
   for (int q = 0; q < 2; ++q) {
     AL(P.x[q], 3 * B);
     AL(P.px[q], k.periodic ? 3 * B : 1);
+    AL(P.xf[q], B);
   }
   AL(P.v, 3 * B); AL(P.a, 3 * B); AL(P.f, 3 * B);
   AL(A.lcl, B); AL(A.lcls, k.lc); AL(A.mass, B); AL(A.exv_rad, B); AL(A.charge, B); AL(A.rl2, k.rl2);
@@ -1223,6 +1230,9 @@ int relayout(tis_ctx *c, const std::vector<const tis_system *> &extra, double gr
         rc = fail(c, TIS_ERR_HIP, "state copy of a new layout failed");
     }
     c->d2d_state += (int64_t)(9 * n * 8);
+    if (!h.d.periodic)
+      hipLaunchKernelGGL(k_near, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, P, P.x[cu], P.xf[cu],
+                         h.d.off, h.d.nmp);
     if (rc == 0 && (hipMemcpyAsync(A.charge + sn, OA.charge + so, n * 8, hipMemcpyDeviceToDevice, c->stream) !=
                         hipSuccess ||
                     (h.d.nst > 0 && hipMemcpyAsync(A.st_coef + 4 * (size_t)h.d.soff,
@@ -1456,7 +1466,13 @@ int32_t tis_state_set(tis_ctx *c, int32_t isys, int32_t which, const double *buf
     c->h2d_state += (int64_t)(comp.size() * sizeof(double));
     HIPCHK(c, hipStreamSynchronize(c->stream));
   }
-  if (which == 0) { c->lists_valid = false; c->lv_init = false; }
+  if (which == 0) {
+    c->lists_valid = false;
+    c->lv_init = false;
+    if (!h.d.periodic)
+      hipLaunchKernelGGL(k_near, dim3((h.d.nmp + 255) / 256), dim3(256), 0, c->stream, c->P, Xc(c), c->P.xf[c->cur],
+                         h.d.off, h.d.nmp);
+  }
   return TIS_OK;
 }
 
@@ -1484,7 +1500,7 @@ static int rebuild_lists(tis_ctx *c, int32_t isys) {
   Range r = range_of(c, isys);
   for (int attempt = 0; attempt < 4; ++attempt) {
     HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
-    launch_lists(c, r, Xc(c), PXc(c), nullptr, 0, 0);
+    launch_lists(c, r, c->cur, 0, 0);
     hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
     HIPCHK(c, hipGetLastError());
     unsigned long long ovf = 0;
@@ -1572,12 +1588,21 @@ int32_t tis_pairs_get(tis_ctx *c, int32_t isys, int32_t which, int32_t *pairs, d
                  : TIS_OK;
 }
 
+// Launches of k_main with at most this many tiles take six waves per tile
+// instead of two: 5.9 against 8.1 us at 160 tiles, 7.3 against 9.2 at 320, even
+// at 640 (10.8), 17.5 against 13.6 at 1,280.
+constexpr int kMainWideTiles = 512;
+
 // k_force (terms, electrostatic chunk pairs, bonded terms), the Ewald
-// passes, then k_main.  Steps draw noise/valence numbers for step
+// passes, then k_main, at the positions in buffer ix (the next ones go to the
+// other).  Steps draw noise/valence numbers for step
 // stepbase+t+1; a stand-alone force evaluation or the initial acceleration
 // uses stepbase.
-static void launch_force_pair(tis_ctx *c, const Range &r, const double *X, const double *PX, double *XN,
-                              double *PXN, int t_local, int mode, int count_step = 0) {
+static void launch_force_pair(tis_ctx *c, const Range &r, int ix, int t_local, int mode, int count_step = 0) {
+  const double *X = c->P.x[ix], *PX = c->P.px[ix];
+  const float4 *XF = c->P.xf[ix];
+  double *XN = c->P.x[ix ^ 1], *PXN = c->P.px[ix ^ 1];
+  float4 *XFN = c->P.xf[ix ^ 1];
   const int32_t pre_t = mode == 1 ? (int32_t)t_local : -1;  // valence draws at the force step
   // timing events on this stream: e[0] start, e[3] before k_main; e[1]/e[2]
   // and e[4]/e[5] are bound to the k_force and k_main dispatches (start and
@@ -1625,14 +1650,17 @@ static void launch_force_pair(tis_ctx *c, const Range &r, const double *X, const
   }
   if (c->timing) (void)hipEventRecord(e3[3], c->stream);
   const int32_t ele_on = c->any_ele ? 1 : 0;
+  // few tiles: six waves per tile instead of two (see kMainWideTiles)
+  const bool wide = r.btn <= kMainWideTiles;
+  auto km = wide ? k_main<4> : k_main<0>;
+  const dim3 bm(kTile * (wide ? 6 : 2));
+  const Tile *mt = r.all ? c->d_btiles_xcd : c->d_btiles + r.bt0;
   if (r.btn > 0 && c->timing)
-    hipExtLaunchKernelGGL(k_main, dim3(r.btn), dim3(kTile * 2), 0, c->stream, e3[4], e3[5], 0, c->P, X, PX, XN,
-                          PXN, r.all ? c->d_btiles_xcd : c->d_btiles + r.bt0, r.btn, (int32_t)t_local, mode, ele_on,
-                          count_step);
+    hipExtLaunchKernelGGL(km, dim3(r.btn), bm, 0, c->stream, e3[4], e3[5], 0, c->P, X, PX, XF, XN, PXN, XFN, mt, r.btn,
+                          (int32_t)t_local, mode, ele_on, count_step);
   else if (r.btn > 0)
-    hipLaunchKernelGGL(k_main, dim3(r.btn), dim3(kTile * 2), 0, c->stream, c->P, X, PX, XN, PXN,
-                       r.all ? c->d_btiles_xcd : c->d_btiles + r.bt0, r.btn, (int32_t)t_local, mode, ele_on,
-                       count_step);
+    hipLaunchKernelGGL(km, dim3(r.btn), bm, 0, c->stream, c->P, X, PX, XF, XN, PXN, XFN, mt, r.btn, (int32_t)t_local,
+                       mode, ele_on, count_step);
   else if (c->timing) {
     (void)hipEventRecord(e3[4], c->stream);
     (void)hipEventRecord(e3[5], c->stream);
@@ -1647,7 +1675,7 @@ int32_t tis_force_sumup(tis_ctx *c, int32_t isys, double *force_out) {
   if (!c->lists_valid) { rc = rebuild_lists(c, -1); if (rc) return rc; }
   Range r = range_of(c, isys);
   // force evaluation at the current coordinates; valence draws use step = stepbase
-  launch_force_pair(c, r, Xc(c), PXc(c), nullptr, nullptr, 0, 0);
+  launch_force_pair(c, r, c->cur, 0, 0);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (isys >= 0 && force_out) return tis_state_get(c, isys, 3, force_out);
@@ -1965,18 +1993,18 @@ int32_t tis_langevin_init(tis_ctx *c, double tstep, int32_t rebuild_every, uint6
   const int cu = c->cur;
   if (init_accel < 0) {
     // per system: new accelerations (mode 2) or kept ones (mode 3)
-    launch_force_pair(c, r, c->P.x[cu], c->P.px[cu], c->P.x[cu ^ 1], c->P.px[cu ^ 1], 0, 4);
+    launch_force_pair(c, r, cu, 0, 4);
   } else if (init_accel) {
     // a = F(x)/m + c1 xi(step0), then x_pred (mode 2)
-    launch_force_pair(c, r, c->P.x[cu], c->P.px[cu], c->P.x[cu ^ 1], c->P.px[cu ^ 1], 0, 2);
+    launch_force_pair(c, r, cu, 0, 2);
   } else {
     // keep the stored a; forces at x give the hbond state, then predict
-    launch_force_pair(c, r, c->P.x[cu], c->P.px[cu], c->P.x[cu ^ 1], c->P.px[cu ^ 1], 0, 3);
+    launch_force_pair(c, r, cu, 0, 3);
   }
   HIPCHK(c, hipGetLastError());
   if (c->any_periodic)
     hipLaunchKernelGGL(k_prep, dim3(c->nbtile), dim3(kTile), 0, c->stream, c->P, c->P.x[cu], c->P.px[cu],
-                       c->P.px[cu ^ 1], c->d_btiles, 0, c->nbtile, c->d_qtiles, 0, 0, 1, 0);
+                       c->P.px[cu ^ 1], c->P.xf[cu], c->P.xf[cu ^ 1], c->d_btiles, 0, c->nbtile, c->d_qtiles, 0, 0, 1, 0);
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->lv_init = true;
   c->t_since_init = 0;
@@ -1990,9 +2018,9 @@ static void eager_lists(tis_ctx *c, int32_t isys) {
   const int cu = c->cur;
   Range r = range_of(c, isys);
   if (c->P.dyn) {
-    launch_lists(c, r, c->P.x[cu], c->P.px[cu], c->P.px[cu ^ 1], 1, 1);
+    launch_lists(c, r, cu, 1, 1);
   } else if (c->t_since_init % c->rebuild_every == 0) {
-    launch_lists(c, r, c->P.x[cu], c->P.px[cu], c->P.px[cu ^ 1], 1, 0);
+    launch_lists(c, r, cu, 1, 0);
     if (isys <= 0) hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
   }
 }
@@ -2001,7 +2029,7 @@ static void eager_lists(tis_ctx *c, int32_t isys) {
 static void eager_forces(tis_ctx *c, int32_t isys, int count_step) {
   const int cu = c->cur;
   Range r = range_of(c, isys);
-  launch_force_pair(c, r, c->P.x[cu ^ 1], c->P.px[cu ^ 1], c->P.x[cu], c->P.px[cu], 0, 1, count_step);
+  launch_force_pair(c, r, cu ^ 1, 0, 1, count_step);
 }
 
 static int eager_step(tis_ctx *c, int32_t isys) {
@@ -2027,12 +2055,12 @@ static int capture_graph(tis_ctx *c, int parity) {
   const bool one = !c->P.dyn && L == c->rebuild_every;
   for (int t = 0; t < L; ++t) {
     if (c->P.dyn) {
-      launch_lists(c, r, c->P.x[cu], c->P.px[cu], c->P.px[cu ^ 1], 1, 1);
+      launch_lists(c, r, cu, 1, 1);
     } else if (t % c->rebuild_every == 0) {
-      launch_lists(c, r, c->P.x[cu], c->P.px[cu], c->P.px[cu ^ 1], 1, 0);
+      launch_lists(c, r, cu, 1, 0);
       if (!one) hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
     }
-    launch_force_pair(c, r, c->P.x[cu ^ 1], c->P.px[cu ^ 1], c->P.x[cu], c->P.px[cu], t, 1, 1);
+    launch_force_pair(c, r, cu ^ 1, t, 1, 1);
     cu ^= 1;
   }
   hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)L,
@@ -2150,18 +2178,18 @@ int32_t tis_tune(tis_ctx *c, int32_t reps, int32_t *shape_out, double *ms_out) {
   for (int w = 0; w < 4; ++w)
     for (int k = 0; k < kCand; ++k) {
       c->shape = cand[k];
-      launch_force_pair(c, r, Xc(c), PXc(c), nullptr, nullptr, 0, 0);
+      launch_force_pair(c, r, c->cur, 0, 0);
     }
   std::vector<std::vector<double>> t(kCand);
   for (int rep = 0; rep < reps; ++rep) {
     // an untimed pass after the host's wait, then every candidate once,
     // starting from a different one each round
-    launch_force_pair(c, r, Xc(c), PXc(c), nullptr, nullptr, 0, 0);
+    launch_force_pair(c, r, c->cur, 0, 0);
     c->timing = true;
     c->tev_used = 0;
     for (int i = 0; i < kCand; ++i) {
       c->shape = cand[(rep + i) % kCand];
-      launch_force_pair(c, r, Xc(c), PXc(c), nullptr, nullptr, 0, 0);
+      launch_force_pair(c, r, c->cur, 0, 0);
     }
     c->timing = false;
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess) {

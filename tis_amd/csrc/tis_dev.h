@@ -61,6 +61,7 @@ struct DSys {
   int32_t ele_form, dh_type;
   double box[3];
   double exv_a, exv_dist, exv_dist_PS, exv_inf;
+  float exv_near2;           // (largest contact distance + kNearMargin)^2
   double hb_cut, margin;
   double cutoff_ele, ele_coef, cdist, rcdist, ele_rl2, dh_cut2, dh_ecut2;
   double beta_hb, tempk;
@@ -131,7 +132,7 @@ constexpr int kLdsBytes = 160 * 1024;
 // depend on the system; rows is the part of the excluded-volume lists held
 // (the rest is read from memory).
 struct WinLds {
-  int32_t x, e, g, pp, je, sptab, mask, rl2, ene, bd, ba, st, hb, qic, slot, meta, cnt, val, list, inc, incoff, nb, bdm,
+  int32_t x, xf, e, g, pp, je, sptab, mask, rl2, ene, bd, ba, st, hb, qic, slot, meta, cnt, val, list, inc, incoff, nb, bdm,
       bam, stm, hbm, hbsite, seq, qidx, qb, spec, stat, inl, total;
 };
 
@@ -142,10 +143,10 @@ __host__ __device__ inline int win_slots(const DSys &d) {
 __host__ __device__ inline WinLds win_layout(const DSys &d, int rows) {
   WinLds L;
   int32_t at = 0;
-  auto take = [&](int32_t bytes) { const int32_t o = at; at += (bytes + 7) & ~7; return o; };
+  auto take = [&](int32_t bytes) { const int32_t o = at; at += (bytes + 15) & ~15; return o; };
   const int nb3 = 24 * d.nmp, nqt = d.ele_form >= 0 ? d.nqt : 0, nq = d.ele_form >= 0 ? d.nq : 0;
   const int np = nqt * (nqt + 1) / 2, ns = win_slots(d), nv = d.hb_excess_possible ? d.nhb : 0;
-  L.x = take(nb3); L.e = take(2 * nb3); L.g = take(nb3);
+  L.x = take(nb3); L.xf = take(16 * d.nmp); L.e = take(2 * nb3); L.g = take(nb3);
   L.pp = take(np * 6 * kTile * 8);
   L.je = take(nqt * (int)sizeof(EleWave));
   L.sptab = take(d.nspecies * d.nspecies * (int)sizeof(SpPair));
@@ -169,12 +170,20 @@ __host__ __device__ inline WinLds win_layout(const DSys &d, int rows) {
   return L;
 }
 
+// Excluded-volume neighbours are sifted in FP32 first: a pair whose FP32
+// squared distance exceeds exv_near2 is beyond contact in FP64 too, by a
+// margin above the rounding of coordinates up to kNearMax (2 x 0.002 A per
+// component).  Beads farther out (or not finite) get a NaN, which no
+// comparison excludes.
+constexpr double kNearMargin = 0.05, kNearMax = 5.0e4;
+
 // All device pointers of a context, passed by value to kernels.
 struct DevPtrs {
   const DSys *sys;
   int32_t nsys, ntot, nqtot;
   // beads
   double *x[2], *px[2];      // [3][ntot] each
+  float4 *xf[2];             // [ntot] their positions in FP32 (wrapped ones of periodic systems): near_pos
   double *v, *a, *f;         // [3][ntot]
   LangClass *lcls;           // Langevin classes of every system (DSys::lc0 ..)
   const uint8_t *lcl;        // [ntot] class of each bead within its system

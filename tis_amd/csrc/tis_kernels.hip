@@ -61,6 +61,13 @@ __device__ inline void vsub(const XA &X, int a, int b, double v[3]) {
   v[0] = X(0, a) - X(0, b); v[1] = X(1, a) - X(1, b); v[2] = X(2, a) - X(2, b);
 }
 
+// The FP32 record of a bead (see kNearMargin): position and excluded-volume
+// species.
+__device__ inline float4 near_pos(double x, double y, double z, int species) {
+  const bool ok = fabs(x) <= kNearMax && fabs(y) <= kNearMax && fabs(z) <= kNearMax;
+  return make_float4(ok ? (float)x : __builtin_nanf(""), (float)y, (float)z, __int_as_float(species));
+}
+
 // The value of v at lane r (the same for every lane) of the wave.
 __device__ inline double at_lane(double v, int r) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(v);
@@ -1185,18 +1192,21 @@ __device__ inline double langevin_update(const double r[4], double rcm, double t
 }
 
 __device__ inline void integrate(const DevPtrs &P, const DSys &s, int g, const BeadState &b, const double gs[3],
-                                 const double F[3], double *XN, double *PXN, int mode, double dxo[3]) {
+                                 const double F[3], double *XN, double *PXN, float4 *XFN, int mode, double dxo[3]) {
 #pragma clang fp contract(off)
   const int n = P.ntot;
+  double y[3];
   for (int d = 0; d < 3; ++d) {
     double v = b.v[d], a = b.a[d];
     const double dx = langevin_update(b.r, b.rcm, P.tstep2, mode, F[d], gs[d], v, a);
     P.v[d * n + g] = v;
     P.a[d * n + g] = a;
     dxo[d] = dx;
-    XN[d * n + g] = b.x[d] + dx;
-    if (s.periodic) PXN[d * n + g] = b.px[d] + dx;
+    y[d] = b.x[d] + dx;
+    XN[d * n + g] = y[d];
+    if (s.periodic) { y[d] = b.px[d] + dx; PXN[d * n + g] = y[d]; }
   }
+  XFN[g] = near_pos(y[0], y[1], y[2], P.species[g]);
 }
 
 // The boxes of a tile of 64 positions (one per lane of the wave): the tile's
@@ -1230,16 +1240,10 @@ __device__ inline void tile_boxes(double p0, double p1, double p2, BBox *tile, B
 // excluded-volume neighbours in groups of four, group k of the list in E of
 // k mod 4 -- a fixed order that every pass keeps (k_main, k_window), however
 // it shares the parts out, so results are bitwise reproducible.
-__device__ inline void exv_entries(const DevPtrs &P, int g, int m0, int cnt, uint32_t e[4]) {
-  // entries past cnt re-read entry cnt - 1 (m0 < cnt) and are skipped
-#pragma unroll
-  for (int u = 0; u < 4; ++u) e[u] = P.nb[(size_t)min(m0 + u, cnt - 1) * P.ntot + g];
-}
-
 // One neighbour within its contact distance (force_exv_dt15.F90:53-115): the
 // mWCA factor (a/dr)^14 amplifies rounding 14-fold, so this formula runs in
 // FP64 (only pairs within D_ij reach it).  Returns whether it was clamped.
-__device__ inline bool exv_contact(double a, double dij, double coef, const double v[3], double d2, double F[3]) {
+__device__ inline bool exv_contact(double a, double dij, double coef, const double v[3], double d2, double (&F)[3]) {
   const double dist = sqrt(d2);
   const double dr = dist + a - dij;
   const double id = 1.0 / dr, ar = a * id, r2 = ar * ar, r6 = r2 * r2 * r2, r12 = r6 * r6;
@@ -1250,38 +1254,110 @@ __device__ inline bool exv_contact(double a, double dij, double coef, const doub
   return cl;
 }
 
-// The wave's group of four neighbours at m0, added to E[hi]; e: the group's
-// list entries (exv_entries); the entries of the wave's next group (m0 + 8)
-// are loaded into en while this group's neighbours are read
-__device__ inline void exv_group(const DevPtrs &P, const DSys &s, const double *Y, int g, int m0, int cnt,
-                                 double xi0, double xi1, double xi2, const SpPair *tab, double (&E)[2][3], bool hi,
-                                 unsigned &nclamp, const uint32_t e[4], uint32_t en[4]) {
-  const int n = P.ntot;
-  // every load of the group is issued before the arithmetic
-  double y0[4], y1[4], y2[4];
-  SpPair tp[4];
+// Excluded volume of one bead: the neighbour groups k mod 4 = k0 in E[0] and,
+// with NE = 2, k mod 4 = k0 + 2 in E[1].
+// Bound: the gathers.  Two or three of a hundred listed pairs are in contact
+// (the list radius is 11.2 A for a contact distance of 3.2 A), so the list is
+// sifted in FP32 first: one 16-byte load per neighbour (position and species),
+// eight in flight with the next eight list entries behind them, and the pairs
+// that may touch go to a queue of the lane in LDS.  The queue's pairs are
+// evaluated in FP64, two at a time: as many rounds as the fullest queue of the
+// wave needs, where evaluating in list order took a round for almost every
+// entry, some lane of 64 being in contact in it.  Each lane keeps its list
+// order, so the sums keep their bits.
+constexpr int kNearQueue = 16;
+// a wave's queue: list entries and species (LDS: k_main runs four waves per
+// SIMD up to 20 KB a block)
+struct NearQueue { uint32_t e[kNearQueue * kTile]; uint8_t sp[kNearQueue * kTile]; };
+
+template <int NE>
+__device__ inline unsigned exv_bead(const DevPtrs &P, const DSys &s, const double *Y, const float4 *XF, int g, int k0,
+                                    int cnt, const SpPair *tab, NearQueue &queue,
+                                    double (&E)[NE][3]) {
+  constexpr int kStep = NE == 2 ? 8 : 16;   // list entries from one group of the wave to the next
+  const int n = P.ntot, lane = threadIdx.x & (kTile - 1);
+  const float4 fi = XF[g];
+  unsigned nclamp = 0;
+  int nq = 0;
+  uint32_t his = 0;   // bit q: queue entry q belongs to E[1]
+  auto entries = [&](int m0, uint32_t (&e)[8]) {
+    // entries past cnt re-read entry cnt - 1 and are skipped
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int j = (int)(e[u] & kIdxMask);
-    y0[u] = Y[j]; y1[u] = Y[n + j]; y2[u] = Y[2 * n + j];
-    tp[u] = tab[P.species[j]];
-  }
-  if (m0 + 8 < cnt) exv_entries(P, g, m0 + 8, cnt, en);
-  const double a = s.exv_a;
+    for (int u = 0; u < 8; ++u) e[u] = P.nb[(size_t)min(m0 + (u & 3) + kStep * (u >> 2), cnt - 1) * n + g];
+  };
+  // kFl queue entries a round: two where the chip is idle (NE = 1), one where
+  // registers decide how many waves run
+  constexpr int kFl = NE == 1 ? 2 : 1;
+  auto flush = [&]() {
+    if (__any(nq > 0)) {
+      const double xi[3] = {Y[g], Y[n + g], Y[2 * n + g]};
+      for (int q = 0; __any(q < nq); q += kFl) {
+        if (q >= nq) continue;
+        uint32_t qe[kFl];
+        double y[kFl][3];
+        SpPair t[kFl];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    if (m0 + u >= cnt) continue;
-    double v[3] = {y0[u] - xi0, y1[u] - xi1, y2[u] - xi2};
-    if (s.periodic) {
-      const int code = (int)(e[u] >> kMirrorShift);
-      for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, code, d);
+        for (int u = 0; u < kFl; ++u) {
+          const int at = min(q + u, nq - 1) * kTile + lane;
+          qe[u] = queue.e[at];
+          const int j = (int)(qe[u] & kIdxMask);
+          y[u][0] = Y[j]; y[u][1] = Y[n + j]; y[u][2] = Y[2 * n + j];
+          t[u] = tab[queue.sp[at]];
+        }
+#pragma unroll
+        for (int u = 0; u < kFl; ++u) {
+          if (q + u >= nq) continue;
+          double v[3] = {y[u][0] - xi[0], y[u][1] - xi[1], y[u][2] - xi[2]};
+          if (s.periodic) {
+            const int code = (int)(qe[u] >> kMirrorShift);
+            for (int d = 0; d < 3; ++d) v[d] += mirror_shift(s, code, d);
+          }
+          const double d2 = dot3(v, v);
+          if (d2 > t[u].dij2) continue;
+          const bool cl = NE == 2 && ((his >> (q + u)) & 1u) ? exv_contact(s.exv_a, t[u].dij, t[u].coef, v, d2, E[NE - 1])
+                                                     : exv_contact(s.exv_a, t[u].dij, t[u].coef, v, d2, E[0]);
+          if (cl && g < (int)(qe[u] & kIdxMask)) ++nclamp;
+        }
+      }
     }
-    const SpPair t = tp[u];
-    const double d2 = dot3(v, v);
-    if (d2 > t.dij2) continue;
-    const bool cl = hi ? exv_contact(a, t.dij, t.coef, v, d2, E[1]) : exv_contact(a, t.dij, t.coef, v, d2, E[0]);
-    if (cl && g < (int)(e[u] & kIdxMask)) ++nclamp;
+    nq = 0;
+    his = 0;
+  };
+  // (the entries in flight do not live across a flush: registers)
+  int m0 = 4 * k0;
+  while (__any(m0 < cnt)) {
+    uint32_t e[8] = {}, en[8] = {};
+    if (m0 < cnt) entries(m0, e);
+    do {
+      if (m0 < cnt) {
+        float4 f[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) f[u] = XF[e[u] & kIdxMask];
+        if (m0 + 2 * kStep < cnt) entries(m0 + 2 * kStep, en);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          float v0 = f[u].x - fi.x, v1 = f[u].y - fi.y, v2 = f[u].z - fi.z;
+          if (s.periodic) {
+            const int code = (int)(e[u] >> kMirrorShift);
+            v0 += (float)mirror_shift(s, code, 0); v1 += (float)mirror_shift(s, code, 1);
+            v2 += (float)mirror_shift(s, code, 2);
+          }
+          const bool far = v0 * v0 + v1 * v1 + v2 * v2 > s.exv_near2;
+          if (!far && m0 + (u & 3) + kStep * (u >> 2) < cnt) {
+            queue.e[nq * kTile + lane] = e[u];
+            queue.sp[nq * kTile + lane] = (uint8_t)__float_as_int(f[u].w);
+            if (NE == 2) his |= (uint32_t)(u >> 2) << nq;
+            ++nq;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) e[u] = en[u];
+      }
+      m0 += 2 * kStep;
+    } while (__any(m0 < cnt) && !__any(nq > kNearQueue - 8));
+    flush();
   }
+  return nclamp;
 }
 
 // The two largest values over the wave (merge of top-2 pairs).
@@ -1351,30 +1427,40 @@ __device__ inline uint64_t noise_step(const DevPtrs &P, const DSys &s, int32_t t
   return *P.stepbase + (uint64_t)t_local + (mode == 2 ? 0u : 1u) - s.step_origin;
 }
 
-// Forces of one bead from the two waves' partial sums, then the integrator
-// with the noise gs; returns the squared displacement since the last
+// A bead's force stored, then the integrator with the noise gs; returns the squared displacement since the last
 // rebuild before this step's update (and accumulates the update) when
 // rebuilds are displacement-triggered.
-__device__ inline double main_tail(const DevPtrs &P, const DSys &s, int g, const double S[3], const double E02[3],
-                                   double (*red)[2][kTile], const BeadState &b, const double gs[3], int lane, double *XN, double *PXN,
-                                   int mode) {
+__device__ inline double main_tail(const DevPtrs &P, const DSys &s, int g, const double F[3], const BeadState &b,
+                                   const double gs[3], double *XN, double *PXN, float4 *XFN, int mode) {
   const int n = P.ntot;
-  double F[3];
-  for (int d = 0; d < 3; ++d) F[d] = (S[d] + red[d][0][lane]) + (E02[d] + red[d][1][lane]);
   P.f[g] = F[0]; P.f[n + g] = F[1]; P.f[2 * n + g] = F[2];
   if (mode == 0) return -1.0;
   double dx[3];
-  integrate(P, s, g, b, gs, F, XN, PXN, resolve_mode(s, mode), dx);
+  integrate(P, s, g, b, gs, F, XN, PXN, XFN, resolve_mode(s, mode), dx);
   if (!P.dyn) return -1.0;
   return accumulate_displacement(P, g, b.o, dx);
 }
 
 
-__global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, const double *PX,
-                                                    double *XN, double *PXN, const Tile *tiles,
-                                                    int ntile, int32_t t_local, int mode, int do_dh,
-                                                    int count_step) {
-  __shared__ double red[3][2][kTile], gsh[3][kTile];
+// XW = 0: two waves share a tile of 64 beads: wave 0 sums each bead's bonded
+// slots, wave 1 draws its Langevin noise and adds its electrostatic sums, and
+// each takes half of the excluded-volume groups; XW = 4: those two and four
+// more waves, each a quarter of the groups, for launches that leave the chip
+// idle, where a tile's chain of loads sets the time.  Wave 0 integrates after
+// the barrier, from state loaded before it.
+// Bound: latency (incidence -> slot; list entry -> position; contact pairs),
+// four waves per SIMD; then the state and slots it moves (75 MB).  576
+// systems, 237,111 beads: 33.2 us with every listed pair evaluated in FP64,
+// 26.8 sifted (19.6 without excluded volume, 21.3 without the slots).  A
+// 2,000-nt chain (94 tiles): 12.0 us, 11.5 sifted by two waves, 9.5 by six;
+// 10 tiles: 8.4 by two, 5.7 by six.
+template <int XW>
+__global__ __launch_bounds__(kTile *(2 + XW)) __attribute__((amdgpu_waves_per_eu(4))) void k_main(
+    DevPtrs P, const double *X, const double *PX, const float4 *XF, double *XN, double *PXN, float4 *XFN,
+    const Tile *tiles, int ntile, int32_t t_local, int mode, int do_dh, int count_step) {
+  constexpr int kEw = XW ? XW : 2;   // waves with excluded-volume groups
+  __shared__ double red[2][3][kTile], rex[kEw][3][kTile], gsh[3][kTile];
+  __shared__ NearQueue queue[kEw];
   if (run_stopped(P)) return;
   // steps completed in the current run (the host resumes a stopped run
   // after the last of them)
@@ -1390,9 +1476,8 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
   const bool valid = li < s.nmp;
   const int g = s.off + (valid ? li : 0);
   const int n = P.ntot;
-  // wave 0: the bonded slots S, wave 1: the electrostatic sums Q, in F; both:
-  // their excluded-volume groups (k mod 4 = w and w + 2) in E
-  double F[3] = {0.0, 0.0, 0.0}, E[2][3] = {};
+  // wave 0: the bonded slots S, wave 1: the electrostatic sums Q, in F
+  double F[3] = {0.0, 0.0, 0.0};
   if (valid) {
     if (w == 1) {
       // the Langevin noise of the bead (wave 0 integrates after the
@@ -1404,12 +1489,12 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
         gsh[0][lane] = gs[0]; gsh[1][lane] = gs[1]; gsh[2][lane] = gs[2];
       }
       if (do_dh && s.ele_form >= 0) ele_sums(P, s, g, F);
-    } else {
+    } else if (w == 0) {
       // bonded slots in incidence order, eight loads in flight at a time
       // (slots past ie re-read slot ie - 1 and are not added)
       // (the next eight slot indices load while these slots are read)
       const int ib = P.inc_off[g], ie = P.inc_off[g + 1];
-      int64_t at[8] = {}, atn[8] = {};
+      int32_t at[8] = {}, atn[8] = {};
       if (ib < ie) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) at[u] = P.inc_slot[min(ib + u, ie - 1)];
@@ -1418,7 +1503,7 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
         float sl[8][3];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const float *q = P.fslot + 3 * at[u];
+          const float *q = P.fslot + 3 * (int64_t)at[u];
           sl[u][0] = q[0]; sl[u][1] = q[1]; sl[u][2] = q[2];
         }
         if (k0 + 8 < ie) {
@@ -1432,26 +1517,19 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
         for (int u = 0; u < 8; ++u) at[u] = atn[u];
       }
     }
-    // excluded volume (force_exv_dt15.F90:53-115), owner view of each pair;
-    // the two waves take alternate groups of four neighbours
-    const double *Y = s.periodic ? PX : X;
-    const double xi0 = Y[g], xi1 = Y[n + g], xi2 = Y[2 * n + g];
-    const SpPair *tab = P.sptab + s.sptab + (int)P.species[g] * s.nspecies;
-    const int cnt = min(P.nb_cnt[g], P.nb_cap);
-    unsigned nclamp = 0;
-    uint32_t e[4] = {0u, 0u, 0u, 0u}, en[4] = {0u, 0u, 0u, 0u};
-    if (4 * w < cnt) exv_entries(P, g, 4 * w, cnt, e);
-    for (int m0 = 4 * w; m0 < cnt; m0 += 8) {
-      exv_group(P, s, Y, g, m0, cnt, xi0, xi1, xi2, tab, E, (m0 & 8) != 0, nclamp, e, en);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) e[u] = en[u];
+    if (w < 2)
+      for (int d = 0; d < 3; ++d) red[w][d][lane] = F[d];
+    // excluded volume (force_exv_dt15.F90:53-115), owner view of each pair
+    if (XW == 0 || w >= 2) {
+      const int k0 = XW ? w - 2 : w;
+      const double *Y = s.periodic ? PX : X;
+      const SpPair *tab = P.sptab + s.sptab + (int)P.species[g] * s.nspecies;
+      double E[XW ? 1 : 2][3] = {};
+      const unsigned nclamp = exv_bead(P, s, Y, XF, g, k0, min(P.nb_cnt[g], P.nb_cap), tab, queue[k0], E);
+      if (nclamp) atomicAdd(&P.counters[0], (unsigned long long)nclamp);
+      for (int d = 0; d < 3; ++d) rex[k0][d][lane] = XW ? E[0][d] : E[0][d] + E[XW ? 0 : 1][d];
     }
-    if (nclamp) atomicAdd(&P.counters[0], (unsigned long long)nclamp);
   }
-  double Ew[3];   // wave 0: E0 + E2, wave 1: E1 + E3
-  for (int d = 0; d < 3; ++d) Ew[d] = E[0][d] + E[1][d];
-  if (w == 1)
-    for (int d = 0; d < 3; ++d) { red[d][0][lane] = F[d]; red[d][1][lane] = Ew[d]; }
   BeadState bs;
   if (w == 0 && valid && mode != 0) load_state(P, s, g, X, PX, bs);
   __syncthreads();
@@ -1459,7 +1537,12 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
   double d2 = -1.0;   // squared displacement since the last rebuild, before this update
   if (valid) {
     const double gs[3] = {gsh[0][lane], gsh[1][lane], gsh[2][lane]};
-    d2 = main_tail(P, s, g, F, Ew, red, bs, gs, lane, XN, PXN, mode);
+    for (int d = 0; d < 3; ++d) {
+      const double E02 = XW ? rex[0][d][lane] + rex[kEw - 2][d][lane] : rex[0][d][lane];
+      const double E13 = XW ? rex[1][d][lane] + rex[kEw - 1][d][lane] : rex[1][d][lane];
+      F[d] = (red[0][d][lane] + red[1][d][lane]) + (E02 + E13);
+    }
+    d2 = main_tail(P, s, g, F, bs, gs, XN, PXN, XFN, mode);
   }
   if (P.dyn && mode != 0) {
     const int it = s.bt0 + tl.start / kTile;
@@ -1484,24 +1567,34 @@ __global__ __launch_bounds__(kTile * 2) void k_main(DevPtrs P, const double *X, 
   }
 }
 
+template __global__ void k_main<0>(DevPtrs, const double *, const double *, const float4 *, double *, double *,
+                                   float4 *, const Tile *, int, int32_t, int, int, int);
+template __global__ void k_main<4>(DevPtrs, const double *, const double *, const float4 *, double *, double *,
+                                   float4 *, const Tile *, int, int32_t, int, int, int);
+
 // ------------------------------------------------------------------ lists
 // util_periodic.F90:26-36 on the current coordinates; with with_pred the
 // predicted wrapped positions px + (c4 v + dt^2/2 a) are refreshed too.
 __device__ inline void wrap_bead(const DevPtrs &P, const DSys &s, const double *X, double *PXc, double *PXp,
-                                 int g, int with_pred) {
+                                 float4 *XFc, float4 *XFp, int g, int with_pred) {
 #pragma clang fp contract(off)
   const int n = P.ntot;
+  double yc[3], yp[3] = {0.0, 0.0, 0.0};
   for (int d = 0; d < 3; ++d) {
     double pw = s.box[d], pmax = 0.5 * pw, pmin = -0.5 * pw;
     double tx = X[d * n + g];
     if (tx > pmax) tx = tx - pw * (double)((int)((tx - pmax) / pw) + 1);
     else if (tx < pmin) tx = tx + pw * (double)((int)((pmin - tx) / pw) + 1);
+    yc[d] = tx;
     PXc[d * n + g] = tx;
     if (with_pred) {
       double dx = P.lcls[s.lc0 + P.lcl[g]].r[3] * P.v[d * n + g] + P.tstep2 * P.a[d * n + g];
-      PXp[d * n + g] = tx + dx;
+      yp[d] = tx + dx;
+      PXp[d * n + g] = yp[d];
     }
   }
+  XFc[g] = near_pos(yc[0], yc[1], yc[2], P.species[g]);
+  if (with_pred) XFp[g] = near_pos(yp[0], yp[1], yp[2], P.species[g]);
 }
 
 // DT15 keep rule for lo < hi (neighbor_assign.F90:481-559)
@@ -2031,8 +2124,14 @@ __device__ inline bool system_trigger(const DevPtrs &P, const DSys &s) {
   return sqrt(a) + sqrt(b) > s.margin;
 }
 
-__global__ __launch_bounds__(kTile) void k_prep(DevPtrs P, const double *X, double *PXc, double *PXp,
-                                                const Tile *btiles, int bt0, int nbt, const Tile *qtiles, int qt0,
+// the FP32 positions of [g0, g0 + n) from x (state uploads)
+__global__ __launch_bounds__(256) void k_near(DevPtrs P, const double *X, float4 *XF, int g0, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, g = g0 + i, N = P.ntot;
+  if (i < n) XF[g] = near_pos(X[g], X[N + g], X[2 * (size_t)N + g], P.species[g]);
+}
+
+__global__ __launch_bounds__(kTile) void k_prep(DevPtrs P, const double *X, double *PXc, double *PXp, float4 *XFc,
+                                                float4 *XFp, const Tile *btiles, int bt0, int nbt, const Tile *qtiles, int qt0,
                                                 int nqt, int with_pred, int gate) {
   if (run_stopped(P)) return;
   const int b = (int)blockIdx.x;
@@ -2051,7 +2150,7 @@ __global__ __launch_bounds__(kTile) void k_prep(DevPtrs P, const double *X, doub
     const int li = tl.start + (int)threadIdx.x;
     if (li < s.nmp) {
       const int g = s.off + li, n = P.ntot;
-      if (s.periodic) wrap_bead(P, s, X, PXc, PXp, g, with_pred);
+      if (s.periodic) wrap_bead(P, s, X, PXc, PXp, XFc, XFp, g, with_pred);
       if (gate)
         for (int d = 0; d < 3; ++d) P.dxyz[d * n + g] = P.dlast[d * n + g];
     }
@@ -2190,6 +2289,7 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
   if (from == n && cb == ce) return;
   const WinLds L = win_layout(s, rows);
   const int tid = (int)threadIdx.x, lane = tid & (kTile - 1), w = tid / kTile, N = P.ntot, nb = s.nmp;
+  float4 *xf = (float4 *)(lds + L.xf);
   double *x = (double *)(lds + L.x), *e = (double *)(lds + L.e), *gn = (double *)(lds + L.g),
          *pp = (double *)(lds + L.pp), *hene = (double *)(lds + L.ene), *rl2 = (double *)(lds + L.rl2),
          *bdp = (double *)(lds + L.bd), *bap = (double *)(lds + L.ba), *stp = (double *)(lds + L.st),
@@ -2231,6 +2331,7 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
   const int ib0 = P.inc_off[s.off];
   if (own) {
     for (int d = 0; d < 3; ++d) x[d * nb + tid] = XP[(size_t)d * N + g];
+    xf[tid] = near_pos(x[tid], x[nb + tid], x[2 * nb + tid], P.species[g]);
     meta[tid] = (uint32_t)(uint8_t)P.mptype[g] | (uint32_t)(uint8_t)P.iclass[g] << 8 | (uint32_t)P.unit[g] << 16;
     incoff[tid] = (uint16_t)(P.inc_off[g] - ib0);
     qidx[tid] = (int16_t)(nq > 0 && P.qidx[g] >= 0 ? P.qidx[g] - s.qoff : -1);
@@ -2549,45 +2650,39 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
         // h + 2 (exv_group's order)
         const int h = k & 1, i = (k >> 1) * kTile + lane;
         if (i < nb) {
-          const double xi0 = x[i], xi1 = x[nb + i], xi2 = x[2 * nb + i];
-          const int cnt = nbc[i];
+          const double xi[3] = {x[i], x[nb + i], x[2 * nb + i]};
+          const float4 fi = xf[i];
+          const int cnt = nbc[i], half = (cnt >> 3) * 4 + min(max((cnt & 7) - 4 * h, 0), 4);   // its entries
           const SpPair *tab = sptab + (int)spec[i] * s.nspecies;
           double E[2][3] = {};
-          int en[4], enn[4] = {0, 0, 0, 0};
-          auto entries = [&](int m0, int (&o)[4]) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int m = min(m0 + u, cnt - 1);
-              if (m < rows) {
-                o[u] = list[m * nb + i];
-              } else {
-                const int j = (int)(P.nb[(size_t)m * N + s.off + i] & kIdxMask) - s.off;
-                o[u] = j | (int)spec[j] << 10;
-              }
-            }
+          // entry q of the half
+          auto entry = [&](int q) {
+            const int m = (q >> 2) * 8 + 4 * h + (q & 3);
+            if (m < rows) return (int)list[m * nb + i];
+            const int j = (int)(P.nb[(size_t)m * N + s.off + i] & kIdxMask) - s.off;
+            return j | (int)spec[j] << 10;
           };
-          if (4 * h < cnt) entries(4 * h, en);
-          for (int m0 = 4 * h; m0 < cnt; m0 += 8) {
-            double d2[4], dv[4][3], lim[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int j = en[u] & 1023;
-              dv[u][0] = x[j] - xi0; dv[u][1] = x[nb + j] - xi1; dv[u][2] = x[2 * nb + j] - xi2;
-              lim[u] = tab[en[u] >> 10].dij2;
+          // sifted in FP32, 32 entries at a time, as in exv_bead; the pairs
+          // that may touch then in FP64
+          for (int q0 = 0; q0 < half; q0 += 32) {
+            uint32_t near = 0;
+#pragma unroll 4
+            for (int q = q0; q < min(q0 + 32, half); ++q) {
+              const float4 f = xf[entry(q) & 1023];
+              const float v0 = f.x - fi.x, v1 = f.y - fi.y, v2 = f.z - fi.z;
+              const bool far = v0 * v0 + v1 * v1 + v2 * v2 > s.exv_near2;
+              near |= (uint32_t)(far ? 0 : 1) << (q - q0);
             }
-            if (m0 + 8 < cnt) entries(m0 + 8, enn);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) d2[u] = dot3(dv[u], dv[u]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              if (m0 + u >= cnt || d2[u] > lim[u]) continue;
-              const SpPair tp = tab[en[u] >> 10];
-              const bool cl = (m0 & 8) ? exv_contact(s.exv_a, tp.dij, tp.coef, dv[u], d2[u], E[1])
-                                       : exv_contact(s.exv_a, tp.dij, tp.coef, dv[u], d2[u], E[0]);
-              if (cl && i < (en[u] & 1023)) ++clamp_exv;
+            for (; near; near &= near - 1) {
+              const int q = q0 + (int)__builtin_ctz(near), en = entry(q), j = en & 1023;
+              const double v[3] = {x[j] - xi[0], x[nb + j] - xi[1], x[2 * nb + j] - xi[2]};
+              const double d2 = dot3(v, v);
+              const SpPair tp = tab[en >> 10];
+              if (d2 > tp.dij2) continue;
+              const bool cl = q & 4 ? exv_contact(s.exv_a, tp.dij, tp.coef, v, d2, E[1])
+                                    : exv_contact(s.exv_a, tp.dij, tp.coef, v, d2, E[0]);
+              if (cl && i < j) ++clamp_exv;
             }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) en[u] = enn[u];
           }
           for (int d = 0; d < 3; ++d) e[(3 * h + d) * nb + i] = E[0][d] + E[1][d];
         }
@@ -2642,6 +2737,7 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
         x[d * nb + tid] = xp[d];
         if (last) P.f[(size_t)d * N + g] = F;
       }
+      xf[tid] = near_pos(xp[0], xp[1], xp[2], spec[tid]);
       if (q >= 0) {
         EleWave &E = je[q / kTile];
         const int c = stage_at(q % kTile, dir);
@@ -2664,6 +2760,10 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
   // ---- the state back: at the end of the launch, or (t < n) before the step
   // whose rebuild overflowed, in the buffers of the launch's start
   const int cw = t == n ? ce : cu;
+  if (own) {
+    P.xf[cw][g] = near_pos(xc[0], xc[1], xc[2], spec[tid]);
+    P.xf[cw ^ 1][g] = xf[tid];
+  }
   if (own)
     for (int d = 0; d < 3; ++d) {
       const size_t o = (size_t)d * N + g;
