@@ -37,7 +37,9 @@ __global__ void k_lpair(DevPtrs, const double *, const double *, const EwTask *,
                         int, int);
 __global__ void k_advance(uint64_t *, uint64_t, uint64_t, uint64_t, unsigned long long *);
 __global__ void k_window(DevPtrs, const int32_t *, int, int, int, int, int);
-__global__ void k_count_rebuild(unsigned long long *);
+__global__ void k_run_report(unsigned long long *, unsigned long long *);
+__global__ void k_state_out(const double *, int, int, int, double *, const unsigned long long *, unsigned long long *);
+__global__ void k_state_in(DevPtrs, double *, int, int, const double *, float4 *);
 __global__ void k_energy(DevPtrs, const double *, const double *, const EwTask *, const int32_t *, int, double *, int);
 __global__ void k_energy_sum(const int32_t *, const int32_t *, int, const double *, double *, int);
 __global__ void k_label_apply(DevPtrs, LabelDev, const int32_t *, const int32_t *, const double *);
@@ -100,7 +102,7 @@ struct ArenaBufs {
          *st_coef = nullptr, *tst_nat = nullptr, *tst_coef = nullptr, *hb_nat = nullptr, *hb_coef = nullptr;
   int32_t *tst2st = nullptr, *tst_excl = nullptr, *tst_sys = nullptr, *hb_site = nullptr, *hb_tert = nullptr,
           *hb_sys = nullptr, *site_val = nullptr, *st_exoff = nullptr, *st_ex = nullptr, *ststat = nullptr;
-  double *ewh = nullptr, *ewc = nullptr, *energy = nullptr;
+  double *ewh = nullptr, *ewc = nullptr;
   unsigned long long *counters = nullptr;
   uint64_t *stepbase = nullptr;
 };
@@ -170,14 +172,10 @@ struct tis_ctx {
   int32_t win_rows = 0, win_lds = 0;     // its list rows and bytes in LDS; win_lds 0: per-step passes
   std::vector<int32_t> systask_of;       // index into d_systask per system or -1
   int32_t *d_ststat = nullptr;           // st_status output of tis_term_status [nsttot]
-  double *d_energy = nullptr;
   EwTask *d_etask = nullptr;             // energy tasks (system, part, parts) in live order
   int32_t *d_efirst = nullptr;           // first task of each live system, and the end
   double *d_epart = nullptr;             // their sums [n_etask][kEnergyTerms]
   int32_t n_etask = 0;
-  int32_t *d_eset = nullptr;             // tis_energy_sumup_set: live positions, then task list
-  double *d_eset_out = nullptr;
-  size_t eset_cap = 0, eset_out_cap = 0;
   double *d_eunit = nullptr;   // raw per-unit-pair energies [nunit^2][25], then their parts
   size_t eunit_cap = 0;
   unsigned long long *d_counters = nullptr;
@@ -195,6 +193,14 @@ struct tis_ctx {
   int32_t rebuild_every = 10;
   int64_t t_since_init = 0;
   uint64_t step_host = 0;                // the device step counter (stepbase) as the host knows it
+  // one block of pinned host memory that kernels read and write themselves:
+  // a report of two words (k_run_report, k_state_out), a ring that calls'
+  // inputs are copied into (the stream is waited for when it comes round),
+  // and the outputs of a call that waits for them
+  char *pin = nullptr, *pin_in = nullptr, *pin_out = nullptr;
+  size_t pin_in_cap = 0, pin_in_at = 0, pin_out_cap = 0;
+  unsigned long long *report = nullptr;
+  int64_t rebuilds_host = 0;             // whole-batch rebuilds counted by the host (TIS_CNT_REBUILDS)
   // payload bytes since creation: uploads of topology and launch tables,
   // state uploads (tis_state_set), state downloads (tis_state_get), state
   // carried device to device by a new arena layout
@@ -221,9 +227,6 @@ struct tis_ctx {
   bool labels_dirty = false;
   std::vector<void *> label_bufs;         // device copies of the label sets
   LabelDev label_dev{};
-  int32_t *d_lab_args = nullptr;          // [2][cap] isys, label
-  double *d_lab_scale = nullptr;          // [cap]
-  int32_t lab_cap = 0;
 };
 
 namespace tis {
@@ -254,6 +257,55 @@ int fail(tis_ctx *c, int code, const char *fmt, ...) {
     if (e_ != hipSuccess)                                                               \
       return fail(ctx, TIS_ERR_HIP, "%s failed: %s", #expr, hipGetErrorString(e_));     \
   } while (0)
+
+// The pinned block with at least `in` bytes of ring and `out` bytes of output
+// (64 KB in all if that is enough: larger blocks cost hundreds of
+// microseconds, which is why a batch's is laid out at its upload).
+int pin_reserve(tis_ctx *c, size_t in, size_t out) {
+  if (c->pin && in <= c->pin_in_cap && out <= c->pin_out_cap) return 0;
+  constexpr size_t kHead = 256, kSmall = 64 << 10;
+  in = std::max((in + 255) & ~(size_t)255, c->pin_in_cap);
+  out = std::max((out + 255) & ~(size_t)255, c->pin_out_cap);
+  if (kHead + in + out < kSmall) in = kSmall - kHead - out;
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if (c->pin) (void)hipHostFree(c->pin);
+  c->pin = nullptr;
+  c->pin_in_cap = c->pin_in_at = c->pin_out_cap = 0;
+  const hipError_t e = hipHostMalloc((void **)&c->pin, kHead + in + out);
+  if (e != hipSuccess) {
+    c->pin = nullptr;
+    return fail(c, TIS_ERR_NOMEM, "hipHostMalloc(%zu) failed: %s", kHead + in + out, hipGetErrorString(e));
+  }
+  c->report = (unsigned long long *)c->pin;
+  c->pin_in = c->pin + kHead;
+  c->pin_out = c->pin_in + in;
+  c->pin_in_cap = in;
+  c->pin_out_cap = out;
+  c->report[0] = c->report[1] = 0;
+  return 0;
+}
+
+// room for `bytes` of a call's input in the ring: the memory may be read by
+// kernels queued after this call, and is reused after the stream has caught up
+int pin_input(tis_ctx *c, size_t bytes, void **p) {
+  bytes = (bytes + 255) & ~(size_t)255;
+  if (int rc = pin_reserve(c, bytes, 0)) return rc;
+  if (c->pin_in_at + bytes > c->pin_in_cap) {
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->pin_in_at = 0;
+  }
+  *p = c->pin_in + c->pin_in_at;
+  c->pin_in_at += bytes;
+  return 0;
+}
+
+// room for `bytes` of output of the call in hand, which waits for the stream
+// before it reads them (taken before the call's inputs: growth moves both)
+int pin_output(tis_ctx *c, size_t bytes, void **p) {
+  if (int rc = pin_reserve(c, 0, bytes)) return rc;
+  *p = c->pin_out;
+  return 0;
+}
 
 template <typename T>
 int dalloc(tis_ctx *c, T **p, size_t n) {
@@ -319,6 +371,7 @@ void free_all(tis_ctx *c) {
   c->d_eunit = nullptr;
   c->eunit_cap = 0;
   c->nsys = c->nbeads = c->nlive = 0;
+  c->rebuilds_host = 0;
   c->lists_valid = false;
   c->lv_init = false;
 }
@@ -912,7 +965,7 @@ int alloc_arena(tis_ctx *c, const Caps &k, std::vector<void *> &list, DevPtrs &P
   AL(P.sys_flag, k.nsys); AL(P.win_at, k.nsys);
   AL(P.pp, k.pp); AL(P.qmask, k.m); AL(P.qmirror, k.mi); AL(P.lcnt, k.lp * kTile);
   AL(A.ewh, 3 * k.k); AL(A.ewc, k.k); AL(P.psk, k.psk); AL(P.pf, k.pf);
-  AL(A.counters, TIS_CNT_MAX); AL(A.stepbase, 1); AL(A.energy, 25 * k.nsys);
+  AL(A.counters, TIS_CNT_MAX); AL(A.stepbase, 1);
 #undef AL
   P.lcl = A.lcl; P.lcls = A.lcls; P.mass = A.mass; P.exv_rad = A.exv_rad; P.charge = A.charge; P.rl2 = A.rl2;
   P.mptype = A.mptype; P.iclass = A.iclass; P.unit = A.unit; P.qidx = A.qidx; P.qbead = A.qbead;
@@ -1208,7 +1261,7 @@ int relayout(tis_ctx *c, const std::vector<const tis_system *> &extra, double gr
   c->ab = A;
   c->caps = caps;
   c->stage = std::move(g);
-  c->d_sys = A.sys; c->d_ststat = A.ststat; c->d_energy = A.energy;
+  c->d_sys = A.sys; c->d_ststat = A.ststat;
   c->d_counters = A.counters; c->d_stepbase = A.stepbase;
   c->d_eunit = nullptr;
   c->eunit_cap = 0;
@@ -1292,6 +1345,11 @@ int append_systems(tis_ctx *c, int32_t nadd, const tis_system *sys, const uint32
   }
   int rc = upload_stage(c, c->stage, m);
   if (rc) return rc;
+  int32_t most = 0;
+  for (const HostSys &h : c->hs)
+    if (h.live) most = std::max(most, h.d.nmp);
+  const size_t one = 3 * sizeof(double) * (size_t)most;
+  if ((rc = pin_reserve(c, one, std::max(one, 25 * sizeof(double) * (size_t)c->nsys)))) return rc;
   c->nbeads = c->stage.nbead; c->nqtot = c->stage.nq; c->nhbtot = c->stage.nhb; c->ntsttot = c->stage.ntst;
   c->nsttot = c->stage.nst;
   return build_tables(c);
@@ -1339,10 +1397,7 @@ int32_t tis_ctx_destroy(tis_ctx *c) {
   free_all(c);
   bd_free(c);
   for (void *p : c->label_bufs) (void)hipFree(p);
-  if (c->d_lab_args) (void)hipFree(c->d_lab_args);
-  if (c->d_lab_scale) (void)hipFree(c->d_lab_scale);
-  if (c->d_eset) (void)hipFree(c->d_eset);
-  if (c->d_eset_out) (void)hipFree(c->d_eset_out);
+  if (c->pin) (void)hipHostFree(c->pin);
   for (hipEvent_t e : c->tev) (void)hipEventDestroy(e);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -1456,24 +1511,26 @@ int32_t tis_state_set(tis_ctx *c, int32_t isys, int32_t which, const double *buf
   if (isys < 0) return fail(c, TIS_ERR_ARG, "tis_state_set needs one system");
   HIPCHK(c, hipSetDevice(c->device));
   const HostSys &h = c->hs[isys];
-  double *base = which == 0 ? Xc(c) : (which == 1 ? c->P.v : c->P.a);
   if (which < 0 || which > 2) return fail(c, TIS_ERR_ARG, "bad state index %d", which);
-  std::vector<double> comp(h.d.nmp);
-  for (int d = 0; d < 3; ++d) {
-    for (int i = 0; i < h.d.nmp; ++i) comp[i] = buf[3 * i + d];
-    HIPCHK(c, hipMemcpyAsync(base + (size_t)d * c->P.ntot + h.d.off, comp.data(), comp.size() * sizeof(double),
-                             hipMemcpyHostToDevice, c->stream));
-    c->h2d_state += (int64_t)(comp.size() * sizeof(double));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-  }
-  if (which == 0) {
-    c->lists_valid = false;
-    c->lv_init = false;
-    if (!h.d.periodic)
-      hipLaunchKernelGGL(k_near, dim3((h.d.nmp + 255) / 256), dim3(256), 0, c->stream, c->P, Xc(c), c->P.xf[c->cur],
-                         h.d.off, h.d.nmp);
-  }
+  double *base = which == 0 ? Xc(c) : (which == 1 ? c->P.v : c->P.a);
+  const size_t bytes = 3 * (size_t)h.d.nmp * sizeof(double);
+  void *in = nullptr;
+  if ((rc = pin_input(c, bytes, &in))) return rc;
+  std::memcpy(in, buf, bytes);
+  hipLaunchKernelGGL(k_state_in, dim3((h.d.nmp + 255) / 256), dim3(256), 0, c->stream, c->P, base, h.d.off, h.d.nmp,
+                     (const double *)in, which == 0 && !h.d.periodic ? c->P.xf[c->cur] : (float4 *)nullptr);
+  HIPCHK(c, hipGetLastError());
+  c->h2d_state += (int64_t)bytes;
+  if (which == 0) { c->lists_valid = false; c->lv_init = false; }
   return TIS_OK;
+}
+
+// `n` beads of base at off into the pinned buffer out (n = 0: none), and the
+// overflow flag to c->report when asked
+static void launch_state_out(tis_ctx *c, const double *base, int off, int n, void *out, bool report) {
+  hipLaunchKernelGGL(k_state_out, dim3((3 * n + 255) / 256 + (n == 0 ? 1 : 0)), dim3(256), 0, c->stream, base,
+                     c->P.ntot, off, n, (double *)out, (const unsigned long long *)c->d_counters,
+                     report ? c->report : nullptr);
 }
 
 int32_t tis_state_get(tis_ctx *c, int32_t isys, int32_t which, double *buf) {
@@ -1485,39 +1542,46 @@ int32_t tis_state_get(tis_ctx *c, int32_t isys, int32_t which, double *buf) {
   HIPCHK(c, hipSetDevice(c->device));
   const HostSys &h = c->hs[isys];
   const double *base = which == 0 ? Xc(c) : (which == 1 ? c->P.v : (which == 2 ? c->P.a : c->P.f));
-  std::vector<double> comp(h.d.nmp);
-  for (int d = 0; d < 3; ++d) {
-    HIPCHK(c, hipMemcpyAsync(comp.data(), base + (size_t)d * c->P.ntot + h.d.off, comp.size() * sizeof(double),
-                             hipMemcpyDeviceToHost, c->stream));
-    c->d2h_bytes += (int64_t)(comp.size() * sizeof(double));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (int i = 0; i < h.d.nmp; ++i) buf[3 * i + d] = comp[i];
-  }
+  const size_t bytes = 3 * (size_t)h.d.nmp * sizeof(double);
+  void *out = nullptr;
+  if ((rc = pin_output(c, bytes, &out))) return rc;
+  launch_state_out(c, base, h.d.off, h.d.nmp, out, false);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  std::memcpy(buf, out, bytes);
+  c->d2h_bytes += (int64_t)bytes;
   return TIS_OK;
 }
 
+// larger list capacity for `need` entries (nb keeps its stride); captured
+// graphs hold the old one
+static int new_nb(tis_ctx *c, unsigned long long need) {
+  const int newcap = (int)(need + need / 2 + 16);
+  uint32_t *nb = nullptr;
+  int rc = dalloc(c, &nb, (size_t)newcap * c->P.ntot);
+  if (rc) return rc;
+  c->P.nb = nb;  // the old buffer stays in allocs until the batch is freed
+  c->P.nb_cap = newcap;
+  for (int k = 0; k < 2; ++k)
+    if (c->graph[k]) { (void)hipGraphExecDestroy(c->graph[k]); c->graph[k] = nullptr; }
+  return TIS_OK;
+}
+
+// The lists of the range, built again with a larger capacity as long as they
+// overflow it (the flag is zero between calls).
 static int rebuild_lists(tis_ctx *c, int32_t isys) {
   Range r = range_of(c, isys);
   for (int attempt = 0; attempt < 4; ++attempt) {
-    HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
     launch_lists(c, r, c->cur, 0, 0);
-    hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
+    launch_state_out(c, nullptr, 0, 0, nullptr, true);
     HIPCHK(c, hipGetLastError());
-    unsigned long long ovf = 0;
-    HIPCHK(c, hipMemcpyAsync(&ovf, c->d_counters + TIS_CNT_NB_OVERFLOW, sizeof(ovf), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (ovf == 0) { c->lists_valid = true; return 0; }
-    // grow the per-bead capacity and rebuild
-    int newcap = (int)(ovf + ovf / 2 + 16);
-    uint32_t *nb = nullptr;
-    int rc = dalloc(c, &nb, (size_t)newcap * c->P.ntot);
+    const unsigned long long ovf = c->report[0];
+    if (ovf == 0) { c->lists_valid = true; c->rebuilds_host += 1; return 0; }
+    HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
+    int rc = new_nb(c, ovf);
     if (rc) return rc;
-    c->P.nb = nb;  // the old buffer stays in allocs until the batch is freed
-    c->P.nb_cap = newcap;
-    for (int k = 0; k < 2; ++k)
-      if (c->graph[k]) { (void)hipGraphExecDestroy(c->graph[k]); c->graph[k] = nullptr; }
   }
-  (void)hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream);
   return fail(c, TIS_ERR_OVERFLOW, "neighbour list capacity could not be grown");
 }
 
@@ -1672,13 +1736,33 @@ int32_t tis_force_sumup(tis_ctx *c, int32_t isys, double *force_out) {
   int rc = check_sys(c, isys);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  if (!c->lists_valid) { rc = rebuild_lists(c, -1); if (rc) return rc; }
-  Range r = range_of(c, isys);
-  // force evaluation at the current coordinates; valence draws use step = stepbase
-  launch_force_pair(c, r, c->cur, 0, 0);
-  HIPCHK(c, hipGetLastError());
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (isys >= 0 && force_out) return tis_state_get(c, isys, 3, force_out);
+  const Range r = range_of(c, isys);
+  const bool want = isys >= 0 && force_out;
+  const HostSys *h = want ? &c->hs[isys] : nullptr;
+  const size_t bytes = want ? 3 * (size_t)h->d.nmp * sizeof(double) : 0;
+  void *out = nullptr;
+  if (want && (rc = pin_output(c, bytes, &out))) return rc;
+  for (int attempt = 0; attempt < 2; ++attempt) {
+    // missing lists are built in front of the force pass, which does nothing
+    // after an overflow: one wait for the whole call unless that happens
+    const bool build = !c->lists_valid;
+    if (build) launch_lists(c, range_of(c, -1), c->cur, 0, 0);
+    // force evaluation at the current coordinates; valence draws use step = stepbase
+    launch_force_pair(c, r, c->cur, 0, 0);
+    launch_state_out(c, c->P.f, want ? h->d.off : 0, want ? h->d.nmp : 0, out, build);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (!build) break;
+    const unsigned long long ovf = c->report[0];
+    if (ovf == 0) { c->lists_valid = true; c->rebuilds_host += 1; break; }
+    HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
+    if ((rc = new_nb(c, ovf))) return rc;
+    if ((rc = rebuild_lists(c, -1))) return rc;
+  }
+  if (want) {
+    std::memcpy(force_out, out, bytes);
+    c->d2h_bytes += (int64_t)bytes;
+  }
   return TIS_OK;
 }
 
@@ -1700,17 +1784,18 @@ int32_t tis_energy_sumup(tis_ctx *c, int32_t isys, double *energy_out) {
   // every live system (in live-list order) or one; the output is by system
   // index, zeros for retired systems
   const int nsel = isys < 0 ? c->nlive : 1, pos0 = isys < 0 ? 0 : c->hs[isys].live_pos;
+  void *pe = nullptr;
+  if ((rc = pin_output(c, 25 * sizeof(double) * (size_t)nsel, &pe))) return rc;
+  double *e = (double *)pe;
   const int t0 = isys < 0 ? 0 : c->hs[isys].et_begin, nt = isys < 0 ? c->n_etask : c->hs[isys].et_count;
   hipLaunchKernelGGL(k_energy, dim3(nt), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c), c->d_etask,
                      (const int32_t *)nullptr, t0, c->d_epart, 0);
   hipLaunchKernelGGL(k_energy_sum, dim3(nsel), dim3(kTile), 0, c->stream, c->d_efirst, (const int32_t *)nullptr, pos0,
-                     c->d_epart, c->d_energy, 0);
+                     c->d_epart, e, 0);
   HIPCHK(c, hipGetLastError());
-  std::vector<double> e(25 * (size_t)nsel);
-  HIPCHK(c, hipMemcpyAsync(e.data(), c->d_energy, e.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (isys >= 0) {
-    std::memcpy(energy_out, e.data(), 25 * sizeof(double));
+    std::memcpy(energy_out, e, 25 * sizeof(double));
   } else {
     for (int is = 0; is < c->nsys; ++is) {
       const HostSys &h = c->hs[is];
@@ -1748,29 +1833,20 @@ int32_t tis_energy_sumup_set(tis_ctx *c, int32_t n, const int32_t *isys, double 
     seen[h.live_pos] = 1;
     for (int q = 0; q < h.et_count; ++q) arg.push_back(h.et_begin + q);
   }
-  if (arg.size() > c->eset_cap) {
-    if (c->d_eset) { (void)hipFree(c->d_eset); c->d_eset = nullptr; c->dev_bytes -= c->eset_cap * sizeof(int32_t); }
-    c->eset_cap = 0;
-    HIPCHK(c, hipMalloc(&c->d_eset, arg.size() * sizeof(int32_t)));
-    c->eset_cap = arg.size();
-    c->dev_bytes += c->eset_cap * sizeof(int32_t);
-  }
-  if ((size_t)n * 25 > c->eset_out_cap) {
-    if (c->d_eset_out) { (void)hipFree(c->d_eset_out); c->d_eset_out = nullptr; c->dev_bytes -= c->eset_out_cap * sizeof(double); }
-    c->eset_out_cap = 0;
-    HIPCHK(c, hipMalloc(&c->d_eset_out, (size_t)n * 25 * sizeof(double)));
-    c->eset_out_cap = (size_t)n * 25;
-    c->dev_bytes += c->eset_out_cap * sizeof(double);
-  }
-  HIPCHK(c, hipMemcpyAsync(c->d_eset, arg.data(), arg.size() * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+  void *pin = nullptr, *pout = nullptr;
+  const size_t obytes = (size_t)n * 25 * sizeof(double);
+  if ((rc = pin_reserve(c, arg.size() * sizeof(int32_t), obytes))) return rc;   // (before either is taken)
+  if ((rc = pin_output(c, obytes, &pout))) return rc;
+  if ((rc = pin_input(c, arg.size() * sizeof(int32_t), &pin))) return rc;
+  std::memcpy(pin, arg.data(), arg.size() * sizeof(int32_t));
+  const int32_t *darg = (const int32_t *)pin;
   hipLaunchKernelGGL(k_energy, dim3((unsigned)(arg.size() - n)), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c),
-                     c->d_etask, c->d_eset + n, 0, c->d_epart, 0);
-  hipLaunchKernelGGL(k_energy_sum, dim3(n), dim3(kTile), 0, c->stream, c->d_efirst, c->d_eset, 0, c->d_epart,
-                     c->d_eset_out, 0);
+                     c->d_etask, darg + n, 0, c->d_epart, 0);
+  hipLaunchKernelGGL(k_energy_sum, dim3(n), dim3(kTile), 0, c->stream, c->d_efirst, darg, 0, c->d_epart,
+                     (double *)pout, 0);
   HIPCHK(c, hipGetLastError());
-  HIPCHK(c, hipMemcpyAsync(energy_out, c->d_eset_out, (size_t)n * 25 * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
+  std::memcpy(energy_out, pout, obytes);
   return TIS_OK;
 }
 
@@ -1921,23 +1997,18 @@ int32_t tis_label_apply(tis_ctx *c, int32_t n, const int32_t *isys, const int32_
     if ((rc = up(uo.data(), uo.size() * sizeof(int64_t), &p))) return rc; c->label_dev.u0off = (const int64_t *)p;
     c->labels_dirty = false;
   }
-  if (c->lab_cap < n) {
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (c->d_lab_args) (void)hipFree(c->d_lab_args);
-    if (c->d_lab_scale) (void)hipFree(c->d_lab_scale);
-    c->d_lab_args = nullptr; c->d_lab_scale = nullptr;
-    HIPCHK(c, hipMalloc((void **)&c->d_lab_args, 2 * sizeof(int32_t) * (size_t)n));
-    HIPCHK(c, hipMalloc((void **)&c->d_lab_scale, sizeof(double) * (size_t)n));
-    c->lab_cap = n;
-  }
-  HIPCHK(c, hipMemcpyAsync(c->d_lab_args, isys, sizeof(int32_t) * n, hipMemcpyHostToDevice, c->stream));
-  HIPCHK(c, hipMemcpyAsync(c->d_lab_args + c->lab_cap, label, sizeof(int32_t) * n, hipMemcpyHostToDevice, c->stream));
-  if (vscale) HIPCHK(c, hipMemcpyAsync(c->d_lab_scale, vscale, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(k_label_apply, dim3(n), dim3(256), 0, c->stream, c->P, c->label_dev, c->d_lab_args,
-                     c->d_lab_args + c->lab_cap, vscale ? (const double *)c->d_lab_scale : nullptr);
+  // the arguments stay in the ring until the kernel has read them
+  void *pin = nullptr;
+  if ((rc = pin_input(c, (size_t)n * (sizeof(double) + 2 * sizeof(int32_t)), &pin))) return rc;
+  double *psc = (double *)pin;
+  int32_t *parg = (int32_t *)(psc + n);
+  std::memcpy(parg, isys, sizeof(int32_t) * n);
+  std::memcpy(parg + n, label, sizeof(int32_t) * n);
+  if (vscale) std::memcpy(psc, vscale, sizeof(double) * n);
+  hipLaunchKernelGGL(k_label_apply, dim3(n), dim3(256), 0, c->stream, c->P, c->label_dev, (const int32_t *)parg,
+                     (const int32_t *)(parg + n), vscale ? (const double *)psc : nullptr);
   HIPCHK(c, hipGetLastError());
   for (int k = 0; k < n; ++k) copy_t_fields(c->hs[isys[k]].d, c->labels[label[k]].d);
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   return TIS_OK;
 }
 
@@ -2021,7 +2092,8 @@ static void eager_lists(tis_ctx *c, int32_t isys) {
     launch_lists(c, r, cu, 1, 1);
   } else if (c->t_since_init % c->rebuild_every == 0) {
     launch_lists(c, r, cu, 1, 0);
-    if (isys <= 0) hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
+    if (isys <= 0) hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)0, (uint64_t)1,
+                                      (uint64_t)0, c->d_counters);
   }
 }
 
@@ -2058,7 +2130,8 @@ static int capture_graph(tis_ctx *c, int parity) {
       launch_lists(c, r, cu, 1, 1);
     } else if (t % c->rebuild_every == 0) {
       launch_lists(c, r, cu, 1, 0);
-      if (!one) hipLaunchKernelGGL(k_count_rebuild, dim3(1), dim3(1), 0, c->stream, c->d_counters);
+      if (!one) hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)0, (uint64_t)1,
+                                   (uint64_t)0, c->d_counters);
     }
     launch_force_pair(c, r, cu ^ 1, t, 1, 1);
     cu ^= 1;
@@ -2294,7 +2367,6 @@ int32_t tis_langevin_steps(tis_ctx *c, int64_t nsteps, int32_t mode) {
   if (mode != TIS_MODE_GRAPH && mode != TIS_MODE_EAGER && mode != TIS_MODE_PLAIN)
     return fail(c, TIS_ERR_ARG, "unknown mode %d", mode);
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, 2 * sizeof(unsigned long long), c->stream));
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
   int64_t nlaunch = 0, remaining = nsteps;
   for (int attempt = 0;; ++attempt) {
@@ -2303,12 +2375,13 @@ int32_t tis_langevin_steps(tis_ctx *c, int64_t nsteps, int32_t mode) {
     const uint64_t step0 = c->step_host;
     int rc = run_steps(c, remaining, mode, &nlaunch);
     if (rc) return rc;
-    unsigned long long st[2] = {0ull, 0ull};  // overflow need, steps completed
-    HIPCHK(c, hipMemcpyAsync(st, c->d_counters + TIS_CNT_NB_OVERFLOW, sizeof(st), hipMemcpyDeviceToHost, c->stream));
+    hipLaunchKernelGGL(k_run_report, dim3(1), dim3(1), 0, c->stream, c->d_counters, c->report);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    const unsigned long long st[2] = {c->report[0], c->report[1]};  // overflow need, steps completed
     if (st[0] == 0ull) {
       c->step_host = step0 + (uint64_t)remaining;
-      HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, 2 * sizeof(unsigned long long), c->stream));
       break;
     }
     // a rebuild overflowed the list capacity: the run stopped at the start
@@ -2337,8 +2410,6 @@ int32_t tis_langevin_steps(tis_ctx *c, int64_t nsteps, int32_t mode) {
     HIPCHK(c, hipMemcpy(c->d_stepbase, &sb, sizeof(sb), hipMemcpyHostToDevice));
     remaining -= completed;
   }
-  HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-  HIPCHK(c, hipEventSynchronize(c->ev1));
   float ms = 0.0f;
   (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
   c->last_total_ms = ms;
@@ -2369,6 +2440,7 @@ int32_t tis_status_counters(tis_ctx *c, int64_t *counters) {
   HIPCHK(c, hipMemcpyAsync(h, c->d_counters, sizeof(h), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   for (int k = 0; k < TIS_CNT_MAX; ++k) counters[k] = (int64_t)h[k];
+  counters[TIS_CNT_REBUILDS] += c->rebuilds_host;
   return TIS_OK;
 }
 

@@ -2124,10 +2124,46 @@ __device__ inline bool system_trigger(const DevPtrs &P, const DSys &s) {
   return sqrt(a) + sqrt(b) > s.margin;
 }
 
-// the FP32 positions of [g0, g0 + n) from x (state uploads)
+// ------------------------------------------------------------------ state transfers
+// A system's state between the caller's (3, n) order, in pinned host memory
+// that the kernels read and write themselves, and the arena's [3][ntot]: one
+// launch each way.  (Three pageable copies with a wait each took 67 us for a
+// system of any size; about 12 now.)
+
+// buf[3 i + d] = base[d][off + i]; report (may be null) gets the overflow
+// flag, and n may be 0 for that alone
+__global__ __launch_bounds__(256) void k_state_out(const double *base, int ntot, int off, int n, double *buf,
+                                                   const unsigned long long *counters, unsigned long long *report) {
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k < 3 * n) buf[k] = base[(size_t)(k % 3) * ntot + off + k / 3];
+  if (k == 0 && report) report[0] = counters[5];
+}
+
+// base[d][off + i] = buf[3 i + d], with the FP32 records when xf is given (the
+// coordinates of a system that is not periodic)
+__global__ __launch_bounds__(256) void k_state_in(DevPtrs P, double *base, int off, int n, const double *buf,
+                                                  float4 *xf) {
+  const int i = blockIdx.x * 256 + threadIdx.x, N = P.ntot, g = off + i;
+  if (i >= n) return;
+  const double x = buf[3 * i], y = buf[3 * i + 1], z = buf[3 * i + 2];
+  base[g] = x; base[N + g] = y; base[2 * (size_t)N + g] = z;
+  if (xf) xf[g] = near_pos(x, y, z, P.species[g]);
+}
+
+// the FP32 records of [g0, g0 + n) from x (a new layout)
 __global__ __launch_bounds__(256) void k_near(DevPtrs P, const double *X, float4 *XF, int g0, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, g = g0 + i, N = P.ntot;
+  const int i = blockIdx.x * 256 + threadIdx.x, g = g0 + i, N = P.ntot;
   if (i < n) XF[g] = near_pos(X[g], X[N + g], X[2 * (size_t)N + g], P.species[g]);
+}
+
+// The end of a run: its stop flag and completed steps to the host; both are
+// zero between calls (the host clears them itself when the run has to resume).
+__global__ void k_run_report(unsigned long long *counters, unsigned long long *report) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    report[0] = counters[5];
+    report[1] = counters[6];
+    if (counters[5] == 0ull) counters[6] = 0ull;
+  }
 }
 
 __global__ __launch_bounds__(kTile) void k_prep(DevPtrs P, const double *X, double *PXc, double *PXp, float4 *XFc,
@@ -2807,10 +2843,6 @@ __global__ void k_advance(uint64_t *stepbase, uint64_t by, uint64_t rebuilds, ui
   if (threadIdx.x == 0 && blockIdx.x == 0 && counters[5] == 0ull) {
     *stepbase += by; counters[4] += by; counters[3] += rebuilds; counters[6] += completed;
   }
-}
-
-__global__ void k_count_rebuild(unsigned long long *counters) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && counters[5] == 0ull) counters[3] += 1;
 }
 
 // ------------------------------------------------------------------ energies

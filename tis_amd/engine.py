@@ -196,7 +196,7 @@ class Engine:
         self._chk(self.L.tis_state_set(self.ctx, isys, which, _fp(a)), "tis_state_set")
 
     def get_state(self, isys, which):
-        a = np.zeros((self.systems[isys].nmp, 3))
+        a = np.empty((self.systems[isys].nmp, 3))
         self._chk(self.L.tis_state_get(self.ctx, isys, which, _fp(a)), "tis_state_get")
         return a
 
@@ -232,7 +232,7 @@ class Engine:
         return (pairs, coef[:cnt]) if which == LIST_ELE else pairs
 
     def force_sumup(self, isys):
-        f = np.zeros((self.systems[isys].nmp, 3))
+        f = np.empty((self.systems[isys].nmp, 3))
         self._chk(self.L.tis_force_sumup(self.ctx, isys, _fp(f)), "tis_force_sumup")
         return f
 
