@@ -1,0 +1,90 @@
+"""The full-panel Cholesky kernel (16 x 16 tiles on the FP64 matrix cores) at
+the edges of its tiles, panels and outer blocks against the FP64 factor, its
+pivot check, and the step's products and forces at the edges of their blocks.
+The wait states of its DPP multiply-adds are checked on the generated code."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+import test_dpp_hazards as hz
+from tis_amd.bdhi import bead_spring_chain
+from tis_amd.engine import BDEngine, load_library
+
+
+def _factor(D, L):
+    fn = load_library().tis_bdhi_factor_noalloc
+    fn.restype = ctypes.c_int32
+    fn.argtypes = [ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p]
+    info = ctypes.c_int32(-1)
+    rc = fn(0, D.data_ptr(), L.data_ptr(), len(D), None, ctypes.byref(info))
+    return rc, info.value
+
+
+def _spd(n):
+    g = np.random.default_rng(n).standard_normal((n, n))
+    return g @ g.T / n + np.eye(n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 80, 127, 128, 129, 191, 192, 193, 255, 256, 257, 320, 511, 577])
+def test_factor_sizes(n):
+    import torch
+    a = _spd(n)
+    print(f"[factor] n={n}", flush=True)
+    D = torch.from_numpy(a).cuda()
+    L = torch.empty_like(D)
+    rc, info = _factor(D, L)
+    assert rc == 0 and info == 0
+    l64 = np.linalg.cholesky(a)
+    err = np.abs(L.T.cpu().numpy() - l64).max() / np.abs(l64).max()
+    # one panel is FP64 throughout; further ones take products in FP32
+    assert err <= (1e-13 if n <= 64 else 2e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("p", [0, 15, 16, 47, 63, 64, 100, 129])
+def test_pivot_check(p):
+    import torch
+    a = _spd(130)
+    a[p, p] = -1.0
+    print(f"[pivot] {p}", flush=True)
+    D = torch.from_numpy(a).cuda()
+    rc, info = _factor(D, torch.empty_like(D))
+    assert rc != 0 and info == p + 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 3, 21, 22, 64, 65, 66, 130])
+def test_forces_and_step(n):
+    """Lanes of one bead's pairs (64 and more), rows and columns of the step's
+    products at the edges of their blocks; bounds as for the chains of the
+    step and force tests."""
+    s, x = bead_spring_chain(n, seed=n)
+    print(f"[bd] n={n}", flush=True)
+    e = BDEngine(s, key=9, seed=11)
+    e.set_coords(x)
+    f, fo = e.forces(), oracle.bd_forces(s, x)
+    assert np.abs(f - fo).max() <= 1e-12 * max(1.0, np.abs(fo).max())
+    e.steps(3, tstep=0.05, refactor_every=1, step0=100)
+    xo = oracle.bdhi_run(s, x, 3, tstep=0.05, refactor_every=1, seed=11, key=9, step0=100)
+    assert np.abs(e.coords() - xo).max() <= 1e-5
+    e.close()
+
+
+@pytest.mark.skipif(not os.path.exists(hz.HIPCC), reason="hipcc not available")
+def test_full_panel_dpp_wait_states(tmp_path):
+    import subprocess
+    out = tmp_path / "bdhi.s"
+    subprocess.run([hz.HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "--cuda-device-only", "-S", hz.SRC, "-o", str(out)], check=True,
+                   capture_output=True)
+    lines = out.read_text().splitlines()
+    start = next(i for i, l in enumerate(lines) if l.startswith("_ZN3tis12k_chol_block"))
+    end = next(i for i in range(start, len(lines)) if lines[i].startswith(".Lfunc_end"))
+    n, bad = hz.dpp_hazards(lines[start:end])
+    # 105 + 120 multiply-adds of a 16 x 16 tile and its inverse, and more moves
+    assert n >= 225
+    assert not bad, bad[:3]

@@ -24,7 +24,9 @@
 namespace tis {
 
 constexpr int kCb = 64;         // Cholesky block size
-constexpr int kGemvRows = 256;  // rows per block of the step products
+constexpr int kGemvRows = 64;   // rows per block of the step products
+constexpr int kGemvWaves = 4;   // waves sharing a block's columns
+constexpr int kGemvThreads = kGemvRows * kGemvWaves;
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 struct BdDev {
@@ -48,15 +50,21 @@ struct BdDev {
 };
 
 // ---------------------------------------------------------------- forces
-// force_fene.F90:40-57 and force_wca.F90:64-96, owner-computes: each bead
-// sums its own bonds and pairs in list order (no atomics).  with_noise also
-// draws the bead's Gaussian triple for step `step`.
-__global__ __launch_bounds__(256) void k_bd_force(BdDev B, uint64_t step, int with_noise) {
+// force_fene.F90:40-57 and force_wca.F90:64-96, owner-computes: a wave per
+// bead, the bead's bonds and pairs over its lanes in list order, the lanes'
+// sums added by a fixed tree (no atomics).  with_noise also draws the bead's
+// Gaussian triple for step `step`.  Bound by latency: a bead of a chain has a
+// pair with every other bead, and one thread per bead walked them one after
+// the other: 22.3 us at 300 beads, 8.0 us by waves.
+constexpr int kForceBeads = 4;   // beads per block
+
+__global__ __launch_bounds__(64 * kForceBeads) void k_bd_force(BdDev B, uint64_t step, int with_noise) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int i = blockIdx.x * kForceBeads + (int)__builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int lane = threadIdx.x & 63;
   if (i >= B.n) return;
   double F[3] = {0.0, 0.0, 0.0};
-  for (int e = B.fb_off[i]; e < B.fb_off[i + 1]; ++e) {
+  for (int e = B.fb_off[i] + lane; e < B.fb_off[i + 1]; e += 64) {
     const uint32_t ent = (uint32_t)B.fb[e];
     const int b = (int)(ent & 0x7fffffffu);
     const int i0 = B.fene_mp[2 * b], j0 = B.fene_mp[2 * b + 1];
@@ -68,7 +76,7 @@ __global__ __launch_bounds__(256) void k_bd_force(BdDev B, uint64_t step, int wi
     const double sg = (ent >> 31) ? 1.0 : -1.0;
     for (int d = 0; d < 3; ++d) F[d] += sg * (fr * v[d]);
   }
-  for (int e = B.wb_off[i]; e < B.wb_off[i + 1]; ++e) {
+  for (int e = B.wb_off[i] + lane; e < B.wb_off[i + 1]; e += 64) {
     const uint32_t ent = (uint32_t)B.wb[e];
     const int k = (int)(ent & 0x7fffffffu);
     const int i0 = B.wca_mp[2 * k], j0 = B.wca_mp[2 * k + 1];
@@ -85,11 +93,15 @@ __global__ __launch_bounds__(256) void k_bd_force(BdDev B, uint64_t step, int wi
     const double sg = (ent >> 31) ? 1.0 : -1.0;
     for (int d = 0; d < 3; ++d) F[d] += sg * (dv * v[d]);
   }
-  for (int d = 0; d < 3; ++d) B.f[3 * i + d] = F[d];
+  for (int m = 32; m > 0; m >>= 1)
+    for (int d = 0; d < 3; ++d) F[d] += __shfl_xor(F[d], m, 64);
+  if (lane == 0)
+    for (int d = 0; d < 3; ++d) B.f[3 * i + d] = F[d];
   if (with_noise) {
     double g[3];
     gauss3(B.seed, B.key, step, (uint32_t)i, g);
-    for (int d = 0; d < 3; ++d) B.xi[3 * i + d] = g[d];
+    if (lane == 0)
+      for (int d = 0; d < 3; ++d) B.xi[3 * i + d] = g[d];
   }
 }
 
@@ -100,6 +112,7 @@ __global__ __launch_bounds__(256) void k_bd_force(BdDev B, uint64_t step, int wi
 __global__ __launch_bounds__(256) void k_rpy_fill(BdDev B) {
 #pragma clang fp contract(off)
   const int i = blockIdx.x * 16 + threadIdx.x, j = blockIdx.y * 16 + threadIdx.y;
+  if (i == 0 && j == 0) *B.info = 0;
   if (i >= B.n || j >= B.n || i > j) return;
   const int n3 = B.n3;
   if (i == j) {
@@ -376,11 +389,11 @@ __device__ __forceinline__ void solve_cols(double (&x)[kCb], const double *Ls, c
 // 32 (P column k at P + k * mpad), in the accumulator layout of
 // v_mfma_f32_32x32x2f32 with the columns' entries as the first operand: the
 // operands and the order of the sums are those of k_chol_update.  Operands
-// come straight from memory (L2), eight k pairs ahead.
+// come straight from memory (L2), 16 k pairs ahead.
 __device__ inline floatx16 quad_product(const float *P, int mpad, int ra, int rb, int K, int lane) {
   floatx16 acc;
   for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-  constexpr int kU = 8;   // k pairs per batch of loads
+  constexpr int kU = 16;   // k pairs per batch of loads
   const int l = lane & 31;
   const float *pa = P + (size_t)(lane >> 5) * mpad + ra + l;
   const float *pb = P + (size_t)(lane >> 5) * mpad + rb + l;
@@ -551,6 +564,275 @@ __global__ __launch_bounds__(kPanelThreads) void k_chol_panel(BdDev B, int kk, i
   }
 }
 
+// ---------------------------------------------------------------- full panels
+// A panel of 64 full columns in tiles of 16 x 16 on the FP64 matrix cores
+// (v_mfma_f64_16x16x4f64): operand A lane l holds A[l % 16][l / 16], B lane l
+// holds B[l / 16][l % 16], D register v of lane l holds D[l / 16 + 4 v][l % 16].
+// A tile is kept transposed in that layout (lane: row l % 16, register v:
+// column l / 16 + 4 v), and then its registers are, as they stand, both the B
+// operand of the transposed tile and the A operand of the tile, register v at
+// k = 4 v: the tile algebra below moves nothing between lanes.
+// Bound: the serial chain of 64 pivots (broadcast, reciprocal, scale, next
+// entry), about 190 cycles each.  k_chol_panel runs it over 64 rows with the
+// columns published in LDS, 12 us, and solves the rows below by 64 dependent
+// steps, 6 us more; here the chain runs in registers, 16 columns at a time
+// (2,984 cycles), the inverses of the 16 x 16 factors come with it, and the
+// rows below are products.  A panel at 3n = 900: 27.7 us by k_chol_panel, 24.5
+// us here; the factor 450 -> 404 us there, 1.60 -> 1.45 ms at 3n = 3000, 7.8
+// -> 7.4 ms at 9000.  The chain's broadcasts are DPP operands of the
+// multiply-adds: as two moves (with their old values) and an fma the tile took
+// 9,004 cycles, as lane-masked moves 6,352.
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+// D = C + A B of 16 x 16 tiles, K = 16
+__device__ __forceinline__ doublex4 tile_fma(const doublex4 &a, const doublex4 &b, doublex4 c) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], b[k], c, 0, 0, 0);
+  return c;
+}
+
+// v0 .. v3 for q = 0 .. 3 (of values: a choice among array elements would put
+// the array in scratch memory)
+__device__ __forceinline__ double one_of4(int q, double v0, double v1, double v2, double v3) {
+  const double lo = q & 1 ? v1 : v0, hi = q & 1 ? v3 : v2;
+  return q & 2 ? hi : lo;
+}
+
+// the value of v at lane N of the lane's row of 16
+template <int N>
+__device__ __forceinline__ double row_value(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, 0x150 + N, 0xF, 0xF, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0x150 + N, 0xF, 0xF, true);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// One 16 x 16 diagonal tile as L D L^T, row r = lane % 16 in a[] (every row of
+// 16 lanes holds a copy), right-looking; t[] takes the same row operations on
+// the identity, L^-1.  On return a[] is the row of the Cholesky factor L
+// sqrt(D), t[] the row of L^-1 and rs 1 / sqrt(D[r]).  bad: the first pivot
+// that is not positive, as kk + column + 1 (0xffffffff: none).  Entries above
+// the diagonal are left to take what the rows below take (no entry on or below
+// it reads them) and cleared at the end; the next column's entry is written by
+// the compiler's own fma, so that the waits before the lane reads of the chain
+// are the compiler's too.
+template <int C, int J>
+__device__ __forceinline__ void factor16_update(double (&a)[16], double u, double ns) {
+  if constexpr (J < 16) {
+    fmac_row_bcast<J>(a[J], u, ns);
+    factor16_update<C, J + 1>(a, u, ns);
+  }
+}
+template <int C, int K>
+__device__ __forceinline__ void factor16_inverse(double (&t)[16], double ns) {
+  if constexpr (K < C) {
+    fmac_row_bcast<C>(t[K], t[K], ns);
+    factor16_inverse<C, K + 1>(t, ns);
+  }
+}
+template <int C>
+__device__ __forceinline__ void factor16_step(double (&a)[16], double (&t)[16], double &piv, int kk, unsigned &bad) {
+  if constexpr (C < 16) {
+    const int r = threadIdx.x & 15;
+    const double u = a[C];
+    const double d = row_value<C>(u);
+    const double ns = -u * rcp_nr(d);
+    if constexpr (C + 1 < 16) a[C + 1] = fma(row_value<C + 1>(u), ns, a[C + 1]);
+    factor16_update<C, C + 2>(a, u, ns);
+    const double nt = r > C ? ns : 0.0;
+    factor16_inverse<C, 0>(t, nt);
+    t[C] = r == C ? 1.0 : nt;
+    piv = r == C ? d : piv;
+    bad = min(bad, d > 0.0 ? 0xffffffffu : (unsigned)(kk + C + 1));
+    factor16_step<C + 1>(a, t, piv, kk, bad);
+  }
+}
+template <int C>
+__device__ __forceinline__ void factor16_scale(double (&a)[16], double rs) {
+  if constexpr (C < 16) {
+    a[C] = (int)(threadIdx.x & 15) >= C ? a[C] * row_value<C>(rs) : 0.0;
+    factor16_scale<C + 1>(a, rs);
+  }
+}
+__device__ __forceinline__ void factor16(double (&a)[16], double (&t)[16], double &rs, int kk, unsigned &bad) {
+  double piv = 1.0;
+  factor16_step<0>(a, t, piv, kk, bad);
+  rs = rsqrt_nr(piv);
+  factor16_scale<0>(a, rs);
+}
+
+// As k_chol_panel for a panel whose 64 columns are all there: wave 0 factors
+// the diagonal block, tile (i, j) of its lower triangle in yt[i (i + 1) / 2 +
+// j]; waves 1-3 form the earlier panels' product for the block's rows
+// meanwhile (the diagonal block's, by all four waves, comes first:
+// quad_product, the bits of k_chol_update); then each wave solves 16 rows.
+// The tiles are in LDS and the loops over them are not unrolled: every panel
+// runs this code once, and straight-line code for all of it (tiles in
+// registers) took 60,000 cycles instead of 25,400, most of them waiting for
+// instructions.
+__global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(1))) void k_chol_block(BdDev B, int kk,
+                                                                                                     int k0, float *P,
+                                                                                                     int mpad) {
+  __shared__ float Td[kCb][kCb + 1], Tr[kCb][kCb + 1];
+  // tiles and, per 16 columns, the inverse factor as operands; the diagonal
+  // tiles of the factor [s][column][row]
+  __shared__ double yt[10][4][kCb], op[4][4][kCb], cd[4][16][16];
+  const int lane = threadIdx.x & (kCb - 1), w = threadIdx.x / kCb, n3 = B.n3;
+  const int r16 = lane & 15, c4 = lane >> 4;
+  const int K = kk - k0;
+  const int r0w = kk + kCb * (int)blockIdx.x;   // the block's first row (blocks 1..)
+  const bool rows = blockIdx.x > 0 && r0w < n3;
+  const int p = kk / kCb;
+  // every wave: columns [16 w, 16 w + 16) of the diagonal block's rows, and 16
+  // of the block's rows (unconditional loads, rows past n3 clamped)
+  double dg[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) dg[c] = B.L[(size_t)(kk + lane) + (size_t)(kk + 16 * w + c) * n3];
+  doublex4 x[4];
+  const int r = r0w + 16 * w + r16;
+  if (rows) {
+    const size_t row = (size_t)min(r, n3 - 1);
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[q][v] = B.L[row + (size_t)(kk + 16 * q + c4 + 4 * v) * n3];
+  }
+  if (w == 3 && blockIdx.x == 0 && p > 0) {
+    // the previous panel's diagonal factor (see k_chol_panel)
+    const double *sp = B.stash + (size_t)((p - 1) & 1) * kCb * kCb;
+    const int kp = kk - kCb;
+#pragma unroll 8
+    for (int c = 0; c < kCb; ++c) B.L[(size_t)(kp + lane) + (size_t)(kp + c) * n3] = sp[c * kCb + lane];
+  }
+  const int l32 = lane & 31, c32 = 4 * (lane >> 5);   // accumulator e: row l32, column c32 + 8 (e / 4) + e % 4
+  // quadrants quad, quad + step, .. of the product for rows from ra
+  auto product = [&](float (*T)[kCb + 1], int ra, int quad, int step) {
+#pragma unroll 1
+    for (; quad < 4; quad += step) {
+      const int qi = quad >> 1, qj = quad & 1;
+      const floatx16 acc = quad_product(P, mpad, ra - k0 + 32 * qi, kk - k0 + 32 * qj, K, lane);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) T[32 * qi + l32][32 * qj + c32 + 8 * (e >> 2) + (e & 3)] = acc[e];
+    }
+  };
+  if (K > 0) product(Td, kk, w, 4);
+  __syncthreads();
+  // the diagonal block less its product into tiles: this wave's 16 columns are
+  // tile column w, row lane of tile row lane / 16
+  {
+    const int i = lane >> 4;
+    if (i >= w) {
+      double(*t)[kCb] = yt[i * (i + 1) / 2 + w];
+#pragma unroll
+      for (int c = 0; c < 16; ++c)
+        t[c >> 2][16 * (c & 3) + r16] = K > 0 ? dg[c] - (double)Td[lane][16 * w + c] : dg[c];
+    }
+  }
+  __syncthreads();
+  if (w == 0) {
+    unsigned bad = 0xffffffffu;
+#pragma unroll 1
+    for (int sx = 0; sx < 4; ++sx) {
+      double a[16], t[16], rs = 0.0;
+      double(*yd)[kCb] = yt[sx * (sx + 1) / 2 + sx];
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) a[4 * v + q] = yd[v][16 * q + r16];
+      factor16(a, t, rs, kk + 16 * sx, bad);
+      doublex4 inv;   // row r16, columns c4 + 4 v of the inverse factor
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        inv[v] = one_of4(c4, t[4 * v], t[4 * v + 1], t[4 * v + 2], t[4 * v + 3]) * rs;
+        op[sx][v][lane] = inv[v];
+        cd[sx][4 * v + c4][r16] = one_of4(c4, a[4 * v], a[4 * v + 1], a[4 * v + 2], a[4 * v + 3]);
+      }
+      // the column's tiles, then what they take from the tiles to the right:
+      // every load first, independent products side by side
+      doublex4 y[4], o[4][4];
+#pragma unroll
+      for (int i = 1; i < 4; ++i)
+        if (i > sx) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) y[i][v] = yt[i * (i + 1) / 2 + sx][v][lane];
+#pragma unroll
+          for (int j = 1; j <= i; ++j)
+            if (j > sx)
+#pragma unroll
+              for (int v = 0; v < 4; ++v) o[i][j][v] = yt[i * (i + 1) / 2 + j][v][lane];
+        }
+#pragma unroll
+      for (int i = 1; i < 4; ++i)
+        if (i > sx) {
+          y[i] = tile_fma(inv, y[i], doublex4{0.0, 0.0, 0.0, 0.0});
+#pragma unroll
+          for (int v = 0; v < 4; ++v) yt[i * (i + 1) / 2 + sx][v][lane] = y[i][v];
+        }
+#pragma unroll
+      for (int j = 1; j < 4; ++j)
+        if (j > sx) {
+          const doublex4 nj = -y[j];
+#pragma unroll
+          for (int i = j; i < 4; ++i) {
+            o[i][j] = tile_fma(nj, y[i], o[i][j]);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) yt[i * (i + 1) / 2 + j][v][lane] = o[i][j][v];
+          }
+        }
+    }
+    if (blockIdx.x == 0 && lane == 0 && bad != 0xffffffffu) atomicCAS(B.info, 0, (int)bad);
+  } else if (K > 0 && rows) {
+    product(Tr, r0w, w - 1, 3);
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    // the factor goes to the stash, or, from a panel of one block, to its
+    // place: this wave's 16 columns, zeros above the diagonal
+    double *fo = gridDim.x > 1 ? B.stash + (size_t)(p & 1) * kCb * kCb : B.L + (size_t)kk + (size_t)kk * n3;
+    const size_t ld = gridDim.x > 1 ? (size_t)kCb : (size_t)n3;
+    const int i = lane >> 4;
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      const double val = i > w ? yt[i * (i + 1) / 2 + w][c >> 2][16 * (c & 3) + r16] : (i == w ? cd[w][c][r16] : 0.0);
+      fo[(size_t)lane + (16 * w + c) * ld] = val;
+    }
+    return;
+  }
+  if (!rows) return;
+  if (K > 0) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[q][v] -= (double)Tr[16 * w + r16][16 * q + c4 + 4 * v];
+  }
+  doublex4 nx[4];   // the solved tiles, negated
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+#pragma unroll
+    for (int e = 0; e < q; ++e) {
+      doublex4 c;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) c[v] = yt[q * (q + 1) / 2 + e][v][lane];
+      x[q] = tile_fma(c, nx[e], x[q]);
+    }
+    doublex4 inv;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) inv[v] = op[q][v][lane];
+    x[q] = tile_fma(inv, x[q], doublex4{0.0, 0.0, 0.0, 0.0});
+    nx[q] = -x[q];
+  }
+  const bool live = r < n3;
+  const int rl = r - k0, q0 = kk - k0;   // row and first column of P
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int c = 16 * q + c4 + 4 * v;
+      if (live) B.L[(size_t)r + (size_t)(kk + c) * n3] = x[q][v];
+      if (rl < mpad) P[(size_t)(q0 + c) * mpad + rl] = live ? (float)x[q][v] : 0.0f;
+    }
+}
+
 // C -= A B^T on 64x64 tiles of the lower part of L, FP32 matrix cores
 // (v_mfma_f32_32x32x2f32, each of four waves a 32x32 quadrant), the sum
 // over K columns of P in chunks of 64 staged through LDS, subtracted from
@@ -639,18 +921,37 @@ static __device__ __align__(256) float scratch[kScratchStash + 4 * kCb * kCb];  
 
 // ---------------------------------------------------------------- step
 // Partial products over a column chunk: yD = D[:, chunk] F[chunk],
-// yL = L[:, chunk] xi[chunk] (lower part only); one thread per row.
-__global__ __launch_bounds__(kGemvRows) void k_bd_gemv(BdDev B, double *ypart, int chunk) {
-  const int k = blockIdx.x * kGemvRows + threadIdx.x;
-  const int c = blockIdx.y, n3 = B.n3;
-  const int l0 = c * chunk, l1 = min(n3, l0 + chunk);
-  if (k >= n3) return;
+// yL = L[:, chunk] xi[chunk] (lower part only).  A block has 64 rows, a lane
+// each, and shares the chunk's columns among its four waves, whose sums are
+// added through LDS.  Bound by the reads of D and L (12 n3^2 bytes), at a few
+// hundred rows by their latency: 16 columns' loads are under way at a time.
+// At 900 rows 57.8 us with one wave per 64 rows and 113 columns and a load
+// at a time, 10.5 us now.
+__global__ __launch_bounds__(kGemvThreads) void k_bd_gemv(BdDev B, double *ypart, int chunk) {
+  __shared__ double part[2][kGemvWaves][kGemvRows];
+  const int lane = threadIdx.x & (kGemvRows - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kGemvRows);
+  const int r0 = blockIdx.x * kGemvRows, n3 = B.n3;
+  const int k = min(r0 + lane, n3 - 1);
+  const int c = blockIdx.y, cw = (chunk + kGemvWaves - 1) / kGemvWaves;
+  const int end = min(n3, (c + 1) * chunk);
+  const int l0 = c * chunk + w * cw, l1 = min(end, l0 + cw);
   double aD = 0.0, aL = 0.0;
+#pragma unroll 16
   for (int l = l0; l < l1; ++l) aD += B.D[(size_t)l * n3 + k] * B.f[l];
-  const int lL = min(l1, k + 1);
-  for (int l = l0; l < lL; ++l) aL += B.L[(size_t)l * n3 + k] * B.xi[l];
-  ypart[(size_t)(2 * c) * n3 + k] = aD;
-  ypart[(size_t)(2 * c + 1) * n3 + k] = aL;
+  const int lL = min(l1, r0 + kGemvRows);
+#pragma unroll 16
+  for (int l = l0; l < lL; ++l) {
+    const double v = B.L[(size_t)l * n3 + k];
+    aL += (l <= k ? v : 0.0) * B.xi[l];
+  }
+  part[0][w][lane] = aD;
+  part[1][w][lane] = aL;
+  __syncthreads();
+  if (w < 2 && r0 + lane < n3) {
+    double y = part[w][0][lane];
+    for (int q = 1; q < kGemvWaves; ++q) y += part[w][q][lane];
+    ypart[(size_t)(2 * c + w) * n3 + k] = y;
+  }
 }
 
 // time_integral.F90:440-446: dx = (dt/kT) D F + sqrt(2 dt) L xi
@@ -660,6 +961,7 @@ __global__ __launch_bounds__(kGemvRows) void k_bd_update(BdDev B, const double *
   const int k = blockIdx.x * kGemvRows + threadIdx.x;
   if (k >= B.n3) return;
   double a = 0.0, b = 0.0;
+#pragma unroll 8
   for (int c = 0; c < nchunk; ++c) { a += ypart[(size_t)(2 * c) * B.n3 + k]; b += ypart[(size_t)(2 * c + 1) * B.n3 + k]; }
   B.x[k] += c1 * a + c2 * b;
 }
@@ -791,7 +1093,6 @@ BdState *need(tis_ctx *c) {
 void launch_fill(tis_ctx *c, BdState *b) {
   hipStream_t st = ctx_stream(c);
   const BdDev &d = b->d;
-  hipLaunchKernelGGL(k_bd_reset, dim3(1), dim3(64), 0, st, d);
   const int gb = (d.n + 15) / 16;
   hipLaunchKernelGGL(k_rpy_fill, dim3(gb, gb), dim3(16, 16), 0, st, d);
 }
@@ -808,7 +1109,11 @@ void factor_launches(const BdDev &d, float *P, hipStream_t st) {
       const int kk = k0 + j * kCb;
       const int m = n3 - kk - kCb;
       const int nbp = m > 0 ? (m + kPanelRowsPerBlock - 1) / kPanelRowsPerBlock : 0;
-      hipLaunchKernelGGL(k_chol_panel, dim3(1 + nbp), dim3(kPanelThreads), 0, st, d, kk, k0, P, mpad);
+      // the last panel of a size that is no multiple of 64 has columns missing
+      if (n3 - kk >= kCb)
+        hipLaunchKernelGGL(k_chol_block, dim3(1 + nbp), dim3(kPanelThreads), 0, st, d, kk, k0, P, mpad);
+      else
+        hipLaunchKernelGGL(k_chol_panel, dim3(1 + nbp), dim3(kPanelThreads), 0, st, d, kk, k0, P, mpad);
     }
     const int kt = k0 + kNb;
     if (kt >= n3) break;
@@ -967,7 +1272,8 @@ int32_t tis_bdhi_setup(tis_ctx *c, const tis_bd_system *s, uint32_t key, uint64_
   if ((rc = balloc(c, b, &b->P, (size_t)kNb * b->mpad))) return rc;
   // step products: ~1024+ blocks
   const int rows = (int)((n3 + kGemvRows - 1) / kGemvRows);
-  b->nchunk = std::max(1, std::min((int)((n3 + 127) / 128), (1024 + rows - 1) / rows));
+  // at least 16 columns a wave, no more blocks than fill the chip twice over
+  b->nchunk = std::max(1, std::min((int)((n3 + 63) / 64), (2048 + rows - 1) / rows));
   b->chunk = (int)((n3 + b->nchunk - 1) / b->nchunk);
   if ((rc = balloc(c, b, &b->ypart, (size_t)2 * b->nchunk * n3))) return rc;
   if ((rc = balloc(c, b, &b->llt_part, (size_t)2 * mt * (mt + 1) / 2))) return rc;
@@ -1014,7 +1320,8 @@ int32_t tis_bdhi_forces(tis_ctx *c, double *force_out) {
   BdState *b = need(c);
   if (!b) return TIS_ERR_STATE;
   BCHK(c, hipSetDevice(ctx_device(c)));
-  hipLaunchKernelGGL(k_bd_force, dim3((b->d.n + 255) / 256), dim3(256), 0, ctx_stream(c), b->d, (uint64_t)0, 0);
+  hipLaunchKernelGGL(k_bd_force, dim3((b->d.n + kForceBeads - 1) / kForceBeads), dim3(64 * kForceBeads), 0, ctx_stream(c), b->d,
+                     (uint64_t)0, 0);
   BCHK(c, hipGetLastError());
   if (force_out) return tis_bdhi_state_get(c, 1, force_out);
   BCHK(c, hipStreamSynchronize(ctx_stream(c)));
@@ -1098,8 +1405,8 @@ int32_t tis_bdhi_steps(tis_ctx *c, double tstep, int64_t nsteps, int32_t refacto
         fill_ms += a; fact_ms += f;
       }
     }
-    hipLaunchKernelGGL(k_bd_force, dim3((d.n + 255) / 256), dim3(256), 0, st, d, step0 + (uint64_t)t + 1u, 1);
-    hipLaunchKernelGGL(k_bd_gemv, dim3(rows, b->nchunk), dim3(kGemvRows), 0, st, d, b->ypart, b->chunk);
+    hipLaunchKernelGGL(k_bd_force, dim3((d.n + kForceBeads - 1) / kForceBeads), dim3(64 * kForceBeads), 0, st, d, step0 + (uint64_t)t + 1u, 1);
+    hipLaunchKernelGGL(k_bd_gemv, dim3(rows, b->nchunk), dim3(kGemvThreads), 0, st, d, b->ypart, b->chunk);
     hipLaunchKernelGGL(k_bd_update, dim3(rows), dim3(kGemvRows), 0, st, d, (const double *)b->ypart, b->nchunk,
                        c1, c2);
   }
