@@ -22,7 +22,7 @@
 namespace tis {
 template <int PPW, int TPL>
 __global__ void k_force(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *, int,
-                        BondedRange, int32_t);
+                        const EwTask *, int, BondedRange, int32_t);
 __global__ void k_ewald_sk(DevPtrs, const double *, const EwTask *, int);
 __global__ void k_ewald_f(DevPtrs, const double *, const EwTask *);
 template <int XW>
@@ -119,7 +119,8 @@ struct HostSys {
   int32_t hd_begin = 0, hd_count = 0;   // its entries of the hbond-lane list
   int32_t esk_begin = 0, esk_count = 0;  // Ewald structure-factor tasks
   int32_t ef_begin = 0, ef_count = 0;    // Ewald force tasks
-  int32_t pt_begin = 0, pt_count = 0;    // periodic electrostatic chunk-pair tasks
+  int32_t pt_begin = 0, pt_count = 0;    // electrostatic chunk-pair tasks (not periodic)
+  int32_t xt_begin = 0, xt_count = 0;    // those of a periodic system
   int32_t bp_begin = 0, bp_count = 0;    // bead tile pairs of the tile-pair list build
   int32_t qp_begin = 0, qp_count = 0;    // charge tile pairs
   int32_t et_begin = 0, et_count = 0;    // energy tasks
@@ -181,9 +182,10 @@ struct tis_ctx {
   unsigned long long *d_counters = nullptr;
   uint64_t *d_stepbase = nullptr;
   bool any_ele = false, any_periodic = false;
-  EwTask *d_ewsk = nullptr, *d_ewf = nullptr, *d_ptask = nullptr, *d_ptask_lpt = nullptr, *d_bpair = nullptr,
+  EwTask *d_ewsk = nullptr, *d_ewf = nullptr, *d_ptask = nullptr, *d_ptask_lpt = nullptr, *d_xtask = nullptr,
+         *d_bpair = nullptr,
          *d_qpair = nullptr;
-  int32_t n_ewsk = 0, n_ewf = 0, n_ptask = 0, n_bpair = 0, n_qpair = 0;
+  int32_t n_ewsk = 0, n_ewf = 0, n_ptask = 0, n_xtask = 0, n_bpair = 0, n_qpair = 0;
   // state
   int cur = 0;
   bool lists_valid = false;
@@ -425,9 +427,11 @@ void ewald_kvectors(const tis_params &p, std::vector<double> &hx, std::vector<do
       for (int iy = -hmax; iy <= hmax; ++iy)
         for (int iz = -hmax; iz <= hmax; ++iz) {
           if (ix * ix + iy * iy + iz * iz != r2) continue;
+          // one of h, -h for both, at twice the coefficient
+          if (ix < 0 || (ix == 0 && (iy < 0 || (iy == 0 && iz < 0)))) continue;
           hx.push_back(ix); hy.push_back(iy); hz.push_back(iz);
-          coef.push_back(2.0 * kPi / (L * L * L) * std::exp(-factor * factor * (double)r2 / (4.0 * a * a)) /
-                         (factor * factor * (double)r2));
+          coef.push_back(2.0 * (2.0 * kPi / (L * L * L) * std::exp(-factor * factor * (double)r2 / (4.0 * a * a)) /
+                                (factor * factor * (double)r2)));
         }
 }
 
@@ -460,7 +464,8 @@ struct Range {
   int hd0, hdn;             // hbond lanes
   int b0, nb, a0, na, s0, ns;
   int ek0, ekn, ef0, efn;   // Ewald tasks
-  int pt0, ptn;             // periodic electrostatic chunk-pair tasks
+  int pt0, ptn;             // electrostatic chunk-pair tasks (not periodic)
+  int xt0, xtn;             // those of periodic systems
 };
 
 // Whole-batch launch order of the bead tiles for k_main: workgroup b runs on
@@ -511,7 +516,7 @@ Range range_of(tis_ctx *c, int32_t isys) {
     r.hd0 = 0; r.hdn = c->nhbdense;
     r.b0 = 0; r.nb = c->stage.nbd; r.a0 = 0; r.na = c->stage.nba; r.s0 = 0; r.ns = c->stage.nst;
     r.ek0 = 0; r.ekn = c->n_ewsk; r.ef0 = 0; r.efn = c->n_ewf;
-    r.pt0 = 0; r.ptn = c->n_ptask;
+    r.pt0 = 0; r.ptn = c->n_ptask; r.xt0 = 0; r.xtn = c->n_xtask;
   } else {
     const HostSys &h = c->hs[isys];
     r.isys = isys;
@@ -521,7 +526,7 @@ Range range_of(tis_ctx *c, int32_t isys) {
     r.hd0 = h.hd_begin; r.hdn = h.hd_count;
     r.b0 = h.d.boff; r.nb = h.d.nbd; r.a0 = h.d.aoff; r.na = h.d.nba; r.s0 = h.d.soff; r.ns = h.d.nst;
     r.ek0 = h.esk_begin; r.ekn = h.esk_count; r.ef0 = h.ef_begin; r.efn = h.ef_count;
-    r.pt0 = h.pt_begin; r.ptn = h.pt_count;
+    r.pt0 = h.pt_begin; r.ptn = h.pt_count; r.xt0 = h.xt_begin; r.xtn = h.xt_count;
   }
   return r;
 }
@@ -1098,7 +1103,7 @@ int build_tables(tis_ctx *c) {
   c->tab_allocs.clear();
   c->tab_bytes = 0;
   std::vector<Tile> btiles, qtiles;
-  std::vector<EwTask> ptask, bpair, qpair, ewsk, ewf, etask;
+  std::vector<EwTask> ptask, xtask, bpair, qpair, ewsk, ewf, etask;
   std::vector<int32_t> systask, hbdense, efirst, wsys;
   c->systask_of.assign(c->nsys, -1);
   c->any_ele = false;
@@ -1108,7 +1113,7 @@ int build_tables(tis_ctx *c) {
     HostSys &h = c->hs[is];
     DSys &d = h.d;
     h.bt_begin = h.bt_count = h.qt_begin = h.qt_count = h.esk_begin = h.esk_count = 0;
-    h.ef_begin = h.ef_count = h.pt_begin = h.pt_count = h.bp_begin = h.bp_count = h.qp_begin = h.qp_count = 0;
+    h.ef_begin = h.ef_count = h.pt_begin = h.pt_count = h.xt_begin = h.xt_count = h.bp_begin = h.bp_count = h.qp_begin = h.qp_count = 0;
     h.hd_begin = h.hd_count = h.et_begin = h.et_count = 0;
     if (!h.live) { std::memset(&dsys[is], 0, sizeof(DSys)); dsys[is].nmp = 0; continue; }
     if (d.periodic) c->any_periodic = true;
@@ -1120,12 +1125,15 @@ int build_tables(tis_ctx *c) {
     for (int st0 = 0; st0 < d.nq; st0 += kTile) qtiles.push_back(Tile{is, st0});
     h.qt_count = (int32_t)qtiles.size() - h.qt_begin;
     d.bt0 = h.bt_begin; d.nbt = h.bt_count; d.qt0 = h.qt_begin; d.nqt = h.qt_count;
-    // electrostatic pairs: one wave per chunk pair (I, J), I <= J
+    // electrostatic pairs: one wave per chunk pair (I, J), I <= J, of a
+    // periodic system a block
     h.pt_begin = (int32_t)ptask.size();
+    h.xt_begin = (int32_t)xtask.size();
     if (d.ele_form != TIS_ELE_NONE && d.nq > 0)
       for (int I = 0; I < d.nqt; ++I)
-        for (int J = I; J < d.nqt; ++J) ptask.push_back(EwTask{is, I, J});
+        for (int J = I; J < d.nqt; ++J) (d.periodic ? xtask : ptask).push_back(EwTask{is, I, J});
     h.pt_count = (int32_t)ptask.size() - h.pt_begin;
+    h.xt_count = (int32_t)xtask.size() - h.xt_begin;
     // tile pairs of the periodic list builds (k_lpair; periodic systems
     // only: their number and the count buffer grow as nbt^2)
     h.bp_begin = (int32_t)bpair.size();
@@ -1166,7 +1174,7 @@ int build_tables(tis_ctx *c) {
   c->P.nsys = c->nsys;
   c->nbtile = (int32_t)btiles.size(); c->nqtile = (int32_t)qtiles.size(); c->nsystask = (int32_t)systask.size();
   c->nhbdense = (int32_t)hbdense.size();
-  c->n_ptask = (int32_t)ptask.size(); c->n_bpair = (int32_t)bpair.size(); c->n_qpair = (int32_t)qpair.size();
+  c->n_ptask = (int32_t)ptask.size(); c->n_xtask = (int32_t)xtask.size(); c->n_bpair = (int32_t)bpair.size(); c->n_qpair = (int32_t)qpair.size();
   c->n_ewsk = (int32_t)ewsk.size(); c->n_ewf = (int32_t)ewf.size();
   if (!dsys.empty()) {
     HIPCHK(c, hipMemcpyAsync(c->ab.sys, dsys.data(), dsys.size() * sizeof(DSys), hipMemcpyHostToDevice, c->stream));
@@ -1183,7 +1191,7 @@ int build_tables(tis_ctx *c) {
     const std::vector<Tile> xt = xcd_order(btiles, c->nsys);
     UPT(c->d_btiles_xcd, xt);
   }
-  UPT(c->d_ptask, ptask); UPT(c->d_ptask_lpt, lpt); UPT(c->d_bpair, bpair); UPT(c->d_qpair, qpair);
+  UPT(c->d_ptask, ptask); UPT(c->d_ptask_lpt, lpt); UPT(c->d_xtask, xtask); UPT(c->d_bpair, bpair); UPT(c->d_qpair, qpair);
   UPT(c->d_ewsk, ewsk); UPT(c->d_ewf, ewf); UPT(c->d_systask, systask);
   choose_window(c, wsys);
   UPT(c->d_wsys, wsys);
@@ -1688,29 +1696,30 @@ static void launch_force_pair(tis_ctx *c, const Range &r, int ix, int t_local, i
   // (launch shape: chunk pairs per wave, bonded terms per lane and the
   // order of the chunk pairs; tis_tune chooses it, no result depends on it)
   const int nterm = r.nb + r.na + r.ns;
-  const int npt = c->any_ele ? r.ptn : 0;
+  const int npt = c->any_ele ? r.ptn : 0, nxt = c->any_ele ? r.xtn : 0;
   const int ppw = c->shape.ppw, tpl = c->shape.tpl;
   const int nblk = (r.hdn + kTile * kWaves - 1) / (kTile * kWaves) + (r.taskn + kWaves - 1) / kWaves +
-                   (npt + kWaves * ppw - 1) / (kWaves * ppw) + (nterm + kTile * kWaves * tpl - 1) / (kTile * kWaves * tpl);
+                   nxt + (npt + kWaves * ppw - 1) / (kWaves * ppw) + (nterm + kTile * kWaves * tpl - 1) / (kTile * kWaves * tpl);
   if (nblk > 0) {
     const BondedRange br{r.b0, r.nb, r.a0, r.na, r.s0, r.ns, r.hd0, r.hdn};
     const int32_t *task = c->d_systask + r.task0;
     const EwTask *pt = r.all ? (c->shape.lpt ? c->d_ptask_lpt : c->d_ptask) : c->d_ptask + r.pt0;
+    const EwTask *xt = c->d_xtask + r.xt0;
     // one kernel per launch shape (each with its own register allocation)
     auto kf = ppw == 1 ? (tpl == 1 ? k_force<1, 1> : k_force<1, 2>) : (tpl == 1 ? k_force<2, 1> : k_force<2, 2>);
     if (c->timing)
       hipExtLaunchKernelGGL(kf, dim3(nblk), dim3(kTile * kWaves), 0, c->stream, e3[1], e3[2], 0, c->P, X, PX,
-                            task, r.taskn, pt, npt, br, pre_t);
+                            task, r.taskn, pt, npt, xt, nxt, br, pre_t);
     else
       hipLaunchKernelGGL(kf, dim3(nblk), dim3(kTile * kWaves), 0, c->stream, c->P, X, PX, task, r.taskn, pt, npt,
-                         br, pre_t);
+                         xt, nxt, br, pre_t);
   } else if (c->timing) {
     (void)hipEventRecord(e3[1], c->stream);
     (void)hipEventRecord(e3[2], c->stream);
   }
   if (r.ekn > 0) {
-    hipLaunchKernelGGL(k_ewald_sk, dim3(r.ekn), dim3(kTile), 0, c->stream, c->P, PX, c->d_ewsk + r.ek0, 0);
-    hipLaunchKernelGGL(k_ewald_f, dim3(r.efn), dim3(kTile * kWaves), 0, c->stream, c->P, PX, c->d_ewf + r.ef0);
+    hipLaunchKernelGGL(k_ewald_sk, dim3(r.ekn), dim3(kTile * kWaves), 0, c->stream, c->P, PX, c->d_ewsk + r.ek0, 0);
+    hipLaunchKernelGGL(k_ewald_f, dim3(r.efn), dim3(kEwThreads), 0, c->stream, c->P, PX, c->d_ewf + r.ef0);
   }
   if (c->timing) (void)hipEventRecord(e3[3], c->stream);
   const int32_t ele_on = c->any_ele ? 1 : 0;
@@ -1780,7 +1789,7 @@ int32_t tis_energy_sumup(tis_ctx *c, int32_t isys, double *energy_out) {
   // structure factors at the current coordinates (FP64 sin/cos)
   const int ek0 = isys < 0 ? 0 : c->hs[isys].esk_begin, ekn = isys < 0 ? c->n_ewsk : c->hs[isys].esk_count;
   if (ekn > 0)
-    hipLaunchKernelGGL(k_ewald_sk, dim3(ekn), dim3(kTile), 0, c->stream, c->P, PXc(c), c->d_ewsk + ek0, 1);
+    hipLaunchKernelGGL(k_ewald_sk, dim3(ekn), dim3(kTile * kWaves), 0, c->stream, c->P, PXc(c), c->d_ewsk + ek0, 1);
   // every live system (in live-list order) or one; the output is by system
   // index, zeros for retired systems
   const int nsel = isys < 0 ? c->nlive : 1, pos0 = isys < 0 ? 0 : c->hs[isys].live_pos;
@@ -1819,7 +1828,7 @@ int32_t tis_energy_sumup_set(tis_ctx *c, int32_t n, const int32_t *isys, double 
   for (int k = 0; k < n; ++k) {
     const HostSys &h = c->hs[isys[k]];
     if (h.esk_count > 0)
-      hipLaunchKernelGGL(k_ewald_sk, dim3(h.esk_count), dim3(kTile), 0, c->stream, c->P, PXc(c),
+      hipLaunchKernelGGL(k_ewald_sk, dim3(h.esk_count), dim3(kTile * kWaves), 0, c->stream, c->P, PXc(c),
                          c->d_ewsk + h.esk_begin, 1);
   }
   // the live position of each entry, then the tasks of the systems listed

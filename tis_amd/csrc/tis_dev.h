@@ -69,7 +69,7 @@ struct DSys {
   double cl_cut2, cl_rcinv;
   // Ewald: alpha, 2 alpha / sqrt(pi), alpha^2, 1/L, 2 C (2 pi / L), self energy
   double ew_alpha, ew_beta, ew_a2, ew_invL, ew_fscale, ew_self;
-  int32_t ewk0, nk;          // reciprocal vectors [ewk0, ewk0 + nk)
+  int32_t ewk0, nk;          // reciprocal vectors [ewk0, ewk0 + nk), one of each h, -h
   int32_t nqc, nkc;          // charge chunks of the S pass, k chunks of the force pass
   int64_t psk_off, pf_off;   // partial structure factors [nqc][nk][2], partial forces [nkc][3][nq]
   // electrostatics by chunk-pair tasks: partial forces
@@ -86,7 +86,8 @@ struct EwTask { int32_t sys, a, b; };
 // constants (time_integral_pre.F90:160-170): r[0] the noise amplitude c1,
 // r[1..3] c2, c3, c4, and 1/m.
 struct LangClass { double r[4], rcm, fric, mass, pad; };
-constexpr int kEwKChunk = 256;   // reciprocal vectors per block of the force pass
+constexpr int kEwKChunk = 128;   // reciprocal vectors per block of the force pass
+constexpr int kEwThreads = 512;  // its threads
 
 // Blocks of the energy pass for a system of nmp beads, nqt charge chunks and
 // nk reciprocal vectors: 256 beads or vectors, or two chunk pairs (32 of their
@@ -233,7 +234,7 @@ struct DevPtrs {
   uint8_t *qmirror;          // periodic ele mirror codes
   // Ewald reciprocal space
   const double *ewh;         // [3][nktot] integer h as FP64
-  const double *ewc;         // [nktot] f(h)
+  const double *ewc;         // [nktot] 2 f(h)
   int32_t nktot;
   double *psk;               // partial structure factors
   double *pf;                // partial reciprocal forces

@@ -774,7 +774,6 @@ __device__ inline void ele_pair_task(const DevPtrs &P, const DSys &s, const doub
   const float qiC = (float)(chi * s.ele_coef);
   const double cut2 = FORM == 0 ? s.dh_cut2 : s.cl_cut2;
   const uint32_t *row = P.qmask + s.moff + (int64_t)(valid ? qi : 0) * s.mwords;
-  const uint8_t *mrow = s.periodic ? P.qmirror + s.mioff + (int64_t)(valid ? qi : 0) * s.nq + jt : nullptr;
   uint64_t m64 = 0;
   if (valid) {
     const int wb = jt >> 5;
@@ -790,11 +789,7 @@ __device__ inline void ele_pair_task(const DevPtrs &P, const DSys &s, const doub
     if (last_half) bit = bit && lane < 32;
     // a step with no listed pair in the wave adds zeros: only the sums move
     if (__any(bit)) {
-      double v0 = SX[jl] - xi0, v1 = SY[jl] - xi1, v2 = SZ[jl] - xi2;
-      if (s.periodic) {
-        const int code = bit ? (int)mrow[jl] : 0;
-        v0 += mirror_shift(s, code, 0); v1 += mirror_shift(s, code, 1); v2 += mirror_shift(s, code, 2);
-      }
+      const double v0 = SX[jl] - xi0, v1 = SY[jl] - xi1, v2 = SZ[jl] - xi2;
       const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
       const bool on = bit && d2 <= cut2;
       float dv = ele_dv<FORM>(s, qiC * SQ[jl], on ? (float)d2 : 1.0f, nclamp, on);
@@ -965,17 +960,117 @@ __device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const 
   if (lane == 0 && nclamp) atomicAdd(&P.counters[1], (unsigned long long)nclamp);
 }
 
-// The force pass, one launch with four kinds of blocks: 256 hbond lanes per
+// ele_pair_task for a periodic system, by a block: the four waves take a
+// quarter of the steps each, and the quarters' sums, brought to one order of
+// charges in LDS, are added as (q0 + q1) + (q2 + q3).  A periodic system is
+// one box whose chunk pairs leave most of the chip idle, so the time is one
+// wave's chain; its mirror codes, a byte load per step on that chain before,
+// are loaded ahead for all of a wave's steps (packed four to a word, bit 7: the
+// pair is listed).  640 charges (55 chunk pairs): the force pass took 32.8 us
+// with a wave per chunk pair, 10.8 now.
+template <int FORM, bool DPP>
+__device__ inline void ele_pair_periodic(const DevPtrs &P, const DSys &s, const double *Y, int I, int J, int dir,
+                                         EleLds &lds) {
+  const int tid = (int)threadIdx.x, lane = tid & (kTile - 1);
+  const int part = __builtin_amdgcn_readfirstlane(tid / kTile);
+  const int rd = dir != 0 ? dir : 1;
+  const int n = P.ntot;
+  EleWave &JE = lds.w[0];
+  double(*red)[6][kTile] = reinterpret_cast<double(*)[6][kTile]>(&lds.w[1]);   // quarters 1-3
+  static_assert(sizeof(EleWave) >= 6 * kTile * sizeof(double), "the quarters' sums do not fit");
+  const int qi = I * kTile + lane, jt = J * kTile;
+  const bool valid = qi < s.nq, diag = I == J;
+  const int ns = diag ? 8 : 16, kb = diag ? 1 + 8 * part : 16 * part;   // this wave's steps
+  uint64_t m64 = 0;
+  if (valid) {
+    const uint32_t *row = P.qmask + s.moff + (int64_t)qi * s.mwords;
+    const int wb = jt >> 5;
+    m64 = row[wb];
+    if (wb + 1 < s.mwords) m64 |= (uint64_t)row[wb + 1] << 32;
+  }
+  uint32_t pk[4] = {0u, 0u, 0u, 0u};
+  {
+    const uint8_t *mrow = P.qmirror + s.mioff + (int64_t)(valid ? qi : 0) * s.nq + jt;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      const int k = kb + u, jl = (lane + rd * k) & (kTile - 1);
+      const bool bit = ((m64 >> jl) & 1u) && u < ns && !(diag && k == 32 && lane >= 32);
+      const uint32_t code = mrow[bit ? jl : 0];   // unlisted: the row's first, unused
+      pk[u >> 2] |= (bit ? code | 0x80u : 0u) << (8 * (u & 3));
+    }
+  }
+  double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0, chi = 0.0;
+  if (valid) {
+    const int gi = P.qbead[s.qoff + qi];
+    xi0 = Y[gi]; xi1 = Y[n + gi]; xi2 = Y[2 * n + gi];
+    chi = P.charge[gi];
+  }
+  if (part == 0) {
+    const bool vj = jt + lane < s.nq;
+    const int gj = vj ? P.qbead[s.qoff + jt + lane] : 0;
+    JE.x[lane] = vj ? Y[gj] : 0.0; JE.y[lane] = vj ? Y[n + gj] : 0.0; JE.z[lane] = vj ? Y[2 * n + gj] : 0.0;
+    JE.q[lane] = vj ? (float)P.charge[gj] : 0.0f;
+  }
+  __syncthreads();
+  const float qiC = (float)(chi * s.ele_coef);
+  const double cut2 = FORM == 0 ? s.dh_cut2 : s.cl_cut2;
+  double F[3] = {0.0, 0.0, 0.0}, G[3] = {0.0, 0.0, 0.0};
+  unsigned nclamp = 0;
+  const bool any = __any(m64 != 0);
+#pragma unroll 1
+  for (int k0 = 0; any && k0 < ns; k0 += 4) {
+    const uint32_t w = pk[0];
+    pk[0] = pk[1]; pk[1] = pk[2]; pk[2] = pk[3];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int jl = (lane + rd * (kb + k0 + u)) & (kTile - 1);
+      const int code = (int)((w >> (8 * u)) & 0x7fu);
+      const bool bit = (w >> (8 * u)) & 0x80u;
+      const double v0 = (JE.x[jl] - xi0) + mirror_shift(s, code, 0);
+      const double v1 = (JE.y[jl] - xi1) + mirror_shift(s, code, 1);
+      const double v2 = (JE.z[jl] - xi2) + mirror_shift(s, code, 2);
+      const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
+      const bool on = bit && d2 <= cut2;
+      float dv = ele_dv<FORM>(s, qiC * JE.q[jl], on ? (float)d2 : 1.0f, nclamp, on);
+      const double dd = on ? (double)dv : 0.0;
+      F[0] -= dd * v0; F[1] -= dd * v1; F[2] -= dd * v2;
+      G[0] += dd * v0; G[1] += dd * v1; G[2] += dd * v2;
+      for (int d = 0; d < 3; ++d) G[d] = rot_next<DPP>(G[d]);
+    }
+  }
+  if (nclamp) atomicAdd(&P.counters[1], (unsigned long long)nclamp);
+  // lane l's G is now the sum on charge l + rd (kb + ns)
+  const int turn = rd * (kb + ns);
+  if (part > 0) {
+    for (int d = 0; d < 3; ++d) {
+      red[part - 1][d][lane] = F[d];
+      red[part - 1][3 + d][(lane + turn) & (kTile - 1)] = G[d];
+    }
+  }
+  __syncthreads();
+  if (part > 0) return;
+  double *pp = P.pp + s.pp_off + ele_task_index(I, J, s.nqt) * (6 * kTile);
+  for (int d = 0; d < 3; ++d) {
+    const double g0 = __shfl(G[d], (lane - turn) & (kTile - 1));
+    const double f = (F[d] + red[0][d][lane]) + (red[1][d][lane] + red[2][d][lane]);
+    const double g = (g0 + red[0][3 + d][lane]) + (red[1][3 + d][lane] + red[2][3 + d][lane]);
+    if (!diag) pp[(3 + d) * kTile + lane] = g;
+    pp[d * kTile + lane] = diag ? f + g : f;
+  }
+}
+
+// The force pass, one launch with five kinds of blocks: 256 hbond lanes per
 // block (hbond_lane: the hbonds of systems without valence-limited sites, one
 // lane each, first because each lane is a long FP64 chain), four systems'
 // tertiary stacks and valence-limited hbonds per block (terms_wave, one wave
-// each), four electrostatic chunk pairs per block (ele_pair_task, one wave
-// each), then the bonded terms, 256 lanes per block (bonded_lane).  k_main
+// each), an electrostatic chunk pair of a periodic system per block
+// (ele_pair_periodic), four of others per block (ele_pair_unrolled,
+// ele_pair_task, one wave each), then the bonded terms, 256 lanes per block (bonded_lane).  k_main
 // gathers all of their outputs.
 template <int PPW, int TPL>
 __global__ __launch_bounds__(kTile * kWaves) __attribute__((amdgpu_waves_per_eu(4)))
 void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systask, int ntask,
-             const EwTask *ptasks, int npt, BondedRange br, int32_t t_local) {
+             const EwTask *ptasks, int npt, const EwTask *xtasks, int nxt, BondedRange br, int32_t t_local) {
   constexpr int ppw = PPW, tpl = TPL;
   __shared__ EleLds lds;
   if (run_stopped(P)) return;
@@ -995,9 +1090,25 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
     return;
   }
   b -= ntb;
+  if (b < nxt) {
+    const EwTask tk = xtasks[b];
+    const DSys s = P.sys[tk.sys];
+    const int dir = wave_dir();
+    if (dir != 0) {
+      if (s.ele_form == 0) ele_pair_periodic<0, true>(P, s, PX, tk.a, tk.b, dir, lds);
+      else if (s.ele_form == 1) ele_pair_periodic<1, true>(P, s, PX, tk.a, tk.b, dir, lds);
+      else ele_pair_periodic<2, true>(P, s, PX, tk.a, tk.b, dir, lds);
+    } else {
+      if (s.ele_form == 0) ele_pair_periodic<0, false>(P, s, PX, tk.a, tk.b, dir, lds);
+      else if (s.ele_form == 1) ele_pair_periodic<1, false>(P, s, PX, tk.a, tk.b, dir, lds);
+      else ele_pair_periodic<2, false>(P, s, PX, tk.a, tk.b, dir, lds);
+    }
+    return;
+  }
+  b -= nxt;
   if (b >= npb) {
     // tpl bonded terms per lane, a grid-wide stride apart
-    const int nbb = (int)gridDim.x - nhdb - ntb - npb;
+    const int nbb = (int)gridDim.x - nhdb - ntb - nxt - npb;
     for (int i = 0; i < tpl; ++i)
       bonded_lane(P, X, PX, br, (b - npb + i * nbb) * (kTile * kWaves) + (int)threadIdx.x);
     return;
@@ -1020,31 +1131,23 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
     }
     const EwTask tk = ptasks[task];
     const DSys s = P.sys[tk.sys];
-    const double *Y = s.periodic ? PX : X;
-    if (dir != 0 && !s.periodic && s.ele_form == 0) {
-      ele_pair_unrolled<0>(P, s, Y, tk.a, tk.b, dir, JE);
-    } else if (dir != 0 && !s.periodic && s.ele_form == 1) {
-      ele_pair_unrolled<1>(P, s, Y, tk.a, tk.b, dir, JE);
-    } else if (dir != 0) {
-      if (s.ele_form == 0) ele_pair_task<0, true>(P, s, Y, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-      else if (s.ele_form == 1) ele_pair_task<1, true>(P, s, Y, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-      else ele_pair_task<2, true>(P, s, Y, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-    } else {
-      if (s.ele_form == 0) ele_pair_task<0, false>(P, s, Y, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-      else if (s.ele_form == 1) ele_pair_task<1, false>(P, s, Y, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-      else ele_pair_task<2, false>(P, s, Y, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-    }
+    if (dir != 0 && s.ele_form == 0) ele_pair_unrolled<0>(P, s, X, tk.a, tk.b, dir, JE);
+    else if (dir != 0 && s.ele_form == 1) ele_pair_unrolled<1>(P, s, X, tk.a, tk.b, dir, JE);
+    else if (s.ele_form == 0) ele_pair_task<0, false>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
+    else if (s.ele_form == 1) ele_pair_task<1, false>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
+    else if (dir != 0) ele_pair_task<2, true>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
+    else ele_pair_task<2, false>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
   }
 }
 
 template __global__ void k_force<1, 1>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, BondedRange, int32_t);
+                                       int, const EwTask *, int, BondedRange, int32_t);
 template __global__ void k_force<2, 1>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, BondedRange, int32_t);
+                                       int, const EwTask *, int, BondedRange, int32_t);
 template __global__ void k_force<1, 2>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, BondedRange, int32_t);
+                                       int, const EwTask *, int, BondedRange, int32_t);
 template __global__ void k_force<2, 2>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, BondedRange, int32_t);
+                                       int, const EwTask *, int, BondedRange, int32_t);
 
 // ------------------------------------------------------------------ Ewald reciprocal space
 // force_ele_coulomb_ewld.F90:62-84.  The phase k.r = 2 pi (h . r/L) is
@@ -1052,32 +1155,44 @@ template __global__ void k_force<2, 2>(DevPtrs, const double *, const double *, 
 // turns before the FP32 sincospi, so its rounding does not grow with |h| or
 // the box; structure factors and forces accumulate in FP64.
 //
+// The vectors are one of each pair h, -h, with twice the coefficient: the
+// phase of -h is the negative, exactly, so the other half would repeat the
+// same cosines and opposite sines.
+//
 // Pass 1: partial structure factors.  One lane per reciprocal vector of a
-// 64-vector tile, over one 64-charge chunk staged in LDS (broadcast reads).
+// 64-vector tile, over one 64-charge chunk staged in LDS (broadcast reads),
+// a quarter of the chunk per wave, the quarters added as (q0 + q1) + (q2 +
+// q3): bound by the sines' arithmetic, which a wave per tile and chunk left
+// to a few waves and their latency.  |h| <= 10, 640 charges: 10.5 us for all
+// vectors with a wave per tile and chunk, 5.4 now.
 // exact = 1 (energy evaluation) takes sin/cos in FP64.
-__global__ __launch_bounds__(kTile) void k_ewald_sk(DevPtrs P, const double *PX, const EwTask *tasks, int exact) {
+__global__ __launch_bounds__(kTile * kWaves) void k_ewald_sk(DevPtrs P, const double *PX, const EwTask *tasks,
+                                                             int exact) {
   __shared__ double fx[kTile], fy[kTile], fz[kTile], fq[kTile];
+  __shared__ double red[kWaves - 1][2][kTile];
   if (run_stopped(P)) return;
   const EwTask tk = tasks[blockIdx.x];
   const DSys s = P.sys[tk.sys];
-  const int lane = threadIdx.x, n = P.ntot;
-  const int qi = tk.b * kTile + lane;
-  if (qi < s.nq) {
-    const int g = P.qbead[s.qoff + qi];
-    fx[lane] = PX[g] * s.ew_invL; fy[lane] = PX[n + g] * s.ew_invL; fz[lane] = PX[2 * n + g] * s.ew_invL;
-    fq[lane] = P.charge[g];
-  } else {
-    fx[lane] = fy[lane] = fz[lane] = 0.0; fq[lane] = 0.0;
+  const int lane = threadIdx.x & (kTile - 1), w = threadIdx.x / kTile, n = P.ntot;
+  const int k = tk.a * kTile + lane;
+  const int kg = s.ewk0 + min(k, s.nk - 1);
+  const double hx = P.ewh[kg], hy = P.ewh[P.nktot + kg], hz = P.ewh[2 * P.nktot + kg];
+  if (w == 0) {
+    const int qi = tk.b * kTile + lane;
+    if (qi < s.nq) {
+      const int g = P.qbead[s.qoff + qi];
+      fx[lane] = PX[g] * s.ew_invL; fy[lane] = PX[n + g] * s.ew_invL; fz[lane] = PX[2 * n + g] * s.ew_invL;
+      fq[lane] = P.charge[g];
+    } else {
+      fx[lane] = fy[lane] = fz[lane] = 0.0; fq[lane] = 0.0;
+    }
   }
   __syncthreads();
-  const int k = tk.a * kTile + lane;
-  if (k >= s.nk) return;
-  const int kg = s.ewk0 + k;
-  const double hx = P.ewh[kg], hy = P.ewh[P.nktot + kg], hz = P.ewh[2 * P.nktot + kg];
-  const int jn = min(kTile, s.nq - tk.b * kTile);
+  constexpr int kPart = kTile / kWaves;
+  const int j0 = w * kPart, j1 = min(j0 + kPart, s.nq - tk.b * kTile);
   double sc = 0.0, ss = 0.0;
   if (exact) {
-    for (int j = 0; j < jn; ++j) {
+    for (int j = j0; j < j1; ++j) {
       double t = hx * fx[j] + hy * fy[j] + hz * fz[j];
       t -= rint(t);
       double sn, cs;
@@ -1086,7 +1201,8 @@ __global__ __launch_bounds__(kTile) void k_ewald_sk(DevPtrs P, const double *PX,
       ss += fq[j] * sn;
     }
   } else {
-    for (int j = 0; j < jn; ++j) {
+#pragma unroll 4
+    for (int j = j0; j < j1; ++j) {
       double t = hx * fx[j] + hy * fy[j] + hz * fz[j];
       t -= rint(t);
       float sn, cs;
@@ -1095,57 +1211,75 @@ __global__ __launch_bounds__(kTile) void k_ewald_sk(DevPtrs P, const double *PX,
       ss += fq[j] * (double)sn;
     }
   }
+  if (w > 0) {
+    red[w - 1][0][lane] = sc;
+    red[w - 1][1][lane] = ss;
+  }
+  __syncthreads();
+  if (w > 0 || k >= s.nk) return;
   double *o = P.psk + s.psk_off + 2 * ((int64_t)tk.b * s.nk + k);
-  o[0] = sc; o[1] = ss;
+  o[0] = (sc + red[0][0][lane]) + (red[1][0][lane] + red[2][0][lane]);
+  o[1] = (ss + red[0][1][lane]) + (red[1][1][lane] + red[2][1][lane]);
 }
 
-// Pass 2: forces.  A block takes a 64-charge tile and a chunk of 256
+// Pass 2: forces.  A block takes a 64-charge tile and a chunk of kEwKChunk
 // reciprocal vectors: it first sums the partial structure factors of its
-// vectors (fixed chunk order) into LDS, then each wave sweeps 64 of them for
-// its lane's charge; partial forces per chunk go to pf (summed by k_main).
-__global__ __launch_bounds__(kTile * kWaves) void k_ewald_f(DevPtrs P, const double *PX, const EwTask *tasks) {
-  __shared__ double shx[kEwKChunk], shy[kEwKChunk], shz[kEwKChunk], sfc[kEwKChunk], ssc[kEwKChunk], sss[kEwKChunk];
-  __shared__ double red[3][kWaves][kTile];
+// vectors into LDS (even charge chunks, odd ones, then both), then each wave
+// sweeps an eighth of them for its lane's charge; partial forces per chunk go
+// to pf (summed by k_main).  Bound as pass 1: 14.9 us for all vectors in
+// chunks of 256 by four waves, 7.8 now, and k_main 11.1 -> 8.1 us with half as
+// many partial forces to add.
+__global__ __launch_bounds__(kEwThreads) void k_ewald_f(DevPtrs P, const double *PX, const EwTask *tasks) {
+  constexpr int kW = kEwThreads / kTile, kPart = kEwKChunk / kW;
+  static_assert(kEwThreads == 4 * kEwKChunk, "a thread per vector, component and half of the charge chunks");
+  __shared__ double shx[kEwKChunk], shy[kEwKChunk], shz[kEwKChunk], sfc[kEwKChunk];
+  __shared__ double sum[2][2][kEwKChunk];   // [half][cosine, sine][vector]
+  __shared__ double red[3][kW][kTile];
   if (run_stopped(P)) return;
   const EwTask tk = tasks[blockIdx.x];
   const DSys s = P.sys[tk.sys];
   const int tid = threadIdx.x, n = P.ntot;
-  {
-    const int k = tk.b * kEwKChunk + tid;
-    double sc = 0.0, ss = 0.0, fc = 0.0, hx = 0.0, hy = 0.0, hz = 0.0;
-    if (k < s.nk) {
-      const double *ps = P.psk + s.psk_off + 2 * (int64_t)k;
-      for (int c = 0; c < s.nqc; ++c) { sc += ps[2 * (int64_t)c * s.nk]; ss += ps[2 * (int64_t)c * s.nk + 1]; }
-      const int kg = s.ewk0 + k;
-      fc = P.ewc[kg]; hx = P.ewh[kg]; hy = P.ewh[P.nktot + kg]; hz = P.ewh[2 * P.nktot + kg];
-    }
-    shx[tid] = hx; shy[tid] = hy; shz[tid] = hz; sfc[tid] = fc; ssc[tid] = sc; sss[tid] = ss;
-  }
-  __syncthreads();
   const int lane = tid & (kTile - 1), w = tid / kTile;
   const int qi = tk.a * kTile + lane;
   const bool valid = qi < s.nq;
-  double f0 = 0.0, f1 = 0.0, f2 = 0.0;
-  if (valid) {
-    const int g = P.qbead[s.qoff + qi];
-    const double x0 = PX[g] * s.ew_invL, x1 = PX[n + g] * s.ew_invL, x2 = PX[2 * n + g] * s.ew_invL;
-    const int kb = w * kTile, ke = min(kb + kTile, s.nk - tk.b * kEwKChunk);
-    for (int k = kb; k < ke; ++k) {
-      double t = shx[k] * x0 + shy[k] * x1 + shz[k] * x2;
-      t -= rint(t);
-      float sn, cs;
-      sincospif((float)(2.0 * t), &sn, &cs);
-      const double term = sfc[k] * ((double)sn * ssc[k] - (double)cs * sss[k]);
-      f0 += term * shx[k]; f1 += term * shy[k]; f2 += term * shz[k];
+  const int g = P.qbead[s.qoff + min(qi, s.nq - 1)];
+  const double x0 = PX[g] * s.ew_invL, x1 = PX[n + g] * s.ew_invL, x2 = PX[2 * n + g] * s.ew_invL;
+  {
+    const int v = tid & (kEwKChunk - 1), part = tid / kEwKChunk, comp = part & 1, half = part >> 1;
+    const int k = tk.b * kEwKChunk + v;
+    double a = 0.0, fc = 0.0, hx = 0.0, hy = 0.0, hz = 0.0;
+    if (k < s.nk) {
+      const double *ps = P.psk + s.psk_off + 2 * (int64_t)k + comp;
+#pragma unroll 8
+      for (int c = half; c < s.nqc; c += 2) a += ps[2 * (int64_t)c * s.nk];
+      const int kg = s.ewk0 + k;
+      if (part == 0) {
+        fc = P.ewc[kg]; hx = P.ewh[kg]; hy = P.ewh[P.nktot + kg]; hz = P.ewh[2 * P.nktot + kg];
+      }
     }
+    sum[half][comp][v] = a;
+    if (part == 0) { shx[v] = hx; shy[v] = hy; shz[v] = hz; sfc[v] = fc; }
+  }
+  __syncthreads();
+  double f0 = 0.0, f1 = 0.0, f2 = 0.0;
+  const int kb = w * kPart, ke = min(kb + kPart, s.nk - tk.b * kEwKChunk);
+#pragma unroll 4
+  for (int k = kb; k < ke; ++k) {
+    double t = shx[k] * x0 + shy[k] * x1 + shz[k] * x2;
+    t -= rint(t);
+    float sn, cs;
+    sincospif((float)(2.0 * t), &sn, &cs);
+    const double sck = sum[0][0][k] + sum[1][0][k], ssk = sum[0][1][k] + sum[1][1][k];
+    const double term = sfc[k] * ((double)sn * sck - (double)cs * ssk);
+    f0 += term * shx[k]; f1 += term * shy[k]; f2 += term * shz[k];
   }
   red[0][w][lane] = f0; red[1][w][lane] = f1; red[2][w][lane] = f2;
   __syncthreads();
-  if (w == 0 && valid) {
-    const double scale = s.ew_fscale * P.charge[P.qbead[s.qoff + qi]];
-    for (int d = 0; d < 3; ++d)
-      P.pf[s.pf_off + ((int64_t)tk.b * 3 + d) * s.nq + qi] =
-          scale * (((red[d][0][lane] + red[d][1][lane]) + red[d][2][lane]) + red[d][3][lane]);
+  if (w < 3 && valid) {
+    const double scale = s.ew_fscale * P.charge[g];
+    double f = red[w][0][lane];
+    for (int q = 1; q < kW; ++q) f += red[w][q][lane];
+    P.pf[s.pf_off + ((int64_t)tk.b * 3 + w) * s.nq + qi] = scale * f;
   }
 }
 
@@ -1415,6 +1549,7 @@ __device__ inline void ele_sums(const DevPtrs &P, const DSys &s, int g, double F
   }
   if (s.ele_form == 2) {
     const double *pf = P.pf + s.pf_off + lq;
+#pragma unroll 4
     for (int c = 0; c < s.nkc; ++c)
       for (int d = 0; d < 3; ++d) F[d] += pf[((int64_t)c * 3 + d) * s.nq];
   }
