@@ -1,13 +1,14 @@
 """Periodic chunk pairs (a block each, a quarter of the steps per wave) and the
 reciprocal pass (half of the vectors, quarters of the charge chunks) at the
-edges of their tiles, every electrostatic form, against the FP64 oracle."""
+edges of their tiles, with the lists
+of such systems, every electrostatic form, against the FP64 oracle."""
 import numpy as np
 import pytest
 
 import oracle
 from systems import force_error
 from tis_amd import topology as T
-from tis_amd.engine import Engine
+from tis_amd.engine import LIST_ELE, LIST_EXV, Engine
 from tis_amd.sysdesc import ELE_COULOMB, ELE_DH, ELE_EWALD
 
 pytestmark = pytest.mark.gpu
@@ -42,6 +43,11 @@ def test_forces_and_energies(nq, form, hmax):
     en = e.energy_sumup(0)
     o = oracle.Oracle(s)
     o.neighbor(x)
+    for which, k in ((LIST_EXV, 0), (LIST_ELE, 1)):
+        a, b = e.pairs(0, which), o.lists(k)
+        (a, ac), (b, bc) = (a, b) if k else ((a, np.zeros(len(a))), (b, np.zeros(len(b))))
+        p, q = np.lexsort(a.T[::-1]), np.lexsort(b.T[::-1])
+        assert np.array_equal(a[p], b[q]) and np.array_equal(ac[p], bc[q])
     fo, _ = o.force(x, seed=0, sys_id=0, step=0)
     eo = o.energy(x, np.zeros_like(x))
     err = force_error(f, fo).max()

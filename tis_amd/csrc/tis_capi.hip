@@ -22,8 +22,8 @@
 namespace tis {
 template <int PPW, int TPL>
 __global__ void k_force(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *, int,
-                        const EwTask *, int, BondedRange, int32_t);
-__global__ void k_ewald_sk(DevPtrs, const double *, const EwTask *, int);
+                        const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
+__global__ void k_ewald_sk(DevPtrs, const double *, const EwTask *);
 __global__ void k_ewald_f(DevPtrs, const double *, const EwTask *);
 template <int XW>
 __global__ void k_main(DevPtrs, const double *, const double *, const float4 *, double *, double *, float4 *,
@@ -33,8 +33,8 @@ __global__ void k_prep(DevPtrs, const double *, double *, double *, float4 *, fl
                        const Tile *, int, int, int, int);
 __global__ void k_lists(DevPtrs, const double *, const double *, const Tile *, int, int, const Tile *, int, int, int,
                         int, int);
-__global__ void k_lpair(DevPtrs, const double *, const double *, const EwTask *, int, const EwTask *, int, int, int,
-                        int, int);
+__global__ void k_lpair(DevPtrs, const double *, const EwTask *, int, const EwTask *, int);
+__global__ void k_lpair_put(DevPtrs, const double *, const EwTask *, int, int);
 __global__ void k_advance(uint64_t *, uint64_t, uint64_t, uint64_t, unsigned long long *);
 __global__ void k_window(DevPtrs, const int32_t *, int, int, int, int, int);
 __global__ void k_run_report(unsigned long long *, unsigned long long *);
@@ -183,8 +183,7 @@ struct tis_ctx {
   uint64_t *d_stepbase = nullptr;
   bool any_ele = false, any_periodic = false;
   EwTask *d_ewsk = nullptr, *d_ewf = nullptr, *d_ptask = nullptr, *d_ptask_lpt = nullptr, *d_xtask = nullptr,
-         *d_bpair = nullptr,
-         *d_qpair = nullptr;
+         *d_bpair = nullptr, *d_qpair = nullptr;
   int32_t n_ewsk = 0, n_ewf = 0, n_ptask = 0, n_xtask = 0, n_bpair = 0, n_qpair = 0;
   // state
   int cur = 0;
@@ -531,17 +530,15 @@ Range range_of(tis_ctx *c, int32_t isys) {
   return r;
 }
 
-static void launch_lpair(tis_ctx *c, const Range &r, const double *X, const double *PX, int mode, int h0, int nh) {
+static void launch_lpair(tis_ctx *c, const Range &r, const double *PX, int gate) {
   const int bp0 = r.all ? 0 : c->hs[r.isys].bp_begin, nbp = r.all ? c->n_bpair : c->hs[r.isys].bp_count;
   const int qp0 = r.all ? 0 : c->hs[r.isys].qp_begin, nqp = r.all ? c->n_qpair : c->hs[r.isys].qp_count;
-  const int nbb = (nbp + kWaves - 1) / kWaves, nqb = (nqp + kWaves - 1) / kWaves;
-  const int nhb = (nh + kTile * kWaves - 1) / (kTile * kWaves);
-  if (nbb + nqb + nhb > 0)
-    hipLaunchKernelGGL(k_lpair, dim3(nbb + nqb + nhb), dim3(kTile * kWaves), 0, c->stream, c->P, X, PX,
-                       c->d_bpair + bp0, nbp, c->d_qpair + qp0, nqp, h0, nh, mode, 0);
-  if (nbb > 0)
-    hipLaunchKernelGGL(k_lpair, dim3(nbb), dim3(kTile * kWaves), 0, c->stream, c->P, X, PX, c->d_bpair + bp0, nbp,
-                       c->d_qpair + qp0, nqp, h0, 0, mode, 1);
+  if (nbp + nqp > 0)
+    hipLaunchKernelGGL(k_lpair, dim3(nbp + nqp), dim3(kTile * kWaves), 0, c->stream, c->P, PX, c->d_bpair + bp0, nbp,
+                       c->d_qpair + qp0, gate);
+  if (nbp > 0)
+    hipLaunchKernelGGL(k_lpair_put, dim3((nbp + kWaves - 1) / kWaves), dim3(kTile * kWaves), 0, c->stream, c->P, PX,
+                       c->d_bpair + bp0, nbp, gate);
 }
 
 // The lists of the range from the positions in buffer cu (wrapped copies into
@@ -571,7 +568,7 @@ int launch_lists(tis_ctx *c, const Range &r, int cu, int with_pred, int gate) {
   if (nblk > 0)
     hipLaunchKernelGGL(k_lists, dim3(nblk), dim3(kTile), 0, c->stream, c->P, X, PXcur, c->d_btiles, r.bt0, r.btn,
                        c->d_qtiles, r.qt0, r.qtn, h0, nh, gate);
-  if (periodic) launch_lpair(c, r, X, PXcur, gate ? 3 : 2, h0, 0);
+  if (periodic) launch_lpair(c, r, PXcur, gate);
   return 0;
 }
 
@@ -968,7 +965,7 @@ int alloc_arena(tis_ctx *c, const Caps &k, std::vector<void *> &list, DevPtrs &P
   AL(P.nb, (size_t)P.nb_cap * B);
   AL(P.dxyz, 3 * B); AL(P.dlast, 3 * B);
   AL(P.sys_flag, k.nsys); AL(P.win_at, k.nsys);
-  AL(P.pp, k.pp); AL(P.qmask, k.m); AL(P.qmirror, k.mi); AL(P.lcnt, k.lp * kTile);
+  AL(P.pp, k.pp); AL(P.qmask, k.m); AL(P.qmirror, k.mi); AL(P.lmask, k.lp * kTile);
   AL(A.ewh, 3 * k.k); AL(A.ewc, k.k); AL(P.psk, k.psk); AL(P.pf, k.pf);
   AL(A.counters, TIS_CNT_MAX); AL(A.stepbase, 1);
 #undef AL
@@ -1665,8 +1662,8 @@ int32_t tis_pairs_get(tis_ctx *c, int32_t isys, int32_t which, int32_t *pairs, d
 // at 640 (10.8), 17.5 against 13.6 at 1,280.
 constexpr int kMainWideTiles = 512;
 
-// k_force (terms, electrostatic chunk pairs, bonded terms), the Ewald
-// passes, then k_main, at the positions in buffer ix (the next ones go to the
+// k_force (structure factors, terms, electrostatic chunk pairs, bonded terms),
+// the second Ewald pass, then k_main, at the positions in buffer ix (the next ones go to the
 // other).  Steps draw noise/valence numbers for step
 // stepbase+t+1; a stand-alone force evaluation or the initial acceleration
 // uses stepbase.
@@ -1690,35 +1687,34 @@ static void launch_force_pair(tis_ctx *c, const Range &r, int ix, int t_local, i
     c->tev_used += kTev;
     (void)hipEventRecord(e3[0], c->stream);
   }
-  // k_force: hbond lanes, per-system tertiary stacks and valence-limited
-  // hbonds, the electrostatic chunk pairs, then the bonded terms in blocks of
-  // 256 lanes
+  // k_force: the structure factors' tiles, hbond lanes, per-system tertiary
+  // stacks and valence-limited hbonds, the electrostatic chunk pairs, then the
+  // bonded terms in blocks of 256 lanes
   // (launch shape: chunk pairs per wave, bonded terms per lane and the
   // order of the chunk pairs; tis_tune chooses it, no result depends on it)
   const int nterm = r.nb + r.na + r.ns;
   const int npt = c->any_ele ? r.ptn : 0, nxt = c->any_ele ? r.xtn : 0;
   const int ppw = c->shape.ppw, tpl = c->shape.tpl;
-  const int nblk = (r.hdn + kTile * kWaves - 1) / (kTile * kWaves) + (r.taskn + kWaves - 1) / kWaves +
+  const int nblk = r.ekn + (r.hdn + kTile * kWaves - 1) / (kTile * kWaves) + (r.taskn + kWaves - 1) / kWaves +
                    nxt + (npt + kWaves * ppw - 1) / (kWaves * ppw) + (nterm + kTile * kWaves * tpl - 1) / (kTile * kWaves * tpl);
   if (nblk > 0) {
     const BondedRange br{r.b0, r.nb, r.a0, r.na, r.s0, r.ns, r.hd0, r.hdn};
     const int32_t *task = c->d_systask + r.task0;
     const EwTask *pt = r.all ? (c->shape.lpt ? c->d_ptask_lpt : c->d_ptask) : c->d_ptask + r.pt0;
-    const EwTask *xt = c->d_xtask + r.xt0;
+    const EwTask *xt = c->d_xtask + r.xt0, *kt = c->d_ewsk + r.ek0;
     // one kernel per launch shape (each with its own register allocation)
     auto kf = ppw == 1 ? (tpl == 1 ? k_force<1, 1> : k_force<1, 2>) : (tpl == 1 ? k_force<2, 1> : k_force<2, 2>);
     if (c->timing)
       hipExtLaunchKernelGGL(kf, dim3(nblk), dim3(kTile * kWaves), 0, c->stream, e3[1], e3[2], 0, c->P, X, PX,
-                            task, r.taskn, pt, npt, xt, nxt, br, pre_t);
+                            task, r.taskn, pt, npt, xt, nxt, kt, r.ekn, br, pre_t);
     else
       hipLaunchKernelGGL(kf, dim3(nblk), dim3(kTile * kWaves), 0, c->stream, c->P, X, PX, task, r.taskn, pt, npt,
-                         xt, nxt, br, pre_t);
+                         xt, nxt, kt, r.ekn, br, pre_t);
   } else if (c->timing) {
     (void)hipEventRecord(e3[1], c->stream);
     (void)hipEventRecord(e3[2], c->stream);
   }
-  if (r.ekn > 0) {
-    hipLaunchKernelGGL(k_ewald_sk, dim3(r.ekn), dim3(kTile * kWaves), 0, c->stream, c->P, PX, c->d_ewsk + r.ek0, 0);
+  if (r.efn > 0) {
     hipLaunchKernelGGL(k_ewald_f, dim3(r.efn), dim3(kEwThreads), 0, c->stream, c->P, PX, c->d_ewf + r.ef0);
   }
   if (c->timing) (void)hipEventRecord(e3[3], c->stream);
@@ -1789,7 +1785,7 @@ int32_t tis_energy_sumup(tis_ctx *c, int32_t isys, double *energy_out) {
   // structure factors at the current coordinates (FP64 sin/cos)
   const int ek0 = isys < 0 ? 0 : c->hs[isys].esk_begin, ekn = isys < 0 ? c->n_ewsk : c->hs[isys].esk_count;
   if (ekn > 0)
-    hipLaunchKernelGGL(k_ewald_sk, dim3(ekn), dim3(kTile * kWaves), 0, c->stream, c->P, PXc(c), c->d_ewsk + ek0, 1);
+    hipLaunchKernelGGL(k_ewald_sk, dim3(ekn), dim3(kTile * kWaves), 0, c->stream, c->P, PXc(c), c->d_ewsk + ek0);
   // every live system (in live-list order) or one; the output is by system
   // index, zeros for retired systems
   const int nsel = isys < 0 ? c->nlive : 1, pos0 = isys < 0 ? 0 : c->hs[isys].live_pos;
@@ -1829,7 +1825,7 @@ int32_t tis_energy_sumup_set(tis_ctx *c, int32_t n, const int32_t *isys, double 
     const HostSys &h = c->hs[isys[k]];
     if (h.esk_count > 0)
       hipLaunchKernelGGL(k_ewald_sk, dim3(h.esk_count), dim3(kTile * kWaves), 0, c->stream, c->P, PXc(c),
-                         c->d_ewsk + h.esk_begin, 1);
+                         c->d_ewsk + h.esk_begin);
   }
   // the live position of each entry, then the tasks of the systems listed
   // (each system's once, however often it is listed)

@@ -195,7 +195,7 @@ struct DevPtrs {
   const SpPair *sptab;
   BBox *bbox, *qbbox;          // per bead tile / per charge tile
   BBox *sbox;                  // per 16-bead group of each bead tile [4 * nbtile]
-  int *lcnt;                   // exv entry counts per (bead tile pair, lane) of the tile-pair build
+  uint64_t *lmask;             // per (bead tile pair, lane) of a periodic list build: the listed beads
   const double *exv_rad;
   const float *exv_eps;
   const double *charge;

@@ -1059,7 +1059,90 @@ __device__ inline void ele_pair_periodic(const DevPtrs &P, const DSys &s, const 
   }
 }
 
-// The force pass, one launch with five kinds of blocks: 256 hbond lanes per
+// ------------------------------------------------------------------ Ewald reciprocal space
+// force_ele_coulomb_ewld.F90:62-84.  The phase k.r = 2 pi (h . r/L) is
+// formed in FP64 from fractional coordinates and reduced to (-1/2, 1/2]
+// turns before the FP32 sincospi, so its rounding does not grow with |h| or
+// the box; structure factors and forces accumulate in FP64.
+//
+// The vectors are one of each pair h, -h, with twice the coefficient: the
+// phase of -h is the negative, exactly, so the other half would repeat the
+// same cosines and opposite sines.
+//
+// Pass 1: partial structure factors.  One lane per reciprocal vector of a
+// 64-vector tile, over one 64-charge chunk staged in LDS (broadcast reads),
+// a quarter of the chunk per wave, the quarters added as (q0 + q1) + (q2 +
+// q3): bound by the sines' arithmetic, which a wave per tile and chunk left
+// to a few waves and their latency.  |h| <= 10, 640 charges: 10.5 us for all
+// vectors with a wave per tile and chunk, 5.4 now.
+// EXACT (energy evaluation) takes sin/cos in FP64.
+struct EwLds {
+  double fx[kTile], fy[kTile], fz[kTile], fq[kTile];
+  double red[kWaves - 1][2][kTile];
+};
+template <bool EXACT>
+__device__ inline void ewald_sk_block(const DevPtrs &P, const double *PX, const EwTask &tk, EwLds &L) {
+  auto &fx = L.fx; auto &fy = L.fy; auto &fz = L.fz; auto &fq = L.fq; auto &red = L.red;
+  const DSys s = P.sys[tk.sys];
+  const int lane = threadIdx.x & (kTile - 1), w = threadIdx.x / kTile, n = P.ntot;
+  const int k = tk.a * kTile + lane;
+  const int kg = s.ewk0 + min(k, s.nk - 1);
+  const double hx = P.ewh[kg], hy = P.ewh[P.nktot + kg], hz = P.ewh[2 * P.nktot + kg];
+  if (w == 0) {
+    const int qi = tk.b * kTile + lane;
+    if (qi < s.nq) {
+      const int g = P.qbead[s.qoff + qi];
+      fx[lane] = PX[g] * s.ew_invL; fy[lane] = PX[n + g] * s.ew_invL; fz[lane] = PX[2 * n + g] * s.ew_invL;
+      fq[lane] = P.charge[g];
+    } else {
+      fx[lane] = fy[lane] = fz[lane] = 0.0; fq[lane] = 0.0;
+    }
+  }
+  __syncthreads();
+  constexpr int kPart = kTile / kWaves;
+  const int j0 = w * kPart, j1 = min(j0 + kPart, s.nq - tk.b * kTile);
+  double sc = 0.0, ss = 0.0;
+  if (EXACT) {
+    for (int j = j0; j < j1; ++j) {
+      double t = hx * fx[j] + hy * fy[j] + hz * fz[j];
+      t -= rint(t);
+      double sn, cs;
+      sincospi(2.0 * t, &sn, &cs);
+      sc += fq[j] * cs;
+      ss += fq[j] * sn;
+    }
+  } else {
+#pragma unroll 4
+    for (int j = j0; j < j1; ++j) {
+      double t = hx * fx[j] + hy * fy[j] + hz * fz[j];
+      t -= rint(t);
+      float sn, cs;
+      sincospif((float)(2.0 * t), &sn, &cs);
+      sc += fq[j] * (double)cs;
+      ss += fq[j] * (double)sn;
+    }
+  }
+  if (w > 0) {
+    red[w - 1][0][lane] = sc;
+    red[w - 1][1][lane] = ss;
+  }
+  __syncthreads();
+  if (w > 0 || k >= s.nk) return;
+  double *o = P.psk + s.psk_off + 2 * ((int64_t)tk.b * s.nk + k);
+  o[0] = (sc + red[0][0][lane]) + (red[1][0][lane] + red[2][0][lane]);
+  o[1] = (ss + red[0][1][lane]) + (red[1][1][lane] + red[2][1][lane]);
+}
+
+// for the energies: sines in FP64 (the force pass runs its own in k_force)
+__global__ __launch_bounds__(kTile * kWaves) void k_ewald_sk(DevPtrs P, const double *PX, const EwTask *tasks) {
+  __shared__ EwLds lds;
+  if (run_stopped(P)) return;
+  ewald_sk_block<true>(P, PX, tasks[blockIdx.x], lds);
+}
+
+// The force pass, one launch with six kinds of blocks: a tile of reciprocal
+// vectors over a charge chunk per block (ewald_sk_block, which only the second
+// reciprocal pass reads: a launch of its own took 5.4 us), 256 hbond lanes per
 // block (hbond_lane: the hbonds of systems without valence-limited sites, one
 // lane each, first because each lane is a long FP64 chain), four systems'
 // tertiary stacks and valence-limited hbonds per block (terms_wave, one wave
@@ -1070,11 +1153,18 @@ __device__ inline void ele_pair_periodic(const DevPtrs &P, const DSys &s, const 
 template <int PPW, int TPL>
 __global__ __launch_bounds__(kTile * kWaves) __attribute__((amdgpu_waves_per_eu(4)))
 void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systask, int ntask,
-             const EwTask *ptasks, int npt, const EwTask *xtasks, int nxt, BondedRange br, int32_t t_local) {
+             const EwTask *ptasks, int npt, const EwTask *xtasks, int nxt, const EwTask *ktasks, int nkt,
+             BondedRange br, int32_t t_local) {
   constexpr int ppw = PPW, tpl = TPL;
   __shared__ EleLds lds;
   if (run_stopped(P)) return;
   int b = (int)blockIdx.x;
+  if (b < nkt) {
+    static_assert(sizeof(EwLds) <= sizeof(EleLds), "the reciprocal pass works in the pair pass's LDS");
+    ewald_sk_block<false>(P, PX, ktasks[b], reinterpret_cast<EwLds &>(lds));
+    return;
+  }
+  b -= nkt;
   const int nhdb = (br.nhd + kTile * kWaves - 1) / (kTile * kWaves);   // blocks of 256 hbond lanes
   const int npb = (npt + kWaves * ppw - 1) / (kWaves * ppw);   // blocks of 4 ppw chunk pairs
   const int ntb = (ntask + kWaves - 1) / kWaves;   // blocks of four system terms passes
@@ -1108,7 +1198,7 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
   b -= nxt;
   if (b >= npb) {
     // tpl bonded terms per lane, a grid-wide stride apart
-    const int nbb = (int)gridDim.x - nhdb - ntb - nxt - npb;
+    const int nbb = (int)gridDim.x - nkt - nhdb - ntb - nxt - npb;
     for (int i = 0; i < tpl; ++i)
       bonded_lane(P, X, PX, br, (b - npb + i * nbb) * (kTile * kWaves) + (int)threadIdx.x);
     return;
@@ -1141,88 +1231,16 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
 }
 
 template __global__ void k_force<1, 1>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, BondedRange, int32_t);
+                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
 template __global__ void k_force<2, 1>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, BondedRange, int32_t);
+                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
 template __global__ void k_force<1, 2>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, BondedRange, int32_t);
+                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
 template __global__ void k_force<2, 2>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, BondedRange, int32_t);
+                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
 
-// ------------------------------------------------------------------ Ewald reciprocal space
-// force_ele_coulomb_ewld.F90:62-84.  The phase k.r = 2 pi (h . r/L) is
-// formed in FP64 from fractional coordinates and reduced to (-1/2, 1/2]
-// turns before the FP32 sincospi, so its rounding does not grow with |h| or
-// the box; structure factors and forces accumulate in FP64.
-//
-// The vectors are one of each pair h, -h, with twice the coefficient: the
-// phase of -h is the negative, exactly, so the other half would repeat the
-// same cosines and opposite sines.
-//
-// Pass 1: partial structure factors.  One lane per reciprocal vector of a
-// 64-vector tile, over one 64-charge chunk staged in LDS (broadcast reads),
-// a quarter of the chunk per wave, the quarters added as (q0 + q1) + (q2 +
-// q3): bound by the sines' arithmetic, which a wave per tile and chunk left
-// to a few waves and their latency.  |h| <= 10, 640 charges: 10.5 us for all
-// vectors with a wave per tile and chunk, 5.4 now.
-// exact = 1 (energy evaluation) takes sin/cos in FP64.
-__global__ __launch_bounds__(kTile * kWaves) void k_ewald_sk(DevPtrs P, const double *PX, const EwTask *tasks,
-                                                             int exact) {
-  __shared__ double fx[kTile], fy[kTile], fz[kTile], fq[kTile];
-  __shared__ double red[kWaves - 1][2][kTile];
-  if (run_stopped(P)) return;
-  const EwTask tk = tasks[blockIdx.x];
-  const DSys s = P.sys[tk.sys];
-  const int lane = threadIdx.x & (kTile - 1), w = threadIdx.x / kTile, n = P.ntot;
-  const int k = tk.a * kTile + lane;
-  const int kg = s.ewk0 + min(k, s.nk - 1);
-  const double hx = P.ewh[kg], hy = P.ewh[P.nktot + kg], hz = P.ewh[2 * P.nktot + kg];
-  if (w == 0) {
-    const int qi = tk.b * kTile + lane;
-    if (qi < s.nq) {
-      const int g = P.qbead[s.qoff + qi];
-      fx[lane] = PX[g] * s.ew_invL; fy[lane] = PX[n + g] * s.ew_invL; fz[lane] = PX[2 * n + g] * s.ew_invL;
-      fq[lane] = P.charge[g];
-    } else {
-      fx[lane] = fy[lane] = fz[lane] = 0.0; fq[lane] = 0.0;
-    }
-  }
-  __syncthreads();
-  constexpr int kPart = kTile / kWaves;
-  const int j0 = w * kPart, j1 = min(j0 + kPart, s.nq - tk.b * kTile);
-  double sc = 0.0, ss = 0.0;
-  if (exact) {
-    for (int j = j0; j < j1; ++j) {
-      double t = hx * fx[j] + hy * fy[j] + hz * fz[j];
-      t -= rint(t);
-      double sn, cs;
-      sincospi(2.0 * t, &sn, &cs);
-      sc += fq[j] * cs;
-      ss += fq[j] * sn;
-    }
-  } else {
-#pragma unroll 4
-    for (int j = j0; j < j1; ++j) {
-      double t = hx * fx[j] + hy * fy[j] + hz * fz[j];
-      t -= rint(t);
-      float sn, cs;
-      sincospif((float)(2.0 * t), &sn, &cs);
-      sc += fq[j] * (double)cs;
-      ss += fq[j] * (double)sn;
-    }
-  }
-  if (w > 0) {
-    red[w - 1][0][lane] = sc;
-    red[w - 1][1][lane] = ss;
-  }
-  __syncthreads();
-  if (w > 0 || k >= s.nk) return;
-  double *o = P.psk + s.psk_off + 2 * ((int64_t)tk.b * s.nk + k);
-  o[0] = (sc + red[0][0][lane]) + (red[1][0][lane] + red[2][0][lane]);
-  o[1] = (ss + red[0][1][lane]) + (red[1][1][lane] + red[2][1][lane]);
-}
-
-// Pass 2: forces.  A block takes a 64-charge tile and a chunk of kEwKChunk
+// ------------------------------------------------------------------ Ewald reciprocal space, pass 2
+// Forces.  A block takes a 64-charge tile and a chunk of kEwKChunk
 // reciprocal vectors: it first sums the partial structure factors of its
 // vectors into LDS (even charge chunks, odd ones, then both), then each wave
 // sweeps an eighth of them for its lane's charge; partial forces per chunk go
@@ -2040,194 +2058,168 @@ __device__ inline void list_hb_entry(const DevPtrs &P, const DSys &s, const doub
 }
 
 // ------------------------------------------------------------------ lists by tile pairs
-// Periodic systems (no box culling, so one wave per tile would sweep every
-// tile of the box in turn): every (bead tile, bead tile) and (charge tile,
-// charge tile) pair is its own wave.  The excluded-volume lists take two passes: pass 0 counts each
-// bead's entries per tile pair, pass 1 writes them after the counts of the
-// earlier tile pairs of its row, so each list keeps the tile order of
-// list_exv_tile.  mode bit 1 takes only the systems whose trigger fired,
-// bit 2 only the periodic systems.
-
 __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// exv entries of bead tile ia (local index) against bead tile jb: counts
-// them (write = false) or writes them from slot `off` on; returns the count
+// The exv and electrostatic lists of periodic systems by pairs of tiles, which
+// one wave per tile (k_lists) would walk one after the other.  Pass 1, a block
+// per pair: each wave tests a quarter of tile b's beads (or charges) against
+// tile a's, a bit per listed one; the bits of a bead pair go to lmask, those
+// of a charge pair are the list rows themselves, with the mirror codes beside
+// them.  Pass 2 (k_lpair_put), a wave per bead pair: the entries of the set
+// bits from the slot that the bits of the tiles before give, so the order is
+// ascending whatever the split.  Bound by the latency of the tests: 793 beads
+// and 640 charges took 98 us with one wave per pair, 64 tests in a row, twice
+// (the entries counted first), 23.8 us now.
+struct PairLds {
+  double sx[kTile], sy[kTile], sz[kTile];
+  int su[kTile], stc[kTile];
+  double rl2[kRl2Lds * kRl2Lds];
+  uint32_t bits[kWaves][kTile];
+};
+
+// beads j0 .. j1 - 1 of the staged tile at jt listed for this lane's bead, bit
+// 0: j0
 template <bool RL2_LDS>
-__device__ inline int exv_pair_scan_t(const DevPtrs &P, const DSys &s, const double *X, const double *PX, int ia,
-                                      int jb, bool write, int off, ListLds &L) {
-  const int lane = threadIdx.x & (kTile - 1);
-  const int li = ia * kTile + lane;
-  const bool valid = li < s.nmp;
-  const int n = P.ntot;
-  const double *Y = s.periodic ? PX : X;
-  const int g = s.off + (valid ? li : 0);
-  const double cut2 = s.rl2max * (1.0 + 1e-9);
-  if (!s.periodic && box_dmin2(P.bbox[s.bt0 + ia], P.bbox[s.bt0 + jb]) > cut2) return 0;
-  if (RL2_LDS)
-    for (int k = lane; k < s.nunit * s.nunit; k += kTile) L.rl2[k] = P.rl2[s.uoff + k];
-  double xi[3] = {0, 0, 0};
-  int ui = 0, ti = 0, ci = 0;
-  if (valid) { ld3(Y, n, g, xi); ui = P.unit[g]; ti = P.mptype[g]; ci = P.iclass[g]; }
-  const int jt = jb * kTile;
-  const int lj = jt + lane;
-  if (lj < s.nmp) {
-    const int gj = s.off + lj;
-    L.sx[lane] = Y[gj]; L.sy[lane] = Y[n + gj]; L.sz[lane] = Y[2 * n + gj];
-    L.su[lane] = P.unit[gj];
-    L.stc[lane] = (int)P.mptype[gj] | ((int)P.iclass[gj] << 8);
+__device__ inline uint32_t exv_pair_bits(const DevPtrs &P, const DSys &s, int li, const double xi[3], int ui, int ti,
+                                         int ci, int jt, int j0, int j1, const PairLds &L) {
+  uint32_t bits = 0u;
+  for (int k = j0; k < j1; ++k) {
+    const int lj2 = jt + k;
+    const bool own_lo = li < lj2;
+    double v[3];
+    pair_vec(s, L.sx[k], L.sy[k], L.sz[k], xi, own_lo, v);
+    pbneighbor(s, v);
+    const double d2 = sq3_exact(v[0], v[1], v[2]);
+    if (lj2 == li || !(d2 < s.rl2max)) continue;
+    const int uj = L.su[k];
+    const int ulo = own_lo ? ui : uj, uhi = own_lo ? uj : ui;
+    const double r2 = RL2_LDS ? L.rl2[ulo * s.nunit + uhi] : P.rl2[s.uoff + ulo * s.nunit + uhi];
+    if (!(d2 < r2)) continue;
+    const int tj = L.stc[k] & 0xFF, cj = L.stc[k] >> 8;
+    const bool keep = own_lo ? exv_keep(s, ui, uj, ci, ti, li, lj2) : exv_keep(s, uj, ui, cj, tj, lj2, li);
+    if (keep) bits |= 1u << (k - j0);
   }
-  wave_lds_sync();
-  int cnt = 0;
-  const int kend = min(kTile, s.nmp - jt);
-  for (int q0 = 0; q0 < kend; q0 += 16) {
-    if (!s.periodic) {
-      const bool need = valid && point_box_d2(xi, P.sbox[4 * (s.bt0 + jb) + q0 / 16]) <= cut2;
-      if (!__any(need)) continue;
-    }
-    const int q1 = min(q0 + 16, kend);
-    if (valid)
-      for (int k = q0; k < q1; ++k) {
-        const int lj2 = jt + k;
-        if (lj2 == li) continue;
-        const bool own_lo = li < lj2;
-        double v[3];
-        pair_vec(s, L.sx[k], L.sy[k], L.sz[k], xi, own_lo, v);
-        const int code = s.periodic ? pbneighbor(s, v) : 0;
-        const double d2 = sq3_exact(v[0], v[1], v[2]);
-        if (!(d2 < s.rl2max)) continue;
-        const int uj = L.su[k];
-        const int ulo = own_lo ? ui : uj, uhi = own_lo ? uj : ui;
-        const double r2 = RL2_LDS ? L.rl2[ulo * s.nunit + uhi] : P.rl2[s.uoff + ulo * s.nunit + uhi];
-        if (!(d2 < r2)) continue;
-        const int tj = L.stc[k] & 0xFF, cj = L.stc[k] >> 8;
-        const bool keep = own_lo ? exv_keep(s, ui, uj, ci, ti, li, lj2) : exv_keep(s, uj, ui, cj, tj, lj2, li);
-        if (!keep) continue;
-        if (write) {
-          const int slot = off + cnt;
-          const int oc = own_lo ? code : mirror_flip(code);
-          if (slot < P.nb_cap) P.nb[(size_t)slot * n + g] = ((uint32_t)oc << kMirrorShift) | (uint32_t)(s.off + lj2);
-        }
-        ++cnt;
-      }
-  }
-  wave_lds_sync();
-  return cnt;
+  return bits;
 }
 
-__device__ inline int exv_pair_scan(const DevPtrs &P, const DSys &s, const double *X, const double *PX, int ia,
-                                    int jb, bool write, int off, ListLds &L) {
-  return s.nunit <= kRl2Lds ? exv_pair_scan_t<true>(P, s, X, PX, ia, jb, write, off, L)
-                            : exv_pair_scan_t<false>(P, s, X, PX, ia, jb, write, off, L);
-}
-
-// ele bit words of charge tile I's rows for charge tile J (and, periodic,
-// the mirror codes), as list_ele_tile does for one J
-__device__ inline void ele_pair_rows(const DevPtrs &P, const DSys &s, const double *X, const double *PX, int I, int J,
-                                     ListLds &L) {
-  const int lane = threadIdx.x & (kTile - 1);
-  const int qi = I * kTile + lane;
-  const bool valid = qi < s.nq;
-  const int n = P.ntot;
-  const double *Y = s.periodic ? PX : X;
-  double xi[3] = {0, 0, 0};
-  if (valid) ld3(Y, n, P.qbead[s.qoff + qi], xi);
-  uint32_t *row = P.qmask + s.moff + (int64_t)(valid ? qi : 0) * s.mwords;
-  const int jt = J * kTile;
-  const int kend = min(kTile, s.nq - jt);
-  int mode = 2;  // 0 none, 1 all, 2 test
-  if (!s.periodic) {
-    const BBox bi = P.qbbox[s.qt0 + I], bj = P.qbbox[s.qt0 + J];
-    if (box_dmin2(bi, bj) > s.ele_rl2 * (1.0 + 1e-9)) mode = 0;
-    else if (box_dmax2(bi, bj) < s.ele_rl2 * (1.0 - 1e-9)) mode = 1;
-  }
-  uint32_t w[2] = {0u, 0u};
-  if (mode == 1) {
-    w[0] = kend >= 32 ? 0xFFFFFFFFu : ((1u << kend) - 1u);
-    w[1] = kend >= 64 ? 0xFFFFFFFFu : (kend > 32 ? ((1u << (kend - 32)) - 1u) : 0u);
-    if (qi >= jt && qi < jt + kend) w[(qi - jt) >> 5] &= ~(1u << ((qi - jt) & 31));
-  } else if (mode == 2) {
-    const int qj = jt + lane;
-    if (qj < s.nq) {
-      const int gj = P.qbead[s.qoff + qj];
-      L.sx[lane] = Y[gj]; L.sy[lane] = Y[n + gj]; L.sz[lane] = Y[2 * n + gj];
-    }
-    wave_lds_sync();
-    if (valid)
-      for (int k = 0; k < kend; ++k) {
-        const int qj2 = jt + k;
-        if (qj2 == qi) continue;
-        const bool own_lo = qi < qj2;
-        double v[3];
-        pair_vec(s, L.sx[k], L.sy[k], L.sz[k], xi, own_lo, v);
-        const int code = s.periodic ? pbneighbor(s, v) : 0;
-        const double d2 = sq3_exact(v[0], v[1], v[2]);
-        if (!(d2 < s.ele_rl2)) continue;
-        w[k >> 5] |= 1u << (k & 31);
-        if (s.periodic) P.qmirror[s.mioff + (int64_t)qi * s.nq + qj2] = (uint8_t)(own_lo ? code : mirror_flip(code));
-      }
-    wave_lds_sync();
-  }
-  if (valid) {
-    row[jt >> 5] = w[0];
-    if ((jt >> 5) + 1 < s.mwords) row[(jt >> 5) + 1] = w[1];
-  }
-}
-
-__device__ inline bool lpair_take(const DevPtrs &P, int sys, int mode) {
-  return (!(mode & 1) || P.sys_flag[sys] != 0) && (!(mode & 2) || P.sys[sys].periodic != 0);
-}
-
-// pass 0: exv counts of bead tile pairs, ele rows of charge tile pairs and
-// hbond candidates (nh > 0); pass 1: exv entries.  One pair per wave.
-__global__ __launch_bounds__(kTile * kWaves) void k_lpair(DevPtrs P, const double *X, const double *PX,
-                                                          const EwTask *bpairs, int nbp, const EwTask *qpairs,
-                                                          int nqp, int h0, int nh, int mode, int pass) {
-  __shared__ ListLds lds[kWaves];
+// gate: only the systems whose displacement trigger fires (sys_flag)
+__global__ __launch_bounds__(kTile * kWaves) void k_lpair(DevPtrs P, const double *PX, const EwTask *bpairs, int nbp,
+                                                          const EwTask *qpairs, int gate) {
+  __shared__ PairLds L;
   if (run_stopped(P)) return;
-  const int w = (int)threadIdx.x / kTile, lane = (int)threadIdx.x & (kTile - 1);
-  const int nbb = (nbp + kWaves - 1) / kWaves, nqb = (nqp + kWaves - 1) / kWaves;
+  constexpr int kPart = kTile / kWaves;
+  const int tid = (int)threadIdx.x, w = tid / kTile, lane = tid & (kTile - 1), n = P.ntot;
   const int b = (int)blockIdx.x;
-  if (b < nbb) {
-    const int p = b * kWaves + w;
-    if (p >= nbp) return;
-    const EwTask bp = bpairs[p];
-    if (!lpair_take(P, bp.sys, mode)) return;
-    const DSys s = P.sys[bp.sys];
-    int *cnt = P.lcnt + (size_t)(s.lp_off + bp.a * s.nbt) * kTile;   // counts of this row of tile pairs
-    if (pass == 0) {
-      cnt[bp.b * kTile + lane] = exv_pair_scan(P, s, X, PX, bp.a, bp.b, false, 0, lds[w]);
-      return;
+  const EwTask tp = b < nbp ? bpairs[b] : qpairs[b - nbp];
+  if (gate && P.sys_flag[tp.sys] == 0) return;
+  const DSys s = P.sys[tp.sys];
+  const int jt = tp.b * kTile;
+  double xi[3] = {0, 0, 0};
+  if (b < nbp) {
+    const int li = tp.a * kTile + lane, g = s.off + li, kend = min(kTile, s.nmp - jt);
+    const bool valid = li < s.nmp;
+    const bool rl2_lds = s.nunit <= kRl2Lds;
+    if (rl2_lds)
+      for (int k = tid; k < s.nunit * s.nunit; k += kTile * kWaves) L.rl2[k] = P.rl2[s.uoff + k];
+    if (w == 0 && lane < kend) {
+      const int gj = s.off + jt + lane;
+      L.sx[lane] = PX[gj]; L.sy[lane] = PX[n + gj]; L.sz[lane] = PX[2 * n + gj];
+      L.su[lane] = P.unit[gj];
+      L.stc[lane] = (int)P.mptype[gj] | ((int)P.iclass[gj] << 8);
     }
-    int off = 0;
-    for (int j = 0; j < bp.b; ++j) off += cnt[j * kTile + lane];
-    const int c = exv_pair_scan(P, s, X, PX, bp.a, bp.b, true, off, lds[w]);
-    const int li = bp.a * kTile + lane;
-    if (bp.b == s.nbt - 1 && li < s.nmp) {
-      const int tot = off + c, g = s.off + li;
-      P.nb_cnt[g] = tot;
-      if (tot > P.nb_cap) atomicMax(&P.counters[5], (unsigned long long)tot);
+    int ui = 0, ti = 0, ci = 0;
+    if (valid) { ld3(PX, n, g, xi); ui = P.unit[g]; ti = P.mptype[g]; ci = P.iclass[g]; }
+    __syncthreads();
+    const int j0 = w * kPart, j1 = min(j0 + kPart, kend);
+    uint32_t bits = 0u;
+    if (valid)
+      bits = rl2_lds ? exv_pair_bits<true>(P, s, li, xi, ui, ti, ci, jt, j0, j1, L)
+                     : exv_pair_bits<false>(P, s, li, xi, ui, ti, ci, jt, j0, j1, L);
+    L.bits[w][lane] = bits;
+    __syncthreads();
+    if (w == 0) {
+      static_assert(kWaves == 4, "four quarters of 16 bits");
+      const uint32_t lo = L.bits[0][lane] | (L.bits[1][lane] << 16), hi = L.bits[2][lane] | (L.bits[3][lane] << 16);
+      P.lmask[(size_t)(s.lp_off + (int64_t)tp.a * s.nbt + tp.b) * kTile + lane] = (uint64_t)lo | ((uint64_t)hi << 32);
     }
     return;
   }
-  if (pass == 1) return;
-  if (b < nbb + nqb) {
-    const int p = (b - nbb) * kWaves + w;
-    if (p >= nqp) return;
-    const EwTask qp = qpairs[p];
-    if (!lpair_take(P, qp.sys, mode)) return;
-    const DSys s = P.sys[qp.sys];
-    ele_pair_rows(P, s, X, PX, qp.a, qp.b, lds[w]);
-    return;
+  // charge pair: the bit words of tile a's rows for tile b
+  const int qi = tp.a * kTile + lane, kend = min(kTile, s.nq - jt);
+  const bool valid = qi < s.nq;
+  if (valid) ld3(PX, n, P.qbead[s.qoff + qi], xi);
+  if (w == 0 && lane < kend) {
+    const int gj = P.qbead[s.qoff + jt + lane];
+    L.sx[lane] = PX[gj]; L.sy[lane] = PX[n + gj]; L.sz[lane] = PX[2 * n + gj];
   }
-  const int k = (b - nbb - nqb) * (kTile * kWaves) + (int)threadIdx.x;
-  if (k >= nh) return;
-  const int h = h0 + k;
-  if (!lpair_take(P, P.hb_sys[h], mode)) return;
-  list_hb_entry(P, P.sys[P.hb_sys[h]], X, PX, h);
+  __syncthreads();
+  uint32_t bits = 0u;
+  if (valid) {
+    uint8_t *mrow = P.qmirror + s.mioff + (int64_t)qi * s.nq + jt;
+    const int j0 = w * kPart, j1 = min(j0 + kPart, kend);
+    for (int k = j0; k < j1; ++k) {
+      const bool own_lo = qi < jt + k;
+      double v[3];
+      pair_vec(s, L.sx[k], L.sy[k], L.sz[k], xi, own_lo, v);
+      const int code = pbneighbor(s, v);
+      const double d2 = sq3_exact(v[0], v[1], v[2]);
+      if (qi == jt + k || !(d2 < s.ele_rl2)) continue;
+      bits |= 1u << (k - j0);
+      mrow[k] = (uint8_t)(own_lo ? code : mirror_flip(code));
+    }
+  }
+  L.bits[w][lane] = bits;
+  __syncthreads();
+  if (w == 0 && valid) {
+    uint32_t *row = P.qmask + s.moff + (int64_t)qi * s.mwords + (jt >> 5);
+    row[0] = L.bits[0][lane] | (L.bits[1][lane] << 16);
+    if ((jt >> 5) + 1 < s.mwords) row[1] = L.bits[2][lane] | (L.bits[3][lane] << 16);
+  }
+}
+
+__global__ __launch_bounds__(kTile * kWaves) void k_lpair_put(DevPtrs P, const double *PX, const EwTask *bpairs,
+                                                              int nbp, int gate) {
+  __shared__ double sx[kWaves][kTile], sy[kWaves][kTile], sz[kWaves][kTile];
+  if (run_stopped(P)) return;
+  const int w = (int)threadIdx.x / kTile, lane = (int)threadIdx.x & (kTile - 1), n = P.ntot;
+  const int p = (int)blockIdx.x * kWaves + w;
+  if (p >= nbp) return;
+  const EwTask bp = bpairs[p];
+  if (gate && P.sys_flag[bp.sys] == 0) return;
+  const DSys s = P.sys[bp.sys];
+  const int li = bp.a * kTile + lane, g = s.off + li, jt = bp.b * kTile;
+  const uint64_t *row = P.lmask + (size_t)(s.lp_off + (int64_t)bp.a * s.nbt) * kTile + lane;
+  uint64_t mask = row[(size_t)bp.b * kTile];   // 0 in lanes past the system's beads
+  int off = 0;
+#pragma unroll 8
+  for (int j = 0; j < bp.b; ++j) off += __popcll(row[(size_t)j * kTile]);
+  if (bp.b == s.nbt - 1 && li < s.nmp) {
+    const int tot = off + __popcll(mask);
+    P.nb_cnt[g] = tot;
+    if (tot > P.nb_cap) atomicMax(&P.counters[5], (unsigned long long)tot);
+  }
+  if (!__any(mask != 0)) return;
+  if (jt + lane < s.nmp) {
+    const int gj = s.off + jt + lane;
+    sx[w][lane] = PX[gj]; sy[w][lane] = PX[n + gj]; sz[w][lane] = PX[2 * n + gj];
+  }
+  double xi[3] = {0, 0, 0};
+  if (mask) ld3(PX, n, g, xi);
+  wave_lds_sync();
+  for (; mask; mask &= mask - 1, ++off) {
+    const int k = __builtin_ctzll(mask);
+    const bool own_lo = li < jt + k;
+    double v[3];
+    pair_vec(s, sx[w][k], sy[w][k], sz[w][k], xi, own_lo, v);
+    const int code = pbneighbor(s, v);
+    if (off < P.nb_cap)
+      P.nb[(size_t)off * n + g] =
+          ((uint32_t)(own_lo ? code : mirror_flip(code)) << kMirrorShift) | (uint32_t)(s.off + jt + k);
+  }
 }
 
 // The list passes of one rebuild in two launches.  gate = 0 builds for every
