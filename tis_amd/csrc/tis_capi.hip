@@ -20,7 +20,7 @@
 #include "tis_internal.h"
 
 namespace tis {
-template <int PPW, int TPL>
+template <int PPW, int TPL, int WPE>
 __global__ void k_force(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *, int,
                         const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
 __global__ void k_ewald_sk(DevPtrs, const double *, const EwTask *);
@@ -1661,6 +1661,11 @@ int32_t tis_pairs_get(tis_ctx *c, int32_t isys, int32_t which, int32_t *pairs, d
 // instead of two: 5.9 against 8.1 us at 160 tiles, 7.3 against 9.2 at 320, even
 // at 640 (10.8), 17.5 against 13.6 at 1,280.
 constexpr int kMainWideTiles = 512;
+// Launches of k_force with at most this many blocks of four waves have two
+// waves per SIMD at most anyway and take the kernel with the registers of two
+// (no spills): 10.6 against 11.4 us for the chunk pairs, hbonds and bonds of one
+// large system, 10.4 against 10.8 for an Ewald box.
+constexpr int kForceFewBlocks = 512;
 
 // k_force (structure factors, terms, electrostatic chunk pairs, bonded terms),
 // the second Ewald pass, then k_main, at the positions in buffer ix (the next ones go to the
@@ -1703,7 +1708,8 @@ static void launch_force_pair(tis_ctx *c, const Range &r, int ix, int t_local, i
     const EwTask *pt = r.all ? (c->shape.lpt ? c->d_ptask_lpt : c->d_ptask) : c->d_ptask + r.pt0;
     const EwTask *xt = c->d_xtask + r.xt0, *kt = c->d_ewsk + r.ek0;
     // one kernel per launch shape (each with its own register allocation)
-    auto kf = ppw == 1 ? (tpl == 1 ? k_force<1, 1> : k_force<1, 2>) : (tpl == 1 ? k_force<2, 1> : k_force<2, 2>);
+    auto kf = ppw == 1 ? (tpl == 1 ? (nblk <= kForceFewBlocks ? k_force<1, 1, 2> : k_force<1, 1, 4>) : k_force<1, 2, 4>)
+                       : (tpl == 1 ? k_force<2, 1, 4> : k_force<2, 2, 4>);
     if (c->timing)
       hipExtLaunchKernelGGL(kf, dim3(nblk), dim3(kTile * kWaves), 0, c->stream, e3[1], e3[2], 0, c->P, X, PX,
                             task, r.taskn, pt, npt, xt, nxt, kt, r.ekn, br, pre_t);

@@ -1150,8 +1150,8 @@ __global__ __launch_bounds__(kTile * kWaves) void k_ewald_sk(DevPtrs P, const do
 // (ele_pair_periodic), four of others per block (ele_pair_unrolled,
 // ele_pair_task, one wave each), then the bonded terms, 256 lanes per block (bonded_lane).  k_main
 // gathers all of their outputs.
-template <int PPW, int TPL>
-__global__ __launch_bounds__(kTile * kWaves) __attribute__((amdgpu_waves_per_eu(4)))
+template <int PPW, int TPL, int WPE>
+__global__ __launch_bounds__(kTile * kWaves) __attribute__((amdgpu_waves_per_eu(WPE)))
 void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systask, int ntask,
              const EwTask *ptasks, int npt, const EwTask *xtasks, int nxt, const EwTask *ktasks, int nkt,
              BondedRange br, int32_t t_local) {
@@ -1230,14 +1230,16 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
   }
 }
 
-template __global__ void k_force<1, 1>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
-template __global__ void k_force<2, 1>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
-template __global__ void k_force<1, 2>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
-template __global__ void k_force<2, 2>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
-                                       int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
+template __global__ void k_force<1, 1, 4>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
+                                          int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
+template __global__ void k_force<2, 1, 4>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
+                                          int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
+template __global__ void k_force<1, 2, 4>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
+                                          int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
+template __global__ void k_force<2, 2, 4>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
+                                          int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
+template __global__ void k_force<1, 1, 2>(DevPtrs, const double *, const double *, const int32_t *, int, const EwTask *,
+                                          int, const EwTask *, int, const EwTask *, int, BondedRange, int32_t);
 
 // ------------------------------------------------------------------ Ewald reciprocal space, pass 2
 // Forces.  A block takes a 64-charge tile and a chunk of kEwKChunk
