@@ -10,17 +10,29 @@ import pytest
 
 import oracle
 import test_dpp_hazards as hz
+from test_zz_no_alloc import D2H, H2D, _hip
 from tis_amd.bdhi import bead_spring_chain
 from tis_amd.engine import BDEngine, load_library
 
 
-def _factor(D, L):
+def _factor(a):
+    """(return code, failing pivot + 1, factor) of the symmetric matrix a."""
+    hip, n, nbytes = _hip(), len(a), a.nbytes
     fn = load_library().tis_bdhi_factor_noalloc
     fn.restype = ctypes.c_int32
     fn.argtypes = [ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p]
-    info = ctypes.c_int32(-1)
-    rc = fn(0, D.data_ptr(), L.data_ptr(), len(D), None, ctypes.byref(info))
-    return rc, info.value
+    D, L, info = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_int32(-1)
+    assert hip.hipMalloc(ctypes.byref(D), nbytes) == 0 and hip.hipMalloc(ctypes.byref(L), nbytes) == 0
+    try:
+        assert hip.hipMemcpy(D, a.ctypes.data, nbytes, H2D) == 0
+        rc = fn(0, D, L, n, None, ctypes.byref(info))
+        assert hip.hipDeviceSynchronize() == 0
+        out = np.zeros((n, n), order="F")
+        assert hip.hipMemcpy(out.ctypes.data, L, nbytes, D2H) == 0
+    finally:
+        hip.hipFree(D)
+        hip.hipFree(L)
+    return rc, info.value, out
 
 
 def _spd(n):
@@ -31,15 +43,12 @@ def _spd(n):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 80, 127, 128, 129, 191, 192, 193, 255, 256, 257, 320, 511, 577])
 def test_factor_sizes(n):
-    import torch
     a = _spd(n)
     print(f"[factor] n={n}", flush=True)
-    D = torch.from_numpy(a).cuda()
-    L = torch.empty_like(D)
-    rc, info = _factor(D, L)
+    rc, info, L = _factor(a)
     assert rc == 0 and info == 0
     l64 = np.linalg.cholesky(a)
-    err = np.abs(L.T.cpu().numpy() - l64).max() / np.abs(l64).max()
+    err = np.abs(L - l64).max() / np.abs(l64).max()
     # one panel is FP64 throughout; further ones take products in FP32
     assert err <= (1e-13 if n <= 64 else 2e-5)
 
@@ -47,12 +56,10 @@ def test_factor_sizes(n):
 @pytest.mark.gpu
 @pytest.mark.parametrize("p", [0, 15, 16, 47, 63, 64, 100, 129])
 def test_pivot_check(p):
-    import torch
     a = _spd(130)
     a[p, p] = -1.0
     print(f"[pivot] {p}", flush=True)
-    D = torch.from_numpy(a).cuda()
-    rc, info = _factor(D, torch.empty_like(D))
+    rc, info, _ = _factor(a)
     assert rc != 0 and info == p + 1
 
 

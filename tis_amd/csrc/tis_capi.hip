@@ -31,6 +31,7 @@ __global__ void k_main(DevPtrs, const double *, const double *, const float4 *, 
 __global__ void k_near(DevPtrs, const double *, float4 *, int, int);
 __global__ void k_prep(DevPtrs, const double *, double *, double *, float4 *, float4 *, const Tile *, int, int,
                        const Tile *, int, int, int, int);
+template <int W>
 __global__ void k_lists(DevPtrs, const double *, const double *, const Tile *, int, int, const Tile *, int, int, int,
                         int, int);
 __global__ void k_lpair(DevPtrs, const double *, const EwTask *, int, const EwTask *, int);
@@ -541,6 +542,13 @@ static void launch_lpair(tis_ctx *c, const Range &r, const double *PX, int gate)
                        c->d_bpair + bp0, nbp, gate);
 }
 
+// List launches of at most this many tiles take eight waves per tile, larger
+// ones four: 512 chains of 60 to 1,800 beads, rebuilt every ten steps, took 42.0
+// ms with eight waves and 40.1 with four (40.5 with one, 39.9 with two), 128
+// chains under the displacement trigger 9.8 ms with one, 9.4 with two, 9.2 with
+// four.
+constexpr int kListWideBlocks = 1024;
+
 // The lists of the range from the positions in buffer cu (wrapped copies into
 // px[cu], predicted wrapped positions into the other when with_pred): k_prep, then k_lists by
 // bead / charge tile for non-periodic systems and the hbond candidates, and
@@ -551,22 +559,26 @@ int launch_lists(tis_ctx *c, const Range &r, int cu, int with_pred, int gate) {
   double *PXcur = c->P.px[cu], *PXpred = c->P.px[cu ^ 1];
   const int h0 = r.all ? 0 : c->hs[r.isys].d.hoff, nh = r.all ? c->nhbtot : c->hs[r.isys].d.nhb;
   const bool periodic = r.all ? c->any_periodic : c->hs[r.isys].d.periodic != 0;
+  // waves per list block, see kListWideBlocks
+  const bool wide = r.btn + r.qtn <= kListWideBlocks;
+  auto kl = wide ? k_lists<kListWide> : k_lists<kListFew>;
+  const int per = kTile * (wide ? kListWide : kListFew);
   if (gate && !periodic) {
     // displacement-triggered rebuilds of non-periodic systems: k_lists takes
     // the decision and the displacement reset itself and culls by the boxes
     // k_main leaves at the end of each step (gate 2), so k_prep is skipped;
     // each system's bead tiles also rebuild its hbond candidates
     if (r.btn + r.qtn > 0)
-      hipLaunchKernelGGL(k_lists, dim3(r.btn + r.qtn), dim3(kTile), 0, c->stream, c->P, X, PXcur, c->d_btiles, r.bt0,
+      hipLaunchKernelGGL(kl, dim3(r.btn + r.qtn), dim3(per), 0, c->stream, c->P, X, PXcur, c->d_btiles, r.bt0,
                          r.btn, c->d_qtiles, r.qt0, r.qtn, h0, nh, 2);
     return 0;
   }
   if (r.btn + r.qtn > 0)
     hipLaunchKernelGGL(k_prep, dim3(r.btn + r.qtn), dim3(kTile), 0, c->stream, c->P, X, PXcur, PXpred,
                        c->P.xf[cu], c->P.xf[cu ^ 1], c->d_btiles, r.bt0, r.btn, c->d_qtiles, r.qt0, r.qtn, with_pred, gate);
-  const int nblk = r.btn + r.qtn + (nh + kTile - 1) / kTile;
+  const int nblk = r.btn + r.qtn + (nh + per - 1) / per;
   if (nblk > 0)
-    hipLaunchKernelGGL(k_lists, dim3(nblk), dim3(kTile), 0, c->stream, c->P, X, PXcur, c->d_btiles, r.bt0, r.btn,
+    hipLaunchKernelGGL(kl, dim3(nblk), dim3(per), 0, c->stream, c->P, X, PXcur, c->d_btiles, r.bt0, r.btn,
                        c->d_qtiles, r.qt0, r.qtn, h0, nh, gate);
   if (periodic) launch_lpair(c, r, PXcur, gate);
   return 0;

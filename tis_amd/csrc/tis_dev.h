@@ -86,6 +86,7 @@ struct EwTask { int32_t sys, a, b; };
 // constants (time_integral_pre.F90:160-170): r[0] the noise amplitude c1,
 // r[1..3] c2, c3, c4, and 1/m.
 struct LangClass { double r[4], rcm, fric, mass, pad; };
+constexpr int kListWide = 8, kListFew = 4;   // waves of a list block (k_lists)
 constexpr int kEwKChunk = 128;   // reciprocal vectors per block of the force pass
 constexpr int kEwThreads = 512;  // its threads
 

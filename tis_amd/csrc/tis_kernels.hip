@@ -1802,11 +1802,22 @@ __device__ inline double box_dmax2(const BBox &a, const BBox &b) {
 // the reference rounds it.
 constexpr int kRl2Lds = 16;       // unit-pair radius tables up to 16 x 16 units are staged in LDS
 
+__device__ inline void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A list block's waves share the tiles that its own tile may meet out in units
+// of 32 beads (or charges).
+constexpr int kUnit = 32, kUnitsRound = kTile;   // beads of a unit, units per round (one lane's box test each)
+
+template <int W>
 struct ListLds {
-  double sx[kTile], sy[kTile], sz[kTile];
-  int su[kTile], stc[kTile];
-  BBox sb[kTile / 16];                 // boxes of the staged tile's 16-bead groups
+  double sx[W][kUnit], sy[W][kUnit], sz[W][kUnit];
+  int su[W][kUnit], stc[W][kUnit];
   double rl2[kRl2Lds * kRl2Lds];
+  uint32_t bits[kUnitsRound][kTile];   // [unit met][bead]: listed beads of the unit
 };
 
 // The pair vector x_hi - x_lo of the reference's lower-index-first loops
@@ -1849,104 +1860,91 @@ __device__ inline bool exv_listed(const DSys &s, double d2, int li, int ui, int 
   return (lj2 != li) & (d2 < s.rl2max) & (d2 < r2) & keep;
 }
 
-// One wave per bead tile sweeps the system's bead tiles in order; tiles and
-// 16-bead groups whose boxes no bead of the tile can reach within the
-// largest list radius are skipped.  The tile boxes are tested 64 at a time
-// (one lane per tile), the group boxes are staged with the tile, and the
-// unit-pair radii sit in LDS, so neither the culling nor the per-pair tests
-// wait on dependent global loads.
-// One candidate pair of the exv list (neighbor_list.F90 distance test with
-// the unit-pair radius, neighbor_assign.F90 exclusions): this lane's bead
-// li against bead lj2 of the same system (staged coordinates, unit,
-// type | class << 8).  On true, entry = mirror << 27 | global index.
-template <bool RL2_LDS>
-__device__ inline bool exv_candidate(const DevPtrs &P, const DSys &s, const double xi[3], int li, int ui, int ti,
-                                     int ci, int lj2, double xj0, double xj1, double xj2, int uj, int tcj,
-                                     const double *rl2l, uint32_t &entry) {
-  if (lj2 == li) return false;
-  const bool own_lo = li < lj2;
-  double v[3];
-  pair_vec(s, xj0, xj1, xj2, xi, own_lo, v);
-  const int code = s.periodic ? pbneighbor(s, v) : 0;
-  const double d2 = sq3_exact(v[0], v[1], v[2]);
-  if (!(d2 < s.rl2max)) return false;   // rl2max bounds every unit-pair radius
-  const int ulo = own_lo ? ui : uj, uhi = own_lo ? uj : ui;
-  const double r2 = RL2_LDS ? rl2l[ulo * s.nunit + uhi] : P.rl2[s.uoff + ulo * s.nunit + uhi];
-  if (!(d2 < r2)) return false;
-  const int tj = tcj & 0xFF, cj = tcj >> 8;
-  const bool keep = own_lo ? exv_keep(s, ui, uj, ci, ti, li, lj2) : exv_keep(s, uj, ui, cj, tj, lj2, li);
-  if (!keep) return false;
-  const int oc = own_lo ? code : mirror_flip(code);
-  entry = ((uint32_t)oc << kMirrorShift) | (uint32_t)(s.off + lj2);
-  return true;
-}
-
-template <bool RL2_LDS, bool ONE_UNIT>
-__device__ inline void list_exv_tile_t(const DevPtrs &P, const DSys &s, const double *X, const double *PX,
-                                       const Tile tl, int it, ListLds &L) {
-  auto &sx = L.sx; auto &sy = L.sy; auto &sz = L.sz; auto &su = L.su; auto &stc = L.stc;
-  const int lane = threadIdx.x;
+// A block per bead tile: units of 32 beads whose boxes (two of 16 beads) the
+// tile can reach within the largest list radius, tested 64 at a time (one lane
+// each), are dealt out to the waves; a wave stages its unit and forms, for
+// each bead of the tile, a bit per listed bead of the unit.  The bits give
+// each unit's first slot, so that the waves then write their entries, which
+// stay in ascending order.  Bound by the latency of the staging and of the 32
+// tests of a unit: with a wave per tile, which met the tiles one after the
+// other, a build took 122 us for 960 compact beads, 35 us for
+// the 6,000 of a long hairpin; by eight waves 23.6 and 11.8 us.
+template <bool RL2_LDS, bool ONE_UNIT, int W>
+__device__ inline void list_exv_tile_t(const DevPtrs &P, const DSys &s, const double *X, const Tile tl, int it,
+                                       ListLds<W> &L) {
+  const int lane = threadIdx.x & (kTile - 1), w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTile);
   const int li = tl.start + lane;
   const bool valid = li < s.nmp;
   const int n = P.ntot;
-  const double *Y = s.periodic ? PX : X;
   const int g = s.off + (valid ? li : 0);
-  if (RL2_LDS)
-    for (int k = lane; k < s.nunit * s.nunit; k += kTile) L.rl2[k] = P.rl2[s.uoff + k];
+  auto &sx = L.sx[w]; auto &sy = L.sy[w]; auto &sz = L.sz[w];
+  auto &su = L.su[w]; auto &stc = L.stc[w];
+  if (RL2_LDS && !ONE_UNIT) {
+    for (int k = (int)threadIdx.x; k < s.nunit * s.nunit; k += kTile * W) L.rl2[k] = P.rl2[s.uoff + k];
+    __syncthreads();
+  }
   double xi[3] = {0, 0, 0};
   int ui = 0, ti = 0, ci = 0;
-  if (valid) { ld3(Y, n, g, xi); ui = P.unit[g]; ti = P.mptype[g]; ci = P.iclass[g]; }
+  if (valid) { ld3(X, n, g, xi); ui = P.unit[g]; ti = P.mptype[g]; ci = P.iclass[g]; }
   const BBox bi = P.bbox[it];
   const double cut2 = s.rl2max * (1.0 + 1e-9);
+  const int nu = (s.nmp + kUnit - 1) / kUnit;
   int cnt = 0;
-  for (int j0 = 0; j0 < s.nbt; j0 += kTile) {
-    // tiles j0 .. j0 + 63 that a bead of this tile may reach, tested at once
-    const int jl = j0 + lane;
-    const bool reach = jl < s.nbt && (s.periodic || !(box_dmin2(bi, P.bbox[s.bt0 + jl]) > cut2));
-    uint64_t todo = __ballot(reach);
-    while (todo) {
-      const int jtile = j0 + __ffsll((unsigned long long)todo) - 1;
-      todo &= todo - 1;
-      const int jt = jtile * kTile;
-      int lj = jt + lane;
-      if (lj < s.nmp) {
-        int gj = s.off + lj;
-        sx[lane] = Y[gj]; sy[lane] = Y[n + gj]; sz[lane] = Y[2 * n + gj];
+  for (int u0 = 0; u0 < nu; u0 += kUnitsRound) {
+    const int ul = u0 + lane;
+    bool reach = false;
+    if (ul < nu) {
+      const BBox *sb = P.sbox + 4 * s.bt0 + 2 * ul;   // (its second group may be past the last bead)
+      reach = !(box_dmin2(bi, sb[0]) > cut2) || (ul * kUnit + 16 < s.nmp && !(box_dmin2(bi, sb[1]) > cut2));
+    }
+    const uint64_t units = __ballot(reach);   // the same in every wave
+    int q = 0;
+    for (uint64_t todo = units; todo; todo &= todo - 1, ++q) {
+      if ((q & (W - 1)) != w) continue;
+      const int unit = u0 + __builtin_ctzll(todo), jt = unit * kUnit;
+      const int kend = min(kUnit, s.nmp - jt);
+      if (lane < kUnit) {   // past the last bead: its copy, whose bits are dropped
+        const int gj = s.off + min(jt + lane, s.nmp - 1);
+        sx[lane] = X[gj]; sy[lane] = X[n + gj]; sz[lane] = X[2 * n + gj];
         su[lane] = P.unit[gj];
         stc[lane] = (int)P.mptype[gj] | ((int)P.iclass[gj] << 8);
       }
-      if (!s.periodic && lane < kTile / 16) L.sb[lane] = P.sbox[4 * (s.bt0 + jtile) + lane];
-      __syncthreads();
-      const int kend = min(kTile, s.nmp - jt);
-      for (int q0 = 0; q0 < kend; q0 += 16) {
-        if (!s.periodic) {
-          const bool need = valid && point_box_d2(xi, L.sb[q0 / 16]) <= cut2;
-          if (!__any(need)) continue;
-        }
-        const int q1 = min(q0 + 16, kend);
-        if (valid) {
-          // exv_candidate for a non-periodic system, every test evaluated
-          // and combined (no branch per test), the group's staged values
-          // read together
+      wave_lds_sync();
+      uint32_t bits = 0u;
 #pragma unroll
-          for (int dk = 0; dk < 16; ++dk) {
-            const int k = q0 + dk;
-            if (k >= q1) continue;   // (the same for every lane)
-            const int lj2 = jt + k;
-            const double d2 = sq3_separate(sx[k] - xi[0], sy[k] - xi[1], sz[k] - xi[2]);
-            // one unit: its radius is rl2max and both beads are in it
-            if (exv_listed<ONE_UNIT>(s, d2, li, ui, ti, ci, lj2, ONE_UNIT ? ui : su[k], stc[k],
-                                     RL2_LDS ? L.rl2 : P.rl2 + s.uoff)) {
-              if (cnt < P.nb_cap) P.nb[(size_t)cnt * n + g] = (uint32_t)(s.off + lj2);
-              ++cnt;
-            }
-          }
+      for (int h = 0; h < 2; ++h) {
+        if (16 * h >= kend) continue;
+        const bool need = valid && point_box_d2(xi, P.sbox[4 * s.bt0 + 2 * unit + h]) <= cut2;
+        if (!__any(need)) continue;
+        // every test evaluated and combined (no branch per test)
+#pragma unroll
+        for (int dk = 0; dk < 16; ++dk) {
+          const int k = 16 * h + dk;
+          const double d2 = sq3_separate(sx[k] - xi[0], sy[k] - xi[1], sz[k] - xi[2]);
+          // one unit: its radius is rl2max and both beads are in it
+          const bool in = exv_listed<ONE_UNIT>(s, d2, li, ui, ti, ci, jt + k, ONE_UNIT ? ui : su[k], stc[k],
+                                               RL2_LDS ? L.rl2 : P.rl2 + s.uoff);
+          bits |= in && k < kend ? 1u << k : 0u;
         }
       }
-      __syncthreads();
+      wave_lds_sync();
+      L.bits[q][lane] = valid ? bits : 0u;
     }
+    __syncthreads();
+    q = 0;
+    for (uint64_t todo = units; todo; todo &= todo - 1, ++q) {
+      uint32_t bits = L.bits[q][lane];
+      const int c = __popc(bits);
+      if ((q & (W - 1)) == w) {
+        const uint32_t j0 = (uint32_t)(s.off + (u0 + __builtin_ctzll(todo)) * kUnit);
+        for (int slot = cnt; bits; bits &= bits - 1u, ++slot)
+          if (slot < P.nb_cap) P.nb[(size_t)slot * n + g] = j0 + (uint32_t)__builtin_ctz(bits);
+      }
+      cnt += c;
+    }
+    __syncthreads();   // the bits are read before the next round's
   }
-  if (valid) {
+  if (w == 0 && valid) {
     P.nb_cnt[g] = cnt;
     if (cnt > P.nb_cap) atomicMax(&P.counters[5], (unsigned long long)cnt);
   }
@@ -1955,11 +1953,12 @@ __device__ inline void list_exv_tile_t(const DevPtrs &P, const DSys &s, const do
 // the unit-pair radii from LDS when the table fits there (a compile-time
 // choice: a run-time one makes every radius read a generic-pointer load).
 // Non-periodic systems only (k_lpair builds the periodic ones).
-__device__ inline void list_exv_tile(const DevPtrs &P, const DSys &s, const double *X, const double *PX,
-                                     const Tile tl, int it, ListLds &L) {
-  if (s.nunit == 1) list_exv_tile_t<true, true>(P, s, X, PX, tl, it, L);
-  else if (s.nunit <= kRl2Lds) list_exv_tile_t<true, false>(P, s, X, PX, tl, it, L);
-  else list_exv_tile_t<false, false>(P, s, X, PX, tl, it, L);
+template <int W>
+__device__ inline void list_exv_tile(const DevPtrs &P, const DSys &s, const double *X, const Tile tl, int it,
+                                     ListLds<W> &L) {
+  if (s.nunit == 1) list_exv_tile_t<true, true, W>(P, s, X, tl, it, L);
+  else if (s.nunit <= kRl2Lds) list_exv_tile_t<true, false, W>(P, s, X, tl, it, L);
+  else list_exv_tile_t<false, false, W>(P, s, X, tl, it, L);
 }
 
 // ele bit matrix (neighbor_list_ele.F90:123-210): bit (qi, qj) set when the
@@ -1979,65 +1978,55 @@ __device__ inline BBox charge_tile_union_box(const DevPtrs &P, const DSys &s, in
   return b;
 }
 
+// A block per charge tile, its rows' words (32 charges each) dealt out to the
+// waves.
 // (union_boxes: the charge tiles' boxes from the bead tiles' boxes instead of
 // qbbox, which only k_prep computes; conservative, so the decisions below
 // stay exact)
-__device__ inline void list_ele_tile(const DevPtrs &P, const DSys &s, const double *X, const double *PX,
-                                     const Tile tl, int it, ListLds &L, bool union_boxes) {
-  auto &sx = L.sx; auto &sy = L.sy; auto &sz = L.sz;
-  const int lane = threadIdx.x;
+template <int W>
+__device__ inline void list_ele_tile(const DevPtrs &P, const DSys &s, const double *X, const Tile tl, int it,
+                                     ListLds<W> &L, bool union_boxes) {
+  const int lane = threadIdx.x & (kTile - 1), w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTile);
+  auto &sx = L.sx[w]; auto &sy = L.sy[w]; auto &sz = L.sz[w];
   const int qi = tl.start + lane;
   const bool valid = qi < s.nq;
   const int n = P.ntot;
-  const double *Y = s.periodic ? PX : X;
   double xi[3] = {0, 0, 0};
-  if (valid) ld3(Y, n, P.qbead[s.qoff + qi], xi);
+  if (valid) ld3(X, n, P.qbead[s.qoff + qi], xi);
   uint32_t *row = P.qmask + s.moff + (int64_t)(valid ? qi : 0) * s.mwords;
   const BBox bi = union_boxes ? charge_tile_union_box(P, s, tl.start / kTile) : P.qbbox[it];
   for (int j0 = 0; j0 < s.nqt; j0 += kTile) {
     // mode of the tile pairs (it, j0 + lane), decided at once: 0 none, 1 all,
     // 2 test
     int lmode = 2;
-    if (!s.periodic && j0 + lane < s.nqt) {
+    if (j0 + lane < s.nqt) {
       const BBox bj = union_boxes ? charge_tile_union_box(P, s, j0 + lane) : P.qbbox[s.qt0 + j0 + lane];
       if (box_dmin2(bi, bj) > s.ele_rl2 * (1.0 + 1e-9)) lmode = 0;
       else if (box_dmax2(bi, bj) < s.ele_rl2 * (1.0 - 1e-9)) lmode = 1;
     }
-    for (int jtile = j0; jtile < min(s.nqt, j0 + kTile); ++jtile) {
-      const int jt = jtile * kTile;
-      const int kend = min(kTile, s.nq - jt);
-      const int mode = __shfl(lmode, jtile - j0);
-      uint32_t w[2] = {0u, 0u};
+    for (int u = 2 * j0 + w; u < min(s.mwords, 2 * (j0 + kTile)); u += W) {
+      const int jt = u * kUnit, kend = min(kUnit, s.nq - jt);
+      const int mode = __shfl(lmode, u / 2 - j0);
+      uint32_t bits = 0u;
       if (mode == 1) {
-        w[0] = kend >= 32 ? 0xFFFFFFFFu : ((1u << kend) - 1u);
-        w[1] = kend >= 64 ? 0xFFFFFFFFu : (kend > 32 ? ((1u << (kend - 32)) - 1u) : 0u);
-        if (qi >= jt && qi < jt + kend) w[(qi - jt) >> 5] &= ~(1u << ((qi - jt) & 31));
+        bits = kend >= kUnit ? 0xFFFFFFFFu : (1u << kend) - 1u;
+        if (qi >= jt && qi < jt + kend) bits &= ~(1u << (qi - jt));
       } else if (mode == 2) {
-        int qj = jt + lane;
-        if (qj < s.nq) {
-          int gj = P.qbead[s.qoff + qj];
-          sx[lane] = Y[gj]; sy[lane] = Y[n + gj]; sz[lane] = Y[2 * n + gj];
+        if (lane < kUnit) {   // past the last charge: its copy, whose bits are dropped
+          const int gj = P.qbead[s.qoff + min(jt + lane, s.nq - 1)];
+          sx[lane] = X[gj]; sy[lane] = X[n + gj]; sz[lane] = X[2 * n + gj];
         }
-        __syncthreads();
-        if (valid)
-          for (int k = 0; k < kend; ++k) {
-            int qj2 = jt + k;
-            if (qj2 == qi) continue;
-            const bool own_lo = qi < qj2;
-            double v[3];
-            pair_vec(s, sx[k], sy[k], sz[k], xi, own_lo, v);
-            int code = s.periodic ? pbneighbor(s, v) : 0;
-            double d2 = sq3_exact(v[0], v[1], v[2]);
-            if (!(d2 < s.ele_rl2)) continue;
-            w[k >> 5] |= 1u << (k & 31);
-            if (s.periodic) P.qmirror[s.mioff + (int64_t)qi * s.nq + qj2] = (uint8_t)(own_lo ? code : mirror_flip(code));
-          }
-        __syncthreads();
+        wave_lds_sync();
+#pragma unroll 16
+        for (int k = 0; k < kUnit; ++k) {
+          double v[3];
+          pair_vec(s, sx[k], sy[k], sz[k], xi, qi < jt + k, v);
+          const double d2 = sq3_exact(v[0], v[1], v[2]);
+          bits |= d2 < s.ele_rl2 && qi != jt + k && k < kend ? 1u << k : 0u;
+        }
+        wave_lds_sync();
       }
-      if (valid) {
-        row[jt >> 5] = w[0];
-        if ((jt >> 5) + 1 < s.mwords) row[(jt >> 5) + 1] = w[1];
-      }
+      if (valid) row[u] = bits;
     }
   }
 }
@@ -2060,11 +2049,6 @@ __device__ inline void list_hb_entry(const DevPtrs &P, const DSys &s, const doub
 }
 
 // ------------------------------------------------------------------ lists by tile pairs
-__device__ inline void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The exv and electrostatic lists of periodic systems by pairs of tiles, which
 // one wave per tile (k_lists) would walk one after the other.  Pass 1, a block
@@ -2239,7 +2223,7 @@ __global__ __launch_bounds__(kTile * kWaves) void k_lpair_put(DevPtrs P, const d
 // sqrt(m1) + sqrt(m2) > margin.
 __device__ inline bool system_trigger(const DevPtrs &P, const DSys &s) {
   double a = 0.0, b = 0.0;
-  for (int t = (int)threadIdx.x; t < s.nbt; t += kTile) {
+  for (int t = (int)threadIdx.x & (kTile - 1); t < s.nbt; t += kTile) {
     const double t1 = P.ttop[2 * (s.bt0 + t)], t2 = P.ttop[2 * (s.bt0 + t) + 1];
     const double hi = fmax(a, t1), lo = fmax(fmin(a, t1), fmax(b, t2));
     a = hi; b = lo;
@@ -2323,13 +2307,14 @@ __global__ __launch_bounds__(kTile) void k_prep(DevPtrs P, const double *X, doub
   if (!s.periodic) bbox_tile(P, s, X, tl, it, charge);
 }
 
-// k_lists: one wave per block; [0, nbt) exv lists of bead tiles, [nbt,
-// nbt + nqt) ele bit rows of charge tiles, then 64 hbond candidates per
+// k_lists, W waves per block: [0, nbt) exv lists of bead tiles,
+// [nbt, nbt + nqt) ele bit rows of charge tiles, then 64 W hbond candidates per
 // block.
-__global__ __launch_bounds__(kTile) void k_lists(DevPtrs P, const double *X, const double *PX, const Tile *btiles,
+template <int W>
+__global__ __launch_bounds__(kTile * W) void k_lists(DevPtrs P, const double *X, const double *PX, const Tile *btiles,
                                                  int bt0, int nbt, const Tile *qtiles, int qt0, int nqt, int h0,
                                                  int nh, int gate) {
-  __shared__ ListLds lds;
+  __shared__ ListLds<W> lds;
   if (run_stopped(P)) return;
   const int b = (int)blockIdx.x;
   if (b < nbt + nqt) {
@@ -2347,23 +2332,29 @@ __global__ __launch_bounds__(kTile) void k_lists(DevPtrs P, const double *X, con
       if (!fire) return;
       if (!charge) {
         const int li = tl.start + (int)threadIdx.x, n = P.ntot;
-        if (li < s.nmp)
+        if ((int)threadIdx.x < kTile && li < s.nmp)
           for (int d = 0; d < 3; ++d) P.dxyz[d * n + s.off + li] = P.dlast[d * n + s.off + li];
         // the system's hbond candidates, shared out over its bead tiles
-        for (int k = tl.start + (int)threadIdx.x; k < s.nhb; k += s.nbt * kTile) list_hb_entry(P, s, X, PX, s.hoff + k);
+        for (int k = tl.start * W + (int)threadIdx.x; k < s.nhb; k += s.nbt * kTile * W)
+          list_hb_entry(P, s, X, PX, s.hoff + k);
       }
     }
     if (s.periodic) return;   // built by tile pairs (k_lpair)
-    if (charge) list_ele_tile(P, s, X, PX, tl, it, lds, gate == 2);
-    else list_exv_tile(P, s, X, PX, tl, it, lds);
+    if (charge) list_ele_tile(P, s, X, tl, it, lds, gate == 2);
+    else list_exv_tile(P, s, X, tl, it, lds);
     return;
   }
-  const int k = (b - nbt - nqt) * kTile + (int)threadIdx.x;
+  const int k = (b - nbt - nqt) * (kTile * W) + (int)threadIdx.x;
   if (k >= nh) return;
   const int h = h0 + k;
   if (gate && !P.sys_flag[P.hb_sys[h]]) return;
   list_hb_entry(P, P.sys[P.hb_sys[h]], X, PX, h);
 }
+
+template __global__ void k_lists<kListWide>(DevPtrs, const double *, const double *, const Tile *, int, int, const Tile *, int,
+                                    int, int, int, int);
+template __global__ void k_lists<kListFew>(DevPtrs, const double *, const double *, const Tile *, int, int, const Tile *, int,
+                                    int, int, int, int);
 
 // ------------------------------------------------------------------ windows of steps
 // Steps of small systems without leaving the workgroup: one workgroup takes
