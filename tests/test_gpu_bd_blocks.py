@@ -1,15 +1,12 @@
-"""The full-panel Cholesky kernel (16 x 16 tiles on the FP64 matrix cores) at
-the edges of its tiles, panels and outer blocks against the FP64 factor, its
-pivot check, and the step's products and forces at the edges of their blocks.
-The wait states of its DPP multiply-adds are checked on the generated code."""
+"""The Cholesky factor at the edges of panels and outer blocks against the FP64
+factor, its pivot check, and the step's products and forces at the edges of
+their blocks."""
 import ctypes
-import os
 
 import numpy as np
 import pytest
 
 import oracle
-import test_dpp_hazards as hz
 from test_zz_no_alloc import D2H, H2D, _hip
 from tis_amd.bdhi import bead_spring_chain
 from tis_amd.engine import BDEngine, load_library
@@ -79,19 +76,3 @@ def test_forces_and_step(n):
     xo = oracle.bdhi_run(s, x, 3, tstep=0.05, refactor_every=1, seed=11, key=9, step0=100)
     assert np.abs(e.coords() - xo).max() <= 1e-5
     e.close()
-
-
-@pytest.mark.skipif(not os.path.exists(hz.HIPCC), reason="hipcc not available")
-def test_full_panel_dpp_wait_states(tmp_path):
-    import subprocess
-    out = tmp_path / "bdhi.s"
-    subprocess.run([hz.HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-                    "-packed-fp32-ops", "--cuda-device-only", "-S", hz.SRC, "-o", str(out)], check=True,
-                   capture_output=True)
-    lines = out.read_text().splitlines()
-    start = next(i for i, l in enumerate(lines) if l.startswith("_ZN3tis12k_chol_block"))
-    end = next(i for i in range(start, len(lines)) if lines[i].startswith(".Lfunc_end"))
-    n, bad = hz.dpp_hazards(lines[start:end])
-    # 105 + 120 multiply-adds of a 16 x 16 tile and its inverse, and more moves
-    assert n >= 225
-    assert not bad, bad[:3]

@@ -389,7 +389,8 @@ __device__ __forceinline__ void solve_cols(double (&x)[kCb], const double *Ls, c
 // 32 (P column k at P + k * mpad), in the accumulator layout of
 // v_mfma_f32_32x32x2f32 with the columns' entries as the first operand: the
 // operands and the order of the sums are those of k_chol_update.  Operands
-// come straight from memory (L2), 16 k pairs ahead.
+// come straight from memory (L2), 16 k pairs ahead (a factor at 3n = 9000: 7.90
+// ms with eight, 7.68 with 16).
 __device__ inline floatx16 quad_product(const float *P, int mpad, int ra, int rb, int K, int lane) {
   floatx16 acc;
   for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
@@ -562,275 +563,6 @@ __global__ __launch_bounds__(kPanelThreads) void k_chol_panel(BdDev B, int kk, i
       P[(size_t)(q0 + c) * mpad + rl] = (live && c < kb) ? (float)v[c] : 0.0f;
     }
   }
-}
-
-// ---------------------------------------------------------------- full panels
-// A panel of 64 full columns in tiles of 16 x 16 on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64): operand A lane l holds A[l % 16][l / 16], B lane l
-// holds B[l / 16][l % 16], D register v of lane l holds D[l / 16 + 4 v][l % 16].
-// A tile is kept transposed in that layout (lane: row l % 16, register v:
-// column l / 16 + 4 v), and then its registers are, as they stand, both the B
-// operand of the transposed tile and the A operand of the tile, register v at
-// k = 4 v: the tile algebra below moves nothing between lanes.
-// Bound: the serial chain of 64 pivots (broadcast, reciprocal, scale, next
-// entry), about 190 cycles each.  k_chol_panel runs it over 64 rows with the
-// columns published in LDS, 12 us, and solves the rows below by 64 dependent
-// steps, 6 us more; here the chain runs in registers, 16 columns at a time
-// (2,984 cycles), the inverses of the 16 x 16 factors come with it, and the
-// rows below are products.  A panel at 3n = 900: 27.7 us by k_chol_panel, 24.5
-// us here; the factor 450 -> 404 us there, 1.60 -> 1.45 ms at 3n = 3000, 7.8
-// -> 7.4 ms at 9000.  The chain's broadcasts are DPP operands of the
-// multiply-adds: as two moves (with their old values) and an fma the tile took
-// 9,004 cycles, as lane-masked moves 6,352.
-typedef double doublex4 __attribute__((ext_vector_type(4)));
-
-// D = C + A B of 16 x 16 tiles, K = 16
-__device__ __forceinline__ doublex4 tile_fma(const doublex4 &a, const doublex4 &b, doublex4 c) {
-#pragma unroll
-  for (int k = 0; k < 4; ++k) c = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], b[k], c, 0, 0, 0);
-  return c;
-}
-
-// v0 .. v3 for q = 0 .. 3 (of values: a choice among array elements would put
-// the array in scratch memory)
-__device__ __forceinline__ double one_of4(int q, double v0, double v1, double v2, double v3) {
-  const double lo = q & 1 ? v1 : v0, hi = q & 1 ? v3 : v2;
-  return q & 2 ? hi : lo;
-}
-
-// the value of v at lane N of the lane's row of 16
-template <int N>
-__device__ __forceinline__ double row_value(double v) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, 0x150 + N, 0xF, 0xF, true);
-  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), 0x150 + N, 0xF, 0xF, true);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// One 16 x 16 diagonal tile as L D L^T, row r = lane % 16 in a[] (every row of
-// 16 lanes holds a copy), right-looking; t[] takes the same row operations on
-// the identity, L^-1.  On return a[] is the row of the Cholesky factor L
-// sqrt(D), t[] the row of L^-1 and rs 1 / sqrt(D[r]).  bad: the first pivot
-// that is not positive, as kk + column + 1 (0xffffffff: none).  Entries above
-// the diagonal are left to take what the rows below take (no entry on or below
-// it reads them) and cleared at the end; the next column's entry is written by
-// the compiler's own fma, so that the waits before the lane reads of the chain
-// are the compiler's too.
-template <int C, int J>
-__device__ __forceinline__ void factor16_update(double (&a)[16], double u, double ns) {
-  if constexpr (J < 16) {
-    fmac_row_bcast<J>(a[J], u, ns);
-    factor16_update<C, J + 1>(a, u, ns);
-  }
-}
-template <int C, int K>
-__device__ __forceinline__ void factor16_inverse(double (&t)[16], double ns) {
-  if constexpr (K < C) {
-    fmac_row_bcast<C>(t[K], t[K], ns);
-    factor16_inverse<C, K + 1>(t, ns);
-  }
-}
-template <int C>
-__device__ __forceinline__ void factor16_step(double (&a)[16], double (&t)[16], double &piv, int kk, unsigned &bad) {
-  if constexpr (C < 16) {
-    const int r = threadIdx.x & 15;
-    const double u = a[C];
-    const double d = row_value<C>(u);
-    const double ns = -u * rcp_nr(d);
-    if constexpr (C + 1 < 16) a[C + 1] = fma(row_value<C + 1>(u), ns, a[C + 1]);
-    factor16_update<C, C + 2>(a, u, ns);
-    const double nt = r > C ? ns : 0.0;
-    factor16_inverse<C, 0>(t, nt);
-    t[C] = r == C ? 1.0 : nt;
-    piv = r == C ? d : piv;
-    bad = min(bad, d > 0.0 ? 0xffffffffu : (unsigned)(kk + C + 1));
-    factor16_step<C + 1>(a, t, piv, kk, bad);
-  }
-}
-template <int C>
-__device__ __forceinline__ void factor16_scale(double (&a)[16], double rs) {
-  if constexpr (C < 16) {
-    a[C] = (int)(threadIdx.x & 15) >= C ? a[C] * row_value<C>(rs) : 0.0;
-    factor16_scale<C + 1>(a, rs);
-  }
-}
-__device__ __forceinline__ void factor16(double (&a)[16], double (&t)[16], double &rs, int kk, unsigned &bad) {
-  double piv = 1.0;
-  factor16_step<0>(a, t, piv, kk, bad);
-  rs = rsqrt_nr(piv);
-  factor16_scale<0>(a, rs);
-}
-
-// As k_chol_panel for a panel whose 64 columns are all there: wave 0 factors
-// the diagonal block, tile (i, j) of its lower triangle in yt[i (i + 1) / 2 +
-// j]; waves 1-3 form the earlier panels' product for the block's rows
-// meanwhile (the diagonal block's, by all four waves, comes first:
-// quad_product, the bits of k_chol_update); then each wave solves 16 rows.
-// The tiles are in LDS and the loops over them are not unrolled: every panel
-// runs this code once, and straight-line code for all of it (tiles in
-// registers) took 60,000 cycles instead of 25,400, most of them waiting for
-// instructions.
-__global__ __launch_bounds__(kPanelThreads) __attribute__((amdgpu_waves_per_eu(1))) void k_chol_block(BdDev B, int kk,
-                                                                                                     int k0, float *P,
-                                                                                                     int mpad) {
-  __shared__ float Td[kCb][kCb + 1], Tr[kCb][kCb + 1];
-  // tiles and, per 16 columns, the inverse factor as operands; the diagonal
-  // tiles of the factor [s][column][row]
-  __shared__ double yt[10][4][kCb], op[4][4][kCb], cd[4][16][16];
-  const int lane = threadIdx.x & (kCb - 1), w = threadIdx.x / kCb, n3 = B.n3;
-  const int r16 = lane & 15, c4 = lane >> 4;
-  const int K = kk - k0;
-  const int r0w = kk + kCb * (int)blockIdx.x;   // the block's first row (blocks 1..)
-  const bool rows = blockIdx.x > 0 && r0w < n3;
-  const int p = kk / kCb;
-  // every wave: columns [16 w, 16 w + 16) of the diagonal block's rows, and 16
-  // of the block's rows (unconditional loads, rows past n3 clamped)
-  double dg[16];
-#pragma unroll
-  for (int c = 0; c < 16; ++c) dg[c] = B.L[(size_t)(kk + lane) + (size_t)(kk + 16 * w + c) * n3];
-  doublex4 x[4];
-  const int r = r0w + 16 * w + r16;
-  if (rows) {
-    const size_t row = (size_t)min(r, n3 - 1);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) x[q][v] = B.L[row + (size_t)(kk + 16 * q + c4 + 4 * v) * n3];
-  }
-  if (w == 3 && blockIdx.x == 0 && p > 0) {
-    // the previous panel's diagonal factor (see k_chol_panel)
-    const double *sp = B.stash + (size_t)((p - 1) & 1) * kCb * kCb;
-    const int kp = kk - kCb;
-#pragma unroll 8
-    for (int c = 0; c < kCb; ++c) B.L[(size_t)(kp + lane) + (size_t)(kp + c) * n3] = sp[c * kCb + lane];
-  }
-  const int l32 = lane & 31, c32 = 4 * (lane >> 5);   // accumulator e: row l32, column c32 + 8 (e / 4) + e % 4
-  // quadrants quad, quad + step, .. of the product for rows from ra
-  auto product = [&](float (*T)[kCb + 1], int ra, int quad, int step) {
-#pragma unroll 1
-    for (; quad < 4; quad += step) {
-      const int qi = quad >> 1, qj = quad & 1;
-      const floatx16 acc = quad_product(P, mpad, ra - k0 + 32 * qi, kk - k0 + 32 * qj, K, lane);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) T[32 * qi + l32][32 * qj + c32 + 8 * (e >> 2) + (e & 3)] = acc[e];
-    }
-  };
-  if (K > 0) product(Td, kk, w, 4);
-  __syncthreads();
-  // the diagonal block less its product into tiles: this wave's 16 columns are
-  // tile column w, row lane of tile row lane / 16
-  {
-    const int i = lane >> 4;
-    if (i >= w) {
-      double(*t)[kCb] = yt[i * (i + 1) / 2 + w];
-#pragma unroll
-      for (int c = 0; c < 16; ++c)
-        t[c >> 2][16 * (c & 3) + r16] = K > 0 ? dg[c] - (double)Td[lane][16 * w + c] : dg[c];
-    }
-  }
-  __syncthreads();
-  if (w == 0) {
-    unsigned bad = 0xffffffffu;
-#pragma unroll 1
-    for (int sx = 0; sx < 4; ++sx) {
-      double a[16], t[16], rs = 0.0;
-      double(*yd)[kCb] = yt[sx * (sx + 1) / 2 + sx];
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) a[4 * v + q] = yd[v][16 * q + r16];
-      factor16(a, t, rs, kk + 16 * sx, bad);
-      doublex4 inv;   // row r16, columns c4 + 4 v of the inverse factor
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        inv[v] = one_of4(c4, t[4 * v], t[4 * v + 1], t[4 * v + 2], t[4 * v + 3]) * rs;
-        op[sx][v][lane] = inv[v];
-        cd[sx][4 * v + c4][r16] = one_of4(c4, a[4 * v], a[4 * v + 1], a[4 * v + 2], a[4 * v + 3]);
-      }
-      // the column's tiles, then what they take from the tiles to the right:
-      // every load first, independent products side by side
-      doublex4 y[4], o[4][4];
-#pragma unroll
-      for (int i = 1; i < 4; ++i)
-        if (i > sx) {
-#pragma unroll
-          for (int v = 0; v < 4; ++v) y[i][v] = yt[i * (i + 1) / 2 + sx][v][lane];
-#pragma unroll
-          for (int j = 1; j <= i; ++j)
-            if (j > sx)
-#pragma unroll
-              for (int v = 0; v < 4; ++v) o[i][j][v] = yt[i * (i + 1) / 2 + j][v][lane];
-        }
-#pragma unroll
-      for (int i = 1; i < 4; ++i)
-        if (i > sx) {
-          y[i] = tile_fma(inv, y[i], doublex4{0.0, 0.0, 0.0, 0.0});
-#pragma unroll
-          for (int v = 0; v < 4; ++v) yt[i * (i + 1) / 2 + sx][v][lane] = y[i][v];
-        }
-#pragma unroll
-      for (int j = 1; j < 4; ++j)
-        if (j > sx) {
-          const doublex4 nj = -y[j];
-#pragma unroll
-          for (int i = j; i < 4; ++i) {
-            o[i][j] = tile_fma(nj, y[i], o[i][j]);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) yt[i * (i + 1) / 2 + j][v][lane] = o[i][j][v];
-          }
-        }
-    }
-    if (blockIdx.x == 0 && lane == 0 && bad != 0xffffffffu) atomicCAS(B.info, 0, (int)bad);
-  } else if (K > 0 && rows) {
-    product(Tr, r0w, w - 1, 3);
-  }
-  __syncthreads();
-  if (blockIdx.x == 0) {
-    // the factor goes to the stash, or, from a panel of one block, to its
-    // place: this wave's 16 columns, zeros above the diagonal
-    double *fo = gridDim.x > 1 ? B.stash + (size_t)(p & 1) * kCb * kCb : B.L + (size_t)kk + (size_t)kk * n3;
-    const size_t ld = gridDim.x > 1 ? (size_t)kCb : (size_t)n3;
-    const int i = lane >> 4;
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      const double val = i > w ? yt[i * (i + 1) / 2 + w][c >> 2][16 * (c & 3) + r16] : (i == w ? cd[w][c][r16] : 0.0);
-      fo[(size_t)lane + (16 * w + c) * ld] = val;
-    }
-    return;
-  }
-  if (!rows) return;
-  if (K > 0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) x[q][v] -= (double)Tr[16 * w + r16][16 * q + c4 + 4 * v];
-  }
-  doublex4 nx[4];   // the solved tiles, negated
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-#pragma unroll
-    for (int e = 0; e < q; ++e) {
-      doublex4 c;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) c[v] = yt[q * (q + 1) / 2 + e][v][lane];
-      x[q] = tile_fma(c, nx[e], x[q]);
-    }
-    doublex4 inv;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) inv[v] = op[q][v][lane];
-    x[q] = tile_fma(inv, x[q], doublex4{0.0, 0.0, 0.0, 0.0});
-    nx[q] = -x[q];
-  }
-  const bool live = r < n3;
-  const int rl = r - k0, q0 = kk - k0;   // row and first column of P
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int c = 16 * q + c4 + 4 * v;
-      if (live) B.L[(size_t)r + (size_t)(kk + c) * n3] = x[q][v];
-      if (rl < mpad) P[(size_t)(q0 + c) * mpad + rl] = live ? (float)x[q][v] : 0.0f;
-    }
 }
 
 // C -= A B^T on 64x64 tiles of the lower part of L, FP32 matrix cores
@@ -1109,11 +841,7 @@ void factor_launches(const BdDev &d, float *P, hipStream_t st) {
       const int kk = k0 + j * kCb;
       const int m = n3 - kk - kCb;
       const int nbp = m > 0 ? (m + kPanelRowsPerBlock - 1) / kPanelRowsPerBlock : 0;
-      // the last panel of a size that is no multiple of 64 has columns missing
-      if (n3 - kk >= kCb)
-        hipLaunchKernelGGL(k_chol_block, dim3(1 + nbp), dim3(kPanelThreads), 0, st, d, kk, k0, P, mpad);
-      else
-        hipLaunchKernelGGL(k_chol_panel, dim3(1 + nbp), dim3(kPanelThreads), 0, st, d, kk, k0, P, mpad);
+      hipLaunchKernelGGL(k_chol_panel, dim3(1 + nbp), dim3(kPanelThreads), 0, st, d, kk, k0, P, mpad);
     }
     const int kt = k0 + kNb;
     if (kt >= n3) break;
