@@ -47,7 +47,8 @@ enum { TIS_CNT_CLAMP_EXV = 0, TIS_CNT_CLAMP_ELE = 1, TIS_CNT_HB_DELETED = 2,
        TIS_CNT_RESUMES = 7, TIS_CNT_MAX = 8 };
 
 /* Langevin launch modes for tis_langevin_steps */
-enum { TIS_MODE_GRAPH = 0,   /* batched, hipGraph-captured, one step = 2 launches */
+enum { TIS_MODE_GRAPH = 0,   /* batched: many steps per launch (windows of small
+                                systems, else a hipGraph of steps)          */
        TIS_MODE_EAGER = 1,   /* batched, launched eagerly                         */
        TIS_MODE_PLAIN = 2 }; /* one system per launch (plain GPU path)            */
 
