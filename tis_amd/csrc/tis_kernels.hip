@@ -2818,17 +2818,29 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
             const int j = (int)(P.nb[(size_t)m * N + s.off + i] & kIdxMask) - s.off;
             return j | (int)spec[j] << 10;
           };
-          // sifted in FP32, 32 entries at a time, as in exv_bead; the pairs
-          // that may touch then in FP64
+          // sifted in FP32, 32 entries at a time (eight records' reads under
+          // way: 200 steps of a 64-nt hairpin 2,361 -> 2,344 us, of 64 of them
+          // 3,678 -> 3,612), as in exv_bead; the pairs that may touch then in FP64
+          const bool local = __all(cnt <= rows);   // no list past the rows in LDS
           for (int q0 = 0; q0 < half; q0 += 32) {
             uint32_t near = 0;
-#pragma unroll 4
-            for (int q = q0; q < min(q0 + 32, half); ++q) {
-              const float4 f = xf[entry(q) & 1023];
-              const float v0 = f.x - fi.x, v1 = f.y - fi.y, v2 = f.z - fi.z;
-              const bool far = v0 * v0 + v1 * v1 + v2 * v2 > s.exv_near2;
-              near |= (uint32_t)(far ? 0 : 1) << (q - q0);
-            }
+            auto sift = [&](auto at) {
+              for (int q = q0; q < min(q0 + 32, half); q += 8) {
+                float4 f[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) f[u] = xf[at(min(q + u, half - 1)) & 1023];
+                uint32_t b = 0;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                  const float v0 = f[u].x - fi.x, v1 = f[u].y - fi.y, v2 = f[u].z - fi.z;
+                  const bool far = v0 * v0 + v1 * v1 + v2 * v2 > s.exv_near2;
+                  b |= far ? 0u : 1u << u;
+                }
+                near |= (half - q < 8 ? b & ((1u << (half - q)) - 1u) : b) << (q - q0);
+              }
+            };
+            if (local) sift([&](int q) { return (int)list[((q >> 2) * 8 + 4 * h + (q & 3)) * nb + i]; });
+            else sift(entry);
             for (; near; near &= near - 1) {
               const int q = q0 + (int)__builtin_ctz(near), en = entry(q), j = en & 1023;
               const double v[3] = {x[j] - xi[0], x[nb + j] - xi[1], x[2 * nb + j] - xi[2]};
