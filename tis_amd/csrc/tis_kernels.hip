@@ -2366,7 +2366,7 @@ template __global__ void k_lists<kListFew>(DevPtrs, const double *, const double
 // them FP64, on the four SIMDs of one CU; its longest chain is the 32
 // dependent pair steps of a charge chunk.  As two launches per step (k_force,
 // k_main) and three per rebuild every hand-over went through L2: 17.6 us a
-// step for that hairpin against 11.4 here, 64 of them 18.1 against 12.4.
+// step for that hairpin against 10.2 here, 64 of them 18.1 against 11.1.
 // Per step: (1) the terms as tasks of one wave each, longest first, taken
 // from a counter in LDS (chunk pairs of charges, 64 hbonds, 64 stacks, the
 // noise of 64 beads, half the neighbour groups of 64 beads, 64 angles, 64
@@ -2452,7 +2452,8 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
          *hbp = (double *)(lds + L.hb);
   EleWave *je = (EleWave *)(lds + L.je);
   SpPair *sptab = (SpPair *)(lds + L.sptab);
-  uint64_t *mask = (uint64_t *)(lds + L.mask), *seg = (uint64_t *)(lds + L.slot);
+  uint64_t *mask = (uint64_t *)(lds + L.mask);
+  uint32_t *seg = (uint32_t *)(lds + L.slot);
   float *qic = (float *)(lds + L.qic), *slot = (float *)(lds + L.slot);
   uint32_t *meta = (uint32_t *)(lds + L.meta);   // type | class << 8 | unit << 16
   int32_t *scnt = (int32_t *)(lds + L.cnt), *sval = (int32_t *)(lds + L.val);
@@ -2614,33 +2615,40 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
     if (due(t)) {
       // ---- lists from the current positions (k_lists' tests; entries in
       // ascending order); to memory too when no later rebuild of this launch
-      // replaces them
+      // replaces them.  Tasks of 64 beads against 32: an even share for the
+      // waves where 64 against 64 left some with twice the others' (200 steps of
+      // a 64-nt hairpin 2,344 -> 2,038 us, of 64 of them 3,630 -> 3,334).
+      const int nu = (nb + kUnit - 1) / kUnit;
       const bool keep = dyn || t + rebuild >= n;
       if (own)
         for (int d = 0; d < 3; ++d) { xp[d] = x[d * nb + tid]; x[d * nb + tid] = xc[d]; }
       __syncthreads();
       for (;;) {
         int k = take_task(&next[2]);
-        if (k >= nbt * nbt + nqt * nqt) break;
-        if (k < nbt * nbt) {
-          // 64 beads against 64: the accept bits of each lane's bead
-          const int i = (k / nbt) * kTile + lane, j0 = (k % nbt) * kTile, kend = min(kTile, nb - j0);
+        if (k >= nqt * nqt + nbt * nu) break;
+        if (k >= nqt * nqt) {
+          // 64 beads against 32: the accept bits of each lane's bead
+          k -= nqt * nqt;
+          const int i = (k / nu) * kTile + lane, j0 = (k % nu) * kUnit, kend = min(kUnit, nb - j0);
           const int ic = i < nb ? i : 0;
           const double x0 = x[ic], x1 = x[nb + ic], x2 = x[2 * nb + ic];
           const int mi = (int)meta[ic], ui = mi >> 16, ti = mi & 0xFF, ci = (mi >> 8) & 0xFF;
-          uint64_t m = 0;
-#pragma unroll 4
-          for (int q = 0; q < kend; ++q) {
-            const int j = j0 + q, mj = (int)meta[j];
-            const double d2 = sq3_separate(x[j] - x0, x[nb + j] - x1, x[2 * nb + j] - x2);
-            const bool ok = s.nunit == 1 ? exv_listed<true>(s, d2, i, ui, ti, ci, j, ui, mj & 0xFFFF, rl2)
-                                         : exv_listed<false>(s, d2, i, ui, ti, ci, j, mj >> 16, mj & 0xFFFF, rl2);
-            m |= (uint64_t)(ok ? 1 : 0) << q;
-          }
-          if (i < nb) seg[(k % nbt) * nb + i] = m;
+          uint32_t m = 0;
+          auto tests = [&](auto one) {
+            constexpr bool ONE = decltype(one)::value;
+#pragma unroll 8
+            for (int q = 0; q < kend; ++q) {
+              const int j = j0 + q, mj = (int)meta[j];
+              const double d2 = sq3_separate(x[j] - x0, x[nb + j] - x1, x[2 * nb + j] - x2);
+              const bool ok = exv_listed<ONE>(s, d2, i, ui, ti, ci, j, ONE ? ui : mj >> 16, mj & 0xFFFF, rl2);
+              m |= (ok ? 1u : 0u) << q;
+            }
+          };
+          if (s.nunit == 1) tests(std::true_type{});
+          else tests(std::false_type{});
+          if (i < nb) seg[(k % nu) * nb + i] = m;
           continue;
         }
-        k -= nbt * nbt;
         const int I = k / nqt, J = k % nqt, qi = I * kTile + lane, jt = J * kTile;
         if (J < I && !keep) continue;
         const int bi = qi < nq ? qb[qi] : 0, kend = min(kTile, nq - jt);
@@ -2673,18 +2681,18 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
       if (own)
         for (int d = 0; d < 3; ++d) x[d * nb + tid] = xp[d];
       if (tid == 0) next[2] = 0;
-      for (int k = tid; k < nb * nbt; k += T) {
+      for (int k = tid; k < nb * nu; k += T) {
         const int i = k % nb, sg = k / nb;
         int m = 0;
-        for (int q = 0; q < sg; ++q) m += __popcll(seg[q * nb + i]);
-        uint64_t bits = seg[k];
-        const int tot = m + __popcll(bits);
-        for (; bits; bits &= bits - 1, ++m) {
-          const int j = sg * kTile + (int)__builtin_ctzll(bits);
+        for (int q = 0; q < sg; ++q) m += __popc(seg[q * nb + i]);
+        uint32_t bits = seg[k];
+        const int tot = m + __popc(bits);
+        for (; bits; bits &= bits - 1u, ++m) {
+          const int j = sg * kUnit + (int)__builtin_ctz(bits);
           if (m < rows) list[m * nb + i] = (uint16_t)(j | (int)spec[j] << 10);
           if ((keep || m >= rows) && m < P.nb_cap) P.nb[(size_t)m * N + s.off + i] = (uint32_t)(s.off + j);
         }
-        if (sg == nbt - 1) {
+        if (sg == nu - 1) {
           nbc[i] = (uint16_t)tot;
           if (keep) P.nb_cnt[s.off + i] = tot;
           if (tot > P.nb_cap) {
