@@ -1070,9 +1070,8 @@ bool window_fits(const DSys &d) {
 // kWindowBeads).  *wsys gets the systems, the largest first (blocks start in
 // order).
 // Measured, us a step with a rebuild every 10 (per-step passes / k_window), 1
-// system and 512: 95 beads 16.3 / 10.9 and 26 / 20; 254 beads 19.4 / 15.7 and
-// 40 / 31; 446 beads 20.8 / 24.6 and 62 / 50: one workgroup falls behind on
-// its own near 400 beads and stays ahead when the batch fills the chip.
+// system and 512: 95 beads 13.0 / 9.0 and 24 / 18; 254 beads 15.8 / 14.8 and
+// 35 / 30; 446 beads 16.4 and 56 either way.
 constexpr int kWindowBeads = 448;
 constexpr int kWindowSteps = 500;   // steps per k_window launch (a few ms)
 
