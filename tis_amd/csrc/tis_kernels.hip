@@ -442,6 +442,17 @@ __device__ inline bool run_stopped(const DevPtrs &P) {
   return __builtin_nontemporal_load(&P.counters[5]) != 0ull;
 }
 
+// The same, decided once for the whole block: in a kernel whose own blocks
+// raise the flag (a list that overflows), the waves of a block that starts
+// meanwhile could read it differently, and those that go on would work without
+// the others' share.  Contains a barrier: every thread of the block calls it.
+__device__ inline bool block_stopped(const DevPtrs &P) {
+  __shared__ int stop;
+  if (threadIdx.x == 0) stop = run_stopped(P) ? 1 : 0;
+  __syncthreads();
+  return stop != 0;
+}
+
 __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -2315,7 +2326,7 @@ __global__ __launch_bounds__(kTile * W) void k_lists(DevPtrs P, const double *X,
                                                  int bt0, int nbt, const Tile *qtiles, int qt0, int nqt, int h0,
                                                  int nh, int gate) {
   __shared__ ListLds<W> lds;
-  if (run_stopped(P)) return;
+  if (block_stopped(P)) return;
   const int b = (int)blockIdx.x;
   if (b < nbt + nqt) {
     const bool charge = b >= nbt;
@@ -2432,7 +2443,7 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
   __shared__ int next[3];
   __shared__ unsigned over;
   __shared__ double top[W][2];
-  if (run_stopped(P)) return;
+  if (block_stopped(P)) return;
   const int isys = wsys[blockIdx.x];
   const DSys s = P.sys[isys];
   const uint64_t base = *P.stepbase;
