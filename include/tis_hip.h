@@ -205,6 +205,14 @@ int32_t tis_term_status(tis_ctx *ctx, int32_t isys, int32_t *hb_status, int32_t 
  * (const_maxsize.F90, allocate_neighbor.F90). */
 int32_t tis_list_capacity(tis_ctx *ctx, int32_t cap, int32_t *cap_out);
 
+/* The largest capacity that list builds may grow to (cap <= 0: no limit, as a
+ * new context has).  A build that needs more returns TIS_ERR_NOMEM, as it does
+ * when the device has no room for the larger lists.  tis_langevin_steps then
+ * leaves the state of the last step that every system completed; runs by
+ * per-step launches may be continued by another call, a batch run by windows
+ * (small systems, TIS_MODE_GRAPH) after tis_langevin_init. */
+int32_t tis_list_limit(tis_ctx *ctx, int32_t cap);
+
 /* Payload bytes moved since the context was created, bytes[4]:
  * [0] host to device, topology, parameters and launch tables;
  * [1] host to device, dynamic state (tis_state_set);

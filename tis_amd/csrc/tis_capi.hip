@@ -38,6 +38,7 @@ __global__ void k_lpair(DevPtrs, const double *, const EwTask *, int, const EwTa
 __global__ void k_lpair_put(DevPtrs, const double *, const EwTask *, int, int);
 __global__ void k_advance(uint64_t *, uint64_t, uint64_t, uint64_t, unsigned long long *);
 __global__ void k_window(DevPtrs, const int32_t *, int, int, int, int, int);
+__global__ void k_window_back(DevPtrs, const int32_t *, int);
 __global__ void k_run_report(unsigned long long *, unsigned long long *);
 __global__ void k_state_out(const double *, int, int, int, double *, const unsigned long long *, unsigned long long *);
 __global__ void k_state_in(DevPtrs, double *, int, int, const double *, float4 *);
@@ -194,6 +195,7 @@ struct tis_ctx {
   double tstep = 0.0;
   int32_t rebuild_every = 10;
   int64_t t_since_init = 0;
+  int32_t nb_limit = 0;                  // largest list capacity calls may grow to; 0: any (tis_list_limit)
   uint64_t step_host = 0;                // the device step counter (stepbase) as the host knows it
   // one block of pinned host memory that kernels read and write themselves:
   // a report of two words (k_run_report, k_state_out), a ring that calls'
@@ -1212,6 +1214,8 @@ int build_tables(tis_ctx *c) {
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.sbox, 4 * nbt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.ttop, 2 * nbt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->d_epart, (size_t)c->n_etask * kEnergyTerms, &c->tab_bytes))) return rc;
+  if ((rc = dalloc_in(c, c->tab_allocs, &c->P.win_back, wsys.empty() ? 1 : 9 * (size_t)c->P.ntot, &c->tab_bytes)))
+    return rc;
   c->dev_bytes += c->tab_bytes;
   for (int k = 0; k < 2; ++k)
     if (c->graph[k]) { (void)hipGraphExecDestroy(c->graph[k]); c->graph[k] = nullptr; }
@@ -1569,18 +1573,35 @@ int32_t tis_state_get(tis_ctx *c, int32_t isys, int32_t which, double *buf) {
   return TIS_OK;
 }
 
-// larger list capacity for `need` entries (nb keeps its stride); captured
-// graphs hold the old one
-static int new_nb(tis_ctx *c, unsigned long long need) {
-  const int newcap = (int)(need + need / 2 + 16);
+// Larger per-bead list capacity for lists of `need` entries, no larger than
+// the caller's limit (tis_list_limit); with keep, the entries built so far stay
+// (the layout nb[slot][ntot] keeps its stride), so systems whose lists are not
+// rebuilt keep theirs.  Captured graphs hold the old capacity: dropped.
+static int grow_nb(tis_ctx *c, unsigned long long need, bool keep) {
+  int newcap = (int)(need + need / 2 + 16);
+  if (c->nb_limit > 0) newcap = std::min(newcap, c->nb_limit);
+  if ((unsigned long long)newcap < need)
+    return fail(c, TIS_ERR_NOMEM, "a list of %llu entries exceeds the limit of %d", need, c->nb_limit);
+  if (newcap <= c->P.nb_cap) return TIS_OK;
   uint32_t *nb = nullptr;
   int rc = dalloc(c, &nb, (size_t)newcap * c->P.ntot);
   if (rc) return rc;
+  if (keep)
+    HIPCHK(c, hipMemcpyAsync(nb, c->P.nb, sizeof(uint32_t) * (size_t)c->P.nb_cap * c->P.ntot, hipMemcpyDeviceToDevice,
+                             c->stream));
   c->P.nb = nb;  // the old buffer stays in allocs until the batch is freed
   c->P.nb_cap = newcap;
   for (int k = 0; k < 2; ++k)
     if (c->graph[k]) { (void)hipGraphExecDestroy(c->graph[k]); c->graph[k] = nullptr; }
   return TIS_OK;
+}
+
+// A list build that failed: what it left is no list, for force calls or for
+// the steps of a run under way.
+static int lists_lost(tis_ctx *c, int rc) {
+  c->lists_valid = false;
+  c->lv_init = false;
+  return rc;
 }
 
 // The lists of the range, built again with a larger capacity as long as they
@@ -1595,10 +1616,9 @@ static int rebuild_lists(tis_ctx *c, int32_t isys) {
     const unsigned long long ovf = c->report[0];
     if (ovf == 0) { c->lists_valid = true; c->rebuilds_host += 1; return 0; }
     HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
-    int rc = new_nb(c, ovf);
-    if (rc) return rc;
+    if (int rc = grow_nb(c, ovf, false)) return lists_lost(c, rc);
   }
-  return fail(c, TIS_ERR_OVERFLOW, "neighbour list capacity could not be grown");
+  return lists_lost(c, fail(c, TIS_ERR_OVERFLOW, "neighbour list capacity could not be grown"));
 }
 
 int32_t tis_neighbor(tis_ctx *c, int32_t isys) {
@@ -1778,7 +1798,7 @@ int32_t tis_force_sumup(tis_ctx *c, int32_t isys, double *force_out) {
     const unsigned long long ovf = c->report[0];
     if (ovf == 0) { c->lists_valid = true; c->rebuilds_host += 1; break; }
     HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
-    if ((rc = new_nb(c, ovf))) return rc;
+    if ((rc = grow_nb(c, ovf, false))) return lists_lost(c, rc);
     if ((rc = rebuild_lists(c, -1))) return rc;
   }
   if (want) {
@@ -2231,24 +2251,6 @@ static int run_steps(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch)
   return TIS_OK;
 }
 
-// Larger per-bead list capacity; the entries built so far are kept (the
-// layout nb[slot][ntot] keeps its stride), so systems whose lists are not
-// rebuilt keep theirs.  Captured graphs hold the old capacity: dropped.
-static int grow_nb(tis_ctx *c, unsigned long long need) {
-  const int newcap = (int)(need + need / 2 + 16);
-  if (newcap <= c->P.nb_cap) return TIS_OK;
-  uint32_t *nb = nullptr;
-  int rc = dalloc(c, &nb, (size_t)newcap * c->P.ntot);
-  if (rc) return rc;
-  HIPCHK(c, hipMemcpyAsync(nb, c->P.nb, sizeof(uint32_t) * (size_t)c->P.nb_cap * c->P.ntot, hipMemcpyDeviceToDevice,
-                           c->stream));
-  c->P.nb = nb;  // the old buffer stays in allocs until the batch is freed
-  c->P.nb_cap = newcap;
-  for (int k = 0; k < 2; ++k)
-    if (c->graph[k]) { (void)hipGraphExecDestroy(c->graph[k]); c->graph[k] = nullptr; }
-  return TIS_OK;
-}
-
 // ---------------------------------------------------------------- launch-shape tuner
 // The force pass of the whole batch at the current coordinates (mode 0:
 // forces only, no state changes) under each candidate launch shape: after
@@ -2383,6 +2385,77 @@ int32_t tis_list_capacity(tis_ctx *c, int32_t cap, int32_t *cap_out) {
   return TIS_OK;
 }
 
+// A run that cannot go on for an error of the device or a launch: no flag or
+// count of it stays for the next call, which has to set the run up again.
+static int run_lost(tis_ctx *c, int rc) {
+  (void)hipStreamSynchronize(c->stream);
+  (void)hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, 2 * sizeof(unsigned long long), c->stream);
+  return lists_lost(c, rc);
+}
+
+// nsteps in the given mode, resumed with a larger list capacity each time a
+// rebuild overflows it.
+static int run_resumed(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch) {
+  const auto check = [&](hipError_t e, const char *what) {
+    return e == hipSuccess ? 0 : run_lost(c, fail(c, TIS_ERR_HIP, "%s failed: %s", what, hipGetErrorString(e)));
+  };
+  for (int attempt = 0;; ++attempt) {
+    const int cur0 = c->cur;
+    const int64_t t0 = c->t_since_init;
+    const uint64_t step0 = c->step_host;
+    int rc = run_steps(c, nsteps, mode, nlaunch);
+    if (rc) return run_lost(c, rc);
+    hipLaunchKernelGGL(k_run_report, dim3(1), dim3(1), 0, c->stream, c->d_counters, c->report);
+    if ((rc = check(hipGetLastError(), "a launch of the run"))) return rc;
+    if ((rc = check(hipEventRecord(c->ev1, c->stream), "hipEventRecord"))) return rc;
+    if ((rc = check(hipStreamSynchronize(c->stream), "the run"))) return rc;
+    const unsigned long long st[2] = {c->report[0], c->report[1]};  // overflow need, steps completed
+    if (st[0] == 0ull) {
+      c->step_host = step0 + (uint64_t)nsteps;
+      if (nsteps > 0) c->lists_valid = true;   // (not so between a growth that failed and the rebuild made up for)
+      return TIS_OK;
+    }
+    // a rebuild overflowed the list capacity: the run stopped at the start
+    // of the step after the st[1] completed ones; grow the capacity, put the
+    // step counters there (also when it cannot grow) and resume
+    const int64_t completed = (int64_t)st[1];
+    c->cur = cur0 ^ (int)(completed & 1);
+    c->t_since_init = t0 + completed;
+    c->step_host = step0 + (uint64_t)completed;
+    const int grown = attempt < 8 ? grow_nb(c, st[0], true)
+                                  : fail(c, TIS_ERR_OVERFLOW, "neighbour list capacity could not be grown");
+    unsigned long long cnt[TIS_CNT_MAX];
+    uint64_t sb = 0;
+    if ((rc = check(hipMemcpy(cnt, c->d_counters, sizeof(cnt), hipMemcpyDeviceToHost), "hipMemcpy"))) return rc;
+    if ((rc = check(hipMemcpy(&sb, c->d_stepbase, sizeof(sb), hipMemcpyDeviceToHost), "hipMemcpy"))) return rc;
+    cnt[TIS_CNT_STEPS] += c->step_host - sb;
+    cnt[TIS_CNT_NB_OVERFLOW] = 0ull;
+    cnt[TIS_CNT_NB_OVERFLOW + 1] = 0ull;
+    if (grown == 0) cnt[TIS_CNT_RESUMES] += 1ull;
+    sb = c->step_host;
+    if ((rc = check(hipMemcpy(c->d_counters, cnt, sizeof(cnt), hipMemcpyHostToDevice), "hipMemcpy"))) return rc;
+    if ((rc = check(hipMemcpy(c->d_stepbase, &sb, sizeof(sb), hipMemcpyHostToDevice), "hipMemcpy"))) return rc;
+    if (grown) {
+      // per-step launches stand at that step as they would to resume; windows
+      // may have run ahead of it and go back
+      c->lists_valid = false;
+      if (mode == TIS_MODE_GRAPH && c->win_lds > 0) {
+        c->lv_init = false;
+        hipLaunchKernelGGL(k_window_back, dim3(c->nlive), dim3(kWinThreads), 0, c->stream, c->P, c->d_wsys, c->cur);
+        if ((rc = check(hipStreamSynchronize(c->stream), "k_window_back"))) return rc;
+      }
+      return grown;
+    }
+    nsteps -= completed;
+  }
+}
+
+int32_t tis_list_limit(tis_ctx *c, int32_t cap) {
+  if (!c) return TIS_ERR_ARG;
+  c->nb_limit = std::max(cap, 0);
+  return TIS_OK;
+}
+
 int32_t tis_langevin_steps(tis_ctx *c, int64_t nsteps, int32_t mode) {
   if (!c || nsteps < 0) return TIS_ERR_ARG;
   if (!c->lv_init) return fail(c, TIS_ERR_STATE, "tis_langevin_init not called");
@@ -2390,48 +2463,8 @@ int32_t tis_langevin_steps(tis_ctx *c, int64_t nsteps, int32_t mode) {
     return fail(c, TIS_ERR_ARG, "unknown mode %d", mode);
   HIPCHK(c, hipSetDevice(c->device));
   HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-  int64_t nlaunch = 0, remaining = nsteps;
-  for (int attempt = 0;; ++attempt) {
-    const int cur0 = c->cur;
-    const int64_t t0 = c->t_since_init;
-    const uint64_t step0 = c->step_host;
-    int rc = run_steps(c, remaining, mode, &nlaunch);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_run_report, dim3(1), dim3(1), 0, c->stream, c->d_counters, c->report);
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    const unsigned long long st[2] = {c->report[0], c->report[1]};  // overflow need, steps completed
-    if (st[0] == 0ull) {
-      c->step_host = step0 + (uint64_t)remaining;
-      break;
-    }
-    // a rebuild overflowed the list capacity: the run stopped at the start
-    // of the step after the st[1] completed ones; put the step counters
-    // there, grow the capacity and resume
-    if (attempt >= 8) {
-      (void)hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, 2 * sizeof(unsigned long long), c->stream);
-      return fail(c, TIS_ERR_OVERFLOW, "neighbour list capacity could not be grown");
-    }
-    const int64_t completed = (int64_t)st[1];
-    c->cur = cur0 ^ (int)(completed & 1);
-    c->t_since_init = t0 + completed;
-    c->step_host = step0 + (uint64_t)completed;
-    unsigned long long cnt[TIS_CNT_MAX];
-    uint64_t sb = 0;
-    HIPCHK(c, hipMemcpy(cnt, c->d_counters, sizeof(cnt), hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(&sb, c->d_stepbase, sizeof(sb), hipMemcpyDeviceToHost));
-    cnt[TIS_CNT_STEPS] += c->step_host - sb;
-    cnt[TIS_CNT_NB_OVERFLOW] = 0ull;
-    cnt[TIS_CNT_NB_OVERFLOW + 1] = 0ull;
-    cnt[TIS_CNT_RESUMES] += 1ull;
-    sb = c->step_host;
-    rc = grow_nb(c, st[0]);
-    if (rc) return rc;
-    HIPCHK(c, hipMemcpy(c->d_counters, cnt, sizeof(cnt), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_stepbase, &sb, sizeof(sb), hipMemcpyHostToDevice));
-    remaining -= completed;
-  }
+  int64_t nlaunch = 0;
+  if (int rc = run_resumed(c, nsteps, mode, &nlaunch)) { c->timing = false; return rc; }
   float ms = 0.0f;
   (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
   c->last_total_ms = ms;

@@ -2495,6 +2495,13 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
       xc[d] = XC[(size_t)d * N + g]; v[d] = P.v[(size_t)d * N + g]; a[d] = P.a[(size_t)d * N + g];
       if (dyn) { ds[d] = P.dxyz[(size_t)d * N + g]; dl[d] = P.dlast[(size_t)d * N + g]; }
     }
+    // for k_window_back
+    if (own && from == 0)
+      for (int d = 0; d < 3; ++d) {
+        P.win_back[(size_t)d * N + g] = xc[d];
+        P.win_back[(size_t)(3 + d) * N + g] = v[d];
+        P.win_back[(size_t)(6 + d) * N + g] = a[d];
+      }
   }
   const int ib0 = P.inc_off[s.off];
   if (own) {
@@ -2974,6 +2981,21 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
     if (ndel) atomicAdd(&P.counters[2], (unsigned long long)ndel);
     if (nfire) atomicAdd(&P.counters[3], (unsigned long long)nfire);
   }
+}
+
+// The systems that a k_window launch has left ahead of *stepbase put back to
+// it (positions into buffer cu), for a run that cannot be resumed.
+__global__ __launch_bounds__(kWinThreads) void k_window_back(DevPtrs P, const int32_t *wsys, int cu) {
+  const int isys = wsys[blockIdx.x], i = (int)threadIdx.x, N = P.ntot;
+  const DSys &s = P.sys[isys];
+  if ((P.win_at[isys] >> 1) <= *P.stepbase || i >= s.nmp) return;
+  const int g = s.off + i;
+  for (int d = 0; d < 3; ++d) {
+    P.x[cu][(size_t)d * N + g] = P.win_back[(size_t)d * N + g];
+    P.v[(size_t)d * N + g] = P.win_back[(size_t)(3 + d) * N + g];
+    P.a[(size_t)d * N + g] = P.win_back[(size_t)(6 + d) * N + g];
+  }
+  P.xf[cu][g] = near_pos(P.win_back[g], P.win_back[(size_t)N + g], P.win_back[2 * (size_t)N + g], P.species[g]);
 }
 
 // st_status of the consecutive stacks [s0, s0 + ns) at the given

@@ -54,6 +54,7 @@ def load_library():
     L.tis_system_validate.argtypes = [C.c_int32, C.POINTER(CSystem), C.c_char_p, C.c_int64]
     L.tis_set_system_T.argtypes = [vp, C.c_int32, C.POINTER(CSystem)]
     L.tis_list_capacity.argtypes = [vp, C.c_int32, C.POINTER(C.c_int32)]
+    L.tis_list_limit.argtypes = [vp, C.c_int32]
     L.tis_term_status.argtypes = [vp, C.c_int32, _i32p, _i32p]
     L.tis_transfer_bytes.argtypes = [vp, C.POINTER(C.c_int64)]
     L.tis_system_append.argtypes = [vp, C.c_int32, C.POINTER(CSystem), C.POINTER(C.c_uint32), _i32p]
@@ -81,7 +82,7 @@ def load_library():
     L.tis_last_timing.argtypes = [vp, _f64p, _f64p, _f64p, C.POINTER(C.c_int64)]
     L.tis_last_force_ms.argtypes = [vp, _f64p]
     for fn in ("tis_ctx_create", "tis_ctx_destroy", "tis_system_upload", "tis_system_validate", "tis_set_system_T",
-               "tis_list_capacity", "tis_term_status", "tis_transfer_bytes", "tis_system_append",
+               "tis_list_capacity", "tis_list_limit", "tis_term_status", "tis_transfer_bytes", "tis_system_append",
                "tis_system_retire", "tis_arena_stats", "tis_tune", "tis_launch_shape",
                "tis_state_set",
                "tis_state_get", "tis_neighbor", "tis_pairs_get", "tis_force_sumup", "tis_force_get",
@@ -334,6 +335,10 @@ class Engine:
         out = C.c_int32()
         self._chk(self.L.tis_list_capacity(self.ctx, int(cap), C.byref(out)), "tis_list_capacity")
         return out.value
+
+    def list_limit(self, cap: int = 0):
+        """Largest capacity list builds may grow to, 0: any (tis_list_limit)."""
+        self._chk(self.L.tis_list_limit(self.ctx, int(cap)), "tis_list_limit")
 
     def last_timing(self):
         t, m, p = C.c_double(), C.c_double(), C.c_double()

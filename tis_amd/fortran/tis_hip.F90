@@ -63,7 +63,7 @@ module tis_hip
   end type tis_bd_system_c
 
   public :: tis_ctx_create, tis_ctx_destroy, tis_last_error, tis_system_upload, tis_system_validate, &
-       tis_set_system_T, tis_list_capacity, tis_term_status, tis_transfer_bytes, &
+       tis_set_system_T, tis_list_capacity, tis_list_limit, tis_term_status, tis_transfer_bytes, &
        tis_system_append, tis_system_retire, tis_arena_stats, tis_tune, tis_launch_shape, &
        tis_state_set, tis_state_get, tis_neighbor, tis_pairs_get, tis_force_sumup, tis_force_get, &
        tis_energy_sumup, tis_energy_sumup_set, tis_energy_unit, tis_langevin_init, tis_langevin_steps, tis_system_origin, tis_device_bytes, &
@@ -147,6 +147,11 @@ module tis_hip
        type(c_ptr), value :: ctx
        integer(c_int32_t), value :: cap
        integer(c_int32_t), intent(out) :: cap_out
+     end function
+     integer(c_int32_t) function tis_list_limit(ctx, cap) bind(C, name="tis_list_limit")
+       import :: c_int32_t, c_ptr
+       type(c_ptr), value :: ctx
+       integer(c_int32_t), value :: cap
      end function
      integer(c_int32_t) function tis_set_system_T(ctx, isys, sys) bind(C, name="tis_set_system_T")
        import :: c_int32_t, c_ptr, tis_system_c
