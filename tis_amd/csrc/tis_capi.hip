@@ -17,6 +17,7 @@
 
 #include "../../include/tis_hip.h"
 #include "tis_dev.h"
+#include "tis_host.h"
 #include "tis_internal.h"
 
 namespace tis {
@@ -197,13 +198,7 @@ struct tis_ctx {
   int64_t t_since_init = 0;
   int32_t nb_limit = 0;                  // largest list capacity calls may grow to; 0: any (tis_list_limit)
   uint64_t step_host = 0;                // the device step counter (stepbase) as the host knows it
-  // one block of pinned host memory that kernels read and write themselves:
-  // a report of two words (k_run_report, k_state_out), a ring that calls'
-  // inputs are copied into (the stream is waited for when it comes round),
-  // and the outputs of a call that waits for them
-  char *pin = nullptr, *pin_in = nullptr, *pin_out = nullptr;
-  size_t pin_in_cap = 0, pin_in_at = 0, pin_out_cap = 0;
-  unsigned long long *report = nullptr;
+  PinBlock pin;                          // see tis_host.h; reserved before a batch is uploaded
   int64_t rebuilds_host = 0;             // whole-batch rebuilds counted by the host (TIS_CNT_REBUILDS)
   // payload bytes since creation: uploads of topology and launch tables,
   // state uploads (tis_state_set), state downloads (tis_state_get), state
@@ -263,29 +258,19 @@ int fail(tis_ctx *c, int code, const char *fmt, ...) {
   } while (0)
 
 // The pinned block with at least `in` bytes of ring and `out` bytes of output
-// (64 KB in all if that is enough: larger blocks cost hundreds of
-// microseconds, which is why a batch's is laid out at its upload).
+// (blocks above 64 KB cost hundreds of microseconds, which is why a batch's is
+// laid out at its upload).
 int pin_reserve(tis_ctx *c, size_t in, size_t out) {
-  if (c->pin && in <= c->pin_in_cap && out <= c->pin_out_cap) return 0;
-  constexpr size_t kHead = 256, kSmall = 64 << 10;
-  in = std::max((in + 255) & ~(size_t)255, c->pin_in_cap);
-  out = std::max((out + 255) & ~(size_t)255, c->pin_out_cap);
-  if (kHead + in + out < kSmall) in = kSmall - kHead - out;
+  if (c->pin.holds(in, out)) return 0;
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (c->pin) (void)hipHostFree(c->pin);
-  c->pin = nullptr;
-  c->pin_in_cap = c->pin_in_at = c->pin_out_cap = 0;
-  const hipError_t e = hipHostMalloc((void **)&c->pin, kHead + in + out);
-  if (e != hipSuccess) {
-    c->pin = nullptr;
-    return fail(c, TIS_ERR_NOMEM, "hipHostMalloc(%zu) failed: %s", kHead + in + out, hipGetErrorString(e));
-  }
-  c->report = (unsigned long long *)c->pin;
-  c->pin_in = c->pin + kHead;
-  c->pin_out = c->pin_in + in;
-  c->pin_in_cap = in;
-  c->pin_out_cap = out;
-  c->report[0] = c->report[1] = 0;
+  const auto alloc = [](size_t n) -> void * {
+    void *p = nullptr;
+    if (hipHostMalloc(&p, n) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  };
+  const size_t failed = c->pin.grow(in, out, alloc, [](void *p) { (void)hipHostFree(p); });
+  if (failed) return fail(c, TIS_ERR_NOMEM, "no %zu bytes of pinned host memory", failed);
   return 0;
 }
 
@@ -294,12 +279,12 @@ int pin_reserve(tis_ctx *c, size_t in, size_t out) {
 int pin_input(tis_ctx *c, size_t bytes, void **p) {
   bytes = (bytes + 255) & ~(size_t)255;
   if (int rc = pin_reserve(c, bytes, 0)) return rc;
-  if (c->pin_in_at + bytes > c->pin_in_cap) {
+  if (c->pin.in_at + bytes > c->pin.in_cap) {
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    c->pin_in_at = 0;
+    c->pin.in_at = 0;
   }
-  *p = c->pin_in + c->pin_in_at;
-  c->pin_in_at += bytes;
+  *p = c->pin.in() + c->pin.in_at;
+  c->pin.in_at += bytes;
   return 0;
 }
 
@@ -307,7 +292,7 @@ int pin_input(tis_ctx *c, size_t bytes, void **p) {
 // before it reads them (taken before the call's inputs: growth moves both)
 int pin_output(tis_ctx *c, size_t bytes, void **p) {
   if (int rc = pin_reserve(c, 0, bytes)) return rc;
-  *p = c->pin_out;
+  *p = c->pin.out();
   return 0;
 }
 
@@ -1331,6 +1316,13 @@ int append_systems(tis_ctx *c, int32_t nadd, const tis_system *sys, const uint32
   for (int k = 0; k < nadd; ++k)
     if (int rc = validate_system(&c->err, c->nsys + k, sys[k])) return rc;
   HIPCHK(c, hipSetDevice(c->device));
+  // the pinned block of the calls to come, before anything changes
+  int32_t most = 0;
+  for (const HostSys &h : c->hs)
+    if (h.live) most = std::max(most, h.d.nmp);
+  for (int k = 0; k < nadd; ++k) most = std::max(most, sys[k].nmp);
+  const size_t one = 3 * sizeof(double) * (size_t)most;
+  if (int rc = pin_reserve(c, one, std::max(one, 25 * sizeof(double) * (size_t)(c->nsys + nadd)))) return rc;
   // fits as it is?
   bool fits = false;
   {
@@ -1365,11 +1357,6 @@ int append_systems(tis_ctx *c, int32_t nadd, const tis_system *sys, const uint32
   }
   int rc = upload_stage(c, c->stage, m);
   if (rc) return rc;
-  int32_t most = 0;
-  for (const HostSys &h : c->hs)
-    if (h.live) most = std::max(most, h.d.nmp);
-  const size_t one = 3 * sizeof(double) * (size_t)most;
-  if ((rc = pin_reserve(c, one, std::max(one, 25 * sizeof(double) * (size_t)c->nsys)))) return rc;
   c->nbeads = c->stage.nbead; c->nqtot = c->stage.nq; c->nhbtot = c->stage.nhb; c->ntsttot = c->stage.ntst;
   c->nsttot = c->stage.nst;
   return build_tables(c);
@@ -1417,7 +1404,7 @@ int32_t tis_ctx_destroy(tis_ctx *c) {
   free_all(c);
   bd_free(c);
   for (void *p : c->label_bufs) (void)hipFree(p);
-  if (c->pin) (void)hipHostFree(c->pin);
+  if (c->pin.base) (void)hipHostFree(c->pin.base);
   for (hipEvent_t e : c->tev) (void)hipEventDestroy(e);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
@@ -1546,11 +1533,11 @@ int32_t tis_state_set(tis_ctx *c, int32_t isys, int32_t which, const double *buf
 }
 
 // `n` beads of base at off into the pinned buffer out (n = 0: none), and the
-// overflow flag to c->report when asked
+// overflow flag to the report when asked
 static void launch_state_out(tis_ctx *c, const double *base, int off, int n, void *out, bool report) {
   hipLaunchKernelGGL(k_state_out, dim3((3 * n + 255) / 256 + (n == 0 ? 1 : 0)), dim3(256), 0, c->stream, base,
                      c->P.ntot, off, n, (double *)out, (const unsigned long long *)c->d_counters,
-                     report ? c->report : nullptr);
+                     report ? c->pin.report() : nullptr);
 }
 
 int32_t tis_state_get(tis_ctx *c, int32_t isys, int32_t which, double *buf) {
@@ -1613,7 +1600,7 @@ static int rebuild_lists(tis_ctx *c, int32_t isys) {
     launch_state_out(c, nullptr, 0, 0, nullptr, true);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    const unsigned long long ovf = c->report[0];
+    const unsigned long long ovf = c->pin.report()[0];
     if (ovf == 0) { c->lists_valid = true; c->rebuilds_host += 1; return 0; }
     HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
     if (int rc = grow_nb(c, ovf, false)) return lists_lost(c, rc);
@@ -1795,7 +1782,7 @@ int32_t tis_force_sumup(tis_ctx *c, int32_t isys, double *force_out) {
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (!build) break;
-    const unsigned long long ovf = c->report[0];
+    const unsigned long long ovf = c->pin.report()[0];
     if (ovf == 0) { c->lists_valid = true; c->rebuilds_host += 1; break; }
     HIPCHK(c, hipMemsetAsync(c->d_counters + TIS_CNT_NB_OVERFLOW, 0, sizeof(unsigned long long), c->stream));
     if ((rc = grow_nb(c, ovf, false))) return lists_lost(c, rc);
@@ -2405,11 +2392,11 @@ static int run_resumed(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunc
     const uint64_t step0 = c->step_host;
     int rc = run_steps(c, nsteps, mode, nlaunch);
     if (rc) return run_lost(c, rc);
-    hipLaunchKernelGGL(k_run_report, dim3(1), dim3(1), 0, c->stream, c->d_counters, c->report);
+    hipLaunchKernelGGL(k_run_report, dim3(1), dim3(1), 0, c->stream, c->d_counters, c->pin.report());
     if ((rc = check(hipGetLastError(), "a launch of the run"))) return rc;
     if ((rc = check(hipEventRecord(c->ev1, c->stream), "hipEventRecord"))) return rc;
     if ((rc = check(hipStreamSynchronize(c->stream), "the run"))) return rc;
-    const unsigned long long st[2] = {c->report[0], c->report[1]};  // overflow need, steps completed
+    const unsigned long long st[2] = {c->pin.report()[0], c->pin.report()[1]};  // overflow need, steps completed
     if (st[0] == 0ull) {
       c->step_host = step0 + (uint64_t)nsteps;
       if (nsteps > 0) c->lists_valid = true;   // (not so between a growth that failed and the rebuild made up for)
