@@ -63,7 +63,7 @@ def test_per_step_run_goes_on(mode, rebuild):
 
 @pytest.mark.parametrize("rebuild", [10, 7, 0])
 def test_window_run_starts_again(rebuild):
-    sizes = (40, 64, 107, 120)
+    sizes = (40, 58, 50, 64)
     print(f"[failed growth] windows rebuild {rebuild}", flush=True)
     eng, ref = _engine(sizes, rebuild), _engine(sizes, rebuild)
     done = 0

@@ -52,3 +52,35 @@ def test_pinned_block_survives_a_failed_growth(tmp_path):
   std::memset(b.base, 3, PinBlock::kHead + b.in_cap + b.out_cap);
   put(b.base);
 """)
+
+
+def test_window_rule_takes_the_faster_side(tmp_path):
+    """Both sides measured (us a step, k_window and per-step launches) for
+    batches of equal chains; where they differ by more than a tenth, the rule
+    takes the faster one.  Mixed batches lie between."""
+    # beads, chunk pairs, systems, k_window, per-step launches
+    rows = [(95, 1, 1, 9.1, 13.1), (95, 1, 256, 9.4, 17.5), (95, 1, 512, 18.4, 23.1), (95, 1, 513, 27.2, 23.7),
+            (95, 1, 1024, 36.5, 30.8), (95, 1, 1536, 54.7, 40.3), (95, 1, 2048, 73.0, 49.1),
+            (95, 1, 4096, 145.6, 85.9),
+            (128, 1, 1, 9.3, 13.1), (128, 1, 512, 19.2, 24.1), (128, 1, 1024, 38.0, 32.5), (128, 1, 2048, 75.6, 53.8),
+            (191, 1, 1, 10.1, 13.2), (191, 1, 256, 10.7, 22.6), (191, 1, 512, 20.5, 28.5), (191, 1, 768, 30.7, 36.2),
+            (191, 1, 2048, 81.4, 72.6),
+            (254, 3, 256, 15.2, 26.8), (254, 3, 512, 30.1, 35.0), (254, 3, 513, 44.6, 37.2),
+            (320, 3, 256, 17.4, 28.7), (320, 3, 512, 33.8, 41.1), (320, 3, 2048, 134.4, 148.3),
+            (386, 3, 1, 20.4, 16.0), (386, 3, 256, 21.6, 31.0), (386, 3, 2048, 165.4, 184.2)]
+    body = "std::vector<WindowLoad> b;\n"
+    for beads, pairs, n, win, step in rows:
+        assert abs(win - step) > 0.09 * min(win, step)
+        body += f"b.assign({n}, WindowLoad{{{beads}, {pairs}}}); CHECK(window_pays(b, false, false) == {int(win < step)});\n"
+    body += """
+  for (int n : {1, 300, 5000}) { b.assign(n, WindowLoad{119, 1}); CHECK(window_pays(b, true, false)); }
+  // one long chain holds no batch of short ones back, nor 255 short ones a long one
+  b.assign(255, WindowLoad{95, 1});
+  b.insert(b.begin(), WindowLoad{320, 3});
+  CHECK(window_pays(b, false, false));
+  // 128 chains of up to 389 beads (24 / 20 us; 21 / 27 under the trigger)
+  b.assign(127, WindowLoad{190, 1});
+  b.insert(b.begin(), WindowLoad{389, 6});
+  CHECK(!window_pays(b, false, false) && window_pays(b, false, true));
+"""
+    _run(tmp_path, body)

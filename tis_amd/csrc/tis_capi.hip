@@ -174,6 +174,7 @@ struct tis_ctx {
   int32_t nhbdense = 0;
   int32_t *d_wsys = nullptr;             // live systems, largest first, when k_window takes the batch
   int32_t win_rows = 0, win_lds = 0;     // its list rows and bytes in LDS; win_lds 0: per-step passes
+  bool win_pays[2] = {false, false};     // taken with a fixed rebuild interval, with the displacement trigger
   std::vector<int32_t> systask_of;       // index into d_systask per system or -1
   int32_t *d_ststat = nullptr;           // st_status output of tis_term_status [nsttot]
   EwTask *d_etask = nullptr;             // energy tasks (system, part, parts) in live order
@@ -1053,13 +1054,10 @@ bool window_fits(const DSys &d) {
          d.nsite < 0xFFFF;
 }
 
-// Batched runs take k_window when every live system fits it and is small (see
-// kWindowBeads).  *wsys gets the systems, the largest first (blocks start in
-// order).
-// Measured, us a step with a rebuild every 10 (per-step passes / k_window), 1
-// system and 512: 95 beads 13.0 / 9.0 and 24 / 18; 254 beads 15.8 / 14.8 and
-// 35 / 30; 446 beads 16.4 and 56 either way.
-constexpr int kWindowBeads = 448;
+// Batched runs take k_window when every live system fits it and the batch is
+// faster by it (window_pays, for fixed rebuild intervals and for the trigger).  *wsys gets the systems, the largest first (blocks
+// start in order).
+constexpr int kWindowBeads = 448;   // (with more, the arrays seldom fit the LDS and one system is slower by it)
 constexpr int kWindowSteps = 500;   // steps per k_window launch (a few ms)
 
 void choose_window(tis_ctx *c, std::vector<int32_t> &wsys) {
@@ -1077,6 +1075,16 @@ void choose_window(tis_ctx *c, std::vector<int32_t> &wsys) {
   }
   if (wsys.empty()) return;
   std::stable_sort(wsys.begin(), wsys.end(), [&](int a, int b) { return c->hs[a].d.nmp > c->hs[b].d.nmp; });
+  std::vector<WindowLoad> load;
+  bool valence = false;
+  for (int is : wsys) {
+    const DSys &d = c->hs[is].d;
+    const int nqt = d.ele_form != TIS_ELE_NONE ? d.nqt : 0;
+    load.push_back(WindowLoad{d.nmp, nqt * (nqt + 1) / 2});
+    valence = valence || d.hb_excess_possible;
+  }
+  for (int trigger = 0; trigger < 2; ++trigger) c->win_pays[trigger] = window_pays(load, valence, trigger != 0);
+  if (!c->win_pays[0] && !c->win_pays[1]) { wsys.clear(); return; }
   int bytes = 0;
   for (int is : wsys) bytes = std::max(bytes, win_layout(c->hs[is].d, rows).total);
   if (hipFuncSetAttribute((const void *)k_window, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
@@ -2176,12 +2184,16 @@ static int capture_graph(tis_ctx *c, int parity) {
   return 0;
 }
 
+static bool takes_window(const tis_ctx *c, int32_t mode) {
+  return mode == TIS_MODE_GRAPH && c->win_lds > 0 && c->win_pays[c->P.dyn ? 1 : 0];
+}
+
 // The steps of one run in the given mode; a stop (list overflow) makes the
 // remaining launches return at once.
 static int run_steps(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch) {
   int64_t done = 0;
   const int L = steps_per_graph(c);
-  if (mode == TIS_MODE_GRAPH && c->win_lds > 0) {
+  if (takes_window(c, mode)) {
     // every system small: launches of up to kWindowSteps steps
     while (done < nsteps) {
       const int n = (int)std::min<int64_t>(nsteps - done, kWindowSteps);
@@ -2426,7 +2438,7 @@ static int run_resumed(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunc
       // per-step launches stand at that step as they would to resume; windows
       // may have run ahead of it and go back
       c->lists_valid = false;
-      if (mode == TIS_MODE_GRAPH && c->win_lds > 0) {
+      if (takes_window(c, mode)) {
         c->lv_init = false;
         hipLaunchKernelGGL(k_window_back, dim3(c->nlive), dim3(kWinThreads), 0, c->stream, c->P, c->d_wsys, c->cur);
         if ((rc = check(hipStreamSynchronize(c->stream), "k_window_back"))) return rc;
