@@ -1062,7 +1062,7 @@ constexpr int kWindowSteps = 500;   // steps per k_window launch (a few ms)
 
 void choose_window(tis_ctx *c, std::vector<int32_t> &wsys) {
   c->win_rows = c->win_lds = 0;
-  const int room = kLdsBytes - 256;
+  const int room = kLdsBytes - 256;   // (k_window's static part: under 256 bytes)
   int rows = kWinRows;
   for (int is = 0; is < c->nsys; ++is) {
     const HostSys &h = c->hs[is];
@@ -1087,7 +1087,9 @@ void choose_window(tis_ctx *c, std::vector<int32_t> &wsys) {
   if (!c->win_pays[0] && !c->win_pays[1]) { wsys.clear(); return; }
   int bytes = 0;
   for (int is : wsys) bytes = std::max(bytes, win_layout(c->hs[is].d, rows).total);
-  if (hipFuncSetAttribute((const void *)k_window, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+  // (the limit is the kernel's, for every context of the process: the same
+  // value whoever sets it)
+  if (hipFuncSetAttribute((const void *)k_window, hipFuncAttributeMaxDynamicSharedMemorySize, room) != hipSuccess) {
     (void)hipGetLastError();
     wsys.clear();
     return;
