@@ -1900,7 +1900,11 @@ int32_t tis_energy_unit(tis_ctx *c, int32_t isys, int32_t style, double *energy_
   const size_t nn = (size_t)nu * nu;
   if (nu < 1 || nn > 65535) return fail(c, TIS_ERR_ARG, "system %d has %d units", isys, nu);
   const HostSys &h = c->hs[isys];
-  const size_t nraw = nn * (25 + (size_t)kEnergyTerms * h.et_count);
+  // parts of each unit pair: the system's where there are few pairs, otherwise
+  // no more than fill the chip (250 units of 35 beads: 376 ms and 2.1 GB by the
+  // system's 120 parts, 90 ms and 17 MB by one)
+  const size_t parts = std::min<size_t>((size_t)h.et_count, std::max<size_t>(1, kEnergyUnitBlocks / nn));
+  const size_t nraw = nn * (25 + kEnergyTerms * parts);
   if (c->eunit_cap < nraw) {
     if (c->d_eunit) {
       (void)hipFree(c->d_eunit);
@@ -1912,10 +1916,10 @@ int32_t tis_energy_unit(tis_ctx *c, int32_t isys, int32_t style, double *energy_
     if (rc) return rc;
     c->eunit_cap = nraw;
   }
-  hipLaunchKernelGGL(k_energy, dim3(h.et_count, (unsigned)nn), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c),
+  hipLaunchKernelGGL(k_energy, dim3((unsigned)parts, (unsigned)nn), dim3(256), 0, c->stream, c->P, Xc(c), PXc(c),
                      c->d_etask, (const int32_t *)nullptr, h.et_begin, c->d_eunit + nn * 25, 1);
   hipLaunchKernelGGL(k_energy_sum, dim3(1, (unsigned)nn), dim3(kTile), 0, c->stream, c->d_efirst,
-                     (const int32_t *)nullptr, h.live_pos, c->d_eunit + nn * 25, c->d_eunit, 1);
+                     (const int32_t *)nullptr, h.live_pos, c->d_eunit + nn * 25, c->d_eunit, (int)parts);
   HIPCHK(c, hipGetLastError());
   std::vector<double> raw(nn * 25);
   HIPCHK(c, hipMemcpyAsync(raw.data(), c->d_eunit, raw.size() * sizeof(double), hipMemcpyDeviceToHost, c->stream));

@@ -96,6 +96,7 @@ constexpr int kEwThreads = 512;  // its threads
 // the call below against 116), per block, up to four blocks per CU.
 constexpr int kEnergyTerms = 9;
 constexpr int kEnergyPartsMax = 1024;
+constexpr size_t kEnergyUnitBlocks = 4096;   // of all unit pairs (tis_energy_unit)
 inline int energy_parts(int nmp, int nqt, int nk) {
   const int64_t pairs = (int64_t)nqt * (nqt + 1) / 2;
   int64_t p = (nmp + 255) / 256;

@@ -3121,18 +3121,20 @@ __device__ inline double ele_energy(const DevPtrs &P, const DSys &s, const doubl
 
 // One block per task (system, part of its nparts): task ids[blockIdx.x], or
 // t0 + blockIdx.x without ids; the sums of task k go to part[k].
-// unit_mode 1: block (x, y) sums only the terms whose unit pair, taken as
-// energy_sumup.F90's terms take it, is (y mod nunit, y / nunit): raw
-// energy_unit entries (the Ewald terms add none, as in
-// energy_ele_coulomb_ewld.F90:168-170); their sums go to part[y ntask + k - t0].
+// unit_mode 1: block (x, y) is part x of gridDim.x of the system of task t0
+// and sums only the terms whose unit pair, taken as energy_sumup.F90's terms
+// take it, is (y mod nunit, y / nunit): raw energy_unit entries (the Ewald
+// terms add none, as in energy_ele_coulomb_ewld.F90:168-170); their sums go to
+// part[y gridDim.x + x].
 __global__ __launch_bounds__(kEBlock) __attribute__((amdgpu_waves_per_eu(4))) void k_energy(DevPtrs P, const double *X, const double *PX,
                                                     const EwTask *tasks, const int32_t *ids, int t0, double *part,
                                                     int unit_mode) {
   __shared__ double red[kEBlock / kTile][kNE];
-  const int task = ids ? ids[blockIdx.x] : t0 + (int)blockIdx.x;
+  const int task = ids ? ids[blockIdx.x] : t0 + (unit_mode ? 0 : (int)blockIdx.x);
   const EwTask tk = tasks[task];
   const DSys s = P.sys[tk.sys];
-  const int t = tk.a * kEBlock + (int)threadIdx.x, nt = tk.b * kEBlock;   // this thread of the system's
+  const int tp = unit_mode ? (int)blockIdx.x : tk.a, np = unit_mode ? (int)gridDim.x : tk.b;
+  const int t = tp * kEBlock + (int)threadIdx.x, nt = np * kEBlock;   // this thread of the system's
   const int n = P.ntot;
   const int ua = unit_mode ? (int)blockIdx.y % s.nunit : 0, ub = unit_mode ? (int)blockIdx.y / s.nunit : 0;
   auto take = [&](int gi, int gj) { return !unit_mode || (P.unit[gi] == ua && P.unit[gj] == ub); };
@@ -3220,6 +3222,7 @@ __global__ __launch_bounds__(kEBlock) __attribute__((amdgpu_waves_per_eu(4))) vo
     const double a = s.exv_a;
     for (int li = t; li < s.nmp; li += nt) {
       const int g = s.off + li;
+      if (unit_mode && P.unit[g] != ua) continue;
       double xi[3];
       ld3(Y, n, g, xi);
       const int cnt = min(P.nb_cnt[g], P.nb_cap);
@@ -3287,13 +3290,14 @@ __global__ __launch_bounds__(kEBlock) __attribute__((amdgpu_waves_per_eu(4))) vo
 }
 
 // The parts of entry k (tasks [first[i], first[i + 1]) with i = pos[k], or k0
-// + k without pos; unit_mode: all parts of block row blockIdx.y) added in a
-// fixed order into the 25 E_TYPE slots of out[k]; TOTAL excludes VELO.
+// + k without pos; unit_parts > 0: the unit_parts parts of block row
+// blockIdx.y) added in a fixed order into the 25 E_TYPE slots of out[k]; TOTAL
+// excludes VELO.
 __global__ __launch_bounds__(kTile) void k_energy_sum(const int32_t *first, const int32_t *pos, int k0,
-                                                      const double *part, double *out, int unit_mode) {
+                                                      const double *part, double *out, int unit_parts) {
   const int i = pos ? pos[blockIdx.x] : k0 + (int)blockIdx.x, t = (int)threadIdx.x;
-  const int np = first[i + 1] - first[i];
-  const double *p = part + (unit_mode ? (size_t)blockIdx.y * np : (size_t)first[i]) * kNE;
+  const int np = unit_parts ? unit_parts : first[i + 1] - first[i];
+  const double *p = part + (unit_parts ? (size_t)blockIdx.y * np : (size_t)first[i]) * kNE;
   // lane l adds parts l, l + 64, ..; then the lanes' sums
   double tot[kNE];
 #pragma unroll
