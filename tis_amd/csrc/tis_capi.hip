@@ -1902,7 +1902,7 @@ int32_t tis_energy_unit(tis_ctx *c, int32_t isys, int32_t style, double *energy_
   const HostSys &h = c->hs[isys];
   // parts of each unit pair: the system's where there are few pairs, otherwise
   // no more than fill the chip (250 units of 35 beads: 376 ms and 2.1 GB by the
-  // system's 120 parts, 90 ms and 17 MB by one)
+  // system's 473 parts, 90 ms and 17 MB by one)
   const size_t parts = std::min<size_t>((size_t)h.et_count, std::max<size_t>(1, kEnergyUnitBlocks / nn));
   const size_t nraw = nn * (25 + kEnergyTerms * parts);
   if (c->eunit_cap < nraw) {
