@@ -3101,6 +3101,8 @@ __device__ inline double ele_energy(const DevPtrs &P, const DSys &s, const doubl
       if (unit_mode && __builtin_amdgcn_readlane(ui, r) != ua) continue;
       bool on = (row >> lane) & 1u;
       if (unit_mode) on = on && uj == ub;
+      // (every lane read stands before the branch: lane r may be off behind it)
+      const double cr = at_lane(ci, r);
       double v[3] = {xj[0] - at_lane(xi[0], r), xj[1] - at_lane(xi[1], r), xj[2] - at_lane(xi[2], r)};
       if (s.periodic) {
         const int c = on ? (int)P.qmirror[s.mioff + (int64_t)(I * kTile + r) * s.nq + qj] : 26;
@@ -3109,7 +3111,7 @@ __device__ inline double ele_energy(const DevPtrs &P, const DSys &s, const doubl
       const double d2 = dot3(v, v);
       if (!on || d2 > cut2) continue;
       const double d1 = sqrt(d2);
-      const double cij = (at_lane(ci, r) * cj) * s.ele_coef;
+      const double cij = (cr * cj) * s.ele_coef;
       if (s.ele_form == 0) e += cij / d1 * exp(-d1 * s.rcdist);
       else if (s.ele_form == 1) e += cij * (1.0 / d1 - s.cl_rcinv);
       else e += cij * erfc(s.ew_alpha * d1) / d1;
