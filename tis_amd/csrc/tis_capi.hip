@@ -38,8 +38,8 @@ __global__ void k_lists(DevPtrs, const double *, const double *, const Tile *, i
 __global__ void k_lpair(DevPtrs, const double *, const EwTask *, int, const EwTask *, int);
 __global__ void k_lpair_put(DevPtrs, const double *, const EwTask *, int, int);
 __global__ void k_advance(uint64_t *, uint64_t, uint64_t, uint64_t, unsigned long long *);
-__global__ void k_window(DevPtrs, const int32_t *, int, int, int, int, int);
-__global__ void k_window_back(DevPtrs, const int32_t *, int);
+__global__ void k_window(DevPtrs, const int32_t *, double *, int, int, int, int, int);
+__global__ void k_window_back(DevPtrs, const int32_t *, const double *, int);
 __global__ void k_run_report(unsigned long long *, unsigned long long *);
 __global__ void k_state_out(const double *, int, int, int, double *, const unsigned long long *, unsigned long long *);
 __global__ void k_state_in(DevPtrs, double *, int, int, const double *, float4 *);
@@ -173,6 +173,7 @@ struct tis_ctx {
   int32_t *d_hbdense = nullptr;          // hbond lanes (DevPtrs::hb_dense)
   int32_t nhbdense = 0;
   int32_t *d_wsys = nullptr;             // live systems, largest first, when k_window takes the batch
+  double *d_win_back = nullptr;          // state at a window's start [9][ntot]
   int32_t win_rows = 0, win_lds = 0;     // its list rows and bytes in LDS; win_lds 0: per-step passes
   bool win_pays[2] = {false, false};     // taken with a fixed rebuild interval, with the displacement trigger
   std::vector<int32_t> systask_of;       // index into d_systask per system or -1
@@ -1209,7 +1210,7 @@ int build_tables(tis_ctx *c) {
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.sbox, 4 * nbt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.ttop, 2 * nbt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->d_epart, (size_t)c->n_etask * kEnergyTerms, &c->tab_bytes))) return rc;
-  if ((rc = dalloc_in(c, c->tab_allocs, &c->P.win_back, wsys.empty() ? 1 : 9 * (size_t)c->P.ntot, &c->tab_bytes)))
+  if ((rc = dalloc_in(c, c->tab_allocs, &c->d_win_back, wsys.empty() ? 1 : 9 * (size_t)c->P.ntot, &c->tab_bytes)))
     return rc;
   c->dev_bytes += c->tab_bytes;
   for (int k = 0; k < 2; ++k)
@@ -2207,7 +2208,7 @@ static int run_steps(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunch)
       const int phase = re > 0 ? (int)(c->t_since_init % re) : 0;
       const int nreb = re > 0 ? (phase + n - 1) / re + (phase == 0 ? 1 : 0) : 0;   // multiples of re in [phase, phase + n)
       hipLaunchKernelGGL(k_window, dim3(c->nlive), dim3(kWinThreads), c->win_lds, c->stream, c->P, c->d_wsys,
-                         c->win_rows, c->cur, n, phase, re);
+                         c->d_win_back, c->win_rows, c->cur, n, phase, re);
       hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, c->stream, c->d_stepbase, (uint64_t)n, (uint64_t)nreb,
                          (uint64_t)n, c->d_counters);
       c->cur ^= n & 1;
@@ -2446,7 +2447,8 @@ static int run_resumed(tis_ctx *c, int64_t nsteps, int32_t mode, int64_t *nlaunc
       c->lists_valid = false;
       if (takes_window(c, mode)) {
         c->lv_init = false;
-        hipLaunchKernelGGL(k_window_back, dim3(c->nlive), dim3(kWinThreads), 0, c->stream, c->P, c->d_wsys, c->cur);
+        hipLaunchKernelGGL(k_window_back, dim3(c->nlive), dim3(kWinThreads), 0, c->stream, c->P, c->d_wsys,
+                           (const double *)c->d_win_back, c->cur);
         if ((rc = check(hipStreamSynchronize(c->stream), "k_window_back"))) return rc;
       }
       return grown;

@@ -251,7 +251,6 @@ struct DevPtrs {
   // k_window: the step a system has reached ahead of *stepbase (a launch that
   // another system's list overflow cut short), << 1 | the buffer of its x
   uint64_t *win_at;          // [nsys]
-  double *win_back;          // [9][ntot] x, v, a at *stepbase, of systems that are ahead of it
   // counters / timing
   unsigned long long *counters;  // TIS_CNT_*
   uint64_t *stepbase;

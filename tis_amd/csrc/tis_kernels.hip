@@ -2437,7 +2437,7 @@ __device__ inline void chunk_pair(int k, int nqt, int &I, int &J) {
 }
 
 __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_window(
-    DevPtrs P, const int32_t *wsys, int rows, int cu, int n, int phase, int rebuild) {
+    DevPtrs P, const int32_t *wsys, double *back, int rows, int cu, int n, int phase, int rebuild) {
   extern __shared__ __align__(16) char lds[];
   constexpr int T = kWinThreads, W = T / kTile;
   __shared__ int next[3];
@@ -2498,9 +2498,9 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
     // for k_window_back
     if (own && from == 0)
       for (int d = 0; d < 3; ++d) {
-        P.win_back[(size_t)d * N + g] = xc[d];
-        P.win_back[(size_t)(3 + d) * N + g] = v[d];
-        P.win_back[(size_t)(6 + d) * N + g] = a[d];
+        back[(size_t)d * N + g] = xc[d];
+        back[(size_t)(3 + d) * N + g] = v[d];
+        back[(size_t)(6 + d) * N + g] = a[d];
       }
   }
   const int ib0 = P.inc_off[s.off];
@@ -2985,17 +2985,18 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
 
 // The systems that a k_window launch has left ahead of *stepbase put back to
 // it (positions into buffer cu), for a run that cannot be resumed.
-__global__ __launch_bounds__(kWinThreads) void k_window_back(DevPtrs P, const int32_t *wsys, int cu) {
+__global__ __launch_bounds__(kWinThreads) void k_window_back(DevPtrs P, const int32_t *wsys, const double *back,
+                                                             int cu) {
   const int isys = wsys[blockIdx.x], i = (int)threadIdx.x, N = P.ntot;
   const DSys &s = P.sys[isys];
   if ((P.win_at[isys] >> 1) <= *P.stepbase || i >= s.nmp) return;
   const int g = s.off + i;
   for (int d = 0; d < 3; ++d) {
-    P.x[cu][(size_t)d * N + g] = P.win_back[(size_t)d * N + g];
-    P.v[(size_t)d * N + g] = P.win_back[(size_t)(3 + d) * N + g];
-    P.a[(size_t)d * N + g] = P.win_back[(size_t)(6 + d) * N + g];
+    P.x[cu][(size_t)d * N + g] = back[(size_t)d * N + g];
+    P.v[(size_t)d * N + g] = back[(size_t)(3 + d) * N + g];
+    P.a[(size_t)d * N + g] = back[(size_t)(6 + d) * N + g];
   }
-  P.xf[cu][g] = near_pos(P.win_back[g], P.win_back[(size_t)N + g], P.win_back[2 * (size_t)N + g], P.species[g]);
+  P.xf[cu][g] = near_pos(back[g], back[(size_t)N + g], back[2 * (size_t)N + g], P.species[g]);
 }
 
 // st_status of the consecutive stacks [s0, s0 + ns) at the given
