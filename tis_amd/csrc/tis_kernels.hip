@@ -699,9 +699,7 @@ __device__ inline float ele_dv(const DSys &s, float qq, float d2, unsigned &ncla
   }
 }
 
-// Staging of the J chunk of each wave's chunk pair: ele_pair_task uses the
-// first 64 entries of each array, ele_pair_unrolled keeps the chunk twice over
-// (so that its reads need no wrap-around).
+// Staging of the J chunk of each wave's chunk pair.
 struct EleLds {
   EleWave w[kWaves];
 };
@@ -717,132 +715,42 @@ __device__ inline double wave_rot(double v) {
   const uint64_t lo = wave_rot((uint32_t)b), hi = wave_rot((uint32_t)(b >> 32));
   return __longlong_as_double((long long)(lo | (hi << 32)));
 }
-// +1 or 63 (= -1 mod 64) when wave_rot is a uniform rotation of the wave,
-// else 0
+// The lane's number within its wave, counted where it is needed: k_force's pair
+// blocks would otherwise keep threadIdx in scratch from the kernel's start (29.3
+// us on the batch of 576 systems, 28.1 without).
+__device__ inline int wave_lane() { return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)); }
+// +1 or 63 (= -1 mod 64): which neighbour's value wave_rot brings
 __device__ inline int wave_dir() {
-  const int lane = threadIdx.x & (kTile - 1);
-  const int d = ((int)wave_rot((uint32_t)lane) - lane) & (kTile - 1);
-  const int d0 = __shfl(d, 0);
-  const bool ok = (d0 == 1 || d0 == kTile - 1) && __all(d == d0);
-  return ok ? d0 : 0;
+  const int lane = wave_lane();
+  return __builtin_amdgcn_readfirstlane(((int)wave_rot((uint32_t)lane) - lane) & (kTile - 1));
 }
 
 // force_ele_DH.F90:68-118, force_ele_coulomb.F90:63-84 and the real-space
-// loop of force_ele_coulomb_ewld.F90:118-137.  One wave per chunk pair
-// (I, J), I <= J, of a system's charges (chunks of 64), four pairs per
-// block.  At iteration k lane l pairs its charge i of chunk I with
-// j = (l + dir k) mod 64 of chunk J (staged in the wave's LDS slice); the
-// force on i accumulates in the lane, the opposite force on j in a register
-// that rotates with the schedule, so after 64 iterations lane l holds the
-// sum for j = l.  The diagonal chunk (J = I) runs k = 1..32 (k = 32 for
-// lanes < 32 only), which meets every unordered pair of the chunk once.
-// List membership from the bit matrix, cutoff test in FP64, pair arithmetic
-// in FP32, accumulation in FP64; periodic pairs take the mirror code the list
+// loop of force_ele_coulomb_ewld.F90:118-137, by chunk pairs (I, J), I <= J, of
+// a system's charges (chunks of 64).  At step k lane l pairs its charge i of
+// chunk I with j = (l + dir k) mod 64 of chunk J (staged in LDS); the force on
+// i accumulates in the lane, the opposite force on j in a register that
+// rotates with the schedule, so after 64 steps lane l holds the sum for j = l.
+// The diagonal chunk (J = I) runs k = 1..32 (k = 32 for lanes < 32 only),
+// which meets every unordered pair of the chunk once.  List membership from
+// the bit matrix, cutoff test in FP64, pair arithmetic in FP32, accumulation
+// in FP64; periodic pairs (ele_pair_periodic) take the mirror code the list
 // stored for them (v = x_j - x_i + shift, util_pbneighbor.F90:22-35).  The
 // forces on chunk I go to slot 0 of the task's partial buffer, those on
 // chunk J (I < J) to slot 1, and k_main sums a charge's slots in task order:
-// a fixed order, so results are bitwise reproducible.  Charges beyond nq are
-// staged as zeros with their bits clear.  dir = 0 (no whole-wave DPP
-// rotation) rotates with __shfl instead.
+// a fixed order, so results are bitwise reproducible.
 __host__ __device__ inline int64_t ele_task_index(int I, int J, int nch) {
   return (int64_t)I * (2 * nch - I + 1) / 2 + (J - I);
 }
 
-// the next value of the rotating sums: DPP when the whole-wave rotation is
-// available (decided once per wave, so the step loop has no branch), else
-// __shfl
-template <bool DPP>
-__device__ inline double rot_next(double v) {
-  if (DPP) return wave_rot(v);
-  const int lane = threadIdx.x & (kTile - 1);
-  return __shfl(v, (lane + 1) & (kTile - 1));
-}
-
-template <int FORM, bool DPP>
-__device__ inline void ele_pair_task(const DevPtrs &P, const DSys &s, const double *Y, int I, int J, int dir,
-                                     double *SX, double *SY, double *SZ, float *SQ) {
-  const int lane = threadIdx.x & (kTile - 1);
-  const int rd = dir != 0 ? dir : 1;
-  const int n = P.ntot;
-  const int qi = I * kTile + lane;
-  const bool valid = qi < s.nq;
-  double xi0 = 0.0, xi1 = 0.0, xi2 = 0.0, chi = 0.0;
-  if (valid) {
-    const int gi = P.qbead[s.qoff + qi];
-    xi0 = Y[gi]; xi1 = Y[n + gi]; xi2 = Y[2 * n + gi];
-    chi = P.charge[gi];
-  }
-  const int jt = J * kTile;
-  {
-    const bool vj = jt + lane < s.nq;
-    const int gj = vj ? P.qbead[s.qoff + jt + lane] : 0;
-    SX[lane] = vj ? Y[gj] : 0.0; SY[lane] = vj ? Y[n + gj] : 0.0; SZ[lane] = vj ? Y[2 * n + gj] : 0.0;
-    SQ[lane] = vj ? (float)P.charge[gj] : 0.0f;
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const float qiC = (float)(chi * s.ele_coef);
-  const double cut2 = FORM == 0 ? s.dh_cut2 : s.cl_cut2;
-  const uint32_t *row = P.qmask + s.moff + (int64_t)(valid ? qi : 0) * s.mwords;
-  uint64_t m64 = 0;
-  if (valid) {
-    const int wb = jt >> 5;
-    m64 = row[wb];
-    if (wb + 1 < s.mwords) m64 |= (uint64_t)row[wb + 1] << 32;
-  }
-  const bool diag = I == J;
-  double F0 = 0.0, F1 = 0.0, F2 = 0.0, G0 = 0.0, G1 = 0.0, G2 = 0.0;
-  unsigned nclamp = 0;
-  auto pair = [&](int k, bool last_half) {
-    const int jl = (lane + rd * k) & (kTile - 1);
-    bool bit = (m64 >> jl) & 1u;
-    if (last_half) bit = bit && lane < 32;
-    // a step with no listed pair in the wave adds zeros: only the sums move
-    if (__any(bit)) {
-      const double v0 = SX[jl] - xi0, v1 = SY[jl] - xi1, v2 = SZ[jl] - xi2;
-      const double d2 = v0 * v0 + v1 * v1 + v2 * v2;
-      const bool on = bit && d2 <= cut2;
-      float dv = ele_dv<FORM>(s, qiC * SQ[jl], on ? (float)d2 : 1.0f, nclamp, on);
-      dv = on ? dv : 0.0f;
-      const double dd = (double)dv;
-      F0 -= dd * v0; F1 -= dd * v1; F2 -= dd * v2;
-      G0 += dd * v0; G1 += dd * v1; G2 += dd * v2;
-    }
-    G0 = rot_next<DPP>(G0); G1 = rot_next<DPP>(G1); G2 = rot_next<DPP>(G2);
-  };
-  if (__any(m64 != 0)) {
-    if (diag) {
-#pragma unroll 1
-      for (int k = 1; k < 32; ++k) pair(k, false);
-      pair(32, true);
-    } else {
-#pragma unroll 1
-      for (int k = 0; k < kTile; ++k) pair(k, false);
-    }
-  }
-  double *pp = P.pp + s.pp_off + ele_task_index(I, J, s.nqt) * (6 * kTile);
-  if (diag) {
-    const int src = (lane - rd * 33) & (kTile - 1);
-    F0 += __shfl(G0, src); F1 += __shfl(G1, src); F2 += __shfl(G2, src);
-  } else {
-    pp[3 * kTile + lane] = G0; pp[4 * kTile + lane] = G1; pp[5 * kTile + lane] = G2;
-  }
-  pp[lane] = F0; pp[kTile + lane] = F1; pp[2 * kTile + lane] = F2;
-  if (nclamp) atomicAdd(&P.counters[1], (unsigned long long)nclamp);
-}
-
-// ele_pair_task for a non-periodic system with the whole-wave DPP rotation
-// (dir = 1 or 63): the same pairs in the same order and the same FP64
-// distances, cutoff tests and accumulation (the DH exponent takes its scale
-// as one constant, -rcd log2(e), so its FP32 rounding can differ by an ulp),
-// in fewer instructions per step: the J chunk is
-// staged twice over in an order where lane l meets, at step k, entry c + k
-// (c = l for dir = 1, 63 - l for dir = 63), so the reads of eight
+// ele_pair_unrolled, a chunk pair of a non-periodic system per wave: the J
+// chunk is staged twice over in an order where lane l meets, at step k, entry
+// c + k (c = l for dir = 1, 63 - l for dir = 63), so the reads of eight
 // consecutive steps take immediate offsets from one address; the list bits
 // are turned into the same order once (bit k of mr is the pair of step k); a
 // pair that is not on gets charge product 0, so its force is exactly zero
-// and adds nothing, with no branch; the DE_MAX clamps are counted per wave.
+// and adds nothing, with no branch; the DE_MAX clamps are counted per wave; the
+// DH exponent takes its scale as one constant, -rcd log2(e).
 // Absent charges sit far apart (kFar, charge 0; -kFar on the I side): their
 // pairs stay finite and off.
 constexpr double kFar = 1e15;
@@ -854,11 +762,11 @@ __device__ inline int stage_at(int lane, int dir) { return dir == 1 ? lane : kTi
 // product factor, list bits m64 of its row against chunk J, nj charges) and
 // the staged chunk J: sums on chunk I in F, on chunk J in G (the diagonal
 // chunk's are added to F).  Returns the clamps (the same on every lane).
-template <int FORM, bool DPP>
+template <int FORM>
 __device__ inline uint32_t ele_pair_sums(const DSys &s, bool diag, int nj, bool valid, uint64_t m64, double xi0,
                                          double xi1, double xi2, float qiC, int dir, const EleWave *JE, double F[3],
                                          double G[3]) {
-  const int lane = threadIdx.x & (kTile - 1);
+  const int lane = wave_lane();
   const int c = stage_at(lane, dir);
   const double cut2 = FORM == 0 ? s.dh_cut2 : s.cl_cut2;
   // bit k of mr: the pair of step k, j = (lane + dir k) mod 64
@@ -897,7 +805,7 @@ __device__ inline uint32_t ele_pair_sums(const DSys &s, bool diag, int nj, bool 
       const double dd = (double)dv;
       F0 -= dd * v0; F1 -= dd * v1; F2 -= dd * v2;
       G0 += dd * v0; G1 += dd * v1; G2 += dd * v2;
-      G0 = rot_next<DPP>(G0); G1 = rot_next<DPP>(G1); G2 = rot_next<DPP>(G2);
+      G0 = wave_rot(G0); G1 = wave_rot(G1); G2 = wave_rot(G2);
     }
   };
   if (__any(m64 != 0)) {
@@ -928,7 +836,7 @@ __device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const 
   // the chunk pair is the wave's: uniform, so the step loops are scalar
   I = __builtin_amdgcn_readfirstlane(I);
   J = __builtin_amdgcn_readfirstlane(J);
-  const int lane = threadIdx.x & (kTile - 1);
+  const int lane = wave_lane();
   const int c = stage_at(lane, dir);
   const int n = P.ntot;
   const int qi = I * kTile + lane;
@@ -962,7 +870,7 @@ __device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const 
   const bool diag = I == J;
   const int nj = s.nq - jt < kTile ? s.nq - jt : kTile;
   double F[3], G[3];
-  const uint32_t nclamp = ele_pair_sums<FORM, true>(s, diag, nj, valid, m64, xi0, xi1, xi2, qiC, dir, JE, F, G);
+  const uint32_t nclamp = ele_pair_sums<FORM>(s, diag, nj, valid, m64, xi0, xi1, xi2, qiC, dir, JE, F, G);
   double *pp = P.pp + s.pp_off + ele_task_index(I, J, s.nqt) * (6 * kTile);
   if (!diag) {
     pp[3 * kTile + lane] = G[0]; pp[4 * kTile + lane] = G[1]; pp[5 * kTile + lane] = G[2];
@@ -971,7 +879,7 @@ __device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const 
   if (lane == 0 && nclamp) atomicAdd(&P.counters[1], (unsigned long long)nclamp);
 }
 
-// ele_pair_task for a periodic system, by a block: the four waves take a
+// A chunk pair of a periodic system, by a block: the four waves take a
 // quarter of the steps each, and the quarters' sums, brought to one order of
 // charges in LDS, are added as (q0 + q1) + (q2 + q3).  A periodic system is
 // one box whose chunk pairs leave most of the chip idle, so the time is one
@@ -979,12 +887,11 @@ __device__ inline void ele_pair_unrolled(const DevPtrs &P, const DSys &s, const 
 // are loaded ahead for all of a wave's steps (packed four to a word, bit 7: the
 // pair is listed).  640 charges (55 chunk pairs): the force pass took 32.8 us
 // with a wave per chunk pair, 10.8 now.
-template <int FORM, bool DPP>
+template <int FORM>
 __device__ inline void ele_pair_periodic(const DevPtrs &P, const DSys &s, const double *Y, int I, int J, int dir,
                                          EleLds &lds) {
   const int tid = (int)threadIdx.x, lane = tid & (kTile - 1);
   const int part = __builtin_amdgcn_readfirstlane(tid / kTile);
-  const int rd = dir != 0 ? dir : 1;
   const int n = P.ntot;
   EleWave &JE = lds.w[0];
   double(*red)[6][kTile] = reinterpret_cast<double(*)[6][kTile]>(&lds.w[1]);   // quarters 1-3
@@ -1004,7 +911,7 @@ __device__ inline void ele_pair_periodic(const DevPtrs &P, const DSys &s, const 
     const uint8_t *mrow = P.qmirror + s.mioff + (int64_t)(valid ? qi : 0) * s.nq + jt;
 #pragma unroll
     for (int u = 0; u < 16; ++u) {
-      const int k = kb + u, jl = (lane + rd * k) & (kTile - 1);
+      const int k = kb + u, jl = (lane + dir * k) & (kTile - 1);
       const bool bit = ((m64 >> jl) & 1u) && u < ns && !(diag && k == 32 && lane >= 32);
       const uint32_t code = mrow[bit ? jl : 0];   // unlisted: the row's first, unused
       pk[u >> 2] |= (bit ? code | 0x80u : 0u) << (8 * (u & 3));
@@ -1034,7 +941,7 @@ __device__ inline void ele_pair_periodic(const DevPtrs &P, const DSys &s, const 
     pk[0] = pk[1]; pk[1] = pk[2]; pk[2] = pk[3];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int jl = (lane + rd * (kb + k0 + u)) & (kTile - 1);
+      const int jl = (lane + dir * (kb + k0 + u)) & (kTile - 1);
       const int code = (int)((w >> (8 * u)) & 0x7fu);
       const bool bit = (w >> (8 * u)) & 0x80u;
       const double v0 = (JE.x[jl] - xi0) + mirror_shift(s, code, 0);
@@ -1046,12 +953,12 @@ __device__ inline void ele_pair_periodic(const DevPtrs &P, const DSys &s, const 
       const double dd = on ? (double)dv : 0.0;
       F[0] -= dd * v0; F[1] -= dd * v1; F[2] -= dd * v2;
       G[0] += dd * v0; G[1] += dd * v1; G[2] += dd * v2;
-      for (int d = 0; d < 3; ++d) G[d] = rot_next<DPP>(G[d]);
+      for (int d = 0; d < 3; ++d) G[d] = wave_rot(G[d]);
     }
   }
   if (nclamp) atomicAdd(&P.counters[1], (unsigned long long)nclamp);
-  // lane l's G is now the sum on charge l + rd (kb + ns)
-  const int turn = rd * (kb + ns);
+  // lane l's G is now the sum on charge l + dir (kb + ns)
+  const int turn = dir * (kb + ns);
   if (part > 0) {
     for (int d = 0; d < 3; ++d) {
       red[part - 1][d][lane] = F[d];
@@ -1158,8 +1065,8 @@ __global__ __launch_bounds__(kTile * kWaves) void k_ewald_sk(DevPtrs P, const do
 // lane each, first because each lane is a long FP64 chain), four systems'
 // tertiary stacks and valence-limited hbonds per block (terms_wave, one wave
 // each), an electrostatic chunk pair of a periodic system per block
-// (ele_pair_periodic), four of others per block (ele_pair_unrolled,
-// ele_pair_task, one wave each), then the bonded terms, 256 lanes per block (bonded_lane).  k_main
+// (ele_pair_periodic), four of others per block (ele_pair_unrolled, one wave
+// each), then the bonded terms, 256 lanes per block (bonded_lane).  k_main
 // gathers all of their outputs.
 template <int PPW, int TPL, int WPE>
 __global__ __launch_bounds__(kTile * kWaves) __attribute__((amdgpu_waves_per_eu(WPE)))
@@ -1195,15 +1102,9 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
     const EwTask tk = xtasks[b];
     const DSys s = P.sys[tk.sys];
     const int dir = wave_dir();
-    if (dir != 0) {
-      if (s.ele_form == 0) ele_pair_periodic<0, true>(P, s, PX, tk.a, tk.b, dir, lds);
-      else if (s.ele_form == 1) ele_pair_periodic<1, true>(P, s, PX, tk.a, tk.b, dir, lds);
-      else ele_pair_periodic<2, true>(P, s, PX, tk.a, tk.b, dir, lds);
-    } else {
-      if (s.ele_form == 0) ele_pair_periodic<0, false>(P, s, PX, tk.a, tk.b, dir, lds);
-      else if (s.ele_form == 1) ele_pair_periodic<1, false>(P, s, PX, tk.a, tk.b, dir, lds);
-      else ele_pair_periodic<2, false>(P, s, PX, tk.a, tk.b, dir, lds);
-    }
+    if (s.ele_form == 0) ele_pair_periodic<0>(P, s, PX, tk.a, tk.b, dir, lds);
+    else if (s.ele_form == 1) ele_pair_periodic<1>(P, s, PX, tk.a, tk.b, dir, lds);
+    else ele_pair_periodic<2>(P, s, PX, tk.a, tk.b, dir, lds);
     return;
   }
   b -= nxt;
@@ -1214,11 +1115,9 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
       bonded_lane(P, X, PX, br, (b - npb + i * nbb) * (kTile * kWaves) + (int)threadIdx.x);
     return;
   }
-  const int w = (int)threadIdx.x / kTile;
   const int dir = wave_dir();
+  const int w = (int)threadIdx.x / kTile;
   EleWave *JE = &lds.w[w];
-  double *SX = JE->x, *SY = JE->y, *SZ = JE->z;
-  float *SQ = JE->q;
   // ppw consecutive chunk pairs per wave, one after the other through the
   // wave's LDS slice
 #pragma unroll 1
@@ -1232,12 +1131,9 @@ void k_force(DevPtrs P, const double *X, const double *PX, const int32_t *systas
     }
     const EwTask tk = ptasks[task];
     const DSys s = P.sys[tk.sys];
-    if (dir != 0 && s.ele_form == 0) ele_pair_unrolled<0>(P, s, X, tk.a, tk.b, dir, JE);
-    else if (dir != 0 && s.ele_form == 1) ele_pair_unrolled<1>(P, s, X, tk.a, tk.b, dir, JE);
-    else if (s.ele_form == 0) ele_pair_task<0, false>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-    else if (s.ele_form == 1) ele_pair_task<1, false>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-    else if (dir != 0) ele_pair_task<2, true>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
-    else ele_pair_task<2, false>(P, s, X, tk.a, tk.b, dir, SX, SY, SZ, SQ);
+    // (an Ewald system is periodic: not among these)
+    if (s.ele_form == 0) ele_pair_unrolled<0>(P, s, X, tk.a, tk.b, dir, JE);
+    else ele_pair_unrolled<1>(P, s, X, tk.a, tk.b, dir, JE);
   }
 }
 
@@ -2388,6 +2284,7 @@ template __global__ void k_lists<kListFew>(DevPtrs, const double *, const double
 // Every term, list and sum is that of the per-step passes, in their order, so
 // results do not depend on which of them ran.
 //
+// back: [9][ntot], takes x, v and a of the launch's start (k_window_back).
 // cu: the buffer of the current positions at *stepbase; phase: steps since
 // the last fixed rebuild was due; rebuild: the interval, 0 for the
 // displacement trigger.  A rebuild that overflows the list capacity raises
@@ -2477,7 +2374,7 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
   const int nq = s.ele_form >= 0 ? s.nq : 0, nqt = s.ele_form >= 0 ? s.nqt : 0, np = nqt * (nqt + 1) / 2;
   const int nbt = s.nbt, nbd = s.nbd, nba = s.nba, nst = s.nst, nhb = s.nhb;
   const bool vlim = s.hb_excess_possible != 0, dyn = rebuild == 0;
-  const int wdir = wave_dir(), dir = wdir ? wdir : 1;   // 0: rotation by shuffles (ele_pair_task)
+  const int dir = wave_dir();
   // slot bases within the system
   const int lb_ba = 2 * nbd, lb_st = lb_ba + 3 * nba, lb_hb = lb_st + 7 * nst;
   float *hslot = slot + 3 * lb_hb;
@@ -2797,14 +2694,10 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
         const double x0 = val ? je[I].x[c] : -kFar, x1 = val ? je[I].y[c] : -kFar, x2 = val ? je[I].z[c] : -kFar;
         const int nj = nq - J * kTile < kTile ? nq - J * kTile : kTile;
         double F[3], G[3];
-        auto sums = [&](auto form, auto dpp) {
-          return ele_pair_sums<decltype(form)::value, decltype(dpp)::value>(s, I == J, nj, val, mask[k * kTile + lane],
-                                                                            x0, x1, x2, qic[qi], dir, &je[J], F, G);
-        };
-        using F0 = std::integral_constant<int, 0>;
-        using F1 = std::integral_constant<int, 1>;
-        const uint32_t nc = wdir ? (s.ele_form == 0 ? sums(F0{}, std::true_type{}) : sums(F1{}, std::true_type{}))
-                                 : (s.ele_form == 0 ? sums(F0{}, std::false_type{}) : sums(F1{}, std::false_type{}));
+        const uint64_t m64 = mask[k * kTile + lane];
+        const uint32_t nc = s.ele_form == 0
+            ? ele_pair_sums<0>(s, I == J, nj, val, m64, x0, x1, x2, qic[qi], dir, &je[J], F, G)
+            : ele_pair_sums<1>(s, I == J, nj, val, m64, x0, x1, x2, qic[qi], dir, &je[J], F, G);
         double *o = pp + (size_t)k * (6 * kTile) + lane;
         for (int d = 0; d < 3; ++d) { o[d * kTile] = F[d]; o[(3 + d) * kTile] = G[d]; }
         clamp_ele += nc;
