@@ -1511,7 +1511,7 @@ __device__ inline double main_tail(const DevPtrs &P, const DSys &s, int g, const
 // idle, where a tile's chain of loads sets the time.  Wave 0 integrates after
 // the barrier, from state loaded before it.
 // Bound: latency (incidence -> slot; list entry -> position; contact pairs),
-// four waves per SIMD; then the state and slots it moves (75 MB).  576
+// four waves per SIMD; then the state, records and slots it moves (107 MB).  576
 // systems, 237,111 beads: 33.2 us with every listed pair evaluated in FP64,
 // 26.8 sifted (19.6 without excluded volume, 21.3 without the slots).  A
 // 2,000-nt chain (94 tiles): 12.0 us, 11.5 sifted by two waves, 9.5 by six;
@@ -2273,7 +2273,7 @@ template __global__ void k_lists<kListFew>(DevPtrs, const double *, const double
 // them FP64, on the four SIMDs of one CU; its longest chain is the 32
 // dependent pair steps of a charge chunk.  As two launches per step (k_force,
 // k_main) and three per rebuild every hand-over went through L2: 17.6 us a
-// step for that hairpin against 10.2 here, 64 of them 18.1 against 11.1.
+// step for that hairpin against 10.1 here, 64 of them 18.1 against 10.3.
 // Per step: (1) the terms as tasks of one wave each, longest first, taken
 // from a counter in LDS (chunk pairs of charges, 64 hbonds, 64 stacks, the
 // noise of 64 beads, half the neighbour groups of 64 beads, 64 angles, 64
@@ -2532,7 +2532,8 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
       // ascending order); to memory too when no later rebuild of this launch
       // replaces them.  Tasks of 64 beads against 32: an even share for the
       // waves where 64 against 64 left some with twice the others' (200 steps of
-      // a 64-nt hairpin 2,344 -> 2,038 us, of 64 of them 3,630 -> 3,334).
+      // a 64-nt hairpin and its frame 2,344 -> 2,038 us; a ladder of 64 of them,
+      // with its frames and exchange, 3,630 -> 3,334).
       const int nu = (nb + kUnit - 1) / kUnit;
       const bool keep = dyn || t + rebuild >= n;
       if (own)
@@ -2722,7 +2723,7 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
       k -= nbt;
       if (k < 2 * nbt) {
         // half h of the neighbour groups of 64 beads: groups k mod 4 = h and
-        // h + 2 (exv_group's order)
+        // h + 2, as exv_bead takes them
         const int h = k & 1, i = (k >> 1) * kTile + lane;
         if (i < nb) {
           const double xi[3] = {x[i], x[nb + i], x[2 * nb + i]};
@@ -2738,8 +2739,8 @@ __global__ __launch_bounds__(kWinThreads) __attribute__((amdgpu_waves_per_eu(2))
             return j | (int)spec[j] << 10;
           };
           // sifted in FP32, 32 entries at a time (eight records' reads under
-          // way: 200 steps of a 64-nt hairpin 2,361 -> 2,344 us, of 64 of them
-          // 3,678 -> 3,612), as in exv_bead; the pairs that may touch then in FP64
+          // way: the cases of the list build's comment 2,361 -> 2,344 and 3,678 ->
+          // 3,612 us), as in exv_bead; the pairs that may touch then in FP64
           const bool local = __all(cnt <= rows);   // no list past the rows in LDS
           for (int q0 = 0; q0 < half; q0 += 32) {
             uint32_t near = 0;
