@@ -1209,9 +1209,12 @@ int build_tables(tis_ctx *c) {
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.qbbox, nqt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.sbox, 4 * nbt, &c->tab_bytes))) return rc;
   if ((rc = dalloc_in(c, c->tab_allocs, &c->P.ttop, 2 * nbt, &c->tab_bytes))) return rc;
-  if ((rc = dalloc_in(c, c->tab_allocs, &c->d_epart, (size_t)c->n_etask * kEnergyTerms, &c->tab_bytes))) return rc;
-  if ((rc = dalloc_in(c, c->tab_allocs, &c->d_win_back, wsys.empty() ? 1 : 9 * (size_t)c->P.ntot, &c->tab_bytes)))
+  // the energy tasks' sums and a window's start state, one allocation (each
+  // costs some 100 us)
+  const size_t ne = (size_t)c->n_etask * kEnergyTerms;
+  if ((rc = dalloc_in(c, c->tab_allocs, &c->d_epart, ne + (wsys.empty() ? 0 : 9 * (size_t)c->P.ntot), &c->tab_bytes)))
     return rc;
+  c->d_win_back = c->d_epart + ne;
   c->dev_bytes += c->tab_bytes;
   for (int k = 0; k < 2; ++k)
     if (c->graph[k]) { (void)hipGraphExecDestroy(c->graph[k]); c->graph[k] = nullptr; }
